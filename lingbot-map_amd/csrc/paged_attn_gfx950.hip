@@ -117,6 +117,9 @@ __device__ __forceinline__ float swap_max(float x) {
   swap_halves(x, lo, hi);
   return max2(lo, hi);
 }
+// A float's bits.  Vector elements go through it: __builtin_bit_cast(unsigned, v[i]) on an
+// ext_vector lvalue takes the vector's address and so returns element 0 whatever i is.
+__device__ __forceinline__ unsigned float_bits(float x) { return __builtin_bit_cast(unsigned, x); }
 
 // loads of this wavefront still allowed in flight (expcnt and lgkmcnt untouched); its LDS accesses done
 #define LBM_LOADS_LEFT(N) asm volatile("s_waitcnt vmcnt(%0)" : : "i"(N) : "memory")
@@ -696,14 +699,14 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
 #pragma unroll
         for (int db = 0; db < 2; ++db)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) top = max(top, __builtin_bit_cast(unsigned, o[qb][db][i]) & 0x7FFFFFFFu);
+          for (int i = 0; i < 16; ++i) top = max(top, float_bits(o[qb][db][i]) & 0x7FFFFFFFu);
       bad = top >= 0x7F800000u;
       if (lane < 16) {
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
           for (int h2 = 0; h2 < 2; ++h2) {
-            const unsigned lb = __builtin_bit_cast(unsigned, lacc[qb][h2]);
+            const unsigned lb = float_bits(lacc[qb][h2]);
             bad = bad || lb < 0x12800000u /* 2^-90 */ || lb > 0x71800000u /* 2^100 */;
           }
       }
@@ -1056,14 +1059,14 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
 #pragma unroll
       for (int db = 0; db < 2; ++db)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) top = max(top, __builtin_bit_cast(unsigned, o[qb][db][i]) & 0x7FFFFFFFu);
+        for (int i = 0; i < 16; ++i) top = max(top, float_bits(o[qb][db][i]) & 0x7FFFFFFFu);
     bad = top >= 0x7F800000u;
     if (lane < 16) {
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) {
-          const unsigned lb = __builtin_bit_cast(unsigned, lacc[qb][h2]);
+          const unsigned lb = float_bits(lacc[qb][h2]);
           bad = bad || lb < 0x12800000u /* 2^-90 */ || lb > 0x71800000u /* 2^100 */;
         }
     }
