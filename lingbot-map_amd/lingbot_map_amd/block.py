@@ -845,7 +845,7 @@ class HipPagedBlock(nn.Module):
                 if not (is_streaming or is_dense) and self._sub_modules_plain():
                     assert x.shape[1] == num_frames * cache.tokens_per_frame, (
                         f"{x.shape[1]} tokens per stream are not {num_frames} frames of {cache.tokens_per_frame}")
-                    pass_rows = cache.begin_frames(global_idx, num_frames)
+                    pass_rows = cache.begin_frames(global_idx, num_frames, self.attn.kv_cache_sliding_window)
                 if is_streaming or is_dense or pass_rows is not None:
                     return self._run_native(native, x, pos, enable_3d_rope, cache, global_idx, normed, next_norm, pass_rows)
         n1 = self.norm1(x) if (normed is None or stats is not None) else normed

@@ -364,16 +364,17 @@ class HipPagedKVCacheManager:
             return made[2][:, n - made[0]].reshape(-1)
         return self._rows_log.get(n)
 
-    def begin_frames(self, block_idx: int, frames: int) -> Optional[int]:
+    def begin_frames(self, block_idx: int, frames: int, sliding_window: int) -> Optional[int]:
         """``append_frame`` for ``frames`` frames of every stream at once, up to the copy of the rows, for
-        a caller whose producer stores them (``HipPagedBlock``'s anchor pass, attention.py:497-511):
-        the device address of the append rows, ``[streams, frames, tokens_per_frame]``.  None when
-        the frames do not fit the window without an eviction in between - then a frame's pages could
-        come out of an earlier frame's - or this block is not where block 0 was."""
+        a caller whose producer stores them and who would call ``evict_frames`` with ``sliding_window``
+        after every frame (``HipPagedBlock``'s anchor pass, attention.py:497-511): the device address of
+        the append rows, ``[streams, frames, tokens_per_frame]``.  None when the frames do not fit the
+        windows that those calls would keep to without an eviction in between - then a frame's pages
+        could come out of an earlier frame's - or this block is not where block 0 was."""
         ts = self._set(block_idx)
         if self._leads(block_idx):
-            room = all(not a or c.win_count + max(0, c.n_anchor + frames - self.scale_frames) <= w
-                       for a, c, w in zip(self._active, self._counts[ts], self._windows))
+            room = all(not a or c.win_count + max(0, c.n_anchor + frames - self.scale_frames) <= self._window_of(b, sliding_window)
+                       for b, (a, c) in enumerate(zip(self._active, self._counts[ts])))
             if not room or self._others_behind():
                 return None
             T, S = self.tokens_per_frame, self.num_streams

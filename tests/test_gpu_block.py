@@ -370,3 +370,46 @@ def test_anchor_pass_runs_the_hooks_of_its_sub_modules(where):
     with torch.no_grad():
         block(torch.randn(1, frames * tokens, 128, device=dev).to(torch.bfloat16), kv_cache=m, global_idx=0, num_frames=frames)
     assert len(seen) == 1
+
+
+@pytest.mark.parametrize("windows", [4, [4, 2]])
+@pytest.mark.parametrize("own", [0, 1, 2, 3])
+def test_anchor_pass_keeps_to_the_blocks_window(own, windows):
+    """The anchor pass evicts by the block's own ``kv_cache_sliding_window`` (by the streams' own windows where
+    the manager has one per stream), whatever the manager's: page tables, counts and the frame after it
+    as ``append_frame`` + ``evict_frames`` frame by frame leave them, with the fewest frames the window
+    holds and more.  (One table set per block: with shared ones a pass that evicts is refused.)"""
+    from lingbot_map_amd.block import HipPagedBlock, Mlp
+    from lingbot_map_amd.manager import HipPagedKVCacheManager
+    dev, tokens, frames, scale, H = torch.device("cuda:0"), 40, 5, 2, 2
+    streams = len(windows) if isinstance(windows, list) else 1
+    torch.manual_seed(own)
+    blocks = [HipPagedBlock(dim=128, num_heads=H, qk_norm=True, init_values=0.5,
+                            kv_cache_sliding_window=own).to(dev, torch.bfloat16).eval() for _ in range(2)]
+    first = torch.randn(streams, frames * tokens, 128, device=dev).to(torch.bfloat16)
+    later = torch.randn(streams, tokens, 128, device=dev).to(torch.bfloat16)
+
+    def run(native):
+        m = HipPagedKVCacheManager(2, 24, tokens, H, 64, torch.bfloat16, dev, num_special_tokens=5, scale_frames=scale,
+                                   sliding_window=windows, max_total_frames=32, page_size=16, layout="frame_pages",
+                                   num_streams=streams, per_block_tables=True)
+        limit, seen = Mlp.FUSED_MAX_ROWS, []
+        Mlp.FUSED_MAX_ROWS = limit if native else 0
+        try:
+            with torch.no_grad():
+                for x, n in ((first, frames), (later, 1)):
+                    for i, b in enumerate(blocks):
+                        x = b(x, kv_cache=m, global_idx=i, num_frames=n)
+                    seen += [[m.build_visible_page_table(0, s), m.build_visible_page_lens(0, s), m.get_cache_stats(0, s)]
+                             for s in range(streams)]
+        finally:
+            Mlp.FUSED_MAX_ROWS = limit
+        assert m.device_header()["error"] == 0
+        return seen, x.float()
+
+    (seen, x), (ref, y) = run(True), run(False)
+    assert seen == ref
+    for s in range(streams):
+        kept = min(frames - scale, windows[s] if streams > 1 else own)     # (what is asked for, not only that both agree)
+        assert seen[s][2]["live_pages"] == kept * 3
+    assert (x - y).abs().mean().item() <= 0.01 * y.abs().mean().item()     # bf16 noise, as in the pass without evictions
