@@ -623,7 +623,10 @@ class _NativeBlock:
             return False
         rope = self.attn.rope
         if manager is not None:
-            if not hasattr(manager, "begin_block") or manager.dtype != torch.bfloat16:
+            # the producer writes num_heads x 64 values per row into the manager's pool: a manager of another
+            # geometry is left to the calls that refuse it before anything is launched
+            if (not hasattr(manager, "begin_block") or manager.dtype != torch.bfloat16
+                    or manager.num_heads != self.num_heads or manager.head_dim != 64):
                 return False
             if streaming:
                 return rope is None or (bool(enable_3d_rope) and torch.is_tensor(pos) and pos.is_complex())

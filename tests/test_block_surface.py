@@ -121,3 +121,17 @@ def test_scratch_lanes_nest_and_restore():
         with N.scratch_lane(3):
             raise ValueError("body fails")
     assert N.current_scratch_lane() == 0
+
+
+@pytest.mark.parametrize("heads,head_dim,fits", [(2, 64, True), (1, 64, False), (4, 64, False), (2, 128, False)])
+def test_native_call_refuses_a_manager_of_another_geometry(heads, head_dim, fits):
+    """The block's one native call writes K/V rows of its own heads x 64 into the manager's pool, so it takes
+    only a manager laid out for them, streaming and in the anchor pass."""
+    from types import SimpleNamespace
+    from lingbot_map_amd.block import _NativeBlock
+    native = object.__new__(_NativeBlock)      # (laying parameters out needs a GPU; the check does not)
+    native.device, native.num_heads, native.attn = torch.device("cpu"), 2, SimpleNamespace(rope=None)
+    manager = SimpleNamespace(begin_block=None, dtype=torch.bfloat16, num_streams=1, num_heads=heads, head_dim=head_dim)
+    x = torch.zeros(1, 8, 128, dtype=torch.bfloat16)
+    for streaming in (True, False):
+        assert native.covers(x, None, False, manager, streaming) is fits

@@ -413,3 +413,19 @@ def test_anchor_pass_keeps_to_the_blocks_window(own, windows):
         kept = min(frames - scale, windows[s] if streams > 1 else own)     # (what is asked for, not only that both agree)
         assert seen[s][2]["live_pages"] == kept * 3
     assert (x - y).abs().mean().item() <= 0.01 * y.abs().mean().item()     # bf16 noise, as in the pass without evictions
+
+
+@pytest.mark.parametrize("heads", [1, 4])
+@pytest.mark.parametrize("frames", [1, 3])
+def test_manager_of_another_geometry_is_refused_untouched(heads, frames):
+    """A block of two heads on a manager of fewer or more: an AssertionError before anything is stored, streaming
+    and in the anchor pass."""
+    from lingbot_map_amd.block import HipPagedBlock
+    from lingbot_map_amd.manager import HipPagedKVCacheManager
+    dev, tokens = torch.device("cuda:0"), 40
+    block = HipPagedBlock(dim=128, num_heads=2, qk_norm=True).to(dev, torch.bfloat16).eval()
+    m = HipPagedKVCacheManager(1, 24, tokens, heads, 64, torch.bfloat16, dev, num_special_tokens=5, scale_frames=frames,
+                               sliding_window=4, max_total_frames=32, page_size=16, layout="frame_pages")
+    with torch.no_grad(), pytest.raises(AssertionError):
+        block(torch.randn(1, frames * tokens, 128, device=dev).to(torch.bfloat16), kv_cache=m, global_idx=0, num_frames=frames)
+    assert m.frame_count == [0] and m.device_header()["frame_count"] == 0 and not m.kv_caches[0].any()
