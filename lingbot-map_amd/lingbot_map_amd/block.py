@@ -487,12 +487,14 @@ class HipPagedAttention(nn.Module):
         H, D = self.num_heads, self.head_dim
         proj = self._fused_projection(x, x.dtype)
         qkv = None if proj is not None else self.qkv(x).reshape(B * n, -1).contiguous()
+        if qkv is not None and qkv.dtype not in (torch.bfloat16, torch.float32):   # (autocast chooses the projection's type)
+            qkv = qkv.to(x.dtype)
         has_norm = isinstance(self.q_norm, nn.LayerNorm)
         qk_norm = (self._norm_f32(self.q_norm) + self._norm_f32(self.k_norm)) if has_norm else (None,) * 4
         table, layout = self._dense_table(pos, enable_3d_rope, B, n, x.dtype)
         q, k, v = (torch.empty(B * n, H, D, dtype=x.dtype, device=x.device) for _ in range(3))
         p = lambda t: None if t is None else C.c_void_p(t.data_ptr())
-        dt = N.DTYPE_BF16 if x.dtype == torch.bfloat16 else N.DTYPE_F32
+        dt = lambda d: N.DTYPE_BF16 if d == torch.bfloat16 else N.DTYPE_F32
         eps = float(self.q_norm.eps) if has_norm else 1e-5
         stream = N.stream_ptr(x.device)
         # q comes out multiplied by the softmax scale and log2(e) (rounded once), see dense_attention
@@ -504,7 +506,8 @@ class HipPagedAttention(nn.Module):
                 eps, q_scale, p(table), layout, p(q), p(k), p(v), None, None, H, D, 16, stream))
         else:
             N.check(N.lib.lbm_qkv_prepare(
-                p(qkv), dt, p(qk_norm[0]), p(qk_norm[1]), p(qk_norm[2]), p(qk_norm[3]), eps, q_scale, p(table), layout, p(q), p(k), p(v), dt,
+                p(qkv), dt(qkv.dtype), p(qk_norm[0]), p(qk_norm[1]), p(qk_norm[2]), p(qk_norm[3]), eps, q_scale, p(table), layout,
+                p(q), p(k), p(v), dt(x.dtype),
                 None, None, B * n, H, D, 16, stream))
         out = dense_attention(q, k, v, num_streams=B, q_prescaled=True).reshape(B, n, H * D)
         return (out, k, v) if return_kv else out

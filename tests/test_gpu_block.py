@@ -429,3 +429,31 @@ def test_manager_of_another_geometry_is_refused_untouched(heads, frames):
     with torch.no_grad(), pytest.raises(AssertionError):
         block(torch.randn(1, frames * tokens, 128, device=dev).to(torch.bfloat16), kv_cache=m, global_idx=0, num_frames=frames)
     assert m.frame_count == [0] and m.device_header()["frame_count"] == 0 and not m.kv_caches[0].any()
+
+
+@pytest.mark.parametrize("rope", [False, True])
+def test_cacheless_attention_of_float32_rows_under_autocast(rope):
+    """Autocast projects float32 rows to bfloat16: the producer has to read the projection in the type that it
+    came in.  Against the same attention written out in float32 on the projection's bfloat16 values."""
+    from lingbot_map_amd.block import HipPagedAttention, RotaryPositionEmbedding2D, PositionGetter
+    dev, B, h, w, C = torch.device("cuda:0"), 2, 5, 9, 128
+    torch.manual_seed(11)
+    attn = HipPagedAttention(dim=C, num_heads=2, qk_norm=True, rope=RotaryPositionEmbedding2D() if rope else None)
+    attn = attn.to(dev, torch.bfloat16).eval()
+    x = torch.randn(B, h * w, C, device=dev)
+    pos = PositionGetter()(B, h, w, dev) if rope else None
+    with torch.no_grad():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            got = attn.dense_attend_fused(x, pos)
+            qkv = attn.qkv(x)
+        assert qkv.dtype == torch.bfloat16 and got.dtype == torch.float32
+        q, k, v = qkv.float().reshape(B, h * w, 3, 2, 64).permute(2, 0, 3, 1, 4).unbind(0)
+        q, k = (torch.nn.functional.layer_norm(t, (64,), m.weight.float(), m.bias.float(), m.eps)
+                for t, m in ((q, attn.q_norm), (k, attn.k_norm)))
+        if rope:
+            q, k = attn.rope(q, pos), attn.rope(k, pos)
+        ref = (torch.softmax(torch.matmul(q, k.transpose(-1, -2).contiguous()) / 8, -1) @ v).transpose(1, 2).reshape(B, h * w, C)
+    # The producer rounds the LayerNorm and the rotation to the projection's type, 2^-9 of each of the 64 products of
+    # a score four times over: sqrt(64 x 4) x 2^-9 / 8 = 0.004 of a score, which moves a mean of values below 2
+    # by 0.004 times their spread; a projection read in the wrong type is off by the values themselves (0.3).
+    assert (got - ref).abs().max().item() <= 1e-2
