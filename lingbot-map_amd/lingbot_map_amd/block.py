@@ -698,6 +698,7 @@ class HipPagedBlock(nn.Module):
         """x + ls(y) and, when ``norm`` is given, norm(x + ls(y)), in one kernel (block.py:283 and
         :194-195; layer_scale.py:21-22)."""
         import ctypes as C
+        assert y.shape == x.shape, f"branch output {tuple(y.shape)} beside the residual stream {tuple(x.shape)}"
         x, y = x.contiguous(), y.contiguous().to(x.dtype)
         x_out = torch.empty_like(x)
         n_out = torch.empty_like(x) if norm is not None else None

@@ -135,3 +135,11 @@ def test_native_call_refuses_a_manager_of_another_geometry(heads, head_dim, fits
     x = torch.zeros(1, 8, 128, dtype=torch.bfloat16)
     for streaming in (True, False):
         assert native.covers(x, None, False, manager, streaming) is fits
+
+
+def test_residual_kernel_refuses_a_branch_of_another_shape():
+    """The kernel reads a row of the branch per row of the stream."""
+    b, x = make_block(), torch.zeros(1, 8, 128, dtype=torch.bfloat16)
+    for shape in ((1, 7, 128), (1, 8, 64), (8, 128)):
+        with pytest.raises(AssertionError, match="branch output"):
+            b._residual(x, torch.zeros(shape, dtype=torch.bfloat16), b.ls1, b.norm2)
