@@ -566,15 +566,21 @@ class _NativeBlock:
     @staticmethod
     def possible(block: "HipPagedBlock") -> bool:
         attn, mlp = block.attn, block.mlp
-        linears = (attn.qkv, attn.proj, mlp.fc1, mlp.fc2)
+        if not all(type(m) is nn.Linear for m in (attn.qkv, attn.proj, mlp.fc1, mlp.fc2)):
+            return False
         norms = (attn.q_norm, attn.k_norm)
         device = attn.qkv.weight.device
-        return (attn.head_dim == 64 and device.type == "cuda"
-                and all(type(m) is nn.Linear and m.weight.dtype == torch.bfloat16 and m.weight.device == device
-                        and m.in_features % 128 == 0 and m.out_features % 64 == 0 for m in linears)
-                and all(isinstance(ls, (LayerScale, nn.Identity)) for ls in (block.ls1, block.ls2))
+        # the call takes pointers: every parameter has the size that the heads and the hidden rows mean
+        dim, hidden = 64 * attn.num_heads, mlp.fc1.out_features
+        linears = ((attn.qkv, 3 * dim, dim), (attn.proj, dim, dim), (mlp.fc1, hidden, dim), (mlp.fc2, dim, hidden))
+        return (attn.head_dim == 64 and device.type == "cuda" and dim % 128 == 0 and hidden % 128 == 0
+                and all(m.weight.dtype == torch.bfloat16 and m.weight.device == device
+                        and tuple(m.weight.shape) == (n, k) and (m.bias is None or m.bias.numel() == n) for m, n, k in linears)
+                and all(isinstance(ls, nn.Identity) or (isinstance(ls, LayerScale) and ls.gamma.numel() == dim)
+                        for ls in (block.ls1, block.ls2))
                 and (all(isinstance(m, nn.Identity) for m in norms) or
-                     all(type(m) is nn.LayerNorm and m.elementwise_affine and m.bias is not None for m in norms))
+                     all(type(m) is nn.LayerNorm and m.elementwise_affine and m.bias is not None
+                         and tuple(m.normalized_shape) == (64,) for m in norms))
                 and isinstance(mlp.act, nn.GELU) and mlp.act.approximate == "none"
                 and FoldedNorm.possible(block.norm2, mlp.fc1))
 
@@ -748,47 +754,52 @@ class HipPagedBlock(nn.Module):
         return (type(self.attn) is HipPagedAttention
                 and not any(m._forward_hooks or m._forward_pre_hooks for m in self.modules() if m is not self))
 
-    def _run_native(self, native: "_NativeBlock", x: Tensor, pos, enable_3d_rope: bool, kv_cache, global_idx: int,
-                    normed, next_norm, pass_rows: Optional[int] = None):
+    def _run_native(self, native: "_NativeBlock", x: Tensor, n1: Optional[Tensor], stats: Optional["RowStats"], pos,
+                    enable_3d_rope: bool, kv_cache, global_idx: int, next_norm, pass_frames: Optional[int] = None):
         """norm1 + qkv projection + producer, attention, proj + LayerScale + residual, fc1 + GELU, fc2 +
         LayerScale + residual (block.py:245-285) as one native call: five GEMM-shaped launches and the
-        attention, no LayerNorm or residual kernel.  With ``next_norm`` the result is ``(x, RowStats)``:
-        the statistics the next block folds its ``norm1`` from.  ``pass_rows``: the frames of an anchor
-        pass (attention.py:475-511), which attend among themselves and are stored in these rows of
-        the cache."""
+        attention, no LayerNorm or residual kernel.  The input comes with its row statistics or with
+        ``n1 = norm1(x)``.  With ``next_norm`` the result is ``(x, RowStats)``: the statistics the next
+        block folds its ``norm1`` from.  ``pass_frames``: so many frames of an anchor pass
+        (attention.py:475-511), which attend among themselves and are stored in the cache; None, with
+        nothing done, when the cache cannot take them at once.
+
+        The cache is touched last: whatever can be refused is refused before its tables move."""
         attn = self._modules["attn"]
         B, n, C = x.shape
         rows = B * n
         x = x.contiguous()
-        stats = normed if isinstance(normed, RowStats) else None
-        if stats is not None and native.folded is not None:
+        if stats is not None:
             a, weights, stats_ptr, stats_tiles = x, native.folded, stats.stats.data_ptr(), stats.tiles
         else:
-            a = (self.norm1(x) if normed is None or stats is not None else normed).contiguous()
-            weights, stats_ptr, stats_tiles = native.plain, None, 0
+            a, weights, stats_ptr, stats_tiles = n1.contiguous(), native.plain, None, 0
         sizes = native.sizes(rows)
-        scratch = torch.empty(sizes[0], dtype=torch.uint8, device=x.device)
-        if kv_cache is not None and pass_rows is None:
+        streaming = kv_cache is not None and pass_frames is None
+        if streaming:
             assert rows == kv_cache.num_streams * kv_cache.tokens_per_frame, (
                 f"{rows} tokens, the cache takes {kv_cache.num_streams} x {kv_cache.tokens_per_frame}")
             table = attn._interleaved_table(pos, B, n) if attn.rope is not None else None
             layout = N.ROPE_INTERLEAVED
+        else:
+            table, layout = attn._dense_table(pos, enable_3d_rope, B, n, x.dtype)
+            row_table, descriptors, ws = dense_plan(rows, B, attn.num_heads, 64, x.device)
+            kv_rows, streams, n_streams = row_table.data_ptr(), addressof(descriptors), B
+        split = _split_workspace(x.device, sizes[2])
+        scratch = torch.empty(sizes[0], dtype=torch.uint8, device=x.device)
+        out = torch.empty_like(x)
+        stats_out = torch.empty(rows, sizes[1], 2, dtype=torch.float32, device=x.device) if next_norm is not None else None
+        pool, page = (None, 16) if kv_cache is None else (kv_cache.kv_caches[global_idx].data_ptr(), kv_cache.page_size)
+        append, keep_kv, live = None, True, None
+        if streaming:
             append, keep_kv, kv_rows, live, plan, ws = kv_cache.begin_block(
                 global_idx, attn.kv_cache_cross_frame_special, attn.kv_cache_camera_only)
             streams, n_streams = plan[2], plan[3]
-            pool, page = kv_cache.kv_caches[global_idx].data_ptr(), kv_cache.page_size
             if n_streams < kv_cache.num_streams:    # streams without a token to see: zeros
                 scratch[:2 * rows * C].zero_()
-        else:
-            table, layout = attn._dense_table(pos, enable_3d_rope, B, n, x.dtype)
-            append, keep_kv, live, pool, page = pass_rows, True, None, None, 16
-            if pass_rows is not None:
-                pool, page = kv_cache.kv_caches[global_idx].data_ptr(), kv_cache.page_size
-            row_table, descriptors, ws = dense_plan(rows, B, attn.num_heads, 64, x.device)
-            kv_rows, streams, n_streams = row_table.data_ptr(), addressof(descriptors), B
-        out = torch.empty_like(x)
-        stats_out = torch.empty(rows, sizes[1], 2, dtype=torch.float32, device=x.device) if next_norm is not None else None
-        split = _split_workspace(x.device, sizes[2])
+        elif pass_frames is not None:
+            append = kv_cache.begin_frames(global_idx, pass_frames, attn.kv_cache_sliding_window)
+            if append is None:
+                return None
         hints = ((None,) * 4, (0,) * 4)
         if self.PREFETCH_HINTS and torch.cuda.is_current_stream_capturing():
             named = native.hints + (getattr(next_norm, "_lbm_folded_qkv_weight", None),)
@@ -842,20 +853,27 @@ class HipPagedBlock(nn.Module):
         with ``next_norm`` the result is ``(x, next_norm(x))`` or ``(x, RowStats of x)``."""
         is_streaming = kv_cache is not None and (num_frames is None or num_frames <= 1)
         is_dense = kv_cache is None or not hasattr(kv_cache, "append_frame")
-        stats = normed if isinstance(normed, RowStats) else None
+        stats, n1 = normed if isinstance(normed, RowStats) else None, None
         if (x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 3 and not torch.is_grad_enabled()
                 and x.shape[0] * x.shape[1] <= Mlp.FUSED_MAX_ROWS):
             native = self._native_block()
             cache = None if is_dense and not is_streaming else kv_cache
             if native is not None and native.covers(x, pos, enable_3d_rope, cache, is_streaming):
-                pass_rows = None
-                if not (is_streaming or is_dense) and self._sub_modules_plain():
+                pass_frames = None if is_streaming or is_dense else num_frames
+                if pass_frames is not None:
                     assert x.shape[1] == num_frames * cache.tokens_per_frame, (
                         f"{x.shape[1]} tokens per stream are not {num_frames} frames of {cache.tokens_per_frame}")
-                    pass_rows = cache.begin_frames(global_idx, num_frames, self.attn.kv_cache_sliding_window)
-                if is_streaming or is_dense or pass_rows is not None:
-                    return self._run_native(native, x, pos, enable_3d_rope, cache, global_idx, normed, next_norm, pass_rows)
-        n1 = self.norm1(x) if (normed is None or stats is not None) else normed
+                if pass_frames is None or self._sub_modules_plain():
+                    fold = stats if native.folded is not None else None
+                    if fold is None:
+                        n1 = self.norm1(x) if normed is None or stats is not None else normed
+                    # (autocast, for one, runs LayerNorm in float32)
+                    if fold is not None or (n1.dtype == torch.bfloat16 and n1.shape == x.shape and n1.device == x.device):
+                        done = self._run_native(native, x, n1, fold, pos, enable_3d_rope, cache, global_idx, next_norm, pass_frames)
+                        if done is not None:
+                            return done
+        if n1 is None:
+            n1 = self.norm1(x) if (normed is None or stats is not None) else normed
         if is_streaming:
             if self.attn.can_fuse(kv_cache, pos, enable_3d_rope):
                 attn_x = self.attn.stream_attend_fused(kv_cache, global_idx, n1, pos)

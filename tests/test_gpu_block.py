@@ -457,3 +457,58 @@ def test_cacheless_attention_of_float32_rows_under_autocast(rope):
     # a score four times over: sqrt(64 x 4) x 2^-9 / 8 = 0.004 of a score, which moves a mean of values below 2
     # by 0.004 times their spread; a projection read in the wrong type is off by the values themselves (0.3).
     assert (got - ref).abs().max().item() <= 1e-2
+
+
+@pytest.mark.parametrize("kind", ["dense", "streamed", "anchor"])
+def test_block_under_autocast_and_with_foreign_norms(kind):
+    """norm1's result reaches the native call only as bfloat16 of the input's shape: under autocast LayerNorm gives
+    float32, and a caller may hand in a float32 ``normed``, which a bfloat16 projection refuses outside of
+    autocast.  The block under autocast against the block without, which round in different places (bf16 noise), and
+    a refusal leaves the cache untouched."""
+    from lingbot_map_amd.block import HipPagedBlock
+    from lingbot_map_amd.manager import HipPagedKVCacheManager
+    dev, tokens, C = torch.device("cuda:0"), 40, 128
+    torch.manual_seed(12)
+    frames = 3 if kind == "anchor" else 1
+    block = HipPagedBlock(dim=C, num_heads=2, qk_norm=True, init_values=0.5).to(dev, torch.bfloat16).eval()
+    x = torch.randn(1, frames * tokens, C, device=dev).to(torch.bfloat16)
+
+    def run(autocast, **kw):
+        m = None if kind == "dense" else HipPagedKVCacheManager(
+            1, 24, tokens, 2, 64, torch.bfloat16, dev, num_special_tokens=5, scale_frames=frames, sliding_window=4,
+            max_total_frames=32, page_size=16, layout="frame_pages")
+        try:
+            with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+                out = block(x, kv_cache=m, global_idx=0, num_frames=frames, **kw)
+            return out.float(), None if m is None else m.kv_caches[0].float()
+        except RuntimeError:
+            assert m is None or (m.frame_count == [0] and m.device_header()["frame_count"] == 0 and not m.kv_caches[0].any())
+            raise
+
+    (y, pool), (z, pool_z) = run(True), run(False)
+    for a, b in ((y, z), (pool, pool_z)):
+        if a is not None:
+            assert (a - b).abs().mean().item() <= 0.01 * b.abs().mean().item()
+    with torch.no_grad():
+        n1 = block.norm1(x)
+    assert torch.equal(run(False, normed=n1)[0], z)
+    with pytest.raises(RuntimeError):
+        run(False, normed=n1.float())
+    with pytest.raises((RuntimeError, AssertionError)):
+        run(False, normed=n1[:, :-1])
+
+
+def test_parameters_of_other_sizes_do_not_reach_the_native_call():
+    """Parameters whose sizes the heads do not mean (a projection swapped for another, a LayerScale or q/k
+    LayerNorm of another length) are left to the module-by-module calls, which name what does not fit."""
+    from torch import nn
+    from lingbot_map_amd.block import HipPagedBlock, LayerScale, _NativeBlock
+    dev, make = torch.device("cuda:0"), lambda **kw: HipPagedBlock(dim=128, num_heads=2, qk_norm=True, init_values=0.5, **kw)
+    swaps = {"attn.proj": nn.Linear(128, 256), "attn.qkv": nn.Linear(128, 128), "mlp.fc1": nn.Linear(256, 512),
+             "mlp.fc2": nn.Linear(512, 256), "attn.q_norm": nn.LayerNorm(128), "ls1": LayerScale(64), "ls2": LayerScale(1)}
+    assert _NativeBlock.possible(make().to(dev, torch.bfloat16))
+    for name, other in swaps.items():
+        block = make()
+        parent, _, leaf = name.rpartition(".")
+        setattr(block.get_submodule(parent), leaf, other)
+        assert not _NativeBlock.possible(block.to(dev, torch.bfloat16)), name
