@@ -33,6 +33,7 @@ from torch import Tensor, nn
 
 from . import _native as N
 from .dense import dense_attention, dense_plan
+from .manager import HipPagedKVCacheManager
 
 
 def apply_rotary_emb(x: Tensor, freqs: Tensor) -> Tensor:
@@ -555,6 +556,14 @@ class HipPagedAttention(nn.Module):
         return self.proj(out)
 
 
+def _runs_own_calls(kind: type) -> bool:
+    """Whether a manager of this class does in ``step_qkv``, ``append_frame`` and ``evict_frames`` what the
+    native call does in their place: not one that wraps a manager or overrides them."""
+    M = HipPagedKVCacheManager
+    return (getattr(kind, "step_qkv", None) is M.step_qkv and getattr(kind, "append_frame", None) is M.append_frame
+            and getattr(kind, "evict_frames", None) is M.evict_frames)
+
+
 class _NativeBlock:
     """A ``HipPagedBlock``'s parameters laid out for ``lbm_block_run``: ``folded`` with norm1 folded
     into the qkv projection (for an input that comes with ``RowStats``; None when norm1 cannot be
@@ -634,8 +643,9 @@ class _NativeBlock:
         if manager is not None:
             # the producer writes num_heads x 64 values per row into the manager's pool: a manager of another
             # geometry is left to the calls that refuse it before anything is launched
-            if (not hasattr(manager, "begin_block") or manager.dtype != torch.bfloat16
-                    or manager.num_heads != self.num_heads or manager.head_dim != 64):
+            if not _runs_own_calls(type(manager)) or manager.dtype != torch.bfloat16:
+                return False
+            if manager.num_heads != self.num_heads or manager.head_dim != 64:
                 return False
             if streaming:
                 return rope is None or (bool(enable_3d_rope) and torch.is_tensor(pos) and pos.is_complex())

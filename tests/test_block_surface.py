@@ -129,9 +129,11 @@ def test_native_call_refuses_a_manager_of_another_geometry(heads, head_dim, fits
     only a manager laid out for them, streaming and in the anchor pass."""
     from types import SimpleNamespace
     from lingbot_map_amd.block import _NativeBlock
+    from lingbot_map_amd.manager import HipPagedKVCacheManager
     native = object.__new__(_NativeBlock)      # (laying parameters out needs a GPU; the check does not)
     native.device, native.num_heads, native.attn = torch.device("cpu"), 2, SimpleNamespace(rope=None)
-    manager = SimpleNamespace(begin_block=None, dtype=torch.bfloat16, num_streams=1, num_heads=heads, head_dim=head_dim)
+    manager = object.__new__(HipPagedKVCacheManager)
+    manager.__dict__.update(dtype=torch.bfloat16, num_streams=1, num_heads=heads, head_dim=head_dim)
     x = torch.zeros(1, 8, 128, dtype=torch.bfloat16)
     for streaming in (True, False):
         assert native.covers(x, None, False, manager, streaming) is fits

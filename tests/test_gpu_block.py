@@ -512,3 +512,43 @@ def test_parameters_of_other_sizes_do_not_reach_the_native_call():
         parent, _, leaf = name.rpartition(".")
         setattr(block.get_submodule(parent), leaf, other)
         assert not _NativeBlock.possible(block.to(dev, torch.bfloat16)), name
+
+
+@pytest.mark.parametrize("frames", [1, 3])
+@pytest.mark.parametrize("how", ["override", "wrap", "plain"])
+def test_managers_that_change_the_calls_are_called(how, frames):
+    """A manager that overrides ``step_qkv`` or ``append_frame``, or wraps another and shows the reference's call
+    surface only, gets those calls; one that leaves them alone is driven by the native call."""
+    from lingbot_map_amd.block import HipPagedBlock
+    from lingbot_map_amd.manager import HipPagedKVCacheManager
+    calls = []
+
+    class Counting(HipPagedKVCacheManager):
+        def step_qkv(self, *a, **kw):
+            calls.append("step_qkv")
+            return super().step_qkv(*a, **kw)
+
+        def append_frame(self, *a, **kw):
+            calls.append("append_frame")
+            return super().append_frame(*a, **kw)
+
+    class Extended(HipPagedKVCacheManager):
+        def begin_block(self, *a, **kw):
+            calls.append("native")
+            return super().begin_block(*a, **kw)
+
+        def begin_frames(self, *a, **kw):
+            calls.append("native")
+            return super().begin_frames(*a, **kw)
+
+    dev, tokens = torch.device("cuda:0"), 40
+    torch.manual_seed(13)
+    block = HipPagedBlock(dim=128, num_heads=2, qk_norm=True, init_values=0.5).to(dev, torch.bfloat16).eval()
+    m = (Counting if how == "override" else Extended)(
+        1, 24, tokens, 2, 64, torch.bfloat16, dev, num_special_tokens=5, scale_frames=frames, sliding_window=4,
+        max_total_frames=32, page_size=16, layout="frame_pages")
+    with torch.no_grad():
+        block(torch.randn(1, frames * tokens, 128, device=dev).to(torch.bfloat16),
+              kv_cache=ReferenceSurfaceOnly(m) if how == "wrap" else m, global_idx=0, num_frames=frames)
+    assert m.frame_count == [frames]
+    assert calls == {"override": ["step_qkv"] if frames == 1 else ["append_frame"] * frames, "wrap": [], "plain": ["native"]}[how]
