@@ -662,6 +662,10 @@ class HipPagedKVCacheManager:
         ``lbm_attn_run_append`` (``step`` does), which ``_newest_self`` remembers."""
         if keyframe is None:
             keyframe = (not self._skip_append,) * self.num_streams
+        else:
+            keyframe = list(keyframe)
+            if len(keyframe) != self.num_streams:
+                raise IndexError(f"keyframe: {len(keyframe)} flags for {self.num_streams} streams")
         keyframe = [a and bool(x) for a, x in zip(self._active, keyframe)]
         tail = [a and not x for a, x in zip(self._active, keyframe)]
         stores = True in keyframe

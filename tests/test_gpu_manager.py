@@ -367,3 +367,24 @@ def test_one_token_step_stores_its_row(cached):
             outs.append(m.step(0, q, k, v, cross_frame_special=False))
         assert torch.equal(outs[0], outs[1]) and torch.equal(ms[0].kv_caches[0], ms[1].kv_caches[0])
     assert ms[0].device_header()["error"] == 0
+
+
+@pytest.mark.parametrize("flags", [[], [True], [True, False, True], (False,)])
+@pytest.mark.parametrize("block", [0, 1])
+def test_step_refuses_flags_for_another_number_of_streams(flags, block):
+    """``keyframe`` holds one flag per stream; any other number is an IndexError on every block, before the
+    counts or the tables move."""
+    m = make("frame_pages", 16, num_streams=2)
+    g = torch.Generator().manual_seed(1)
+    qkv = [torch.randn(14, 2, 64, generator=g).to("cuda:0", torch.bfloat16) for _ in range(3)]
+    m.step(0, *qkv, keyframe=[True, True])
+    if block == 0:
+        m.step(1, *qkv, keyframe=[True, True])
+    counts, before = list(m.frame_count), [m.get_cache_stats(0, s) for s in range(2)]
+    tables = [m.build_visible_page_table(0, s) for s in range(2)]
+    with pytest.raises(IndexError):
+        m.step(block, *qkv, keyframe=flags)
+    assert m.frame_count == counts and [m.get_cache_stats(0, s) for s in range(2)] == before
+    assert [m.build_visible_page_table(0, s) for s in range(2)] == tables
+    m.step(block, *qkv, keyframe=(True, True))
+    m.check_device_errors()
