@@ -30,6 +30,7 @@ from typing import Callable, Optional
 import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
+from torch.nn.modules.module import _global_forward_hooks, _global_forward_pre_hooks
 
 from . import _native as N
 from .dense import dense_attention, dense_plan
@@ -745,14 +746,19 @@ class HipPagedBlock(nn.Module):
     # ------------------------------------------------------------------ the block as one native call
     def _native_block(self) -> Optional["_NativeBlock"]:
         """The block's parameters as ``lbm_block_run`` takes them, or None when the block is not one
-        it covers; kept until a parameter or a sub-module changes."""
+        it covers; kept until a parameter, a sub-module or a setting that it holds changes."""
         mods = self._modules
-        attn, mlp = mods["attn"]._modules, mods["mlp"]._modules
-        if type(mods["mlp"]) is not Mlp:
+        attn, mlp, norm1, norm2 = mods["attn"], mods["mlp"], mods["norm1"], mods["norm2"]
+        # (a subclass of either may do something else in any of its methods)
+        if type(mlp) is not Mlp or type(attn) is not HipPagedAttention:
             return None
-        leaves = (mods["norm1"], mods["norm2"], mods["ls1"], mods["ls2"], attn["qkv"], attn["q_norm"], attn["k_norm"],
-                  attn["proj"], mlp["fc1"], mlp["act"], mlp["fc2"])
-        key = [(t.data_ptr(), t._version) for m in leaves for t in m._parameters.values() if t is not None]
+        a, m = attn._modules, mlp._modules
+        leaves = (norm1, norm2, mods["ls1"], mods["ls2"], a["qkv"], a["q_norm"], a["k_norm"], a["proj"], m["fc1"], m["act"], m["fc2"], attn)
+        key = [(t.data_ptr(), t._version) for leaf in leaves for t in leaf._parameters.values() if t is not None]
+        # what forward reads of them besides; a module without the attribute is none that the call covers
+        of = lambda leaf, name: leaf.__dict__.get(name)
+        key.append((of(norm1, "eps"), of(norm2, "eps"), of(a["q_norm"], "eps"), of(a["k_norm"], "eps"), of(m["act"], "approximate"),
+                    attn.num_heads, attn.head_dim))
         hit = self.__dict__.get("_native_cache")
         if hit is None or hit[0] != leaves or hit[1] != key:
             hit = self.__dict__["_native_cache"] = (leaves, key, _NativeBlock(self) if _NativeBlock.possible(self) else None)
@@ -760,9 +766,9 @@ class HipPagedBlock(nn.Module):
 
     def _sub_modules_plain(self) -> bool:
         """Whether calling the sub-modules one by one would run nothing that the native call does not: no
-        hooks on them, no subclass of the attention."""
-        return (type(self.attn) is HipPagedAttention
-                and not any(m._forward_hooks or m._forward_pre_hooks for m in self.modules() if m is not self))
+        hooks on them, nor on all modules."""
+        return not (_global_forward_hooks or _global_forward_pre_hooks
+                    or any(m._forward_hooks or m._forward_pre_hooks for m in self.modules() if m is not self))
 
     def _run_native(self, native: "_NativeBlock", x: Tensor, n1: Optional[Tensor], stats: Optional["RowStats"], pos,
                     enable_3d_rope: bool, kv_cache, global_idx: int, next_norm, pass_frames: Optional[int] = None):

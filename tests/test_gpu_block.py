@@ -552,3 +552,71 @@ def test_managers_that_change_the_calls_are_called(how, frames):
               kv_cache=ReferenceSurfaceOnly(m) if how == "wrap" else m, global_idx=0, num_frames=frames)
     assert m.frame_count == [frames]
     assert calls == {"override": ["step_qkv"] if frames == 1 else ["append_frame"] * frames, "wrap": [], "plain": ["native"]}[how]
+
+
+@pytest.mark.parametrize("kind", ["dense", "streamed", "anchor"])
+def test_settings_changed_after_the_first_call_hold(kind):
+    """The settings that a forward pass reads from its sub-modules (epsilons, GELU's approximation) and the class of
+    the attention may change between calls: each result is a new block's with the same settings, bit for bit."""
+    from lingbot_map_amd.block import HipPagedAttention, HipPagedBlock
+    from lingbot_map_amd.manager import HipPagedKVCacheManager
+    dev, tokens, C = torch.device("cuda:0"), 40, 128
+    torch.manual_seed(14)
+    frames = 3 if kind == "anchor" else 1
+    block = HipPagedBlock(dim=C, num_heads=2, qk_norm=True, init_values=0.5).to(dev, torch.bfloat16).eval()
+    x = 0.1 * torch.randn(1, frames * tokens, C, device=dev).to(torch.bfloat16)     # (small enough for an epsilon to show)
+
+    def run(b):
+        m = None if kind == "dense" else HipPagedKVCacheManager(
+            1, 24, tokens, 2, 64, torch.bfloat16, dev, num_special_tokens=5, scale_frames=frames, sliding_window=4,
+            max_total_frames=32, page_size=16, layout="frame_pages")
+        with torch.no_grad():
+            return b(x, kv_cache=m, global_idx=0, num_frames=frames)
+
+    last = run(block)
+    for name, field, value in (("norm2", "eps", 0.5), ("attn.q_norm", "eps", 0.5), ("attn.k_norm", "eps", 0.5), ("mlp.act", "approximate", "tanh"),
+                               ("norm1", "eps", 0.5)):
+        setattr(block.get_submodule(name), field, value)
+        new = HipPagedBlock(dim=C, num_heads=2, qk_norm=True, init_values=0.5).to(dev, torch.bfloat16).eval()
+        new.load_state_dict(block.state_dict())
+        for n in ("norm1", "norm2", "attn.q_norm", "attn.k_norm"):
+            new.get_submodule(n).eps = block.get_submodule(n).eps
+        new.mlp.act.approximate = block.mlp.act.approximate
+        out = run(block)
+        assert torch.equal(out, run(new)), name
+        # (one q_scale and one epsilon for q and k: the producer takes q's, so k's alone changes nothing)
+        assert name in ("mlp.act", "attn.k_norm") or not torch.equal(out, last), name
+        last = out
+
+    seen = []
+
+    class Watched(HipPagedAttention):
+        def stream_attend_fused(self, *a, **kw):
+            seen.append("streamed")
+            return super().stream_attend_fused(*a, **kw)
+
+        def dense_attend_fused(self, *a, **kw):
+            seen.append("dense")
+            return super().dense_attend_fused(*a, **kw)
+
+    block.attn.__class__ = Watched
+    run(block)
+    assert seen == ["streamed" if kind == "streamed" else "dense"]
+
+
+def test_anchor_pass_runs_hooks_of_all_modules():
+    """A hook registered for all modules sees the block's sub-modules in the anchor pass."""
+    from torch.nn.modules.module import register_module_forward_hook
+    from lingbot_map_amd.block import HipPagedAttention, HipPagedBlock, Mlp
+    from lingbot_map_amd.manager import HipPagedKVCacheManager
+    dev, tokens, frames, seen = torch.device("cuda:0"), 40, 3, []
+    block = HipPagedBlock(dim=128, num_heads=2, qk_norm=True).to(dev, torch.bfloat16).eval()
+    m = HipPagedKVCacheManager(1, 24, tokens, 2, 64, torch.bfloat16, dev, num_special_tokens=5, scale_frames=frames,
+                               sliding_window=4, max_total_frames=32, page_size=16, layout="frame_pages")
+    hook = register_module_forward_hook(lambda mod, args, out: seen.append(type(mod)))
+    try:
+        with torch.no_grad():
+            block(torch.randn(1, frames * tokens, 128, device=dev).to(torch.bfloat16), kv_cache=m, global_idx=0, num_frames=frames)
+    finally:
+        hook.remove()
+    assert {HipPagedAttention, Mlp, HipPagedBlock} <= set(seen)
