@@ -272,18 +272,23 @@ class HipAggregatorStream(nn.Module):
             return None
         f0 = self.total_frames_processed if first_frame is None else first_frame
         rope = self.rope3d
+        H, W = H // self.patch_size, W // self.patch_size
+        if type(rope) is not RotaryPositionEmbedding3D:
+            return rope(ppf=frames, pph=H, ppw=W, patch_start_idx=self.num_special_tokens, device=device, f_start=f0, f_end=f0 + frames)
         assert 0 <= f0 and f0 + frames <= rope.max_seq_len, \
             f"frames [{f0}, {f0 + frames}) outside the {rope.max_seq_len} positions of the table"
-        key = (frames, H, W, str(device))
+        version = lambda t: 0 if t.is_inference() else t._version
+        key = (frames, H, W, str(device), self.num_special_tokens, version(rope.inv_freq), version(rope.pair_axis))
         hit = self.__dict__.get("_table_base")
-        if hit is None or hit[0] != key:
+        if hit is None or hit[0] != key or hit[1] is not rope.inv_freq or hit[2] is not rope.pair_axis:
             # the angles of a call that starts at frame 0, and what every frame later adds to them:
             # one launch per call instead of writing down a frame's coordinates again
-            coords = rope.coordinates(frames, H // self.patch_size, W // self.patch_size, self.num_special_tokens, device)
+            coords = rope.coordinates(frames, H, W, self.num_special_tokens, device)
             later = torch.where(rope.pair_axis == 0, rope.inv_freq, torch.zeros_like(rope.inv_freq)).to(device)
             angles = rope.angles(coords)
-            hit = self.__dict__["_table_base"] = (key, angles, later, torch.ones_like(angles))
-        return torch.polar(hit[3], torch.add(hit[1], hit[2], alpha=f0))[None, None]
+            hit = self.__dict__["_table_base"] = (key, rope.inv_freq, rope.pair_axis, angles, later, torch.ones_like(angles))
+        _, _, _, angles, later, ones = hit
+        return torch.polar(ones, torch.add(angles, later, alpha=f0))[None, None]
 
     def forward(self, images: Tensor, selected_idx: Optional[List[int]] = None,
                 num_frame_for_scale: Optional[int] = None, sliding_window_size: Optional[int] = None,
@@ -339,9 +344,11 @@ class HipAggregatorStream(nn.Module):
                     first_group = global_idx < self.aa_block_size
                     if self.rope3d is not None:     # frame index = frames streamed so far (stream.py:464-478)
                         if first_group:
-                            # one complex64 entry per token and stream: the blocks take it as it is
                             table = pos3d if pos3d is not None else self.stream_table(S, H, W, tokens.device)
-                            self._cached_pos3d = table.to(torch.complex64).expand(B, -1, -1, -1).contiguous()
+                            if table.is_complex() and table.dim() == 4:
+                                # one complex64 entry per token and stream: the blocks take it as it is
+                                table = table.to(torch.complex64).expand(B, -1, -1, -1).contiguous()
+                            self._cached_pos3d = table
                         pos_g = self._cached_pos3d
                     else:
                         pos_g = pos.view(B, S * P, 2) if pos is not None else None

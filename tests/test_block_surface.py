@@ -145,3 +145,38 @@ def test_residual_kernel_refuses_a_branch_of_another_shape():
     for shape in ((1, 7, 128), (1, 8, 64), (8, 128)):
         with pytest.raises(AssertionError, match="branch output"):
             b._residual(x, torch.zeros(shape, dtype=torch.bfloat16), b.ls1, b.norm2)
+
+
+def test_stream_table_follows_its_rotary_module():
+    """The aggregator keeps the angles of a first frame and adds what later frames turn by: equal to the rotary
+    module's own table at any frame, for several frames, after the module or its rates are replaced, for a subclass
+    with a forward of its own, and for buffers made in inference mode."""
+    from lingbot_map_amd import HipAggregatorStream
+    from lingbot_map_amd.block import RotaryPositionEmbedding3D
+    model = HipAggregatorStream(embed_dim=64, depth=1, num_heads=1, enable_3d_rope=True, max_frame_num=64)
+
+    def check(frames=1):
+        for f0 in (0, 7, 40):
+            want = model.rope3d(ppf=frames, pph=3, ppw=5, patch_start_idx=model.num_special_tokens, device="cpu", f_start=f0, f_end=f0 + frames)
+            got = model.stream_table(frames, 3 * model.patch_size, 5 * model.patch_size, "cpu", first_frame=f0)
+            # (an angle below 64 in float64: a rounding of the product, one of the sum)
+            assert got.shape == want.shape and got.dtype == want.dtype and (got - want).abs().max().item() <= 64 * 2.0 ** -52
+
+    check()
+    check(frames=3)
+    model.rope3d = RotaryPositionEmbedding3D(64, max_seq_len=64, theta=50.0)
+    check()
+    model.rope3d.inv_freq.mul_(0.5)
+    check()
+
+    class Mirrored(RotaryPositionEmbedding3D):
+        def forward(self, *a, **kw):
+            return super().forward(*a, **kw).conj()
+
+    model.rope3d = Mirrored(64, max_seq_len=64)
+    check()
+    with torch.inference_mode():
+        model.rope3d = RotaryPositionEmbedding3D(64, max_seq_len=64)
+    check()
+    with pytest.raises(AssertionError):
+        model.stream_table(1, 42, 70, "cpu", first_frame=64)
