@@ -2,18 +2,22 @@
 // lingbot_map/layers/flashinfer_cache.py:118-127,372-383), on the bf16 matrix instructions.
 //
 // A float is the exact sum of three bf16 values (8 + 8 + 8 significant bits, same exponent range), so a
-// product of two floats is the sum of nine products of bf16 values, each exact in fp32.  Six of them
-// are computed; the three left out are below 2^-23 of the product together, the size of the
-// rounding that an fp32 multiply-add makes.  Sums run in the fp32 accumulators of the matrix pipe, the
-// small terms of a k-step first.  Against float64 the result is closer than that of
-// v_mfma_f32_16x16x4_f32 (relative error 4.2e-7 against 6.4e-7 at 4,000 tokens: fewer roundings per
-// sum).  A bf16 instruction does 16 times the work of an fp32 one per cycle, so six of them are 2.7
-// times as fast; the kernel runs at 1.05 PFLOP/s of bf16 products (176 TFLOP/s of fp32 ones), the rate
-// the chip's power allows a kernel of this mix (the bf16 kernel's, too): neither fences that spread
-// the operand reads and splits over the MFMAs nor a tenth fewer vector instructions moved it.  Measured,
-// 1,004 rows x 16 heads: 1,004 tokens 49 -> 32 us, 8,032 tokens 337 -> 187 us against the fp32
-// instruction.  Infinities have a
-// pass of their own at the end of the kernel.
+// product of two floats is the sum of nine products of bf16 values, each exact in fp32 (Henry, Tang,
+// Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations",
+// ARITH 2019).  Eight of them are computed; the ninth, of the two smallest terms, is below 2^-31 of the
+// product.  The leading products and the other seven have accumulators of their own, which meet in one
+// fp32 addition: a product alone comes out as fp32 rounds it, and a sum over head dimensions or tokens
+// takes a rounding of its full size per 16 or 32 terms.  Six products in one accumulator were a quarter
+// faster (29 and 187 us below) but left up to 1.2 x 2^-23 of a product out, and took six roundings per 16
+// terms.  Largest error of a score against float64, in units of 2^-24 of its size, for 1 and 64 products,
+// v_mfma_f32_16x16x4_f32 / six / eight: 1.1 / 3.6 / 1.1 and 8.5 / 6.3 / 1.0; relative error of the output at
+// 4,000 tokens 6.5e-7 / 4.3e-7 / 1.7e-7.
+//
+// A bf16 instruction does 16 times the work of an fp32 one per cycle; the kernel runs at 1.1 PFLOP/s of
+// bf16 products (137 TFLOP/s of fp32 ones), the rate the chip's power allows a kernel of this mix (the bf16
+// kernel's, too): neither fences that spread the operand reads and splits over the MFMAs nor a tenth fewer
+// vector instructions moved it.  Measured, 1,004 rows x 16 heads: 1,004 tokens 48 -> 37 us, 8,032 tokens
+// 337 -> 240 us against the fp32 instruction.  Infinities have a pass of their own at the end of the kernel.
 //
 // One workgroup = eight wavefronts on 64 query rows of one head.  A wavefront takes every eighth
 // 32-token tile of the KV list, for all 64 rows (so that a value of K or V is split once per 64 rows),
@@ -82,7 +86,7 @@ __device__ __forceinline__ void split_truncated(const f32x8& x, bf16x8 (&p)[3]) 
   for (int k = 0; k < 3; ++k) p[k] = __builtin_bit_cast(bf16x8, w[k]);
 }
 // the same by rounding to nearest (Q and the numerators: with one operand's remainders of either
-// sign, what the left-out products add has no preferred sign)
+// sign, what the left-out product adds has no preferred sign)
 __device__ __forceinline__ void split_rounded(f32x8 x, bf16x8 (&p)[3]) {
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -93,14 +97,16 @@ __device__ __forceinline__ void split_rounded(f32x8 x, bf16x8 (&p)[3]) {
     }
   }
 }
-// acc[i] += a * b[i] over 16 k's, small terms first, the two sums in turn
-__device__ __forceinline__ void mfma_split(const bf16x8 (&a)[3], const bf16x8 (&b0)[3], const bf16x8 (&b1)[3], f32x16& acc0, f32x16& acc1) {
-  constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+// hi[i] += the leading products of a * b[i] over 16 k's, lo[i] += the seven others, small ones first
+__device__ __forceinline__ void mfma_split(const bf16x8 (&a)[3], const bf16x8 (&b0)[3], const bf16x8 (&b1)[3], f32x16 (&hi)[2], f32x16 (&lo)[2]) {
+  constexpr int pa[7] = {2, 1, 2, 0, 1, 1, 0}, pb[7] = {1, 2, 0, 2, 1, 0, 1};
 #pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[i]], b0[pb[i]], acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[i]], b1[pb[i]], acc1, 0, 0, 0);
+  for (int i = 0; i < 7; ++i) {
+    lo[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[i]], b0[pb[i]], lo[0], 0, 0, 0);
+    lo[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[i]], b1[pb[i]], lo[1], 0, 0, 0);
   }
+  hi[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b0[0], hi[0], 0, 0, 0);
+  hi[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b1[0], hi[1], 0, 0, 0);
 }
 
 // loads of this wavefront still allowed in flight (expcnt and lgkmcnt untouched), and LDS reads done
@@ -216,11 +222,11 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32 
   for (int t = wave; t < n_tiles; t += kWaves) {
     LBM_LOADS_LEFT(9);
     // ---- S^T = K Q^T: s[qb][i] is kv = 8 (i / 4) + 4 g + i % 4, q = 32 qb + n32
-    f32x16 s[2];
+    f32x16 s[2], s_lo[2];
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) s[qb][i] = 0.f;
+      for (int i = 0; i < 16; ++i) s[qb][i] = s_lo[qb][i] = 0.f;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const int c = ks * 4 + g * 2;
@@ -233,8 +239,12 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32 
 #pragma unroll
         for (int k = 0; k < 3; ++k)
           qp[qb][k] = *(const bf16x8*)&lds_q[k * kQPlane + (qb * 32 + n32) * 64 + ((ks * 2 + g) ^ ((n32 >> 1) & 7)) * 8];
-      mfma_split(kp, qp[0], qp[1], s[0], s[1]);
+      mfma_split(kp, qp[0], qp[1], s, s_lo);
     }
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[qb][i] += s_lo[qb][i];
     // ---- the next K tile: its entries have landed, this one's fragments are read
     LBM_LOADS_LEFT(8);
     LBM_LDS_READ();
@@ -282,16 +292,21 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32 
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           x[j] = __builtin_amdgcn_exp2f(s[qb][kk * 8 + j] - m[qb]);
-          l[qb] += x[j];
         }
+        l[qb] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
         split_rounded(x, p[qb][kk]);
       }
-    // ---- O^T += V^T P^T
+    // ---- O^T += V^T P^T, the tile's sums in registers that held the scores before they join O
     LBM_LOADS_LEFT(9);
 #pragma unroll
-    for (int kk = 0; kk < 2; ++kk)
+    for (int db = 0; db < 2; ++db) {
+      f32x16 hi[2], lo[2];
 #pragma unroll
-      for (int db = 0; db < 2; ++db) {
+      for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) hi[qb][i] = lo[qb][i] = 0.f;
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
         f32x8 x;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -300,8 +315,13 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32 
         }
         bf16x8 vp[3];
         split_truncated(x, vp);
-        mfma_split(vp, p[0][kk], p[1][kk], o[0][db], o[1][db]);
+        mfma_split(vp, p[0][kk], p[1][kk], hi, lo);
       }
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[qb][db][i] += hi[qb][i] + lo[qb][i];
+    }
     LBM_LDS_READ();
     load_rows(true);
   }
@@ -350,7 +370,9 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32 
   }
   // A term of the split of an infinity is NaN, and so is every result that one had a part in - also where
   // floats give a number (a key at -inf has no weight) or an infinity.  A workgroup that ends with such a
-  // value walks its rows once more, in plain fp32: eight lanes per row, token by token.
+  // value walks its rows once more, in plain fp32: eight lanes per row, token by token.  A launch with such a
+  // workgroup, or with nothing else, takes 0.44-0.48 ms at 1,004 rows x 1,004 tokens (39 us without) and
+  // 4.4-4.6 ms at 8,032 tokens (260 us).
   float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   unsigned top = bits(l_tot) & 0x7fffffffu;
 #pragma unroll
