@@ -1882,13 +1882,17 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
   }
   ScheduleKey& memo = g_schedules[found];
   if (!hit) {
-    int best_splits[LBM_MAX_STREAMS], cand_splits[LBM_MAX_STREAMS];
+    int best_splits[LBM_MAX_STREAMS], cand_splits[LBM_MAX_STREAMS], wary_splits[LBM_MAX_STREAMS];
     double best = -1.0;
     long long best_tps = 0;
     auto consider = [&](long long tps, bool wary) {
       if (tps < 2) tps = 2;
       if (tps > max_nt) tps = max_nt > 0 ? max_nt : 1;
       const double c = price_candidate(qt, nt, n_streams, num_heads, (int)tps, q_rows, cand_splits, wary);
+      // A stream that the upper estimate leaves whole stays whole: split, its partial results would be rounded
+      // to bf16 on their way through memory, and no time is worth a result with fewer bits.
+      for (int i = 0; !wary && i < n_streams; ++i)
+        if (wary_splits[i] == 1 && cand_splits[i] > 1) return;
       if (best < 0 || c < best) {
         best = c;
         best_tps = tps;
@@ -1925,6 +1929,7 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
       // put 6 % ahead took 71 us against 68).
       consider_all(true);
       const long long wary_tps = best_tps;
+      for (int i = 0; i < n_streams; ++i) wary_splits[i] = best_splits[i];
       best = -1.0;
       consider(wary_tps, false);
       const double wary_choice = best;

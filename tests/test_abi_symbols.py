@@ -71,3 +71,25 @@ def test_host_side_argument_checks_need_no_gpu():
     fake = C.c_void_p(256)   # never dereferenced: the call fails in the argument checks
     rc = N.lib.lbm_tables_step(fake, C.byref(g), 2, ops, fake, None, None, None, None)
     assert rc == N.ERR_INVALID and b"overlap" in N.lib.lbm_last_error()
+
+
+def test_schedule_leaves_whole_what_the_upper_estimate_leaves_whole():
+    """Partial results are rounded to bf16 on their way through memory, so a stream of a ragged launch is split only
+    where the upper estimate splits it; the fitted costs choose among such splits.  Rows of partials show it:
+    (splits x rows of every split stream) x heads x (64 bf16 values + a float)."""
+    from lingbot_map_amd import _native as N
+
+    def partial_rows(heads, *streams):
+        arr, at = (N.AttnStream * len(streams))(), 0
+        for i, (rows, kv) in enumerate(streams):
+            arr[i] = N.AttnStream(at, rows, 0, kv, 0)
+            at += rows
+        per_row = heads * (64 * 2 + 4)
+        size = int(N.lib.lbm_attn_workspace_bytes(arr, len(streams), heads, 64))
+        assert size % per_row == 0
+        return size // per_row
+
+    # 520 rows x 2,787 tokens, 200 x 776 and 530 x 6,222 stay whole beside streams ten times as long
+    assert partial_rows(16, (128, 19598), (520, 2787), (9, 12085)) == 7 * 128 + 5 * 9
+    assert partial_rows(8, (333, 9), (487, 24626), (113, 3), (10, 1), (284, 90), (200, 776)) == 12 * 487
+    assert partial_rows(12, (15, 5868), (530, 6222), (17, 63013), (14, 40299)) == 10 * 17 + 7 * 14
