@@ -216,10 +216,7 @@ size_t lbm_attn_workspace_bytes(const lbm_attn_stream* streams, int32_t n_stream
   if (num_heads <= 0 || head_dim <= 0) return 0;
   LbmAttnSchedule sch;
   lbm_attn_schedule(streams, n_streams, num_heads, &sch);
-  // a batch that takes the split-KV kernel always asks for some, also where nothing is split (the
-  // call itself does not insist on that): a caller sees by it which kernel a batch takes
-  const size_t need = lbm_attn_schedule_bytes(sch, num_heads, head_dim);
-  return need == 0 && sch.small == 0 && sch.total_wgs > 0 ? 256 : need;
+  return lbm_attn_schedule_bytes(sch, num_heads, head_dim);
 }
 
 static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, void* out, const void* self_k,

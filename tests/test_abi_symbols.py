@@ -93,3 +93,12 @@ def test_schedule_leaves_whole_what_the_upper_estimate_leaves_whole():
     assert partial_rows(16, (128, 19598), (520, 2787), (9, 12085)) == 7 * 128 + 5 * 9
     assert partial_rows(8, (333, 9), (487, 24626), (113, 3), (10, 1), (284, 90), (200, 776)) == 12 * 487
     assert partial_rows(12, (15, 5868), (530, 6222), (17, 63013), (14, 40299)) == 10 * 17 + 7 * 14
+
+
+def test_workspace_query_is_zero_where_nothing_is_split():
+    """Eight streams of 1,004 rows x 5,000 tokens: 256 workgroups of the split-KV kernel, each with the whole KV
+    list, no partial results; one frame of 1,004 x 1,004 on the short-KV kernel."""
+    from lingbot_map_amd import _native as N
+    arr = (N.AttnStream * 8)(*[N.AttnStream(i * 1004, 1004, i * 5000, 5000, 0) for i in range(8)])
+    assert N.lib.lbm_attn_workspace_bytes(arr, 8, 16, 64) == 0
+    assert N.lib.lbm_attn_workspace_bytes((N.AttnStream * 1)(N.AttnStream(0, 1004, 0, 1004, 0)), 1, 16, 64) == 0
