@@ -1283,8 +1283,8 @@ __device__ __forceinline__ float max_over_lane_groups(float x) {
   return fmaxf(a, b);
 }
 
-template <int D>
 __global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32 a) {
+  constexpr int D = 128;
   // NG groups of four waves: wave w of every group owns the same 16 query rows, group j takes
   // KV tiles j, j + NG, ... (NG waves per SIMD, so one wave's softmax, LDS waits and barriers
   // overlap the others' matrix work); the partial results are merged through LDS at the end.
@@ -2120,7 +2120,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       return lbm_check_launch("lbm_attn_f32_decode_kernel");
     }
     if (head_dim == 64) return lbm_launch_attn_f32_d64(f, stream);
-    hipLaunchKernelGGL(lbm_attn_f32_kernel<128>, dim3(wg), dim3(512), 0, stream, f);
+    hipLaunchKernelGGL(lbm_attn_f32_kernel, dim3(wg), dim3(512), 0, stream, f);
     return lbm_check_launch("lbm_attn_f32_kernel");
   }
   if (dtype != LBM_DTYPE_BF16) return lbm_fail(LBM_ERR_INVALID, "unknown dtype %d", dtype);
