@@ -1484,7 +1484,7 @@ __global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32 a) {
 // D/4 lanes form a row group that takes a K row and its V row, 16 bytes a lane: a wavefront holds
 // 64 / (D/4) row groups, a workgroup NW times as many, and the tokens of the workgroup's piece of
 // the KV axis are dealt to them one by one.  A group asks for the K AND the V rows of eight
-// or twenty tokens at once (V does not wait for the scores: one trip to memory per batch instead of two), and
+// or eleven tokens at once (V does not wait for the scores: one trip to memory per batch instead of two), and
 // keeps the softmax state of its own tokens - maximum, sum, unnormalised output - in registers, so
 // nothing crosses lanes inside the loop but the D/4-lane sum of a dot product (DPP) and there is no
 // barrier in it; the groups meet through LDS once, at the end.
@@ -1496,9 +1496,12 @@ __global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32 a) {
 namespace {
 constexpr int kDecQ = 8;         // query rows per stream this path takes
 constexpr int kDecBatch = 8;     // tokens a row group has in flight
-constexpr int kDecOneBatch = 20; // the same where one workgroup takes everything: eight waves have the registers
-                                 // for 320 tokens of 128 floats in one trip (16 waves of 8 tokens: 9.4 us for 300
-                                 // tokens in two trips, against 8.0)
+constexpr int kDecOneBatch = 11; // the same where one workgroup takes everything, 16 (head_dim 128) or 32 row groups:
+                                 // a step loads its batch whether the tokens are there or not, so a short list
+                                 // wants few and a long one few trips.  us a launch at head_dim 128, 16 heads, for
+                                 // 6 / 8 / 11 / 20: 64 tokens 3.7 / 4.2 / 4.5 / 6.4, 150 5.8 / 6.6 / 5.4 / 7.1, 300 8.1 / 8.3 /
+                                 // 7.5 / 7.6, 512 10.4 / 10.2 / 9.7 / 11.3; means over 13 lengths from 16 to 512 tokens 6.8 /
+                                 // 7.0 / 6.9 / 8.3, at head_dim 64 5.0 / 5.3 / 5.5 / 6.8
 constexpr int kDecChunk = 256;   // tokens per chunk, as long as that makes at most kDecMaxChunks
 constexpr int kDecMaxChunks = 64;
 constexpr int kDecOneTokens = 512;
