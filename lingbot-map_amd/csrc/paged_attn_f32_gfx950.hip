@@ -57,8 +57,7 @@ constexpr int kLdsBytes = kLoopBytes > kMergeBytes ? kLoopBytes : kMergeBytes;
 static_assert(kLdsBytes <= 160 * 1024, "LDS of a CU");
 constexpr float kSlack = 8.f;           // a score this far above the reference raises it
 
-// value of the other half-wave's lane beside the own one (inline asm: the builtin's two results are
-// folded into one by the compiler)
+// value of the other half-wave's lane beside the own one
 __device__ __forceinline__ void swap_halves(float x, float& lo, float& hi) {
   float a = x, b = x;
   asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));

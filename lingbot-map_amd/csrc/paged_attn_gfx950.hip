@@ -91,9 +91,9 @@ struct AttnArgs : AttnCore {
 
 // Exchange between lane l and lane l^32.  v_permlane32_swap swaps the upper half of its first
 // register with the lower half of its second; fed two copies of x it leaves {x_lo, x_lo} in
-// the first and {x_hi, x_hi} in the second.  Written as inline asm because the compiler
-// folds the builtin's two results into one; the s_nop covers the VALU-write to permlane-read
-// wait states the compiler can no longer see.
+// the first and {x_hi, x_hi} in the second.  Inline asm with the wait states from a VALU write to
+// the permlane's read in it; the builtin compiles to the same instruction, provided that its two results
+// are read by value (see float_bits).
 __device__ __forceinline__ void swap_halves(float x, float& lo, float& hi) {
   float a = x, b = x;
   asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
@@ -734,10 +734,8 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
     // the row sum of query n32 of this block sits in lane n32 % 16, element n32 / 16
-    // (the two elements go through an opaque asm: fed two elements of one vector, the compiler
-    // folds the select below into the permute's data operand, which picks by the wrong lane)
-    float sum_lo = lacc[qb][0], sum_hi = lacc[qb][1];
-    asm volatile("" : "+v"(sum_lo), "+v"(sum_hi));
+    // (both elements by value first, see float_bits)
+    const float sum_lo = lacc[qb][0], sum_hi = lacc[qb][1];
     const float l_lo = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (lane & 15), __builtin_bit_cast(int, sum_lo)));
     const float l_hi = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (lane & 15), __builtin_bit_cast(int, sum_hi)));
     const float l_tot = (n32 & 16) ? l_hi : l_lo;
