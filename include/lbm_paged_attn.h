@@ -336,7 +336,8 @@ typedef struct lbm_block_call {
   float* out_stats;            /* row statistics of out ([rows][lbm_linear_stats_tiles(rows, dim)][2]) or NULL */
   void* scratch;               /* at least lbm_block_scratch_bytes; starts with the attention's output [rows, dim] */
   const float* rope_cs;        /* as lbm_qkv_prepare */
-  void* pool;                  /* NULL: attention over the rows of this call only (kv_rows all negative) */
+  void* pool;                  /* rows of num_heads x 64, as append_rows and kv_rows count them; NULL: attention over the
+                                * rows of this call only (kv_rows all negative) */
   const int32_t* append_rows;  /* NULL: nothing is stored in the pool */
   const int32_t* kv_rows;
   const int32_t* live_kv_tokens;        /* NULL: the streams' counts are the host's */

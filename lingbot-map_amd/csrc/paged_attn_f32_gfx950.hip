@@ -14,10 +14,11 @@
 // 4,000 tokens 6.5e-7 / 4.3e-7 / 1.7e-7.
 //
 // A bf16 instruction does 16 times the work of an fp32 one per cycle; the kernel runs at 1.1 PFLOP/s of
-// bf16 products (137 TFLOP/s of fp32 ones), the rate the chip's power allows a kernel of this mix (the bf16
-// kernel's, too): neither fences that spread the operand reads and splits over the MFMAs nor a tenth fewer
-// vector instructions moved it.  Measured, 1,004 rows x 16 heads: 1,004 tokens 48 -> 37 us, 8,032 tokens
-// 337 -> 240 us against the fp32 instruction.  Infinities have a pass of their own at the end of the kernel.
+// bf16 products (137 TFLOP/s of fp32 ones).  At 8,032 tokens the matrix pipe works 58 % and the vector ALU (7 splits,
+// sums and exponentials per MFMA) 62 % of the cycles, at 1.7 GHz; with six products, fences that spread the
+// operand reads and splits over the MFMAs and a tenth fewer vector instructions changed nothing.  Measured,
+// 1,004 rows x 16 heads: 1,004 tokens 48 -> 37 us, 8,032 tokens 337 -> 240 us against the fp32 instruction.
+// Infinities have a pass of their own at the end of the kernel.
 //
 // One workgroup = eight wavefronts on 64 query rows of one head.  A wavefront takes every eighth
 // 32-token tile of the KV list, for all 64 rows (so that a value of K or V is split once per 64 rows),
