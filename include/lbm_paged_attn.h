@@ -266,7 +266,7 @@ size_t lbm_linear_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t epilo
  * the next one will read - the weights of the layer that follows - names it here: the next
  * lbm_linear, lbm_linear_norm, lbm_qkv_linear_prepare or lbm_qkv_linear_prepare_norm call of the
  * calling host thread then also reads one dword of every 128-byte line of [next_read, next_read +
- * bytes) while it computes (a ninth wavefront per workgroup that does nothing else), which leaves
+ * bytes) while it computes (one wavefront per workgroup that does nothing else), which leaves
  * the lines in the memory-side cache.  The hint is consumed by that one call (launches on
  * 256-row tiles ignore it); results are the same with and without it.  The memory must be
  * readable device memory for as long as that launch can run, replays of a captured graph

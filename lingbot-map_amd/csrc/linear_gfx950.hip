@@ -34,8 +34,11 @@
 // registers and no LDS store instructions in between) in 64-wide slices of K, four LDS stages (three
 // of a 256-column tile), one slice less ahead of the multiply; rows are unpadded and their 16-byte chunks XOR-swizzled by
 // the choice of source address, so the b128 fragment reads are free of bank conflicts.  One
-// workgroup barrier per slice.  The tile leaves through LDS as whole rows: 16-byte stores, and
-// the residual is read the same way.
+// workgroup barrier per slice.  Two more wavefronts do the loading: a CU's vector memory path takes 64 bytes per
+// cycle, so the 32 KB of a 128 x 128 step keep it busy as long as the multiply takes, and a wavefront that
+// issues a load into a full path stands still with its MFMAs behind it (the tiles of 256 columns, whose
+// accumulators leave no registers for a third wavefront per SIMD, load for themselves).  The tile leaves
+// through LDS as whole rows: 16-byte stores, and the residual is read the same way.
 #include <type_traits>
 #include <hip/hip_runtime.h>
 #include "lbm_internal.h"
@@ -59,9 +62,10 @@ typedef __attribute__((ext_vector_type(2))) short s16x2;
 constexpr int kGK = 128;         // K granularity the launches accept
 constexpr int kGM = 128;         // activation rows per tile
 constexpr int kGThreads = 512;
-constexpr int kGTouchThreads = 64;   // lbm_linear_bf16_kernel: one more wavefront that only asks for weight lines ahead of the loop
+constexpr int kGLoadWaves = 2;       // wavefronts that load the operands
+constexpr int kGTouchThreads = 64;   // and one that only asks for the next launch's lines
 // (256 columns: the accumulators leave no registers for a third wavefront per SIMD)
-constexpr int lbm_linear_threads(int tn) { return kGThreads + (tn == 256 ? 0 : kGTouchThreads); }
+constexpr int lbm_linear_threads(int tn) { return kGThreads + (tn == 256 ? 0 : kGLoadWaves * 64 + kGTouchThreads); }
 constexpr int kKS = 64;          // K elements per LDS stage
 constexpr int kStagesG = 4;      // LDS stages: three being loaded while one is multiplied (six stages for the 64-column tile,
                                  // which has the room: slower, 8.4 -> 8.8 us for proj - the longer prologue costs more than the depth gains)
@@ -104,7 +108,7 @@ struct LinearArgs {
   // parks its fp32 partial tile in `split_part` and takes a ticket from the tile's counter; the
   // one that draws the last ticket sums the partials in slice order (the same sum whoever is
   // last) and runs the epilogue.  Counters start at zero and are left at zero.
-  // memory the launch after this one will read (lbm_linear_prefetch_hint): the ninth wavefronts of
+  // memory the launch after this one will read (lbm_linear_prefetch_hint): one wavefront per workgroup of
   // lbm_linear_bf16_kernel ask for it
   const char* touch;
   unsigned touch_lines;          // 128-byte lines
@@ -191,10 +195,159 @@ __device__ __forceinline__ void lbm_tile_of_workgroup(int b, int m_tiles, int n_
   nt = panel * 8 + rem - mt * width;
 }
 
+
+// ---- pieces that the kernels below share
+
+// s_waitcnt vmcnt(N), the other counters untouched
+#define LBM_DMA_WAIT(N) __builtin_amdgcn_s_waitcnt(0x0F70 | ((N) & 15) | (((N) >> 4) << 14))
+
+// What a wavefront beside the computing ones does with a prefetch hint (lbm_linear_prefetch_hint).  It holds
+// no operand and joins no barrier (a wavefront that has ended is not waited for).  In a model every launch
+// finds its weights in HBM - a frame walks through far more weight bytes than the caches hold - and the
+// loop's steps of look-ahead do not cover that latency: the same launch takes 0.6 to 5 us longer on weights
+// that no cache holds.  A caller that knows which memory the launch AFTER this one will read says so, and
+// these wavefronts, all workgroups' together, read one dword of every 128-byte line of it: the lines are
+// then in the memory-side cache (or an L2) when that launch starts, having travelled while this one computed.
+// (plain loads whose results the compiler sees - a load whose result it does not know of could
+// land in a register it has reused: eight in flight per lane, their values folded into a word
+// that is stored only under a condition that never holds)
+__device__ __forceinline__ void touch_lines(const LinearArgs& p, int lane) {
+  unsigned folded = 0;
+  const unsigned stride = gridDim.x * 64u;
+  for (unsigned first = blockIdx.x * 64u + (unsigned)lane; first < p.touch_lines; first += 8u * stride) {
+    unsigned got[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const unsigned line = first + (unsigned)j * stride;
+      got[j] = line < p.touch_lines ? *(const unsigned*)(p.touch + (size_t)line * 128) : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) folded ^= got[j];
+  }
+  if (folded == 0x5bd1e995u && p.M < 0) p.out[lane] = (unsigned short)folded;   // (M is never negative)
+}
+
+// LNA: the statistics of a row, held by four neighbouring lanes that take every fourth (mean, M2) partial each;
+// equal-sized partials merge as mean = avg(mean_i), M2 = sum(M2_i) + n_i * sum((mean_i - mean)^2) (Chan et
+// al.), variance = M2 / K.  Returns (rstd, -mean * rstd).  The partials are asked for before the operand
+// tiles (loads return in order) and merged while those travel.
+constexpr int kLnHeld = 4;     // partials a lane keeps in registers (up to 16 column tiles)
+__device__ __forceinline__ void ask_row_stats(const LinearArgs& p, int row, int part, f32x2 (&held)[kLnHeld]) {
+  const float* st = p.ln_stats + (size_t)row * p.ln_tiles * 2;
+#pragma unroll
+  for (int i = 0; i < kLnHeld; ++i)
+    if (part + 4 * i < p.ln_tiles) held[i] = *(const f32x2*)(st + 2 * (part + 4 * i));
+}
+__device__ __forceinline__ f32x2 merge_row_stats(const LinearArgs& p, int row, int part, const f32x2 (&held)[kLnHeld]) {
+  const float* st = p.ln_stats + (size_t)row * p.ln_tiles * 2;
+  float sm = 0.f;
+#pragma unroll
+  for (int i = 0; i < kLnHeld; ++i)
+    if (part + 4 * i < p.ln_tiles) sm += held[i][0];
+  for (int i = part + 4 * kLnHeld; i < p.ln_tiles; i += 4) sm += st[2 * i];
+  sm += lbm_qkv::lane_xor1(sm);
+  sm += lbm_qkv::lane_xor2(sm);
+  const float mean = sm / (float)p.ln_tiles;
+  const float n_i = (float)p.K / (float)p.ln_tiles;
+  float m2 = 0.f;
+#pragma unroll
+  for (int i = 0; i < kLnHeld; ++i)
+    if (part + 4 * i < p.ln_tiles) {
+      const float d = held[i][0] - mean;
+      m2 += held[i][1] + n_i * d * d;
+    }
+  for (int i = part + 4 * kLnHeld; i < p.ln_tiles; i += 4) {
+    const float d = st[2 * i] - mean;
+    m2 += st[2 * i + 1] + n_i * d * d;
+  }
+  m2 += lbm_qkv::lane_xor1(m2);
+  m2 += lbm_qkv::lane_xor2(m2);
+  const float rstd = __builtin_amdgcn_rsqf(m2 / (float)p.K + p.ln_eps);
+  return f32x2{rstd, -mean * rstd};
+}
+
+// residual + branch, eight bf16 values
+__device__ __forceinline__ u32x4 add_rows(u32x4 x, u32x4 v) {
+  u32x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float s0 = bf16_bits_to_f32(x[e] & 0xffffu) + bf16_bits_to_f32(v[e] & 0xffffu);
+    const float s1 = bf16_bits_to_f32(x[e] >> 16) + bf16_bits_to_f32(v[e] >> 16);
+    o[e] = (unsigned)__builtin_bit_cast(unsigned short, (__bf16)s0) | ((unsigned)__builtin_bit_cast(unsigned short, (__bf16)s1) << 16);
+  }
+  return o;
+}
+
+// (mean, M2) of a row's stored values (v: this lane's eight, from column col on), 64 or 128 columns at a
+// time (shift 6 or 7): the 8 or 16 lanes that hold them are neighbours
+__device__ __forceinline__ void store_row_stats(const LinearArgs& p, u32x4 v, int row, int col, int shift, int lane) {
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    x[2 * e] = bf16_bits_to_f32(v[e] & 0xffffu);
+    x[2 * e + 1] = bf16_bits_to_f32(v[e] >> 16);
+  }
+  float sm = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+  sm = lbm_qkv::sum_of_8(sm);
+  if (shift == 7) sm += lbm_qkv::other_half_of_16(sm);
+  const float mean = sm * (shift == 7 ? 1.0f / 128 : 1.0f / 64);
+  float m2 = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) m2 += (x[e] - mean) * (x[e] - mean);
+  m2 = lbm_qkv::sum_of_8(m2);
+  if (shift == 7) m2 += lbm_qkv::other_half_of_16(m2);
+  if (row < p.M && (lane & ((1 << (shift - 3)) - 1)) == 0) {
+    float* so = p.stats_out + ((size_t)row * (p.N >> shift) + (col >> shift)) * 2;
+    so[0] = mean;
+    so[1] = m2;
+  }
+}
+
+// The pre-attention producer on eight consecutive columns of the projection's output, rounded to bf16 (raw):
+// the lanes of a (token, q|k|v, head) row of 64 are eight neighbours, exactly the producer's layout, so its
+// LayerNorm, rotary embedding and scatter run on the tile as it leaves instead of in a pass of their own
+// (lingbot_map/layers/attention.py:402-426, rope.py:438-461, flashinfer_cache.py:215-218).
+template <int ROPE>
+__device__ __forceinline__ void ask_rotary(const LinearArgs& p, int token, int c8, lbm_qkv::f32x4 (&cs)[4]) {
+  if (ROPE == 1) {
+    const lbm_qkv::f32x4* src = (const lbm_qkv::f32x4*)(p.rope_cs + ((long long)token * 32 + c8 * 4) * 2);
+    cs[0] = src[0]; cs[1] = src[1];
+  } else if (ROPE == 2) {
+    const lbm_qkv::f32x4* src = (const lbm_qkv::f32x4*)(p.rope_cs + ((long long)token * 64 + c8 * 8) * 2);
+    cs[0] = src[0]; cs[1] = src[1]; cs[2] = src[2]; cs[3] = src[3];
+  }
+}
+template <int ROPE, bool NORM>
+__device__ __forceinline__ bf16x8 produce_row(u32x4 raw, int which, int c8, const lbm_qkv::f32x4 (&w4)[2], const lbm_qkv::f32x4 (&b4)[2],
+                                              const lbm_qkv::f32x4 (&cs)[4], float eps, float post) {
+  bf16x8 o8 = __builtin_bit_cast(bf16x8, raw);   // v rows leave as they are
+  if (which < 2) {
+    // q and k rows: the row's last rounding is the conversion that packs it
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = __builtin_bit_cast(float, (i & 1) ? (raw[i >> 1] & 0xffff0000u) : (raw[i >> 1] << 16));
+    lbm_qkv::norm_rope_unrounded<0, ROPE, NORM>(x, w4, b4, cs, c8, eps, post);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) o8[i] = (__bf16)x[i];
+  }
+  return o8;
+}
+__device__ __forceinline__ unsigned short* produced_rows(const LinearArgs& p, int which) { return which == 0 ? p.out : (which == 1 ? p.k_out : p.v_out); }
+__device__ __forceinline__ void store_produced(const LinearArgs& p, unsigned short* plain, bf16x8 o8, int which, int token, int head, int c8, int pool_row) {
+  const int H = p.num_heads;
+  const long long nhd = ((long long)token * H + head) * 64 + c8 * 8;
+  if (plain) *(bf16x8*)(plain + nhd) = o8;
+  if (which > 0 && pool_row >= 0) {
+    const long long row_elems = (long long)H * 64;
+    const long long d = (long long)pool_row * row_elems + (which == 2 ? (long long)p.page_size * row_elems : 0) + head * 64 + c8 * 8;
+    *(bf16x8*)(p.pool + d) = o8;
+  }
+}
+
 // TN: output columns per tile (256, 128 or 64); a wavefront owns 64 x (TN / 2) of the tile.  Every
 // output element is the same sum in the same order whatever TN is: they give the same bits.
 // 256: bound by the multiply (a 64-wide step moves 48 KB for 1,024 cycles of MFMA, where 128 columns move 32 KB
-// for 512); three stages, and no ninth wavefront.
+// for 512); three stages, and no wavefronts beside the computing ones.
 // ROPE / NORM: rotary layout (0 none, 1 interleaved, 2 half-split) and qk-LayerNorm of the
 // kEpiQkvPrepare epilogue; 0 / false otherwise.
 // LNA: the activations' rows are standardised by the store (see LinearArgs).
@@ -259,31 +412,49 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
   const size_t k_first = SPLITK ? (size_t)split * nk * kKS : 0;
   const char* a_base = (const char*)(p.a + k_first);
   const char* w_base = (const char*)(p.w + (size_t)n0 * p.K + k_first);
-  if (wave >= kGThreads / 64) {   // (a scalar condition: the whole wavefront branches)
-    // The ninth wavefront holds no operand and joins no barrier (a wavefront that has ended is not
-    // waited for).  In a model every launch finds its weights in HBM - a frame walks through far
-    // more weight bytes than the caches hold - and the loop's three steps of look-ahead do not
-    // cover that latency: the same launch takes 0.6 to 5 us longer on weights that no cache holds.
-    // A caller that knows which memory the launch AFTER this one will read says so
-    // (lbm_linear_prefetch_hint), and these wavefronts, all workgroups' together, read one dword of
-    // every 128-byte line of it: the lines are then in the memory-side cache (or an L2) when that
-    // launch starts, having travelled while this one computed.
-    // (plain loads whose results the compiler sees - a load whose result it does not know of could
-    // land in a register it has reused: eight in flight per lane, their values folded into a word
-    // that is stored only under a condition that never holds)
-    unsigned folded = 0;
-    const unsigned stride = gridDim.x * 64u;
-    for (unsigned first = blockIdx.x * 64u + (unsigned)lane; first < p.touch_lines; first += 8u * stride) {
-      unsigned got[8];
+  constexpr bool kLoaders = TN != 256;
+  if (kLoaders && wave >= kGThreads / 64 && wave < kGThreads / 64 + kGLoadWaves) {
+    // A loading wavefront: every second KB - eight rows - of each step's operands.  The rows of a step are waited
+    // for before the barrier that the computing wavefronts read them behind, and asked for behind the one that
+    // frees their stage.  (M x N x K 1,004 x 3,072 x 1,024: 13.0 us with every wavefront loading its rows between
+    // its own MFMAs, 11.8 with these; 1,004 x 4,096 x 1,024 + GELU 14.7 -> 13.4; 4,016 x 1,024 x 4,096 35.6 -> 34.0.)
+    const int par = wave - kGThreads / 64, l8 = lane >> 3;
+    constexpr int kUnitsA = kGM / 16, kLoads = kUnitsA + TN / 16;
+    const unsigned chunk = (unsigned)(((lane & 7) ^ (4 * par + (lane >> 4))) * 8);   // rows 8 (2 u + par) + l8: bits 1 .. 3
+    unsigned off[kLoads];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const unsigned line = first + (unsigned)j * stride;
-        got[j] = line < p.touch_lines ? *(const unsigned*)(p.touch + (size_t)line * 128) : 0u;
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) folded ^= got[j];
+    for (int u = 0; u < kLoads; ++u) {
+      const int row = u < kUnitsA ? min(m0 + 8 * (2 * u + par) + l8, p.M - 1) : 8 * (2 * (u - kUnitsA) + par) + l8;
+      off[u] = ((unsigned)row * (unsigned)p.K + chunk) * 2u;
     }
-    if (folded == 0x5bd1e995u && p.M < 0) p.out[lane] = (unsigned short)folded;   // (M is never negative)
+    const unsigned lds_first = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned short*)&lds_ops[0]) + (unsigned)par * 1024u;
+    auto load_step = [&](int s) {
+      const unsigned st = (unsigned)(s % kStages);
+      const unsigned at_a = lds_first + st * (kGM * kKS * 2), at_w = lds_first + (kStages * kGM + st * TN) * (kKS * 2);
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u) {
+        const char* base = (u < kUnitsA ? a_base : w_base) + (size_t)s * (kKS * 2);
+        const unsigned at = u < kUnitsA ? at_a + u * 2048u : at_w + (u - kUnitsA) * 2048u;
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off[u]), "s"(base), "s"(at) : "memory", "m0");
+      }
+    };
+    __builtin_amdgcn_s_setprio(3);     // few instructions, and everybody waits for them
+#pragma unroll
+    for (int s = 0; s < kStages; ++s)
+      if (s < nk) load_step(s);
+    for (int s = -1; s < nk; ++s) {    // the barrier at the top of step s publishes the rows of step s + 1
+      const int behind = nk - 2 - s;   // steps asked for behind those
+      if (s < 0 && behind >= 3) LBM_DMA_WAIT(3 * kLoads);
+      else if (behind >= 2) LBM_DMA_WAIT(2 * kLoads);
+      else if (behind == 1) LBM_DMA_WAIT(kLoads);
+      else LBM_DMA_WAIT(0);
+      __builtin_amdgcn_s_barrier();
+      if (s >= 0 && s + kStages < nk) load_step(s + kStages);
+    }
+    return;
+  }
+  if (wave >= kGThreads / 64) {   // (a scalar condition: the whole wavefront branches)
+    touch_lines(p, lane);
     return;
   }
   // The loads are written as inline assembly: the compiler would otherwise wait for every
@@ -322,9 +493,7 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
                                     : m0_w + (unsigned)(stage * TN * kKS * 2 + 64 * (j - kPassA) * kKS * 2);
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(m0v) : "memory", "m0");
   };
-  // loads of this wavefront still allowed in flight: N (vmcnt(N); expcnt and lgkmcnt untouched)
   constexpr int kDmaPerStep = kPassA + kPassW;
-#define LBM_DMA_WAIT(N) __builtin_amdgcn_s_waitcnt(0x0F70 | ((N) & 15) | (((N) >> 4) << 14))
 
   f32x16 acc[NT][2];   // [column block of W][row block of A]; element i: column 8 (i / 4) + 4 g + i % 4, row n32
 #pragma unroll
@@ -364,19 +533,9 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
         acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[buf][k16][a], af[buf][k16][b], acc[a][b], 0, 0, 0);
   };
 
-  // LNA, row statistics: row r of the tile is handled by threads 4 r .. 4 r + 3, each taking every
-  // fourth (mean, M2) partial; equal-sized partials merge as mean = avg(mean_i),
-  // M2 = sum(M2_i) + n_i * sum((mean_i - mean)^2) (Chan et al.), variance = M2 / K.  The partials
-  // are asked for before the operand tiles (loads return in order) and merged while those travel.
-  constexpr int kLnHeld = 4;     // partials a thread keeps in registers (up to 16 column tiles)
+  // LNA, row statistics: row r of the tile is handled by threads 4 r .. 4 r + 3
   f32x2 ln_part[kLnHeld] = {};
-  const float* ln_st = nullptr;
-  if (LNA) {
-    ln_st = p.ln_stats + (size_t)min(m0 + (tid >> 2), p.M - 1) * p.ln_tiles * 2;
-#pragma unroll
-    for (int i = 0; i < kLnHeld; ++i)
-      if ((tid & 3) + 4 * i < p.ln_tiles) ln_part[i] = *(const f32x2*)(ln_st + 2 * ((tid & 3) + 4 * i));
-  }
+  if (LNA) ask_row_stats(p, min(m0 + (tid >> 2), p.M - 1), tid & 3, ln_part);
   // The per-column vectors of the epilogue (bias, column sums of w, LayerScale) are asked for now
   // and parked in LDS behind the first operand loads; the loop's barriers publish them.
   float cv_bias = 0.f, cv_sum = 0.f, cv_gamma = 1.f;
@@ -389,56 +548,28 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
   // for the first operand tile covers it and the barrier behind that wait publishes it) ...
   if (EPI == LBM_LINEAR_BIAS_GELU && tid < kGeluEntries / 8)
     dma_row((const char*)g_gelu_table, (unsigned)tid * 16u, &gelu_tab[wave * 512]);
-  // ... then three steps ahead: steps 0, 1, 2 on their way before anything else happens
+  // ... then the first steps of the tiles that load for themselves
 #pragma unroll
   for (int i = 0; i < kStages - 1; ++i)
-    if (i < nk) dma_step(i, i);
+    if (!kLoaders && i < nk) dma_step(i, i);
   if (tid < TN) {
     colvec[0][tid] = cv_bias;
     colvec[1][tid] = cv_sum;
     colvec[2][tid] = cv_gamma;
   }
-  if (LNA) {
-    const int r = tid >> 2, part = tid & 3;
-    float sm = 0.f;
-#pragma unroll
-    for (int i = 0; i < kLnHeld; ++i)
-      if (part + 4 * i < p.ln_tiles) sm += ln_part[i][0];
-    for (int i = part + 4 * kLnHeld; i < p.ln_tiles; i += 4) sm += ln_st[2 * i];
-    sm += lbm_qkv::lane_xor1(sm);
-    sm += lbm_qkv::lane_xor2(sm);
-    const float mean = sm / (float)p.ln_tiles;
-    const float n_i = (float)p.K / (float)p.ln_tiles;
-    float m2 = 0.f;
-#pragma unroll
-    for (int i = 0; i < kLnHeld; ++i)
-      if (part + 4 * i < p.ln_tiles) {
-        const float d = ln_part[i][0] - mean;
-        m2 += ln_part[i][1] + n_i * d * d;
-      }
-    for (int i = part + 4 * kLnHeld; i < p.ln_tiles; i += 4) {
-      const float d = ln_st[2 * i] - mean;
-      m2 += ln_st[2 * i + 1] + n_i * d * d;
-    }
-    m2 += lbm_qkv::lane_xor1(m2);
-    m2 += lbm_qkv::lane_xor2(m2);
-    const float rstd = __builtin_amdgcn_rsqf(m2 / (float)p.K + p.ln_eps);
-    if (part == 0) {
-      ln_rows[2 * r] = rstd;
-      ln_rows[2 * r + 1] = -mean * rstd;
-    }
-    // (read in the epilogue, many barriers from here)
+  if (LNA) {   // (read in the epilogue, many barriers from here)
+    const f32x2 row = merge_row_stats(p, min(m0 + (tid >> 2), p.M - 1), tid & 3, ln_part);
+    if ((tid & 3) == 0) *(f32x2*)&ln_rows[2 * (tid >> 2)] = row;
   }
-  // Step 0's fragments: its rows have landed (steps 1 and 2 may still be in flight), barrier, read.
-  if (kStages == 4 && 2 < nk) LBM_DMA_WAIT(2 * kDmaPerStep);
-  else LBM_DMA_WAIT(kDmaPerStep);
+  // Step 0's fragments: its rows have landed (later steps may still be in flight), barrier, read.
+  LBM_DMA_WAIT(kLoaders ? 0 : kDmaPerStep);   // (0: the GELU table)
   __syncthreads();
   read_step(0, 0);
-  if (kStages - 1 < nk) dma_step(kStages - 1, kStages - 1);
-  // Step s: wait until the rows of step s + 1 have landed (the loads of steps s + 2 and, with four
-  // stages, s + 3 may still be in flight), barrier (everyone's rows of step s + 1 are there, and everyone
+  if (!kLoaders && kStages - 1 < nk) dma_step(kStages - 1, kStages - 1);
+  // Step s: the rows of step s + 1 have landed (whoever loads them waits until only the loads of steps
+  // s + 2 and, with four stages, s + 3 are in flight), barrier (everyone's rows of step s + 1 are there, and everyone
   // holds the fragments of step s in registers, so its stage is free), then the MFMAs of step s with the
-  // fragment reads of step s + 1 in between, then the loads of step s + kStages into the freed stage.
+  // fragment reads of step s + 1 in between; the loads of step s + kStages go into the freed stage.
   static_assert(kStages == 4 || kStages == 3, "the waits below are written for a ring of three or four stages");
   constexpr int kUnroll = kStages == 4 ? 4 : 6;   // whole rounds of the ring and of the two fragment buffers
 #define LBM_SGB(mask, n) __builtin_amdgcn_sched_group_barrier(mask, n, 0)
@@ -447,12 +578,13 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
     for (int st = 0; st < kUnroll; ++st) {
       const int sidx = s0 + st;
       if (sidx < nk) {
-        if (kStages == 4 && sidx + 3 < nk) LBM_DMA_WAIT(2 * kDmaPerStep);
-        else if (sidx + 2 < nk) LBM_DMA_WAIT(kDmaPerStep);
-        else LBM_DMA_WAIT(0);
+        if (!kLoaders) {
+          if (sidx + 2 < nk) LBM_DMA_WAIT(kDmaPerStep);
+          else LBM_DMA_WAIT(0);
+        }
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
-        const bool more = sidx + kStages < nk;
+        const bool more = !kLoaders && sidx + kStages < nk;
 #pragma unroll
         for (int k16 = 0; k16 < 2; ++k16) {
           read_slice((st + 1) % kStages, (st + 1) & 1, k16);   // (past the last step: stale rows, never used)
@@ -516,13 +648,7 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
 #pragma unroll
     for (int j = 0; j < kPasses; ++j) {
       const int t = min(m0 + j * kRowsPerPass + tid / kPieces, p.M - 1);
-      if (ROPE == 1 && pq.which < 2) {
-        const qf4* cs = (const qf4*)(p.rope_cs + ((long long)t * 32 + pq.c8 * 4) * 2);
-        pq.cs4[j][0] = cs[0]; pq.cs4[j][1] = cs[1];
-      } else if (ROPE == 2 && pq.which < 2) {
-        const qf4* cs = (const qf4*)(p.rope_cs + ((long long)t * 64 + pq.c8 * 8) * 2);
-        pq.cs4[j][0] = cs[0]; pq.cs4[j][1] = cs[1]; pq.cs4[j][2] = cs[2]; pq.cs4[j][3] = cs[3];
-      }
+      if (pq.which < 2) ask_rotary<ROPE>(p, t, pq.c8, pq.cs4[j]);
       pq.pool_row[j] = -1;
       if (pq.which > 0 && p.append_rows) pq.pool_row[j] = p.append_rows[t];
     }
@@ -644,37 +770,14 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
   }
   __syncthreads();
   if (EPI == kEpiQkvPrepare) {
-    // The staged tile holds the projection's output rounded to bf16, 8 consecutive columns per
-    // thread: exactly the producer's layout (8 lanes per (token, q|k|v, head) row of 64), so its
-    // LayerNorm, rotary embedding and scatter run here instead of in a pass of their own
-    // (lingbot_map/layers/attention.py:402-426, rope.py:438-461, flashinfer_cache.py:215-218).
-    unsigned short* dst_plain = pq.which == 0 ? p.out : (pq.which == 1 ? p.k_out : p.v_out);
+    unsigned short* const plain = produced_rows(p, pq.which);
 #pragma unroll
     for (int j = 0; j < kPasses; ++j) {
       const int r = j * kRowsPerPass + tid / kPieces;
-      const bool valid = m0 + r < p.M;            // rows past M computed on the last token's entries, never stored
       const u32x2 lo = *(const u32x2*)&stage[r * kCStride + pq.c], hi = *(const u32x2*)&stage[r * kCStride + pq.c + 4];
-      const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
-      bf16x8 o8 = __builtin_bit_cast(bf16x8, raw);   // v rows leave as they are
-      if (pq.which < 2) {
-        // q and k rows: the row's last rounding is the conversion that packs it
-        float x[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = __builtin_bit_cast(float, (i & 1) ? (raw[i >> 1] & 0xffff0000u) : (raw[i >> 1] << 16));
-        lbm_qkv::norm_rope_unrounded<0, ROPE, NORM>(x, pq.w4, pq.b4, pq.cs4[j], pq.c8, p.eps, pq.which == 0 ? p.q_scale : 1.0f);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) o8[i] = (__bf16)x[i];
-      }
-      if (valid) {
-        const long long nhd = ((long long)(m0 + r) * H + pq.h) * 64 + pq.c8 * 8;
-        if (dst_plain) *(bf16x8*)(dst_plain + nhd) = o8;
-        if (pq.which > 0 && pq.pool_row[j] >= 0) {
-          const long long row_elems = (long long)H * 64;
-          const long long d = (long long)pq.pool_row[j] * row_elems + (pq.which == 2 ? (long long)p.page_size * row_elems : 0) +
-                              pq.h * 64 + pq.c8 * 8;
-          *(bf16x8*)(p.pool + d) = o8;
-        }
-      }
+      // (rows past M are computed on the last token's entries and never stored)
+      const bf16x8 o8 = produce_row<ROPE, NORM>(u32x4{lo[0], lo[1], hi[0], hi[1]}, pq.which, pq.c8, pq.w4, pq.b4, pq.cs4[j], p.eps, pq.which == 0 ? p.q_scale : 1.0f);
+      if (m0 + r < p.M) store_produced(p, plain, o8, pq.which, m0 + r, pq.h, pq.c8, pq.pool_row[j]);
     }
     return;
   }
@@ -687,47 +790,12 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
     u32x4 v = {lo[0], lo[1], hi[0], hi[1]};
     if (row < p.M) {
       unsigned short* dst = p.out + (size_t)row * p.N + n0 + c;
-      if (EPI == LBM_LINEAR_BIAS_RESIDUAL) {
-        const u32x4 x = res_v[j];
-        u32x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float s0 = bf16_bits_to_f32(x[e] & 0xffffu) + bf16_bits_to_f32(v[e] & 0xffffu);
-          const float s1 = bf16_bits_to_f32(x[e] >> 16) + bf16_bits_to_f32(v[e] >> 16);
-          o[e] = (unsigned)__builtin_bit_cast(unsigned short, (__bf16)s0) | ((unsigned)__builtin_bit_cast(unsigned short, (__bf16)s1) << 16);
-        }
-        v = o;
-      }
+      if (EPI == LBM_LINEAR_BIAS_RESIDUAL) v = add_rows(res_v[j], v);
       *(u32x4*)dst = v;
     }
-    if (EPI == LBM_LINEAR_BIAS_RESIDUAL && p.stats_out) {
-      // (mean, M2) of the row's stored values, 64 or 128 columns at a time: the 8 or 16 lanes that hold
-      // them are neighbours
-      const int shift = TN == 64 ? 6 : p.stats_shift;
-      float x[8];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        x[2 * e] = bf16_bits_to_f32(v[e] & 0xffffu);
-        x[2 * e + 1] = bf16_bits_to_f32(v[e] >> 16);
-      }
-      float sm = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
-      sm = lbm_qkv::sum_of_8(sm);
-      if (shift == 7) sm += lbm_qkv::other_half_of_16(sm);
-      const float mean = sm * (shift == 7 ? 1.0f / 128 : 1.0f / 64);
-      float m2 = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) m2 += (x[e] - mean) * (x[e] - mean);
-      m2 = lbm_qkv::sum_of_8(m2);
-      if (shift == 7) m2 += lbm_qkv::other_half_of_16(m2);
-      if (row < p.M && (tid & ((1 << (shift - 3)) - 1)) == 0) {
-        float* so = p.stats_out + ((size_t)row * (p.N >> shift) + ((n0 + c) >> shift)) * 2;
-        so[0] = mean;
-        so[1] = m2;
-      }
-    }
+    if (EPI == LBM_LINEAR_BIAS_RESIDUAL && p.stats_out) store_row_stats(p, v, row, n0 + c, TN == 64 ? 6 : p.stats_shift, tid);
   }
 }
-
 
 // ---------------------------------------------------------------------------- several streams' rows
 // The same product on 256 x 256 (or 192 x 256) tiles, for launches with enough rows to give most
@@ -956,13 +1024,7 @@ __global__ __launch_bounds__(kGThreads, 1) void lbm_linear_bf16_big_kernel(Linea
 #pragma unroll
     for (int j = 0; j < kGroup; ++j) {
       const int t = min(m0 + (grp * kGroup + j) * kRowsPerPass + pr, p.M - 1);
-      if (ROPE == 1 && which < 2) {
-        const qf4* src = (const qf4*)(p.rope_cs + ((long long)t * 32 + c8 * 4) * 2);
-        cs[j][0] = src[0]; cs[j][1] = src[1];
-      } else if (ROPE == 2 && which < 2) {
-        const qf4* src = (const qf4*)(p.rope_cs + ((long long)t * 64 + c8 * 8) * 2);
-        cs[j][0] = src[0]; cs[j][1] = src[1]; cs[j][2] = src[2]; cs[j][3] = src[3];
-      }
+      if (which < 2) ask_rotary<ROPE>(p, t, c8, cs[j]);
       rows[j] = -1;
       if (which > 0 && p.append_rows) rows[j] = p.append_rows[t];
     }
@@ -1010,34 +1072,15 @@ __global__ __launch_bounds__(kGThreads, 1) void lbm_linear_bf16_big_kernel(Linea
   if (EPI == kEpiQkvPrepare) {
     // the producer on the staged tile, as in the kernel above; the rotary entries and pool rows of
     // four passes are asked for while the four before them are worked on
-    unsigned short* dst_plain = which == 0 ? p.out : (which == 1 ? p.k_out : p.v_out);
+    unsigned short* const plain = produced_rows(p, which);
     const float post = which == 0 ? p.q_scale : 1.0f;
     auto work = [&](int grp, const qf4 (&cs)[kGroup][4], const int (&rows)[kGroup]) {
 #pragma unroll
       for (int j = 0; j < kGroup; ++j) {
         const int r = (grp * kGroup + j) * kRowsPerPass + pr;
-        const bool valid = m0 + r < p.M;
         const u32x2 lo = *(const u32x2*)&stage[r * kBCStride + pc], hi = *(const u32x2*)&stage[r * kBCStride + pc + 4];
-        const u32x4 raw = {lo[0], lo[1], hi[0], hi[1]};
-        bf16x8 o8 = __builtin_bit_cast(bf16x8, raw);   // v rows leave as they are
-        if (which < 2) {
-          // q and k rows: the row's last rounding is the conversion that packs it
-          float x[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) x[i] = __builtin_bit_cast(float, (i & 1) ? (raw[i >> 1] & 0xffff0000u) : (raw[i >> 1] << 16));
-          lbm_qkv::norm_rope_unrounded<0, ROPE, NORM>(x, w4, b4, cs[j], c8, p.eps, post);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) o8[i] = (__bf16)x[i];
-        }
-        if (valid) {
-          const long long nhd = ((long long)(m0 + r) * H + ph) * 64 + c8 * 8;
-          if (dst_plain) *(bf16x8*)(dst_plain + nhd) = o8;
-          if (which > 0 && rows[j] >= 0) {
-            const long long row_elems = (long long)H * 64;
-            const long long d = (long long)rows[j] * row_elems + (which == 2 ? (long long)p.page_size * row_elems : 0) + ph * 64 + c8 * 8;
-            *(bf16x8*)(p.pool + d) = o8;
-          }
-        }
+        const bf16x8 o8 = produce_row<ROPE, NORM>(u32x4{lo[0], lo[1], hi[0], hi[1]}, which, c8, w4, b4, cs[j], p.eps, post);
+        if (m0 + r < p.M) store_produced(p, plain, o8, which, m0 + r, ph, c8, rows[j]);
       }
     };
 #pragma unroll
@@ -1205,7 +1248,7 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
   lbm_take_prefetch_hint(p);
   if (int rc = lbm_set_row_norm(p, a_norm, "lbm_linear_norm")) return rc;
   const bool lna = a_norm != nullptr;
-  const dim3 block(kGThreads), block_s(kGThreads + kGTouchThreads);
+  const dim3 block(kGThreads), block_s(lbm_linear_threads(128));
   if (epilogue == LBM_LINEAR_BIAS || epilogue == LBM_LINEAR_BIAS_GELU) {
     if (const int bm = lbm_linear_big_tiles(p)) {
       const dim3 grid_b((unsigned)(p.m_tiles * p.n_tiles));
@@ -1312,7 +1355,7 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
     wide = false;
     p.n_tiles = N / 64;
   }
-  const dim3 grid((unsigned)(p.m_tiles * p.n_tiles)), block(kGThreads + kGTouchThreads);
+  const dim3 grid((unsigned)(p.m_tiles * p.n_tiles)), block(lbm_linear_threads(128));
 #define LBM_QKV_LAUNCH_L(R, NRM, L)                                                                                   \
   {                                                                                                                   \
     if (wide) hipLaunchKernelGGL((lbm_linear_bf16_kernel<kEpiQkvPrepare, 128, R, NRM, L>), grid, block, 0, stream, p); \
