@@ -245,9 +245,9 @@ int32_t lbm_linear_stats_tiles(int32_t M, int32_t N);
 /* lbm_linear with a_norm (NULL = none; not with the residual epilogue) applied to the
  * activations and / or out_stats (NULL = none; residual epilogue only) written.
  * workspace (NULL = none): device memory of at least lbm_linear_workspace_bytes(M, N, K, epilogue)
- * bytes that lets a launch with few tiles and a long K (fc2 of one frame: 128 tiles, K = 4096)
- * put several workgroups on each tile, each over a slice of K; the one that finishes a tile last
- * sums the slices in a fixed order, so results do not depend on timing.  The first 512 bytes
+ * bytes with which a launch with few tiles and a long K (fc2 of one frame: K = 4096) sums K in two
+ * or four slices that it adds in a fixed order, so results do not depend on timing: up to K = 4096 within a
+ * workgroup, beyond with several workgroups per tile that meet in the workspace.  The first 512 bytes
  * of the workspace hold one counter per tile, for every shape: the caller zero-fills the workspace
  * once, every launch leaves the counters at zero, and launches of different shapes may share it.  Launches that overlap in time on one GPU need
  * workspaces of their own, and with a workspace the residual may not alias out. */

@@ -17,11 +17,13 @@
 //     affine part folded into w and bias by the caller (block.py:194-195, 217; the normalised rows
 //     are then never rounded to bf16, the folded weights are);
 //   * the qkv projection can carry the pre-attention producer as its epilogue (kEpiQkvPrepare);
-//   * a launch with few tiles and a long K can put several workgroups on a tile (SPLITK).
+//   * a launch with few tiles and a long K can sum K in slices, by several workgroups per tile (SPLITK)
+//     or by one (the KS of the small tiles).
 //
 // Shapes this is written for: M about 1,000 rows per stream (one frame), K, N in 1024 .. 4096.
 // At that size a launch has only a few hundred tiles and 16-64 k-steps, so what counts is a
-// tile count that matches the 256 CUs and a short prologue, not asymptotic throughput.
+// tile count that matches the 256 CUs and a short prologue, not asymptotic throughput.  Three kernels: the
+// one described here; smaller tiles for fewer rows and larger ones for more stand below with what differs.
 //
 // One workgroup = 8 wavefronts on a 128 x 128 tile of the output (TN = 64: 128 x 64, 256: 128 x 256).  The product
 // is computed transposed, C^T = W A^T with v_mfma_f32_32x32x16_bf16 (A operand = 32 rows of W, B
@@ -66,6 +68,7 @@ constexpr int kGLoadWaves = 2;       // wavefronts that load the operands
 constexpr int kGTouchThreads = 64;   // and one that only asks for the next launch's lines
 // (256 columns: the accumulators leave no registers for a third wavefront per SIMD)
 constexpr int lbm_linear_threads(int tn) { return kGThreads + (tn == 256 ? 0 : kGLoadWaves * 64 + kGTouchThreads); }
+constexpr int lbm_rows_threads(int tm) { return tm / 32 * 4 * 64 + (kGLoadWaves * 64 + kGTouchThreads); }   // lbm_linear_bf16_rows_kernel
 constexpr int kKS = 64;          // K elements per LDS stage
 constexpr int kStagesG = 4;      // LDS stages: three being loaded while one is multiplied (six stages for the 64-column tile,
                                  // which has the room: slower, 8.4 -> 8.8 us for proj - the longer prologue costs more than the depth gains)
@@ -104,7 +107,7 @@ struct LinearArgs {
   // [M][N >> stats_shift][2], or null
   float* stats_out;
   int stats_shift;               // 6 or 7; 6 where the tiles have 64 columns
-  // SPLITK kernels: k_splits workgroups share a tile, each over its own slice of K.  Every one
+  // K summed in k_splits slices.  SPLITK kernels: k_splits workgroups share a tile, each over its own slice.  Every one
   // parks its fp32 partial tile in `split_part` and takes a ticket from the tile's counter; the
   // one that draws the last ticket sums the partials in slice order (the same sum whoever is
   // last) and runs the epilogue.  Counters start at zero and are left at zero.
@@ -126,7 +129,7 @@ __device__ __forceinline__ float bf16_bits_to_f32(unsigned v) { return __builtin
 // instead it is tabulated for |v| in [2^-12, 2^3) - 15 binades x 128 mantissas x 2 signs, 7.5 KB,
 // exact values rounded once (gen_gelu_table.py) - and each workgroup pulls the table into LDS with
 // one 16-byte LDS-direct load per thread, ahead of its first operand tiles, and looks the
-// elements up, sixteen per lane at a time (gelu_of_16), so that their lookups overlap.
+// elements up, sixteen per lane at a time (gelu_of), so that their lookups overlap.
 // Outside the table the function has closed forms that agree with torch's fp32 evaluation
 // after the rounding to bf16: below 2^-12, 1 + erf differs from 1 by less than 2^-12 and
 // v / 2 is the nearest bf16 value (zeros and denormals included); from 8 up erff is exactly
@@ -146,11 +149,12 @@ static __device__ __attribute__((aligned(16))) const unsigned short g_gelu_table
 // that hold such a value - ten vector instructions per element where one value at a time took 21 (fc1 of
 // 8,040 rows 78.0 -> 75.7 us, 4,016 rows 38.9 -> 37.9, 1,004 rows 14.7 -> 14.5; what is left of the 8 us
 // that GELU costs a 256 x 256 tile is the lookups' bank conflicts).
-__device__ __forceinline__ void gelu_of_16(const f32x4 (&x)[4], const unsigned short* tab, bf16x4 (&y)[4]) {
+template <int C>
+__device__ __forceinline__ void gelu_of(const f32x4 (&x)[C], const unsigned short* tab, bf16x4 (&y)[C]) {
   const u16x2 lo = (unsigned short)(kGeluE0 << 7), hi = (unsigned short)((kGeluE0 << 7) + kGeluHalf - 1);
-  u16x2 in[8], out[8], beyond = {0, 0};
+  u16x2 in[2 * C], out[2 * C], beyond = {0, 0};
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
+  for (int i = 0; i < 2 * C; ++i) {
     unsigned pair = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x[i >> 1][(i & 1) * 2], x[i >> 1][(i & 1) * 2 + 1]}, bf16x2));
     asm("" : "+v"(pair));   // (or the signs are taken from x, one compare and one select each)
     in[i] = __builtin_bit_cast(u16x2, pair);
@@ -164,7 +168,7 @@ __device__ __forceinline__ void gelu_of_16(const f32x4 (&x)[4], const unsigned s
   if (__builtin_amdgcn_ballot_w64(__builtin_bit_cast(unsigned, beyond) != 0u)) {
     // outside the table: v / 2 below it, v or v * 0 above it (see kGeluE0)
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 2 * C; ++i)
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
         const unsigned b16 = in[i][e], mag = b16 & 0x7fffu;
@@ -174,7 +178,7 @@ __device__ __forceinline__ void gelu_of_16(const f32x4 (&x)[4], const unsigned s
       }
   }
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
+  for (int c = 0; c < C; ++c)
     y[c] = __builtin_bit_cast(bf16x4, u32x2{__builtin_bit_cast(unsigned, out[2 * c]), __builtin_bit_cast(unsigned, out[2 * c + 1])});
 }
 
@@ -763,7 +767,7 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
       }
       y[c4] = __builtin_convertvector(x[c4], bf16x4);
     }
-    if (EPI == LBM_LINEAR_BIAS_GELU) gelu_of_16(x, gelu_tab, y);
+    if (EPI == LBM_LINEAR_BIAS_GELU) gelu_of<4>(x, gelu_tab, y);
 #pragma unroll
     for (int c4 = 0; c4 < 4; ++c4)
       *(bf16x4*)&stage[(wm + b * 32 + n32) * kCStride + wn + a * 32 + c4 * 8 + g * 4] = y[c4];
@@ -795,6 +799,231 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
     }
     if (EPI == LBM_LINEAR_BIAS_RESIDUAL && p.stats_out) store_row_stats(p, v, row, n0 + c, TN == 64 ? 6 : p.stats_shift, tid);
   }
+}
+
+// ---------------------------------------------------------------------------- few rows
+// The same product on tiles of 64 columns x 64 or 32 rows, for launches whose 128-row tiles would leave CUs idle
+// (a small image's 261 rows into 1,024 columns: 48 of 256) or share a tile between workgroups that meet in memory.
+// Bound by the fill: a step moves (TM + 64) x 128 bytes through a CU's 64 bytes per cycle for TM x 64 x 64
+// multiplications, a half to a quarter of that time on the matrix pipe, so what counts is how many CUs share the
+// rows, and how little stands around the loop.  A wavefront owns a 32 x 32 block of the tile over its half of
+// every 64-wide slice of K - the sums of the 128-row tiles, in their order: the same bits - and two others load, a
+// 64-wide half each of 128-wide steps (half the barriers), three steps ahead.  Everything the store needs is asked
+// for before the loop.  KS: the launches that sum K in slices (LinearArgs::k_splits) keep KS pairs of sums, one
+// slice behind the other, and add them in slice order at the end: the bits of several workgroups that
+// meet in memory, without the meeting (5 us of an fc2 launch).
+// us per launch, weights rotating through 24 layers, before (128 x 64 tiles) and after: M x N x K 81 x 3,072 x
+// 1,024 with the producer 9.4 -> 6.3, 261 rows 10.1 -> 7.7; 261 x 1,024 x 1,024 8.1 -> 5.2, 1,004 rows 8.4 -> 6.6;
+// 261 x 1,024 x 4,096 12.3 -> 11.2, 512 rows 14.6 -> 11.9, 1,004 rows 18.1 -> 15.5.  (Six stages instead of four: no
+// faster.  What the last are bound by is L2: 256 CUs x 87 bytes per ns against 92 of a bare copy of such rows.)
+template <int EPI, int TM, int KS = 1, int ROPE = 0, bool NORM = false, bool LNA = false>
+__global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_kernel(LinearArgs p) {
+  constexpr int kWaves = TM / 32 * 4;                      // computing wavefronts: (TM / 32) x 2 blocks of 32 x 32, two halves of K each
+  constexpr int kHalf = (TM + 64) * kKS;                   // elements of one 64-wide half of a stage: rows of a, then of w
+  constexpr int kStage = 2 * kHalf;
+  constexpr int kStages = 4;
+  __shared__ __attribute__((aligned(1024))) unsigned short ops[kStages * kStage];
+  __shared__ __attribute__((aligned(16))) unsigned short gelu_tab[EPI == LBM_LINEAR_BIAS_GELU ? kGeluEntries : 8];
+  __shared__ __attribute__((aligned(8))) float ln_rows[LNA ? TM * 2 : 2];                   // per row: rstd, -mean * rstd
+  __shared__ __attribute__((aligned(16))) float colvec[3][64];                              // bias, column sums of w (LNA), LayerScale
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int mt, nt;
+  lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt);
+  const int m0 = mt * TM, n0 = nt * 64;
+  const int nk = p.K / (2 * kKS);                          // 128-wide steps
+
+  if (wave >= kWaves) {
+    if (wave == kWaves + 2) {
+      touch_lines(p, lane);
+      return;
+    }
+    // A loading wavefront, as in the kernel above: one 64-wide half of every step, eight whole rows per load.
+    const int half = wave - kWaves;
+    constexpr int kUnitsA = TM / 8, kUnitsW = 8, kLoads = kUnitsA + kUnitsW;
+    const int l8 = lane >> 3, chunk = (lane & 7) ^ (lane >> 4);
+    unsigned off[kLoads];
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int row = u < kUnitsA ? min(m0 + 8 * u + l8, p.M - 1) : 8 * (u - kUnitsA) + l8;   // rows past M re-read the last row
+      off[u] = ((unsigned)row * (unsigned)p.K + (unsigned)(chunk ^ (4 * (u & 1))) * 8u) * 2u;
+    }
+    const char* a_base = (const char*)(p.a + half * kKS);
+    const char* w_base = (const char*)(p.w + (size_t)n0 * p.K + half * kKS);
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned short*)&ops[0]) + (unsigned)(half * kHalf * 2);
+    auto load_step = [&](int s) {
+      const unsigned st = lds0 + (unsigned)(s % kStages) * (kStage * 2);
+      const size_t at = (size_t)s * (2 * kKS * 2);
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u) {
+        const char* base = (u < kUnitsA ? a_base : w_base) + at;
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off[u]), "s"(base), "s"(st + u * 1024u) : "memory", "m0");
+      }
+    };
+    __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+    for (int i = 0; i < kStages - 1; ++i)
+      if (i < nk) load_step(i);
+    for (int s = -1; s < nk - 1; ++s) {   // the barrier at the top of step s publishes the rows of step s + 1
+      const int behind = nk - 2 - s;      // steps that may be in flight behind those
+      if (behind >= 2) LBM_DMA_WAIT(2 * kLoads);
+      else if (behind == 1) LBM_DMA_WAIT(kLoads);
+      else LBM_DMA_WAIT(0);
+      __builtin_amdgcn_s_barrier();
+      if (s + kStages < nk) load_step(s + kStages);
+    }
+    return;
+  }
+
+  // ---- computing wavefronts
+  const int n32 = lane & 31, g = lane >> 5;
+  const int kh = wave & 1, sub = wave >> 1;
+  const int wm = (sub >> 1) * 32, wn = (sub & 1) * 32;
+  const int r = tid >> 3, c8 = tid & 7;                    // the row and the piece of it that this thread stores
+  const int row = m0 + r, row_held = min(row, p.M - 1);
+  // everything the store will need is asked for before the first step
+  if (EPI == LBM_LINEAR_BIAS_GELU) {
+#pragma unroll
+    for (int i = 0; i < (kGeluEntries / 8 + kWaves * 64 - 1) / (kWaves * 64); ++i) {
+      const int at = i * kWaves * 64 + tid;
+      const unsigned m0v = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned short*)&gelu_tab[0] + (unsigned)(i * kWaves + wave) * 1024u);
+      if (at < kGeluEntries / 8)
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"((unsigned)at * 16u), "s"((const char*)g_gelu_table), "s"(m0v) : "memory", "m0");
+    }
+  }
+  f32x2 ln_part[kLnHeld] = {};
+  const bool ln_lane = LNA && tid < TM * 4;
+  if (ln_lane) ask_row_stats(p, min(m0 + (tid >> 2), p.M - 1), tid & 3, ln_part);
+  // (one value per thread: the vectors need not be aligned)
+  float cv = 0.f;
+  if (wave == 0 && p.bias) cv = p.bias[n0 + lane];
+  if (LNA && wave == 1) cv = p.ln_colsum[n0 + lane];
+  if (EPI == LBM_LINEAR_BIAS_RESIDUAL && wave == 2 && p.gamma) cv = p.gamma[n0 + lane];
+  u32x4 res = {};
+  if (EPI == LBM_LINEAR_BIAS_RESIDUAL) res = *(const u32x4*)(p.res + (size_t)row_held * p.N + n0 + c8 * 8);
+  lbm_qkv::f32x4 w4[2] = {}, b4[2] = {}, cs4[4] = {};
+  int which = 0, head = 0, pool_row = -1;
+  if (EPI == kEpiQkvPrepare) {
+    which = n0 / (p.num_heads * 64);
+    head = nt - which * p.num_heads;
+    if (NORM && which < 2) {
+      const lbm_qkv::f32x4* wp = (const lbm_qkv::f32x4*)((which == 0 ? p.q_norm_w : p.k_norm_w) + c8 * 8);
+      const lbm_qkv::f32x4* bp = (const lbm_qkv::f32x4*)((which == 0 ? p.q_norm_b : p.k_norm_b) + c8 * 8);
+      w4[0] = wp[0]; w4[1] = wp[1];
+      b4[0] = bp[0]; b4[1] = bp[1];
+    }
+    if (which < 2) ask_rotary<ROPE>(p, row_held, c8, cs4);
+    else if (p.append_rows) pool_row = p.append_rows[row_held];
+    if (which == 1 && p.append_rows) pool_row = p.append_rows[row_held];
+  }
+  if (ln_lane) {
+    const f32x2 st = merge_row_stats(p, min(m0 + (tid >> 2), p.M - 1), tid & 3, ln_part);
+    if ((tid & 3) == 0) *(f32x2*)&ln_rows[2 * (tid >> 2)] = st;
+  }
+  if (wave < 3) colvec[wave][lane] = cv;
+
+  // fragments: row n32 of the block (the second half of K takes its columns of w with the halves of 16 swapped,
+  // so that registers 0 .. 7 of either sum are the columns that its wavefront finishes)
+  const int sw = (n32 >> 1) & 7;
+  const unsigned short* fa = ops + (wm + n32) * kKS;
+  const unsigned short* fw = ops + (TM + wn + (n32 ^ (kh * 16))) * kKS;
+  int pos[2];
+#pragma unroll
+  for (int k16 = 0; k16 < 2; ++k16) pos[k16] = ((kh * 4 + k16 * 2 + g) ^ sw) * 8;
+  bf16x8 wf[2][4], af[2][4];
+  int stage_at = 0;          // elements to the stage that is read next
+  auto read_step = [&](int buf) {
+    const int stage = stage_at;
+    stage_at = stage_at == (kStages - 1) * kStage ? 0 : stage_at + kStage;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int at = stage + (i >> 1) * kHalf + pos[i & 1];
+      wf[buf][i] = __builtin_bit_cast(bf16x8, *(const u32x4*)(fw + at));
+      af[buf][i] = __builtin_bit_cast(bf16x8, *(const u32x4*)(fa + at));
+    }
+  };
+  f32x16 part[KS];
+#pragma unroll
+  for (int j = 0; j < KS; ++j)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) part[j][i] = 0.f;
+  auto step_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  step_barrier();
+  read_step(0);
+  const int seg = nk / KS;
+#pragma unroll
+  for (int j = 0; j < KS; ++j) {
+    for (int s0 = 0; s0 < seg; s0 += 2) {
+#pragma unroll
+      for (int st = 0; st < 2; ++st) {
+        if (KS > 1 || s0 + st < seg) {          // (several sums: of an even number of steps each)
+          if (j * seg + s0 + st + 1 < nk) {
+            step_barrier();
+            read_step(st ^ 1);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) part[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[st][i], af[st][i], part[j], 0, 0, 0);
+        }
+      }
+    }
+  }
+  LBM_DMA_WAIT(0);     // (the GELU table)
+  step_barrier();      // everyone is done with the operands
+  // ---- the two halves of K meet
+  float* xch = (float*)&ops[0];              // [wave][KS][2][64 lanes][4]
+  static_assert(kWaves * KS * 2 * 64 * 16 <= kStage * 2 * 2, "the exchanged sums fit the first two stages");
+#pragma unroll
+  for (int j = 0; j < KS; ++j)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) *(f32x4*)&xch[(((wave * KS + j) * 2 + c) * 64 + lane) * 4] = f32x4{part[j][8 + 4 * c], part[j][9 + 4 * c], part[j][10 + 4 * c], part[j][11 + 4 * c]};
+  step_barrier();
+  f32x4 fin[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+#pragma unroll
+    for (int j = 0; j < KS; ++j) {
+      const f32x4 got = *(const f32x4*)&xch[((((wave ^ 1) * KS + j) * 2 + c) * 64 + lane) * 4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float both = part[j][4 * c + e] + got[e];
+        fin[c][e] = j > 0 ? fin[c][e] + both : (KS > 2 ? 0.f + both : both);
+      }
+    }
+  }
+  // ---- epilogue
+  constexpr int kCStride = 64 + 4;
+  unsigned short* stage = &ops[2 * kStage];
+  f32x2 row_f = {1.f, 0.f};
+  if (LNA) row_f = *(const f32x2*)&ln_rows[2 * (wm + n32)];
+  f32x4 x[2];
+  bf16x4 y[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int col = wn + kh * 16 + c * 8 + g * 4;
+    const f32x4 bias4 = *(const f32x4*)&colvec[0][col], colsum4 = *(const f32x4*)&colvec[1][col], gamma4 = *(const f32x4*)&colvec[2][col];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float lin = fin[c][e];
+      if (LNA) lin = __builtin_fmaf(lin, row_f[0], row_f[1] * colsum4[e]);
+      x[c][e] = lin + bias4[e];
+      if (EPI == LBM_LINEAR_BIAS_RESIDUAL && p.gamma) x[c][e] = round_bf16(x[c][e]) * gamma4[e];
+    }
+    y[c] = __builtin_convertvector(x[c], bf16x4);
+  }
+  if (EPI == LBM_LINEAR_BIAS_GELU) gelu_of<2>(x, gelu_tab, y);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) *(bf16x4*)&stage[(wm + n32) * kCStride + wn + kh * 16 + c * 8 + g * 4] = y[c];
+  step_barrier();
+  const u32x2 lo = *(const u32x2*)&stage[r * kCStride + c8 * 8], hi = *(const u32x2*)&stage[r * kCStride + c8 * 8 + 4];
+  u32x4 v = {lo[0], lo[1], hi[0], hi[1]};
+  if (EPI == kEpiQkvPrepare) {
+    const bf16x8 o8 = produce_row<ROPE, NORM>(v, which, c8, w4, b4, cs4, p.eps, which == 0 ? p.q_scale : 1.0f);
+    if (row < p.M) store_produced(p, produced_rows(p, which), o8, which, row, head, c8, pool_row);
+    return;
+  }
+  if (EPI == LBM_LINEAR_BIAS_RESIDUAL) v = add_rows(res, v);
+  if (row < p.M) *(u32x4*)(p.out + (size_t)row * p.N + n0 + c8 * 8) = v;
+  if (EPI == LBM_LINEAR_BIAS_RESIDUAL && p.stats_out) store_row_stats(p, v, row, n0 + c8 * 8, 6, tid);
 }
 
 // ---------------------------------------------------------------------------- several streams' rows
@@ -1063,7 +1292,7 @@ __global__ __launch_bounds__(kGThreads, 1) void lbm_linear_bf16_big_kernel(Linea
         }
         y[c4] = __builtin_convertvector(x[c4], bf16x4);
       }
-      if (EPI == LBM_LINEAR_BIAS_GELU) gelu_of_16(x, gelu_tab, y);
+      if (EPI == LBM_LINEAR_BIAS_GELU) gelu_of<4>(x, gelu_tab, y);
 #pragma unroll
       for (int c4 = 0; c4 < 4; ++c4) *(bf16x4*)&stage[row * kBCStride + wn + a * 32 + c4 * 8 + g * 4] = y[c4];
     }
@@ -1112,6 +1341,23 @@ int lbm_linear_tiles(LinearArgs& p) {
   // (a width of its own, so that the next launch's LayerNorm sums the same values whatever tile made them)
   p.stats_shift = p.N % 128 == 0 && tiles >= 160 ? 7 : 6;
   return tn;
+}
+// 64 or 32 rows per tile of 64 columns in the place of 128 x tn tiles where they need fewer rounds of the CUs x
+// bytes per step (the fill is what bounds either), or 0; sets the row tiles.  With K summed in slices one workgroup
+// walks them all: up to K = 4,096 that is the faster way (M x N x K 31 x 1,024 x 4,096: 10.5 -> 10.4 us,
+// 1,004 rows 17.3 -> 15.6), from there on several workgroups are (512 x 768 x 6,144: 15.4 against 16.2; 81 x
+// 1,024 x 8,192: 13.9 against 18.2); slices of an odd number of 128-wide steps go there too.
+int lbm_linear_rows_tiles(LinearArgs& p, int tn, int splits) {
+  if (tn != 64 || (splits > 1 && (p.K > 4096 || p.K % (splits * 4 * kKS) != 0))) return 0;
+  const int nt = p.N / 64;
+  int best = 0;
+  long long best_cost = ((long long)p.m_tiles * nt + 255) / 256 * (128 + 64);
+  for (int tm : {64, 32}) {
+    const long long cost = ((long long)((p.M + tm - 1) / tm) * nt + 255) / 256 * (tm + 64);
+    if (cost < best_cost) best = tm, best_cost = cost;
+  }
+  if (best) p.m_tiles = (p.M + best - 1) / best;
+  return best;
 }
 // 256 columns where that halves the rounds of the 256 CUs; sets the tile count.  A round of 128 x 256 tiles
 // takes 1.35-1.4 rounds of 128 x 128, so two for one gain (M x N x K 8,040 x 1,024 x 4,096: 61 us against
@@ -1266,19 +1512,35 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
     }
   }
   const bool wide = lbm_linear_tiles(p) == 128;
-  if (workspace) {
-    const int splits = lbm_linear_splits(p, epilogue);
-    if (splits > 1 && workspace_bytes >= lbm_linear_workspace_for(M, N, K, epilogue)) {
-      if (residual == out)   // a workgroup that is not the tile's last would see the other's store
-        return lbm_fail(LBM_ERR_INVALID, "lbm_linear_norm: with a workspace the residual may not alias out");
-      p.k_splits = splits;
-      p.split_counters = (unsigned*)workspace;
-      p.split_part = (float*)((char*)workspace + kSplitCounterBytes);
-      const dim3 grid_s((unsigned)(p.m_tiles * p.n_tiles * splits));
-      // (128 tiles at most, so they have 64 columns)
-      hipLaunchKernelGGL((lbm_linear_bf16_kernel<LBM_LINEAR_BIAS_RESIDUAL, 64, 0, false, false, true>), grid_s, block_s, 0, stream, p);
-      return lbm_check_launch("lbm_linear_bf16_kernel<split K>");
-    }
+  const int splits = workspace && workspace_bytes >= lbm_linear_workspace_for(M, N, K, epilogue) ? lbm_linear_splits(p, epilogue) : 1;
+  if (splits > 1 && residual == out)   // a workgroup that is not the tile's last would see the other's store
+    return lbm_fail(LBM_ERR_INVALID, "lbm_linear_norm: with a workspace the residual may not alias out");
+  if (const int tm = lbm_linear_rows_tiles(p, wide ? 128 : 64, splits)) {
+    const dim3 grid_r((unsigned)(p.m_tiles * p.n_tiles)), block_r(lbm_rows_threads(tm));
+#define LBM_ROWS_LAUNCH(E, S, L)                                                                                                \
+  {                                                                                                                             \
+    if (tm == 64) hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<E, 64, S, 0, false, L>), grid_r, block_r, 0, stream, p);       \
+    else hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<E, 32, S, 0, false, L>), grid_r, block_r, 0, stream, p);                \
+  }
+    if (epilogue == LBM_LINEAR_BIAS && lna) LBM_ROWS_LAUNCH(LBM_LINEAR_BIAS, 1, true)
+    else if (epilogue == LBM_LINEAR_BIAS) LBM_ROWS_LAUNCH(LBM_LINEAR_BIAS, 1, false)
+    else if (epilogue == LBM_LINEAR_BIAS_GELU && lna) LBM_ROWS_LAUNCH(LBM_LINEAR_BIAS_GELU, 1, true)
+    else if (epilogue == LBM_LINEAR_BIAS_GELU) LBM_ROWS_LAUNCH(LBM_LINEAR_BIAS_GELU, 1, false)
+    else if (epilogue == LBM_LINEAR_BIAS_RESIDUAL && splits == 1) LBM_ROWS_LAUNCH(LBM_LINEAR_BIAS_RESIDUAL, 1, false)
+    else if (epilogue == LBM_LINEAR_BIAS_RESIDUAL && splits == 2) LBM_ROWS_LAUNCH(LBM_LINEAR_BIAS_RESIDUAL, 2, false)
+    else if (epilogue == LBM_LINEAR_BIAS_RESIDUAL) LBM_ROWS_LAUNCH(LBM_LINEAR_BIAS_RESIDUAL, 4, false)
+    else return lbm_fail(LBM_ERR_INVALID, "lbm_linear: unknown epilogue %d", epilogue);
+#undef LBM_ROWS_LAUNCH
+    return lbm_check_launch("lbm_linear_bf16_rows_kernel");
+  }
+  if (splits > 1) {
+    p.k_splits = splits;
+    p.split_counters = (unsigned*)workspace;
+    p.split_part = (float*)((char*)workspace + kSplitCounterBytes);
+    const dim3 grid_s((unsigned)(p.m_tiles * p.n_tiles * splits));
+    // (128 tiles at most, so they have 64 columns)
+    hipLaunchKernelGGL((lbm_linear_bf16_kernel<LBM_LINEAR_BIAS_RESIDUAL, 64, 0, false, false, true>), grid_s, block_s, 0, stream, p);
+    return lbm_check_launch("lbm_linear_bf16_kernel<split K>");
   }
   const bool wider = wide && lbm_linear_wider(p);
   const dim3 grid((unsigned)(p.m_tiles * p.n_tiles));
@@ -1354,6 +1616,27 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
   if (wide && (num_heads & 1)) {
     wide = false;
     p.n_tiles = N / 64;
+  }
+  if (const int tm = lbm_linear_rows_tiles(p, wide ? 128 : 64, 1)) {
+    const dim3 grid_r((unsigned)(p.m_tiles * p.n_tiles)), block_r(lbm_rows_threads(tm));
+#define LBM_QKV_ROWS_T(T, R, NRM)                                                                                                       \
+  {                                                                                                                                     \
+    if (lna) hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<kEpiQkvPrepare, T, 1, R, NRM, true>), grid_r, block_r, 0, stream, p);       \
+    else hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<kEpiQkvPrepare, T, 1, R, NRM, false>), grid_r, block_r, 0, stream, p);          \
+  }
+#define LBM_QKV_ROWS(R, NRM)                                                       \
+  {                                                                                \
+    if (tm == 64) LBM_QKV_ROWS_T(64, R, NRM) else LBM_QKV_ROWS_T(32, R, NRM)       \
+  }
+    if (rope == 0 && !norm) LBM_QKV_ROWS(0, false)
+    else if (rope == 0) LBM_QKV_ROWS(0, true)
+    else if (rope == 1 && !norm) LBM_QKV_ROWS(1, false)
+    else if (rope == 1) LBM_QKV_ROWS(1, true)
+    else if (!norm) LBM_QKV_ROWS(2, false)
+    else LBM_QKV_ROWS(2, true)
+#undef LBM_QKV_ROWS
+#undef LBM_QKV_ROWS_T
+    return lbm_check_launch("lbm_linear_bf16_rows_kernel<qkv prepare>");
   }
   const dim3 grid((unsigned)(p.m_tiles * p.n_tiles)), block(lbm_linear_threads(128));
 #define LBM_QKV_LAUNCH_L(R, NRM, L)                                                                                   \

@@ -515,3 +515,49 @@ def test_k_split_launches_of_two_shapes_share_one_workspace():
         torch.cuda.synchronize()
         check(out.cpu(), ref, scale=torch.maximum(res.float().abs(), (ref.float() - res.float()).abs()), bar=2.0 ** -6)
     assert ws[:512].abs().sum().item() == 0
+
+
+@pytest.mark.parametrize("M", [1, 31, 32, 33, 64, 65, 97, 300])
+def test_few_rows_are_exact_on_small_integers(M):
+    """The 64- and 32-row tiles at their edges, with one step of K, an odd number, and K summed in two and four
+    slices: whole numbers up to 2 in magnitude, whose sums are exact in fp32 in any order, so that every epilogue
+    gives the one value its roundings leave.  Vectors that are not 16-byte aligned; rows past M stay as they are."""
+    N = _native()
+    dev = torch.device("cuda:0")
+    g = torch.Generator().manual_seed(M)
+    for K, Nn in ((128, 64), (384, 192), (1024, 1024), (2048, 128), (4096, 64)):
+        a = torch.randint(-2, 3, (M, K), generator=g).to(torch.bfloat16)
+        w = torch.randint(-2, 3, (Nn, K), generator=g).to(torch.bfloat16)
+        bias = torch.randint(-4, 5, (Nn + 1,), generator=g).float().to(dev)[1:]
+        gamma = (2.0 ** torch.randint(-2, 2, (Nn + 1,), generator=g)).to(dev)[1:]
+        res = torch.randint(-64, 65, (M, Nn), generator=g).to(torch.bfloat16)
+        a_d, w_d, r_d = a.to(dev), w.to(dev), res.to(dev)
+        lin = (a.double() @ w.double().T + bias.double().cpu()).to(torch.bfloat16)
+        branch = (lin.float() * gamma.cpu()).to(torch.bfloat16)
+        want = {N.LINEAR_BIAS: lin, N.LINEAR_BIAS_RESIDUAL: (res.float() + branch.float()).to(torch.bfloat16)}
+        need = int(N.lib.lbm_linear_workspace_bytes(M, Nn, K, N.LINEAR_BIAS_RESIDUAL))
+        assert (need > 0) == (K >= 2048)
+        ws = torch.zeros(max(need, 16), dtype=torch.uint8, device=dev)
+        for epi in (N.LINEAR_BIAS, N.LINEAR_BIAS_RESIDUAL, N.LINEAR_BIAS_GELU):
+            for with_ws in ((False, True) if need and epi == N.LINEAR_BIAS_RESIDUAL else (False,)):
+                out = torch.full((M + 1, Nn), 7.0, dtype=torch.bfloat16, device=dev)
+                N.check(N.lib.lbm_linear_norm(ptr(a_d), None, ptr(w_d), ptr(bias), ptr(gamma) if epi == N.LINEAR_BIAS_RESIDUAL else None,
+                                              ptr(r_d) if epi == N.LINEAR_BIAS_RESIDUAL else None, ptr(out), None, M, Nn, K, epi,
+                                              ptr(ws) if with_ws else None, need if with_ws else 0, None))
+                torch.cuda.synchronize()
+                out = out.cpu()
+                assert (out[M] == 7.0).all()
+                if epi == N.LINEAR_BIAS_GELU:   # the exact value rounded once; below -3, where 1 + erf cancels, one bf16 step of GELU(-3)
+                    gelu = torch.nn.functional.gelu(lin.double()).to(torch.bfloat16)
+                    assert torch.equal(out[:M][lin >= -3], gelu[lin >= -3]), (K, Nn)
+                    assert ((out[:M].float() - gelu.float())[lin < -3].abs() <= 2.0 ** -8 * 4.1e-3).all()
+                else:
+                    assert torch.equal(out[:M], want[epi]), (K, Nn, epi, with_ws)
+
+
+@pytest.mark.parametrize("M,H", [(2, 1), (33, 3), (64, 2), (100, 5)])
+def test_few_rows_with_the_producer_as_the_epilogue(M, H):
+    """The producer on the 64- and 32-row tiles: as on the others, bit-equal to the two separate launches."""
+    for norm in (False, True):
+        for rope in ("none", "interleaved", "half_split"):
+            test_qkv_projection_with_the_producer_as_its_epilogue(M, H, 256, norm, rope)
