@@ -1027,29 +1027,38 @@ __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_
 }
 
 // ---------------------------------------------------------------------------- several streams' rows
-// The same product on 256 x 256 (or 192 x 256) tiles, for launches with enough rows to give most
+// The same product on 256 x 256 (192 x 256, 128 x 256) tiles, for launches with enough rows to give most
 // of the 256 CUs such a tile (four streams' 4,016 rows x the qkv projection's 3,072 or fc1's
 // 4,096 columns): a 256 x 256 tile moves 64 KB of operands per 64 of K for 8.4 MFLOP - 128 FLOP
 // per byte on the way from L2 into LDS, which is what bounds the 128 x 128 tiles above at 64.
-// Eight wavefronts, each on 64 rows x 128 columns of the tile (96 x 64 of a 192-row tile) over
-// the whole K slice, no K split inside the workgroup and so no exchange at the end.  Two LDS
+// Eight wavefronts, each on 64 rows x 128 columns of the tile (96 x 64 of a 192-row tile, 64 x 64 of a 128-row
+// one) over the whole K slice, no K split inside the workgroup and so no exchange at the end: one sum per
+// element, the same bits whatever the tile.  Two LDS
 // stages: a 64-wide step is 24-32 MFMAs per wavefront, longer than a trip to memory, so one step
 // of prefetch is enough; the loads of a step are issued at the end of the step before the one
-// they replace, right behind the barrier that frees its stage.  Same operand path (global -> LDS directly, swizzled 16-byte chunks), same
+// they replace, right behind the barrier that frees its stage (a 128-row tile's step is half as long: three
+// stages).  Same operand path (global -> LDS directly, swizzled 16-byte chunks), same
 // epilogue arithmetic and rounding sequence.  Epilogues: bias, bias + GELU, and the
 // pre-attention producer; the folded LayerNorm of the activations; not the residual forms (their
 // 1,024 columns make too few such tiles).  The per-column vectors wait in LDS instead of
-// registers (the accumulators take half the register file).  192-row tiles are for shapes whose
-// 256-row tiles would leave a quarter of the CUs idle (4,016 x 3,072: 192 against 252 tiles).
+// registers (the accumulators take half the register file).  192- and 128-row tiles are for shapes whose
+// 256-row tiles would leave CUs idle (4,016 x 3,072: 192 against 252 tiles; 2,008 x 3,072: 96 against 192:
+// 33 us with the producer on the 132 tiles of 192 rows, 23 on these; 1,350 x 4,096 + GELU 27.7 -> 21.3).
 constexpr int kBN = 256;
 constexpr int kBCStride = kBN + 4;                          // bf16 per staged output row
+constexpr int lbm_big_stages(int bm) { return bm == 128 ? 3 : 2; }
+// Whether two more wavefronts load, as above: where the others can do with 168 registers, that is with
+// 128 rows, and with 192 unless the store holds rotary entries.
+constexpr bool lbm_big_loaders(int bm, int rope) { return bm == 128 || (bm == 192 && rope == 0); }
+constexpr int lbm_big_threads(int bm, int rope) { return kGThreads + (lbm_big_loaders(bm, rope) ? kGLoadWaves * 64 : 0); }
 constexpr int lbm_big_lds_bytes(int bm) {
-  return bm * kBCStride * 2 > 2 * (bm + kBN) * kKS * 2 ? bm * kBCStride * 2 : 2 * (bm + kBN) * kKS * 2;
+  const int stages = lbm_big_stages(bm) * (bm + kBN) * kKS * 2;
+  return bm * kBCStride * 2 > stages ? bm * kBCStride * 2 : stages;
 }
 static_assert(lbm_big_lds_bytes(256) + kGeluEntries * 2 + 2 * kBN * 4 + 256 * 8 <= 160 * 1024, "LDS budget of the 256 x 256 tile");
 
 template <int BM, int EPI, int ROPE = 0, bool NORM = false, bool LNA = false>
-__global__ __launch_bounds__(kGThreads, 1) void lbm_linear_bf16_big_kernel(LinearArgs p) {
+__global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_big_kernel(LinearArgs p) {
   constexpr int kRowGroups = BM == 256 ? 4 : 2;             // wavefronts along the rows of the tile
   constexpr int kColGroups = 8 / kRowGroups;
   constexpr int RB = BM / 32 / kRowGroups, CB = kBN / 32 / kColGroups;   // 32 x 32 blocks per wavefront: 2 x 4 or 3 x 2
@@ -1093,6 +1102,40 @@ __global__ __launch_bounds__(kGThreads, 1) void lbm_linear_bf16_big_kernel(Linea
                  st + BM * kKS * 2 + (64 * (j - kPassA) + 8 * wave) * (kKS * 2));
   };
   constexpr int kDma = kPassA + kPassW;
+  constexpr bool kLoaders = lbm_big_loaders(BM, ROPE);
+  constexpr int kStages = lbm_big_stages(BM);
+  if (kLoaders && wave >= kGThreads / 64) {
+    // a loading wavefront: every second KB of a step's operands (as in the kernel above)
+    const int par = wave - kGThreads / 64, l8 = lane >> 3;
+    constexpr int kUnitsA = BM / 16, kLoads = kUnitsA + kBN / 16;
+    const unsigned chunk = (unsigned)(((lane & 7) ^ (4 * par + (lane >> 4))) * 8);
+    unsigned off[kLoads];
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int row = u < kUnitsA ? min(m0 + 8 * (2 * u + par) + l8, p.M - 1) : 8 * (2 * (u - kUnitsA) + par) + l8;
+      off[u] = ((unsigned)row * (unsigned)p.K + chunk) * 2u;
+    }
+    const unsigned lds_first = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)&lds_raw[0]) + (unsigned)par * 1024u;
+    auto load_step = [&](int s) {
+      const unsigned st = lds_first + (unsigned)(s % kStages) * kStageBytes;
+#pragma unroll
+      for (int u = 0; u < kLoads; ++u) {
+        const char* base = (u < kUnitsA ? a_base : w_base) + (size_t)s * (kKS * 2);
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off[u]), "s"(base), "s"(st + u * 2048u) : "memory", "m0");
+      }
+    };
+    __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+    for (int s = 0; s < kStages - 1; ++s)
+      if (s < nk) load_step(s);
+    for (int s = -1; s < nk; ++s) {    // the barrier of step s hands over the rows of step s + 1 and frees the stage of step s
+      if (kStages > 2 && nk - 2 - s >= 1) LBM_DMA_WAIT(kLoads);
+      else LBM_DMA_WAIT(0);
+      __builtin_amdgcn_s_barrier();
+      if (s + kStages < nk) load_step(s + kStages);
+    }
+    return;
+  }
 
   // the folded LayerNorm's row statistics: two threads per row, each every second partial
   constexpr int kLnHeld = 8;
@@ -1112,7 +1155,7 @@ __global__ __launch_bounds__(kGThreads, 1) void lbm_linear_bf16_big_kernel(Linea
   if (EPI == LBM_LINEAR_BIAS_GELU && tid < kGeluEntries / 8)
     dma_row((const char*)g_gelu_table, (unsigned)tid * 16u, (const unsigned char*)&gelu_tab[wave * 512]);
 #pragma unroll
-  for (int j = 0; j < kDma; ++j) dma_one(0, 0, j);
+  for (int j = 0; j < (kLoaders ? 0 : kDma); ++j) dma_one(0, 0, j);
   if (tid < kBN) {
     colvec[0][tid] = cv_bias;
     colvec[1][tid] = cv_sum;
@@ -1201,19 +1244,19 @@ __global__ __launch_bounds__(kGThreads, 1) void lbm_linear_bf16_big_kernel(Linea
   // loads of the step after the next one, which have a whole step to land.
   constexpr int kQ = CB * RB, kR = CB + RB, kH = kQ / 2;
   auto step = [&](int s, auto stage_c) {
-    constexpr unsigned here = decltype(stage_c)::value * kStageBytes, there = kStageBytes - here;
+    constexpr unsigned here = decltype(stage_c)::value * kStageBytes, there = (decltype(stage_c)::value + 1) % kStages * kStageBytes;
 #pragma unroll
     for (int kq = 0; kq < 3; ++kq) {
       read(here, kq + 1, wf[(kq + 1) & 1], af[(kq + 1) & 1]);
       mfmas(kq, 0, kQ);
 #pragma unroll
       for (int i = 0; i < kR; ++i) { LBM_SGB(0x008, 1); LBM_SGB(0x100, 1); }
-      LBM_SGB(0x008, kQ - kR);
+      if (kQ > kR) LBM_SGB(0x008, kQ - kR);
       __builtin_amdgcn_sched_barrier(0);
     }
     mfmas(3, 0, kH);
     __builtin_amdgcn_sched_barrier(0);
-    LBM_DMA_WAIT(0);
+    if (!kLoaders) LBM_DMA_WAIT(0);
     __syncthreads();   // the other stage has landed everywhere, and everyone has read all of this one
     __builtin_amdgcn_sched_barrier(0);
     read(there, 0, wf[0], af[0]);
@@ -1222,15 +1265,16 @@ __global__ __launch_bounds__(kGThreads, 1) void lbm_linear_bf16_big_kernel(Linea
 #pragma unroll
     for (int i = 0; i < kQ - kH; ++i) { LBM_SGB(0x008, 1); LBM_SGB(0x100, 1); }
     __builtin_amdgcn_sched_barrier(0);
-    if (s + 2 < nk) dma_step(s + 2, here);
+    if (!kLoaders && s + 2 < nk) dma_step(s + 2, here);
   };
   LBM_DMA_WAIT(0);
   __syncthreads();
-  dma_step(1, kStageBytes);
+  if (!kLoaders) dma_step(1, kStageBytes);
   read(0, 0, wf[0], af[0]);
-  for (int s = 0; s < nk; s += 2) {
+  for (int s = 0; s < nk; s += kStages) {
     step(s, std::integral_constant<unsigned, 0>{});
-    step(s + 1, std::integral_constant<unsigned, 1>{});
+    if (kStages == 2 || s + 1 < nk) step(s + 1, std::integral_constant<unsigned, 1>{});
+    if (kStages == 3 && s + 2 < nk) step(s + 2, std::integral_constant<unsigned, kStages - 1>{});
   }
 #undef LBM_SGB
 
@@ -1239,7 +1283,7 @@ __global__ __launch_bounds__(kGThreads, 1) void lbm_linear_bf16_big_kernel(Linea
   constexpr int kPieces = kBN / 8;                    // 16-byte pieces per row of the tile: 32
   constexpr int kRowsPerPass = kGThreads / kPieces;   // 16
   constexpr int kPasses = BM / kRowsPerPass;          // 16 or 12
-  constexpr int kGroup = 4;                           // passes whose rotary entries and pool rows travel together
+  constexpr int kGroup = BM == 128 ? 2 : 4;           // passes whose rotary entries and pool rows travel together
   const int pr = tid / kPieces, pc = (tid % kPieces) * 8;
   typedef lbm_qkv::f32x4 qf4;
   const int H = p.num_heads;
@@ -1373,18 +1417,18 @@ bool lbm_linear_wider(LinearArgs& p) {
 }  // namespace
 
 namespace {
-// 256- or 192-row tiles of 256 columns when they give at least half of the 256 CUs a workgroup
+// Tiles of 256 columns when those of 256 or 192 rows give at least half of the 256 CUs a workgroup
 // (several streams' rows into the 3,072 or 4,096 columns of the qkv projection or fc1): the row
-// count of the tile (the one that needs fewer rounds of the CUs times rows), or 0; sets the tile
-// counts
+// count of the tile (the one that needs the fewest rounds of the CUs times rows, of 128 rows too; as many rows as
+// possible among equals), or 0; sets the tile counts
 int lbm_linear_big_tiles(LinearArgs& p) {
   if (p.N % kBN != 0) return 0;
   const int nt = p.N / kBN;
   int best = 0;
   long long best_cost = 0;
-  for (int bm : {256, 192}) {
+  for (int bm : {256, 192, 128}) {
     const long long tiles = (long long)((p.M + bm - 1) / bm) * nt;
-    if (tiles < 128) continue;
+    if (bm == 128 ? !best : tiles < 128) continue;   // (fewer: the kernel above, whose elements are two sums)
     const long long cost = ((tiles + 255) / 256) * bm;      // rounds of the 256 CUs x rows per tile
     if (!best || cost < best_cost) best = bm, best_cost = cost;
   }
@@ -1501,7 +1545,8 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
 #define LBM_BIG_LAUNCH(E, L)                                                                                         \
       {                                                                                                              \
         if (bm == 256) hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<256, E, 0, false, L>), grid_b, block, 0, stream, p); \
-        else hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<192, E, 0, false, L>), grid_b, block, 0, stream, p);           \
+        else if (bm == 192) hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<192, E, 0, false, L>), grid_b, dim3(lbm_big_threads(192, 0)), 0, stream, p);           \
+        else hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<128, E, 0, false, L>), grid_b, dim3(lbm_big_threads(128, 0)), 0, stream, p);           \
       }
       if (epilogue == LBM_LINEAR_BIAS && lna) LBM_BIG_LAUNCH(LBM_LINEAR_BIAS, true)
       else if (epilogue == LBM_LINEAR_BIAS) LBM_BIG_LAUNCH(LBM_LINEAR_BIAS, false)
@@ -1591,7 +1636,7 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
   const bool norm = q_norm_w != nullptr;
   // 256-wide tiles: four whole heads each, so that a tile does not straddle q | k | v
   if (const int bm = (num_heads & 3) == 0 ? lbm_linear_big_tiles(p) : 0) {
-    const dim3 grid_b((unsigned)(p.m_tiles * p.n_tiles)), block_b(kGThreads);
+    const dim3 grid_b((unsigned)(p.m_tiles * p.n_tiles)), block_b(lbm_big_threads(bm, rope));
 #define LBM_QKV_BIG_M(BM, R, NRM)                                                                                               \
     {                                                                                                                           \
       if (lna) hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<BM, kEpiQkvPrepare, R, NRM, true>), grid_b, block_b, 0, stream, p);  \
@@ -1599,7 +1644,7 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
     }
 #define LBM_QKV_BIG(R, NRM)                                                  \
     {                                                                        \
-      if (bm == 256) LBM_QKV_BIG_M(256, R, NRM) else LBM_QKV_BIG_M(192, R, NRM) \
+      if (bm == 256) LBM_QKV_BIG_M(256, R, NRM) else if (bm == 192) LBM_QKV_BIG_M(192, R, NRM) else LBM_QKV_BIG_M(128, R, NRM) \
     }
     if (rope == 0 && !norm) LBM_QKV_BIG(0, false)
     else if (rope == 0) LBM_QKV_BIG(0, true)

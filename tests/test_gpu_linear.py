@@ -561,3 +561,21 @@ def test_few_rows_with_the_producer_as_the_epilogue(M, H):
     for norm in (False, True):
         for rope in ("none", "interleaved", "half_split"):
             test_qkv_projection_with_the_producer_as_its_epilogue(M, H, 256, norm, rope)
+
+
+@pytest.mark.parametrize("K", [128, 256, 384, 1024])
+@pytest.mark.parametrize("Nn,epilogue", [(3072, "bias"), (4096, "gelu")])
+def test_tile_height_changes_no_bit(K, Nn, epilogue):
+    """2,000 rows run on tiles of 128 rows x 256 columns, 4,016 on 192 (3,072 columns) or 256 (4,096): the rows that
+    both launches hold come out the same, from two steps of K on (fewer than the ring has stages)."""
+    N = _native()
+    epi = {"bias": N.LINEAR_BIAS, "gelu": N.LINEAR_BIAS_GELU}[epilogue]
+    a, w, bias, _ = _inputs(4016, K, Nn, seed=K + Nn)
+    few, many = run_linear(a[:2000], w, bias, epi), run_linear(a, w, bias, epi)
+    assert torch.equal(few, many[:2000])
+
+
+def test_qkv_projection_with_the_producer_on_tiles_of_128_rows():
+    for norm in (False, True):
+        for rope in ("none", "interleaved", "half_split"):
+            test_qkv_projection_with_the_producer_as_its_epilogue(1950, 16, 256, norm, rope)
