@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define LBM_ABI_VERSION 10
+#define LBM_ABI_VERSION 11
 
 #define LBM_OK 0
 #define LBM_ERR_INVALID 1     /* bad argument (null pointer, negative size, bad enum)      */
@@ -311,6 +311,15 @@ int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k,
                         const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads,
                         int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
                         void* workspace, size_t workspace_bytes, void* stream);
+
+/* lbm_attn_run_append for a row table that names no row of append_rows (ABI 11), as the plans of
+ * lbm_tables_step with LBM_OP_PLAN_NEWEST_SELF do: with nobody reading those rows, attention launches that
+ * merge nothing carry the append as well, by workgroups of their own.  Same results. */
+int lbm_attn_run_append_apart(const void* q, void* pool, void* out, const void* new_k, const void* new_v,
+                              const int32_t* kv_rows, const int32_t* append_rows, int32_t append_tokens,
+                              const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads,
+                              int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
+                              void* workspace, size_t workspace_bytes, void* stream);
 
 /* A whole transformer block of the streaming model in one call (ABI 10): qkv projection + producer,
  * attention, proj + LayerScale + residual, fc1 + GELU, fc2 + LayerScale + residual

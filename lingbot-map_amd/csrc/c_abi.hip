@@ -224,7 +224,7 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
                              const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads,
                              int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
                              void* workspace, size_t workspace_bytes, void* stream,
-                             const int32_t* append_rows = nullptr, int32_t append_tokens = 0) {
+                             const int32_t* append_rows = nullptr, int32_t append_tokens = 0, bool append_apart = false) {
   int rc = lbm_check_attn_streams(streams, n_streams, who);
   if (rc != LBM_OK) return rc;
   if (!q || !pool || !out || !kv_rows) return lbm_fail(LBM_ERR_INVALID, "%s: null q, pool, out or kv_rows", who);
@@ -240,7 +240,7 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
   if (need > 0 && (!workspace || workspace_bytes < need))
     return lbm_fail(LBM_ERR_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", who, workspace_bytes, need);
   return lbm_launch_attention(q, pool, out, self_k, self_v, kv_rows, live_kv_tokens, sch, num_heads, head_dim,
-                              page_size, dtype, sm_scale, workspace, (hipStream_t)stream, append_rows, append_tokens);
+                              page_size, dtype, sm_scale, workspace, (hipStream_t)stream, append_rows, append_tokens, append_apart);
 }
 
 int lbm_attn_run(const void* q, const void* pool, void* out, const void* self_k,
@@ -263,6 +263,19 @@ int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k,
   return lbm_attn_run_impl("lbm_attn_run_append", q, pool, out, new_k, new_v, kv_rows, nullptr, streams, n_streams,
                            num_heads, head_dim, page_size, dtype, sm_scale, workspace, workspace_bytes, stream,
                            append_rows, append_tokens);
+}
+
+int lbm_attn_run_append_apart(const void* q, void* pool, void* out, const void* new_k, const void* new_v,
+                              const int32_t* kv_rows, const int32_t* append_rows, int32_t append_tokens,
+                              const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads,
+                              int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
+                              void* workspace, size_t workspace_bytes, void* stream) {
+  if (!new_k || !new_v || !append_rows)
+    return lbm_fail(LBM_ERR_INVALID, "lbm_attn_run_append_apart: null new_k, new_v or append_rows");
+  if (append_tokens < 0) return lbm_fail(LBM_ERR_INVALID, "lbm_attn_run_append_apart: negative append_tokens");
+  return lbm_attn_run_impl("lbm_attn_run_append_apart", q, pool, out, new_k, new_v, kv_rows, nullptr, streams, n_streams,
+                           num_heads, head_dim, page_size, dtype, sm_scale, workspace, workspace_bytes, stream,
+                           append_rows, append_tokens, true);
 }
 
 int lbm_attn_run_live(const void* q, const void* pool, void* out, const void* self_k,

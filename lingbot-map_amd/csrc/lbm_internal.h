@@ -78,6 +78,10 @@ struct AttnArgsF32 {
   int n_streams;
   lbm_attn_stream s[LBM_MAX_STREAMS];
   int wg_begin[LBM_MAX_STREAMS + 1];
+  // the append carried by workgroups behind the attention's (lbm_attn_run_append_apart; 0 tokens: none): row t of
+  // self_k / self_v to pool row append_rows[t]
+  const int32_t* append_rows;
+  int append_tokens;
 };
 // fp32 attention at head_dim 64 on bf16 matrix instructions (paged_attn_f32_gfx950.hip)
 int lbm_launch_attn_f32_d64(AttnArgsF32& a, hipStream_t stream);
@@ -87,7 +91,25 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
                          const LbmAttnSchedule& sch,
                          int num_heads, int head_dim, int page_size, int dtype, float sm_scale,
                          void* workspace, hipStream_t stream,
-                         const int32_t* append_rows = nullptr, int append_tokens = 0);
+                         const int32_t* append_rows = nullptr, int append_tokens = 0, bool append_apart = false);
+
+#ifdef __HIPCC__
+// The append as workgroups of an attention launch: workgroup `wg` of those behind the attention's copies one 16-byte
+// piece of a K row and of the matching V row per thread (row_pieces: 16-byte pieces per row).
+__device__ __forceinline__ void lbm_append_pieces(const void* k, const void* v, void* pool, const int32_t* append_rows,
+                                                  int append_tokens, int row_pieces, int page_size, int wg, int threads) {
+  typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+  const long long idx = (long long)wg * threads + threadIdx.x;
+  if (idx >= (long long)append_tokens * row_pieces) return;
+  const int t = (int)(idx / row_pieces), piece = (int)(idx % row_pieces);
+  const int row = append_rows[t];
+  if (row < 0) return;
+  const u32x4 kk = ((const u32x4*)k)[idx], vv = ((const u32x4*)v)[idx];
+  u32x4* dst = (u32x4*)pool + (long long)row * row_pieces + piece;
+  dst[0] = kk;
+  dst[(long long)page_size * row_pieces] = vv;
+}
+#endif
 
 // Address and size of the library's static device scratch array on the current device (looked
 // up once per device; no allocation).

@@ -183,7 +183,7 @@ class HipPagedKVCacheManager:
         # append rows of a pass of several frames that block 0 made in one go (begin_frames), until block
         # 0 moves on: (appends before it, frames, rows [streams, frames, tokens])
         self._pass_rows = [None] * self._n_sets
-        #: step(): the attention call stores the new frame itself (lbm_attn_run_append), reading it
+        #: step(): the attention call stores the new frame itself (lbm_attn_run_append_apart), reading it
         #: from the caller's tensors meanwhile - no append launch in front of the attention
         self.fuse_append = True
         self._newest_self = [False] * self._n_sets   # the set's row table names the newest frame by the caller's rows
@@ -659,7 +659,7 @@ class HipPagedKVCacheManager:
         reads it from the caller's rows only.
         ``newest_self`` (leading block): the row table names the rows a keyframe appends by the
         caller's own K/V rows; every block of the frame then attends and appends with
-        ``lbm_attn_run_append`` (``step`` does), which ``_newest_self`` remembers."""
+        ``lbm_attn_run_append_apart`` (``step`` does), which ``_newest_self`` remembers."""
         if keyframe is None:
             keyframe = (not self._skip_append,) * self.num_streams
         else:
@@ -706,7 +706,8 @@ class HipPagedKVCacheManager:
                         q_prescaled: bool = False, append_rows: Optional[int] = None) -> Tensor:
         """``q_prescaled``: q already carries 1 / sqrt(D) and log2(e) (``step_qkv``'s producer).
         ``append_rows``: the address of the rows ``self_k`` / ``self_v`` are also stored in, row t in
-        pool row ``append_rows[t]``, once the attention has read the pool (``lbm_attn_run_append``)."""
+        pool row ``append_rows[t]``: pages of this frame, which its plan names by the caller's rows
+        (``lbm_attn_run_append_apart``)."""
         ts = self._set(block_idx)
         if self._newest_self[ts] and append_rows is None:
             raise RuntimeError("this frame's row table names its newest frame by the caller's K/V rows (step() led "
@@ -733,7 +734,7 @@ class HipPagedKVCacheManager:
         tail = (0.0 if q_prescaled else self._sm_scale, ws.data_ptr(), ws.numel(), self._stream_handle())
         tensors = (qc.data_ptr(), self.kv_caches[block_idx].data_ptr(), out.data_ptr(), k_ptr, v_ptr, self._kv_rows_ptr(ts))
         if append_rows is not None:
-            N.check(N.lib.lbm_attn_run_append(*tensors, append_rows, self_k.shape[0], *common, *tail))
+            N.check(N.lib.lbm_attn_run_append_apart(*tensors, append_rows, self_k.shape[0], *common, *tail))
         elif self.device_token_counts:
             N.check(N.lib.lbm_attn_run_live(*tensors, self._live_counts_ptr(ts), *common, *tail))
         else:
