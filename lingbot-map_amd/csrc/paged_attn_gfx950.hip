@@ -1944,7 +1944,7 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
       memo.n_tiles[i] = nt[i];
       memo.n_splits[i] = best_splits[i];
       memo.order[i] = i;
-      tiles[i] = nt[i] > 0 ? (nt[i] + best_splits[i] - 1) / best_splits[i] : 0;
+      tiles[i] = nt[i] > 0 ? (memo.small ? nt[i] : (nt[i] + best_splits[i] - 1) / best_splits[i]) : 0;
     }
     for (int i = 1; i < n_streams; ++i)
       for (int j = i; j > 0 && tiles[memo.order[j]] > tiles[memo.order[j - 1]]; --j) {
@@ -1954,8 +1954,11 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
   if (memo.small) {
     sch.small = memo.small;
     int wg = 0;
-    for (int i = 0; i < n_streams; ++i) {
-      LbmAttnStreamPlan& p = sch.s[i];
+    for (int oi = 0; oi < n_streams; ++oi) {
+      const int i = memo.order[oi];
+      // streams with the longest workgroups first, as below: the launch ends with short ones (261 rows over
+      // 783 tokens and 261 over 2,088 in one launch: a frame of 24 blocks 479 us in the callers' order, 413 so)
+      LbmAttnStreamPlan& p = sch.s[oi];
       p.q_begin = streams[i].q_begin;
       p.q_rows = streams[i].q_rows;
       p.kv_row_begin = streams[i].kv_row_begin;
