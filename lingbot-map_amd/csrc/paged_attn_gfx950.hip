@@ -795,6 +795,9 @@ constexpr int kSmThreads = kSmWaves * 64;
 // XCD's L2 no longer holds for its neighbours (485 rows x 5,820 tokens: 38 us against 29 on the pair).
 constexpr int kSmMaxKv = 4096;
 constexpr int kSmPiece = 32;     // KV tokens per step of a wavefront
+// KV tokens of a launch's longest stream beyond which its workgroups begin at different pieces (lbm_attn_bf16_d64_small_kernel's
+// TURN): 261 rows over 1,305 tokens 9.9 us in order, 10.1 so; 86 over 1,500 13.3, 11.6; 300 over 900 and 2,100 17.3, 16.7.
+constexpr int kSmTurnKv = 1408;
 constexpr int kSmOStride = 68;   // floats per row of a partial output parked in LDS (4-bank shift per row)
 constexpr int kSmPieceBytes = kSmPiece * 64 * 2;                                 // K (or V) rows of a piece, unpadded
 constexpr int kSmOffLists = kSmWaves * 2 * 2 * kSmPieceBytes;                    // behind two stages of K and V per wavefront
@@ -807,8 +810,9 @@ constexpr int lbm_sm_lds_bytes(int rows) {
 static_assert(lbm_sm_lds_bytes(64) <= 160 * 1024, "LDS budget of the short-KV kernel");
 }  // namespace
 
-// QB: 32-row blocks of query rows per workgroup
-template <int QB>
+// QB: 32-row blocks of query rows per workgroup.  TURN: workgroups may begin at different pieces (an
+// instance of its own: what it adds in front of the first load takes 0.2 us, 3 % of a launch on 261 own rows).
+template <int QB, bool TURN>
 __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[lbm_sm_lds_bytes(32 * QB)];
   constexpr int kRows = 32 * QB;
@@ -842,6 +846,19 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
   const int n_pieces = (kv_tokens + kSmPiece - 1) / kSmPiece;
   const int pps = (n_pieces + kSmWaves - 1) / kSmWaves;
   const int p0 = wave * pps, p1 = min(p0 + pps, n_pieces);   // this wavefront's pieces (possibly none)
+  // Where in its pieces it begins.  Over a cache the workgroups of a head, which start together, each begin at
+  // another place and go round: all at the same one, they would ask HBM for the same two pieces per wavefront,
+  // a quarter of what it takes to keep it busy, and wait for them together.  A ragged last piece stays the last
+  // (it is masked there).  Attention to a stream's own rows, just written, keeps the order: an encoder's
+  // results stay what they are.
+  // (24 blocks with pools of their own, us per block: 261 rows over 2,349 tokens 16.3 -> 14.1, 600 over 3,600 25.3 ->
+  // 23.6; 261 over 4,000 tokens, pools rotating through 600 MB, 25.1 -> 19.3.)
+  int go_round = 0, turn = 0;
+  if (TURN && pps > 2 && kv_tokens != sp.q_rows) {
+    go_round = max(p1 - p0 - (p1 == n_pieces && kv_tokens % kSmPiece != 0 ? 1 : 0), 0);
+    turn = min(__builtin_amdgcn_readfirstlane((int)((float)(q_tile * go_round) * __builtin_amdgcn_rcpf((float)sp.n_qtiles))), go_round);
+  }
+  auto piece = [&](int i) { return !TURN ? p0 + i : p0 + i + (i + turn < go_round ? turn : (i < go_round ? turn - go_round : 0)); };   // the i-th it takes
   const unsigned row_bytes = (unsigned)H * 128u;
   const int q_row0 = q_tile * kRows;
   if (n_pieces == 0) {
@@ -871,8 +888,9 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
   const unsigned chunk_k[2] = {(unsigned)(((lane & 7) ^ (lane >> 4)) * 16), (unsigned)(((lane & 7) ^ (4 | (lane >> 4))) * 16)};
   const unsigned chunk_v = (unsigned)(((lane & 7) ^ (((lane >> 4) & 1) * 4)) * 16);
   // (tokens past the last re-read it: finite data, masked below)
-  auto load_entries = [&](int pc) {   // of pieces pc (lanes 0-31) and pc + 1
-    const int32_t* src = rows + min(pc * kSmPiece + lane, last_token);
+  auto load_entries = [&](int i) {   // of the i-th piece (lanes 0-31) and the next
+    const int pa = piece(i), pb = piece(i + 1);
+    const int32_t* src = rows + min(TURN ? (g ? pb : pa) * kSmPiece + n32 : pa * kSmPiece + lane, last_token);
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" : : "v"(src), "s"(m0_entries) : "memory", "m0");
   };
   auto find_rows = [&](int e) {   // negative entries name rows of the caller's own K/V
@@ -890,7 +908,7 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
   };
   // pieces p0 and p0 + 1, as far as there are such, and the entries of the one after them on their way
   auto start = [&]() {
-    load_entries(p0);
+    load_entries(0);
     LBM_LOADS_LEFT(0);
     const int e0 = entries[n32], e1 = entries[kSmPiece + n32];
     find_rows(e0);
@@ -899,7 +917,7 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
     if (p0 + 1 < p1) {
       find_rows(e1);
       LBM_LDS_DONE();
-      load_entries(p0 + 2);
+      load_entries(2);
       load_rows(1);
     }
   };
@@ -968,9 +986,9 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
         ka[ks] = __builtin_bit_cast(bf16x8, *(const u32x4*)&k[n32 * 64 + ((ks * 2 + g) ^ ((n32 >> 1) & 7)) * 8]);
     };
     // AHEAD: 2 - the piece two ahead is asked for, 1 - the next piece is the last, 0 - this one is
-    auto step = [&](int pc, auto AHEAD) {
+    auto step = [&](int at, auto AHEAD) {
       constexpr int kAhead = decltype(AHEAD)::value;
-      const int stage = (pc - p0) & 1;
+      const int stage = at & 1;
       const unsigned short* ring_v = (const unsigned short*)(ring + stage * 2 * kSmPieceBytes + kSmPieceBytes);
       // S^T = K Q^T for the piece's 32 kv rows: sc[qb][i] is kv = 8 (i / 4) + 4 g + i % 4, q = 32 qb + n32
       f32x16 sc[QB];
@@ -986,7 +1004,7 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
 #pragma unroll
         for (int db = 0; db < 2; ++db) va[ks][db] = v_frag(ring_v, ks, db);
       if (kAhead == 0) {   // (the stream's ragged last piece is some wavefront's last piece)
-        const int n_valid = kv_tokens - pc * kSmPiece;
+        const int n_valid = kv_tokens - piece(at) * kSmPiece;
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
@@ -1033,7 +1051,7 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
       }
       if (kAhead == 2) {  // both buffers of this stage are read: the piece two ahead may come
         LBM_LDS_DONE();
-        load_entries(pc + 3);
+        load_entries(at + 3);
         load_rows(stage);
       }
       // O^T += V^T P^T over the piece's two 16-row k-steps
@@ -1048,10 +1066,10 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
     if (p0 + 1 < p1) LBM_LOADS_LEFT(8);
     else LBM_LOADS_LEFT(0);
     read_k(0);
-    int pc = p0;
-    for (; pc + 2 < p1; ++pc) step(pc, std::integral_constant<int, 2>());
-    if (pc + 1 < p1) step(pc++, std::integral_constant<int, 1>());
-    step(pc, std::integral_constant<int, 0>());
+    int at = 0;
+    for (; at + 2 < p1 - p0; ++at) step(at, std::integral_constant<int, 2>());
+    if (at + 1 < p1 - p0) step(at++, std::integral_constant<int, 1>());
+    step(at, std::integral_constant<int, 0>());
   };
   walk(std::false_type());
   // range check of the pass without reference (integer compares, see the main kernel)
@@ -1916,7 +1934,7 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
       }
       const double wary_small = kSmLaunchUs + (rows_us / 256.0 > longest ? rows_us / 256.0 : longest);
       consider_all(true);
-      // (32 and 64 rows per workgroup give the same bits: the fitted costs choose)
+      // (32 and 64 rows per workgroup give the same bits where a stream attends to its own rows: the fitted costs choose)
       if (best < 0 || best >= 0.85 * wary_small)
         memo.small = price_small(nt, n_streams, num_heads, 32, q_rows) < price_small(nt, n_streams, num_heads, 64, q_rows) ? 32 : 64;
     } else {
@@ -2161,8 +2179,13 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       blocks += (unsigned)(((long long)append_tokens * num_heads * 8 + kSmThreads - 1) / kSmThreads);
       *appended = true;
     }
-    if (sch.small == 64) hipLaunchKernelGGL(lbm_attn_bf16_d64_small_kernel<2>, dim3(blocks), dim3(kSmThreads), 0, stream, a);
-    else hipLaunchKernelGGL(lbm_attn_bf16_d64_small_kernel<1>, dim3(blocks), dim3(kSmThreads), 0, stream, a);
+    bool turn = false;   // (the kernel decides per stream, by the live count)
+    for (int i = 0; i < sch.n_streams; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);
+    const dim3 grid(blocks), block(kSmThreads);
+    if (sch.small == 64 && turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, true>), grid, block, 0, stream, a);
+    else if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false>), grid, block, 0, stream, a);
+    else if (turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, false>), grid, block, 0, stream, a);
     return lbm_check_launch("lbm_attn_bf16_d64_small_kernel");
   }
   hipLaunchKernelGGL(lbm_attn_bf16_d64_kernel, dim3(sch.total_wgs), dim3(kThreads), 0, stream, a);
