@@ -794,6 +794,7 @@ constexpr int kSmThreads = kSmWaves * 64;
 // KV tokens up to which the kernel is a candidate.  Beyond them every workgroup would read a KV list that its
 // XCD's L2 no longer holds for its neighbours (485 rows x 5,820 tokens: 38 us against 29 on the pair).
 constexpr int kSmMaxKv = 4096;
+constexpr int kSmMaxCacheKv = 4864;   // the same for one stream that attends to more than its own rows (lbm_attn_schedule)
 constexpr int kSmPiece = 32;     // KV tokens per step of a wavefront
 // KV tokens of a launch's longest stream beyond which its workgroups begin at different pieces (lbm_attn_bf16_d64_small_kernel's
 // TURN): 261 rows over 1,305 tokens 9.9 us in order, 10.1 so; 86 over 1,500 13.3, 11.6; 300 over 900 and 2,100 17.3, 16.7.
@@ -1803,6 +1804,7 @@ double makespan(WorkgroupClass* c, int n) {
 
 struct ScheduleKey {
   int n_streams = -1, num_heads = 0;
+  bool one_cache = false;
   int small = 0;   // query rows per workgroup of the short-KV kernel, 0: the split-KV pair
   int q_rows[LBM_MAX_STREAMS], n_tiles[LBM_MAX_STREAMS];
   int order[LBM_MAX_STREAMS], n_splits[LBM_MAX_STREAMS];
@@ -1882,10 +1884,11 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
   // several streams would take the CUs rounds of such workgroups.
   bool small_ok = n_streams > 0;
   for (int i = 0; i < n_streams; ++i) small_ok = small_ok && streams[i].kv_tokens <= kSmMaxKv;
+  const bool one_cache = n_streams == 1 && streams[0].kv_tokens != streams[0].q_rows && streams[0].kv_tokens <= kSmMaxCacheKv;
   int found = -1;
   for (int j = 0; j < kMemos && found < 0; ++j) {
     const ScheduleKey& m = g_schedules[j];
-    bool hit = m.n_streams == n_streams && m.num_heads == num_heads;
+    bool hit = m.n_streams == n_streams && m.num_heads == num_heads && m.one_cache == one_cache;
     for (int i = 0; hit && i < n_streams; ++i) hit = m.q_rows[i] == q_rows[i] && m.n_tiles[i] == nt[i];
     if (hit) found = j;
   }
@@ -1954,8 +1957,20 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
         consider(wary_tps, false);
       }
     }
+    // One stream's attention to a cache: no encoder makes such a launch (theirs attend to their own rows), so the
+    // fitted costs may give it to the short-KV kernel, up to 4,864 tokens and where they see the pair less than 15 %
+    // ahead: they underrate the pair by 23 % and this kernel by 17 % where K/V come from HBM.  Of 17 random launches
+    // with 80-1,374 rows 11 change over, 0.83 of their time in the mean and none slower.  us per block of a streamed
+    // frame, 24 blocks, pair and this kernel: 400 x 3,600 25.1, 19.4; 261 x 3,393 21.9, 18.5; 261 x 4,437 23.2, 21.9;
+    // 800 x 4,800 31.4, 29.5; 1,004 x 5,020 33.8, 34.4.  Several streams' launches are priced less well and stay.
+    if (!memo.small && one_cache) {
+      const double pair_us = price_candidate(qt, nt, n_streams, num_heads, (int)best_tps, q_rows, cand_splits, false);
+      const double us32 = price_small(nt, n_streams, num_heads, 32, q_rows), us64 = price_small(nt, n_streams, num_heads, 64, q_rows);
+      if ((us32 < us64 ? us32 : us64) < 1.15 * pair_us) memo.small = us32 < us64 ? 32 : 64;
+    }
     memo.n_streams = n_streams;
     memo.num_heads = num_heads;
+    memo.one_cache = one_cache;
     int tiles[LBM_MAX_STREAMS];
     for (int i = 0; i < n_streams; ++i) {
       memo.q_rows[i] = q_rows[i];
