@@ -1958,15 +1958,16 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
       }
     }
     // One stream's attention to a cache: no encoder makes such a launch (theirs attend to their own rows), so the
-    // fitted costs may give it to the short-KV kernel, up to 4,864 tokens and where they see the pair less than 15 %
-    // ahead: they underrate the pair by 23 % and this kernel by 17 % where K/V come from HBM.  Of 17 random launches
+    // fitted costs may give it to the short-KV kernel, up to 4,864 tokens and where they see the pair less than 8 %
+    // ahead: they underrate the pair by 23 % and this kernel by 17 % where K/V come from HBM.  Of 16 random launches
     // with 80-1,374 rows 11 change over, 0.83 of their time in the mean and none slower.  us per block of a streamed
     // frame, 24 blocks, pair and this kernel: 400 x 3,600 25.1, 19.4; 261 x 3,393 21.9, 18.5; 261 x 4,437 23.2, 21.9;
-    // 800 x 4,800 31.4, 29.5; 1,004 x 5,020 33.8, 34.4.  Several streams' launches are priced less well and stay.
+    // 800 x 4,800 31.4, 29.5; 1,004 x 5,020 33.8, 34.4;
+    // 120 x 3,000 17.3, 17.8.  Several streams' launches are priced less well and stay.
     if (!memo.small && one_cache) {
       const double pair_us = price_candidate(qt, nt, n_streams, num_heads, (int)best_tps, q_rows, cand_splits, false);
       const double us32 = price_small(nt, n_streams, num_heads, 32, q_rows), us64 = price_small(nt, n_streams, num_heads, 64, q_rows);
-      if ((us32 < us64 ? us32 : us64) < 1.15 * pair_us) memo.small = us32 < us64 ? 32 : 64;
+      if ((us32 < us64 ? us32 : us64) < 1.08 * pair_us) memo.small = us32 < us64 ? 32 : 64;
     }
     memo.n_streams = n_streams;
     memo.num_heads = num_heads;
