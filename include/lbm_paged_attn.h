@@ -321,6 +321,13 @@ int lbm_attn_run_append_apart(const void* q, void* pool, void* out, const void* 
                               int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
                               void* workspace, size_t workspace_bytes, void* stream);
 
+/* lbm_attn_run over the streams' own rows in order (ABI 11): entry kv_row_begin + t of kv_rows is
+ * -1 - (kv_row_begin + t) for every token t of every stream, which the caller promises and launches that split no
+ * KV rely on instead of reading it.  Same results.  k, v: as self_k, self_v. */
+int lbm_attn_run_own(const void* q, const void* k, const void* v, void* out, const int32_t* kv_rows, const lbm_attn_stream* streams,
+                     int32_t n_streams, int32_t num_heads, int32_t head_dim, int32_t dtype, float sm_scale, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
 /* A whole transformer block of the streaming model in one call (ABI 10): qkv projection + producer,
  * attention, proj + LayerScale + residual, fc1 + GELU, fc2 + LayerScale + residual
  * (lingbot_map/layers/block.py:245-285), i.e. lbm_qkv_linear_prepare_norm, lbm_attn_run (or
@@ -360,6 +367,7 @@ typedef struct lbm_block_call {
                                 * n_streams 0: no attention, the caller filled its output */
   const void* hints[4];        /* lbm_linear_prefetch_hint in front of the four GEMM launches; NULL: none */
   size_t hint_bytes[4];
+  int32_t own_rows;            /* ABI 11; 1: kv_rows is as lbm_attn_run_own takes it (with keep_kv) */
 } lbm_block_call;
 
 size_t lbm_block_scratch_bytes(int32_t rows, int32_t num_heads, int32_t hidden);

@@ -224,7 +224,8 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
                              const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads,
                              int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
                              void* workspace, size_t workspace_bytes, void* stream,
-                             const int32_t* append_rows = nullptr, int32_t append_tokens = 0, bool append_apart = false) {
+                             const int32_t* append_rows = nullptr, int32_t append_tokens = 0, bool append_apart = false,
+                             bool own_rows = false) {
   int rc = lbm_check_attn_streams(streams, n_streams, who);
   if (rc != LBM_OK) return rc;
   if (!q || !pool || !out || !kv_rows) return lbm_fail(LBM_ERR_INVALID, "%s: null q, pool, out or kv_rows", who);
@@ -234,13 +235,15 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
   if (live_kv_tokens)
     for (int i = 0; i < n_streams; ++i)
       if (streams[i].live_at < 0) return lbm_fail(LBM_ERR_INVALID, "%s: stream %d has a negative live_at", who, i);
+  // (rows are addressed by 32-bit byte offsets from the stream's first)
+  for (int i = 0; own_rows && i < n_streams; ++i) own_rows = (long long)streams[i].kv_tokens * num_heads * head_dim * 2 < (1LL << 32);
   LbmAttnSchedule sch;
   lbm_attn_schedule(streams, n_streams, num_heads, &sch);
   const size_t need = lbm_attn_schedule_bytes(sch, num_heads, head_dim);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return lbm_fail(LBM_ERR_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", who, workspace_bytes, need);
   return lbm_launch_attention(q, pool, out, self_k, self_v, kv_rows, live_kv_tokens, sch, num_heads, head_dim,
-                              page_size, dtype, sm_scale, workspace, (hipStream_t)stream, append_rows, append_tokens, append_apart);
+                              page_size, dtype, sm_scale, workspace, (hipStream_t)stream, append_rows, append_tokens, append_apart, own_rows);
 }
 
 int lbm_attn_run(const void* q, const void* pool, void* out, const void* self_k,
@@ -250,6 +253,13 @@ int lbm_attn_run(const void* q, const void* pool, void* out, const void* self_k,
                  void* stream) {
   return lbm_attn_run_impl("lbm_attn_run", q, pool, out, self_k, self_v, kv_rows, nullptr, streams, n_streams,
                            num_heads, head_dim, page_size, dtype, sm_scale, workspace, workspace_bytes, stream);
+}
+
+int lbm_attn_run_own(const void* q, const void* k, const void* v, void* out, const int32_t* kv_rows, const lbm_attn_stream* streams,
+                     int32_t n_streams, int32_t num_heads, int32_t head_dim, int32_t dtype, float sm_scale, void* workspace,
+                     size_t workspace_bytes, void* stream) {
+  return lbm_attn_run_impl("lbm_attn_run_own", q, k, out, k, v, kv_rows, nullptr, streams, n_streams, num_heads, head_dim, 1, dtype,
+                           sm_scale, workspace, workspace_bytes, stream, nullptr, 0, false, true);
 }
 
 int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k, const void* new_v,
@@ -356,7 +366,8 @@ int lbm_block_run(const lbm_block_weights* w, const lbm_block_call* c, void* str
   if (c->n_streams > 0) {
     rc = lbm_attn_run_impl("lbm_block_run", q, c->pool ? c->pool : k, heads, c->keep_kv ? k : nullptr, c->keep_kv ? v : nullptr,
                            c->kv_rows, c->live_kv_tokens, c->streams, c->n_streams, w->num_heads, 64, c->page_size, LBM_DTYPE_BF16,
-                           0.f, c->attn_workspace, c->attn_workspace_bytes, stream);
+                           0.f, c->attn_workspace, c->attn_workspace_bytes, stream, nullptr, 0, false,
+                           c->own_rows && c->keep_kv && !c->live_kv_tokens);
     if (rc != LBM_OK) return rc;
   }
   if (c->hints[1]) lbm_set_prefetch_hint(c->hints[1], c->hint_bytes[1]);

@@ -91,7 +91,8 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
                          const LbmAttnSchedule& sch,
                          int num_heads, int head_dim, int page_size, int dtype, float sm_scale,
                          void* workspace, hipStream_t stream,
-                         const int32_t* append_rows = nullptr, int append_tokens = 0, bool append_apart = false);
+                         const int32_t* append_rows = nullptr, int append_tokens = 0, bool append_apart = false,
+                         bool own_rows = false);
 
 #ifdef __HIPCC__
 // The append as workgroups of an attention launch: workgroup `wg` of those behind the attention's copies one 16-byte

@@ -813,7 +813,10 @@ static_assert(lbm_sm_lds_bytes(64) <= 160 * 1024, "LDS budget of the short-KV ke
 
 // QB: 32-row blocks of query rows per workgroup.  TURN: workgroups may begin at different pieces (an
 // instance of its own: what it adds in front of the first load takes 0.2 us, 3 % of a launch on 261 own rows).
-template <int QB, bool TURN>
+// OWN: token t of a stream is row kv_row_begin + t of the caller's K/V (lbm_attn_run_own): the rows are asked for
+// at once, without the trip to memory for their table entries and the one through LDS for their addresses (261
+// rows 5.5 -> 5.2 us, 1,004 rows 11.4 -> 10.6, 2,000 rows 29.4 -> 26.3).
+template <int QB, bool TURN, bool OWN = false>
 __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[lbm_sm_lds_bytes(32 * QB)];
   constexpr int kRows = 32 * QB;
@@ -897,6 +900,15 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
   auto find_rows = [&](int e) {   // negative entries name rows of the caller's own K/V
     sources[lane] = (unsigned long long)((e < 0 ? own_rows : pool_rows) + (unsigned long long)(unsigned)(e ^ (e >> 31)) * row_bytes);
   };
+  auto load_own_rows = [&](int pc, int stage) {
+    const char* k = (const char*)(a.self_k + (size_t)head * 64) + (size_t)sp.kv_row_begin * row_bytes;
+    const char* v = (const char*)(a.self_v + (size_t)head * 64) + (size_t)sp.kv_row_begin * row_bytes;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {   // K rows in j = 0..3, V rows in 4..7; tokens past the last re-read it
+      const unsigned at = (unsigned)min(pc * kSmPiece + (j & 3) * 8 + (lane >> 3), last_token) * row_bytes + (j < 4 ? chunk_k[j & 1] : chunk_v);
+      asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(at), "s"(j < 4 ? k : v), "s"(m0_ring + (unsigned)(stage * 2 * kSmPieceBytes + j * 1024)) : "memory", "m0");
+    }
+  };
   auto load_rows = [&](int stage) {
     unsigned long long at[8];
 #pragma unroll
@@ -909,6 +921,11 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
   };
   // pieces p0 and p0 + 1, as far as there are such, and the entries of the one after them on their way
   auto start = [&]() {
+    if (OWN) {
+      load_own_rows(p0, 0);
+      if (p0 + 1 < p1) load_own_rows(p0 + 1, 1);
+      return;
+    }
     load_entries(0);
     LBM_LOADS_LEFT(0);
     const int e0 = entries[n32], e1 = entries[kSmPiece + n32];
@@ -923,21 +940,36 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
     }
   };
   const int q_r = max(min(q_row0 + (tid >> 3), sp.q_rows - 1), 0);   // rows past the last one re-read it (never stored)
-  const u32x4 q_raw = *(const u32x4*)(a.q + ((size_t)(sp.q_begin + q_r) * H + head) * 64 + (tid & 7) * 8);
+  u32x4 q_raw = {};
+  if (!OWN) q_raw = *(const u32x4*)(a.q + ((size_t)(sp.q_begin + q_r) * H + head) * 64 + (tid & 7) * 8);
 
   // ---- Q: the workgroup reads its rows once as whole rows, every wavefront picks its fragments up
   // from LDS; scale * log2(e) folded in (as in the main kernel)
   bf16x8 qf[QB][4];
   {
     unsigned short* patch_q = (unsigned short*)(lds_raw + kSmOffQ);
-    if (QB == 2 || tid < kRows * 8) *(u32x4*)&patch_q[(tid >> 3) * kKStride + (tid & 7) * 8] = q_raw;
-    if (p0 < p1) start();
+    if (OWN) {
+      // Q travels to LDS directly as well, in front of K and V and unpadded (chunk c of row r at c ^ ((r >> 1) & 7)): a load
+      // that the compiler sees would make it wait for everything behind
+      if (QB == 2 || wave < 4) {
+        const unsigned short* src = a.q + ((size_t)(sp.q_begin + q_r) * H + head) * 64 + ((tid & 7) ^ ((tid >> 4) & 7)) * 8;
+        asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(src), "s"(lds_at(patch_q) + (unsigned)wave * 1024u) : "memory", "m0");
+      }
+      if (p0 < p1) start();
+      if (p0 + 1 < p1) LBM_LOADS_LEFT(16);
+      else if (p0 < p1) LBM_LOADS_LEFT(8);
+      else LBM_LOADS_LEFT(0);
+    } else {
+      if (QB == 2 || tid < kRows * 8) *(u32x4*)&patch_q[(tid >> 3) * kKStride + (tid & 7) * 8] = q_raw;
+      if (p0 < p1) start();
+    }
     __syncthreads();
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        const bf16x8 rawf = __builtin_bit_cast(bf16x8, *(const u32x4*)&patch_q[(qb * 32 + n32) * kKStride + ks * 16 + g * 8]);
+        const bf16x8 rawf = __builtin_bit_cast(bf16x8, *(const u32x4*)&patch_q[
+            OWN ? (qb * 32 + n32) * 64 + ((ks * 2 + g) ^ ((n32 >> 1) & 7)) * 8 : (qb * 32 + n32) * kKStride + ks * 16 + g * 8]);
         f32x8 f = __builtin_convertvector(rawf, f32x8);
 #pragma unroll
         for (int j = 0; j < 8; ++j) f[j] *= a.scale_log2;
@@ -1047,13 +1079,17 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
       }
       if (kAhead > 0) {   // the next piece has landed: its K fragments travel under this one's last MFMAs
         LBM_LOADS_LEFT(0);
-        if (kAhead == 2) find_rows(entries[n32]);
+        if (kAhead == 2 && !OWN) find_rows(entries[n32]);
         read_k(stage ^ 1);
       }
       if (kAhead == 2) {  // both buffers of this stage are read: the piece two ahead may come
         LBM_LDS_DONE();
-        load_entries(at + 3);
-        load_rows(stage);
+        if (OWN) {
+          load_own_rows(p0 + at + 2, stage);
+        } else {
+          load_entries(at + 3);
+          load_rows(stage);
+        }
       }
       // O^T += V^T P^T over the piece's two 16-row k-steps
 #pragma unroll
@@ -2051,7 +2087,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
                               const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                               const LbmAttnSchedule& sch, int num_heads, int head_dim, int page_size, int dtype,
                               float sm_scale, void* workspace, hipStream_t stream, const int32_t* append_rows,
-                              int append_tokens, bool append_apart, bool* appended);
+                              int append_tokens, bool append_apart, bool own_rows, bool* appended);
 }  // namespace
 
 // append_rows (lbm_attn_run_append): rows of self_k / self_v that are stored in the pool after the
@@ -2064,10 +2100,10 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
                          const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                          const LbmAttnSchedule& sch,
                          int num_heads, int head_dim, int page_size, int dtype, float sm_scale,
-                         void* workspace, hipStream_t stream, const int32_t* append_rows, int append_tokens, bool append_apart) {
+                         void* workspace, hipStream_t stream, const int32_t* append_rows, int append_tokens, bool append_apart, bool own_rows) {
   bool appended = false;
   int rc = lbm_launch_attention_only(q, pool, out, self_k, self_v, kv_rows, live_kv_tokens, sch, num_heads, head_dim,
-                                     page_size, dtype, sm_scale, workspace, stream, append_rows, append_tokens, append_apart, &appended);
+                                     page_size, dtype, sm_scale, workspace, stream, append_rows, append_tokens, append_apart, own_rows, &appended);
   if (rc != LBM_OK || !append_rows || append_tokens <= 0 || appended) return rc;
   return lbm_launch_append(self_k, self_v, dtype, const_cast<void*>(pool), dtype, append_rows, append_tokens, num_heads,
                            head_dim, page_size, stream);
@@ -2078,7 +2114,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
                               const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                               const LbmAttnSchedule& sch, int num_heads, int head_dim, int page_size, int dtype,
                               float sm_scale, void* workspace, hipStream_t stream, const int32_t* append_rows,
-                              int append_tokens, bool append_apart, bool* appended) {
+                              int append_tokens, bool append_apart, bool own_rows, bool* appended) {
   if (head_dim != 64 && !(head_dim == 128 && dtype == LBM_DTYPE_F32))
     return lbm_fail(LBM_ERR_UNSUPPORTED, "attention kernels cover head_dim 64 (bf16, fp32) and 128 (fp32), got %d", head_dim);
   if (dtype == LBM_DTYPE_F32) {
@@ -2194,6 +2230,11 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       a.append_tokens = append_tokens;
       blocks += (unsigned)(((long long)append_tokens * num_heads * 8 + kSmThreads - 1) / kSmThreads);
       *appended = true;
+    }
+    if (own_rows) {
+      if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false, true>), dim3(blocks), dim3(kSmThreads), 0, stream, a);
+      else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, false, true>), dim3(blocks), dim3(kSmThreads), 0, stream, a);
+      return lbm_check_launch("lbm_attn_bf16_d64_small_kernel<own rows>");
     }
     bool turn = false;   // (the kernel decides per stream, by the live count)
     for (int i = 0; i < sch.n_streams; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);

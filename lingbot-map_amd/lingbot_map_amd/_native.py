@@ -83,11 +83,11 @@ class BlockCall(C.Structure):
         "streams", "attn_workspace", "split_workspace")] + \
         [(n, C.c_size_t) for n in ("scratch_bytes", "attn_workspace_bytes", "split_workspace_bytes")] + [("q_scale", C.c_float)] + \
         [(n, C.c_int32) for n in ("rows", "stats_tiles", "rope_layout", "keep_kv", "n_streams", "page_size")] + \
-        [("hints", C.c_void_p * 4), ("hint_bytes", C.c_size_t * 4)]
+        [("hints", C.c_void_p * 4), ("hint_bytes", C.c_size_t * 4), ("own_rows", C.c_int32)]
 
 
 SYMBOLS = ("lbm_abi_version", "lbm_last_error", "lbm_tables_words", "lbm_tables_step",
-           "lbm_rows_from_pages", "lbm_kv_append", "lbm_qkv_prepare", "lbm_residual_norm", "lbm_linear", "lbm_linear_norm", "lbm_linear_stats_tiles", "lbm_linear_workspace_bytes", "lbm_linear_prefetch_hint", "lbm_qkv_linear_prepare", "lbm_qkv_linear_prepare_norm", "lbm_attn_workspace_bytes", "lbm_attn_run", "lbm_attn_run_append", "lbm_attn_run_append_apart", "lbm_attn_run_live",
+           "lbm_rows_from_pages", "lbm_kv_append", "lbm_qkv_prepare", "lbm_residual_norm", "lbm_linear", "lbm_linear_norm", "lbm_linear_stats_tiles", "lbm_linear_workspace_bytes", "lbm_linear_prefetch_hint", "lbm_qkv_linear_prepare", "lbm_qkv_linear_prepare_norm", "lbm_attn_workspace_bytes", "lbm_attn_run", "lbm_attn_run_own", "lbm_attn_run_append", "lbm_attn_run_append_apart", "lbm_attn_run_live",
            "lbm_attn_run_static", "lbm_block_scratch_bytes", "lbm_block_run")
 
 
@@ -131,6 +131,8 @@ def _load():
     lib.lbm_attn_run.restype = C.c_int
     lib.lbm_attn_run.argtypes = [vp, vp, vp, vp, vp, vp, p(AttnStream), i32, i32, i32, i32, i32,
                                  C.c_float, vp, C.c_size_t, vp]
+    lib.lbm_attn_run_own.restype = C.c_int
+    lib.lbm_attn_run_own.argtypes = [vp, vp, vp, vp, vp, p(AttnStream), i32, i32, i32, i32, C.c_float, vp, C.c_size_t, vp]
     lib.lbm_attn_run_append.restype = C.c_int
     lib.lbm_attn_run_append.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, p(AttnStream), i32, i32, i32, i32, i32,
                                         C.c_float, vp, C.c_size_t, vp]

@@ -825,7 +825,7 @@ class HipPagedBlock(nn.Module):
             x.data_ptr(), a.data_ptr(), stats_ptr, out.data_ptr(), None if stats_out is None else stats_out.data_ptr(),
             scratch.data_ptr(), None if table is None else table.data_ptr(), pool, append, kv_rows, live, streams, ws.data_ptr(),
             None if split is None else split.data_ptr(), sizes[0], ws.numel(), 0 if split is None else split.numel(),
-            native.q_scale, rows, stats_tiles, layout, keep_kv, n_streams, page, hints[0], hints[1])
+            native.q_scale, rows, stats_tiles, layout, keep_kv, n_streams, page, hints[0], hints[1], not streaming)
         N.check(N.lib.lbm_block_run(weights, call, N.stream_handle(x.device)))
         return out if next_norm is None else (out, RowStats(stats_out, sizes[1]))
 

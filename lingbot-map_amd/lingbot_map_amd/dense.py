@@ -53,9 +53,8 @@ def dense_attention(q: Tensor, k: Tensor, v: Tensor, num_streams: int = 1, q_pre
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     kv_rows, streams, ws = dense_plan(rows, num_streams, H, D, q.device)
     out = torch.empty_like(q)
-    k_ptr = k.data_ptr()
-    N.check(N.lib.lbm_attn_run(
-        q.data_ptr(), k_ptr, out.data_ptr(), k_ptr, v.data_ptr(), kv_rows.data_ptr(), streams, num_streams, H, D, 16,
+    N.check(N.lib.lbm_attn_run_own(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kv_rows.data_ptr(), streams, num_streams, H, D,
         N.DTYPE_BF16 if q.dtype == torch.bfloat16 else N.DTYPE_F32, 0.0 if q_prescaled else 1.0 / math.sqrt(D),
         ws.data_ptr(), ws.numel(), N.stream_handle(q.device)))
     return out
