@@ -312,21 +312,29 @@ int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k,
                         int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
                         void* workspace, size_t workspace_bytes, void* stream);
 
-/* lbm_attn_run_append for a row table that names no row of append_rows (ABI 11), as the plans of
- * lbm_tables_step with LBM_OP_PLAN_NEWEST_SELF do: with nobody reading those rows, attention launches that
- * merge nothing carry the append as well, by workgroups of their own.  Same results. */
-int lbm_attn_run_append_apart(const void* q, void* pool, void* out, const void* new_k, const void* new_v,
-                              const int32_t* kv_rows, const int32_t* append_rows, int32_t append_tokens,
-                              const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads,
-                              int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
-                              void* workspace, size_t workspace_bytes, void* stream);
-
-/* lbm_attn_run over the streams' own rows in order (ABI 11): entry kv_row_begin + t of kv_rows is
- * -1 - (kv_row_begin + t) for every token t of every stream, which the caller promises and launches that split no
- * KV rely on instead of reading it.  Same results.  k, v: as self_k, self_v. */
-int lbm_attn_run_own(const void* q, const void* k, const void* v, void* out, const int32_t* kv_rows, const lbm_attn_stream* streams,
-                     int32_t n_streams, int32_t num_heads, int32_t head_dim, int32_t dtype, float sm_scale, void* workspace,
-                     size_t workspace_bytes, void* stream);
+/* An attention call as one record (ABI 11): lbm_attn_run, or lbm_attn_run_live with live_kv_tokens, or
+ * lbm_attn_run_append with append_rows (not both), and what only a record's flags say:
+ *   LBM_ATTN_OWN_ROWS      entry kv_row_begin + t of kv_rows is -1 - (kv_row_begin + t) for every token t of every
+ *                          stream: launches that split no KV rely on it instead of reading the table
+ *   LBM_ATTN_APPEND_APART  kv_rows names no row of append_rows, as the plans of lbm_tables_step with
+ *                          LBM_OP_PLAN_NEWEST_SELF do: launches that merge nothing carry the append as well, by
+ *                          workgroups of their own
+ * Same results with and without the flags. */
+#define LBM_ATTN_OWN_ROWS 1
+#define LBM_ATTN_APPEND_APART 2
+typedef struct lbm_attn_call {
+  const void* q;
+  void* pool;
+  void* out;
+  const void *self_k, *self_v;
+  const int32_t *kv_rows, *live_kv_tokens, *append_rows;
+  const lbm_attn_stream* streams;
+  void* workspace;
+  size_t workspace_bytes;
+  float sm_scale;
+  int32_t append_tokens, n_streams, num_heads, head_dim, page_size, dtype, flags;
+} lbm_attn_call;
+int lbm_attn_run_call(const lbm_attn_call* call, void* stream);
 
 /* A whole transformer block of the streaming model in one call (ABI 10): qkv projection + producer,
  * attention, proj + LayerScale + residual, fc1 + GELU, fc2 + LayerScale + residual
@@ -367,7 +375,7 @@ typedef struct lbm_block_call {
                                 * n_streams 0: no attention, the caller filled its output */
   const void* hints[4];        /* lbm_linear_prefetch_hint in front of the four GEMM launches; NULL: none */
   size_t hint_bytes[4];
-  int32_t own_rows;            /* ABI 11; 1: kv_rows is as lbm_attn_run_own takes it (with keep_kv) */
+  int32_t own_rows;            /* ABI 11; 1: kv_rows is as LBM_ATTN_OWN_ROWS says (with keep_kv) */
 } lbm_block_call;
 
 size_t lbm_block_scratch_bytes(int32_t rows, int32_t num_heads, int32_t hidden);

@@ -255,13 +255,6 @@ int lbm_attn_run(const void* q, const void* pool, void* out, const void* self_k,
                            num_heads, head_dim, page_size, dtype, sm_scale, workspace, workspace_bytes, stream);
 }
 
-int lbm_attn_run_own(const void* q, const void* k, const void* v, void* out, const int32_t* kv_rows, const lbm_attn_stream* streams,
-                     int32_t n_streams, int32_t num_heads, int32_t head_dim, int32_t dtype, float sm_scale, void* workspace,
-                     size_t workspace_bytes, void* stream) {
-  return lbm_attn_run_impl("lbm_attn_run_own", q, k, out, k, v, kv_rows, nullptr, streams, n_streams, num_heads, head_dim, 1, dtype,
-                           sm_scale, workspace, workspace_bytes, stream, nullptr, 0, false, true);
-}
-
 int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k, const void* new_v,
                         const int32_t* kv_rows, const int32_t* append_rows, int32_t append_tokens,
                         const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads,
@@ -275,17 +268,14 @@ int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k,
                            append_rows, append_tokens);
 }
 
-int lbm_attn_run_append_apart(const void* q, void* pool, void* out, const void* new_k, const void* new_v,
-                              const int32_t* kv_rows, const int32_t* append_rows, int32_t append_tokens,
-                              const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads,
-                              int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
-                              void* workspace, size_t workspace_bytes, void* stream) {
-  if (!new_k || !new_v || !append_rows)
-    return lbm_fail(LBM_ERR_INVALID, "lbm_attn_run_append_apart: null new_k, new_v or append_rows");
-  if (append_tokens < 0) return lbm_fail(LBM_ERR_INVALID, "lbm_attn_run_append_apart: negative append_tokens");
-  return lbm_attn_run_impl("lbm_attn_run_append_apart", q, pool, out, new_k, new_v, kv_rows, nullptr, streams, n_streams,
-                           num_heads, head_dim, page_size, dtype, sm_scale, workspace, workspace_bytes, stream,
-                           append_rows, append_tokens, true);
+int lbm_attn_run_call(const lbm_attn_call* c, void* stream) {
+  if (!c) return lbm_fail(LBM_ERR_INVALID, "lbm_attn_run_call: null call");
+  if (c->append_rows && (!c->self_k || !c->self_v || c->append_tokens < 0 || c->live_kv_tokens))
+    return lbm_fail(LBM_ERR_INVALID, "lbm_attn_run_call: append_rows with null self_k or self_v, negative append_tokens or live_kv_tokens");
+  return lbm_attn_run_impl("lbm_attn_run_call", c->q, c->pool, c->out, c->self_k, c->self_v, c->kv_rows, c->live_kv_tokens, c->streams,
+                           c->n_streams, c->num_heads, c->head_dim, c->page_size, c->dtype, c->sm_scale, c->workspace,
+                           c->workspace_bytes, stream, c->append_rows, c->append_rows ? c->append_tokens : 0,
+                           (c->flags & LBM_ATTN_APPEND_APART) != 0, (c->flags & LBM_ATTN_OWN_ROWS) && c->self_k && !c->live_kv_tokens);
 }
 
 int lbm_attn_run_live(const void* q, const void* pool, void* out, const void* self_k,

@@ -78,7 +78,7 @@ struct AttnArgsF32 {
   int n_streams;
   lbm_attn_stream s[LBM_MAX_STREAMS];
   int wg_begin[LBM_MAX_STREAMS + 1];
-  // the append carried by workgroups behind the attention's (lbm_attn_run_append_apart; 0 tokens: none): row t of
+  // the append carried by workgroups behind the attention's (LBM_ATTN_APPEND_APART; 0 tokens: none): row t of
   // self_k / self_v to pool row append_rows[t]
   const int32_t* append_rows;
   int append_tokens;

@@ -813,7 +813,7 @@ static_assert(lbm_sm_lds_bytes(64) <= 160 * 1024, "LDS budget of the short-KV ke
 
 // QB: 32-row blocks of query rows per workgroup.  TURN: workgroups may begin at different pieces (an
 // instance of its own: what it adds in front of the first load takes 0.2 us, 3 % of a launch on 261 own rows).
-// OWN: token t of a stream is row kv_row_begin + t of the caller's K/V (lbm_attn_run_own): the rows are asked for
+// OWN: token t of a stream is row kv_row_begin + t of the caller's K/V (LBM_ATTN_OWN_ROWS): the rows are asked for
 // at once, without the trip to memory for their table entries and the one through LDS for their addresses (261
 // rows 5.5 -> 5.2 us, 1,004 rows 11.4 -> 10.6, 2,000 rows 29.4 -> 26.3).
 template <int QB, bool TURN, bool OWN = false>

@@ -6,6 +6,7 @@ from __future__ import annotations
 import contextlib
 import ctypes as C
 import os
+import struct
 
 from .build import LIB_PATH
 
@@ -63,6 +64,17 @@ class AttnStream(C.Structure):
     _fields_ = [(n, C.c_int32) for n in ("q_begin", "q_rows", "kv_row_begin", "kv_tokens", "live_at")]
 
 
+# ``lbm_attn_call`` as two packed pieces, which the caller puts one behind the other: what differs from call to
+# call (nine addresses, 0 for none, the workspace's address and size, the softmax scale) and what a plan's calls
+# have in common (``attn_call_tail``).  0.5 us a call; eighteen arguments one by one take the binding 2.7.
+ATTN_CALL_HEAD = struct.Struct("10PNf")
+ATTN_OWN_ROWS, ATTN_APPEND_APART = 1, 2
+
+
+def attn_call_tail(append_tokens: int, n_streams: int, num_heads: int, head_dim: int, page_size: int, dtype: int, flags: int) -> bytes:
+    return struct.pack("7i", append_tokens, n_streams, num_heads, head_dim, page_size, dtype, flags)
+
+
 class RowNorm(C.Structure):
     """``lbm_row_norm``: a LayerNorm folded into the launch that consumes its output."""
     _fields_ = [("stats", C.c_void_p), ("w_colsum", C.c_void_p), ("stats_tiles", C.c_int32), ("eps", C.c_float)]
@@ -87,7 +99,7 @@ class BlockCall(C.Structure):
 
 
 SYMBOLS = ("lbm_abi_version", "lbm_last_error", "lbm_tables_words", "lbm_tables_step",
-           "lbm_rows_from_pages", "lbm_kv_append", "lbm_qkv_prepare", "lbm_residual_norm", "lbm_linear", "lbm_linear_norm", "lbm_linear_stats_tiles", "lbm_linear_workspace_bytes", "lbm_linear_prefetch_hint", "lbm_qkv_linear_prepare", "lbm_qkv_linear_prepare_norm", "lbm_attn_workspace_bytes", "lbm_attn_run", "lbm_attn_run_own", "lbm_attn_run_append", "lbm_attn_run_append_apart", "lbm_attn_run_live",
+           "lbm_rows_from_pages", "lbm_kv_append", "lbm_qkv_prepare", "lbm_residual_norm", "lbm_linear", "lbm_linear_norm", "lbm_linear_stats_tiles", "lbm_linear_workspace_bytes", "lbm_linear_prefetch_hint", "lbm_qkv_linear_prepare", "lbm_qkv_linear_prepare_norm", "lbm_attn_workspace_bytes", "lbm_attn_run", "lbm_attn_run_append", "lbm_attn_run_live", "lbm_attn_run_call",
            "lbm_attn_run_static", "lbm_block_scratch_bytes", "lbm_block_run")
 
 
@@ -131,13 +143,11 @@ def _load():
     lib.lbm_attn_run.restype = C.c_int
     lib.lbm_attn_run.argtypes = [vp, vp, vp, vp, vp, vp, p(AttnStream), i32, i32, i32, i32, i32,
                                  C.c_float, vp, C.c_size_t, vp]
-    lib.lbm_attn_run_own.restype = C.c_int
-    lib.lbm_attn_run_own.argtypes = [vp, vp, vp, vp, vp, p(AttnStream), i32, i32, i32, i32, C.c_float, vp, C.c_size_t, vp]
     lib.lbm_attn_run_append.restype = C.c_int
     lib.lbm_attn_run_append.argtypes = [vp, vp, vp, vp, vp, vp, vp, i32, p(AttnStream), i32, i32, i32, i32, i32,
                                         C.c_float, vp, C.c_size_t, vp]
-    lib.lbm_attn_run_append_apart.restype = C.c_int
-    lib.lbm_attn_run_append_apart.argtypes = lib.lbm_attn_run_append.argtypes
+    lib.lbm_attn_run_call.restype = C.c_int
+    lib.lbm_attn_run_call.argtypes = [C.c_char_p, vp]
     lib.lbm_attn_run_live.restype = C.c_int
     lib.lbm_attn_run_live.argtypes = [vp, vp, vp, vp, vp, vp, vp, p(AttnStream), i32, i32, i32, i32, i32,
                                       C.c_float, vp, C.c_size_t, vp]
@@ -170,7 +180,6 @@ def check(rc: int) -> None:
 def q_scale_log2(sm_scale: float) -> float:
     """The ``q_scale`` to hand the producers so that ``lbm_attn_run`` can be called with
     ``sm_scale = 0``: the softmax scale times log2(e), as a float32 value."""
-    import struct
     return struct.unpack("f", struct.pack("f", sm_scale * 1.4426950408889634))[0]
 
 

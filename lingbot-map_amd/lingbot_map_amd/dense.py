@@ -7,6 +7,7 @@ of the caller's own K/V, the pool is never read.
 """
 from __future__ import annotations
 
+import ctypes as C
 import math
 from typing import Dict
 
@@ -16,6 +17,7 @@ from torch import Tensor
 from . import _native as N
 
 _plans: Dict[tuple, tuple] = {}          # (rows, streams, H, D, device) -> (row table, stream descriptors, workspace bytes)
+_tails: Dict[tuple, bytes] = {}          # (streams, H, D, dtype) -> what the calls of such a plan have in common
 _workspace: Dict[object, Tensor] = {}
 
 
@@ -51,10 +53,15 @@ def dense_attention(q: Tensor, k: Tensor, v: Tensor, num_streams: int = 1, q_pre
     rows, H, D = q.shape
     assert 1 <= num_streams <= N.MAX_STREAMS and rows % num_streams == 0
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-    kv_rows, streams, ws = dense_plan(rows, num_streams, H, D, q.device)
+    device = q.device
+    kv_rows, streams, ws = dense_plan(rows, num_streams, H, D, device)
+    tail = _tails.get((num_streams, H, D, q.dtype))
+    if tail is None:
+        tail = _tails[(num_streams, H, D, q.dtype)] = N.attn_call_tail(
+            0, num_streams, H, D, 16, N.DTYPE_BF16 if q.dtype == torch.bfloat16 else N.DTYPE_F32, N.ATTN_OWN_ROWS)
     out = torch.empty_like(q)
-    N.check(N.lib.lbm_attn_run_own(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), kv_rows.data_ptr(), streams, num_streams, H, D,
-        N.DTYPE_BF16 if q.dtype == torch.bfloat16 else N.DTYPE_F32, 0.0 if q_prescaled else 1.0 / math.sqrt(D),
-        ws.data_ptr(), ws.numel(), N.stream_handle(q.device)))
+    k_ptr = k.data_ptr()
+    N.check(N.lib.lbm_attn_run_call(N.ATTN_CALL_HEAD.pack(
+        q.data_ptr(), k_ptr, out.data_ptr(), k_ptr, v.data_ptr(), kv_rows.data_ptr(), 0, 0, C.addressof(streams), ws.data_ptr(),
+        ws.numel(), 0.0 if q_prescaled else 1.0 / math.sqrt(D)) + tail, N.stream_handle(device)))
     return out

@@ -183,15 +183,15 @@ class HipPagedKVCacheManager:
         # append rows of a pass of several frames that block 0 made in one go (begin_frames), until block
         # 0 moves on: (appends before it, frames, rows [streams, frames, tokens])
         self._pass_rows = [None] * self._n_sets
-        #: step(): the attention call stores the new frame itself (lbm_attn_run_append_apart), reading it
+        #: step(): the attention call stores the new frame itself (append_rows of lbm_attn_run_call), reading it
         #: from the caller's tensors meanwhile - no append launch in front of the attention
         self.fuse_append = True
         self._newest_self = [False] * self._n_sets   # the set's row table names the newest frame by the caller's rows
         self._n_appends: List[int] = [0] * num_blocks    # appends ever made per block (rollbacks do not count down)
         # what the launches of one plan have in common, kept per table set until the plan's token
         # counts change: (counts, stream descriptors, their address, streams with tokens, workspace
-        # bytes, the arguments of the attention call that follow from it)
-        self._launches = [((), None, 0, 0, 0, ()) for _ in range(self._n_sets)]
+        # bytes, the tail of the attention call's record)
+        self._launches = [((), None, 0, 0, 0, b"") for _ in range(self._n_sets)]
         self._sm_scale = 1.0 / math.sqrt(head_dim)
         self._frame_shape = torch.Size((num_streams * tokens_per_frame, num_heads, head_dim))
         # a step's operations, with the fields that never change filled in
@@ -659,15 +659,19 @@ class HipPagedKVCacheManager:
         reads it from the caller's rows only.
         ``newest_self`` (leading block): the row table names the rows a keyframe appends by the
         caller's own K/V rows; every block of the frame then attends and appends with
-        ``lbm_attn_run_append_apart`` (``step`` does), which ``_newest_self`` remembers."""
-        if keyframe is None:
-            keyframe = (not self._skip_append,) * self.num_streams
+        one call (``step`` does), which ``_newest_self`` remembers."""
+        if keyframe is None and False not in self._active:
+            every, none = (True,) * self.num_streams, (False,) * self.num_streams
+            keyframe, tail = (none, every) if self._skip_append else (every, none)
         else:
-            keyframe = list(keyframe)
-            if len(keyframe) != self.num_streams:
-                raise IndexError(f"keyframe: {len(keyframe)} flags for {self.num_streams} streams")
-        keyframe = [a and bool(x) for a, x in zip(self._active, keyframe)]
-        tail = [a and not x for a, x in zip(self._active, keyframe)]
+            if keyframe is None:
+                keyframe = (not self._skip_append,) * self.num_streams
+            else:
+                keyframe = list(keyframe)
+                if len(keyframe) != self.num_streams:
+                    raise IndexError(f"keyframe: {len(keyframe)} flags for {self.num_streams} streams")
+            keyframe = [a and bool(x) for a, x in zip(self._active, keyframe)]
+            tail = [a and not x for a, x in zip(self._active, keyframe)]
         stores = True in keyframe
         ts = block_idx if self.per_block_tables else 0
         if block_idx == ts:
@@ -707,7 +711,7 @@ class HipPagedKVCacheManager:
         """``q_prescaled``: q already carries 1 / sqrt(D) and log2(e) (``step_qkv``'s producer).
         ``append_rows``: the address of the rows ``self_k`` / ``self_v`` are also stored in, row t in
         pool row ``append_rows[t]``: pages of this frame, which its plan names by the caller's rows
-        (``lbm_attn_run_append_apart``)."""
+        (``LBM_ATTN_APPEND_APART``)."""
         ts = self._set(block_idx)
         if self._newest_self[ts] and append_rows is None:
             raise RuntimeError("this frame's row table names its newest frame by the caller's K/V rows (step() led "
@@ -717,13 +721,13 @@ class HipPagedKVCacheManager:
         if not qc.is_contiguous():
             qc = qc.contiguous()
         out = torch.empty_like(qc)
-        k_ptr = v_ptr = None
+        k_ptr = v_ptr = 0
         if self_k is not None:
             if self_k.dtype != self.dtype:
                 self_k, self_v = self_k.to(self.dtype), self_v.to(self.dtype)
             self_k, self_v = self_k.contiguous(), self_v.contiguous()
             k_ptr, v_ptr = self_k.data_ptr(), self_v.data_ptr()
-        _, streams, _, n, need, common = self._launch_plan(ts)
+        _, _, streams, n, need, tail = self._launch_plan(ts)
         if n < self.num_streams:
             out.zero_()
         if n == 0:
@@ -731,14 +735,10 @@ class HipPagedKVCacheManager:
                 self._scatter(block_idx, self._append_rows[ts], self_k, self_v)
             return out
         ws = self._workspace(need)
-        tail = (0.0 if q_prescaled else self._sm_scale, ws.data_ptr(), ws.numel(), self._stream_handle())
-        tensors = (qc.data_ptr(), self.kv_caches[block_idx].data_ptr(), out.data_ptr(), k_ptr, v_ptr, self._kv_rows_ptr(ts))
-        if append_rows is not None:
-            N.check(N.lib.lbm_attn_run_append_apart(*tensors, append_rows, self_k.shape[0], *common, *tail))
-        elif self.device_token_counts:
-            N.check(N.lib.lbm_attn_run_live(*tensors, self._live_counts_ptr(ts), *common, *tail))
-        else:
-            N.check(N.lib.lbm_attn_run(*tensors, *common, *tail))
+        live = self._live_counts_ptr(ts) if self.device_token_counts and append_rows is None else 0
+        N.check(N.lib.lbm_attn_run_call(N.ATTN_CALL_HEAD.pack(
+            qc.data_ptr(), self.kv_caches[block_idx].data_ptr(), out.data_ptr(), k_ptr, v_ptr, self._kv_rows_ptr(ts), live,
+            append_rows or 0, streams, ws.data_ptr(), ws.numel(), 0.0 if q_prescaled else self._sm_scale) + tail, self._stream_handle()))
         return out
 
     def _launch_plan(self, ts: int):
@@ -753,9 +753,9 @@ class HipPagedKVCacheManager:
                     streams[n] = N.AttnStream(b * T, T, b * self._rows_cap, kv, b * self._table_words)
                     n += 1
             need = int(N.lib.lbm_attn_workspace_bytes(streams, n, self.num_heads, self.head_dim)) if n else 0
-            common = (streams, n, self.num_heads, self.head_dim, self.page_size,
-                      N.DTYPE_BF16 if self.dtype == torch.bfloat16 else N.DTYPE_F32)
-            hit = self._launches[ts] = (counts, streams, C.addressof(streams), n, need, common)
+            tail = N.attn_call_tail(self._frame_shape[0], n, self.num_heads, self.head_dim, self.page_size,
+                                    N.DTYPE_BF16 if self.dtype == torch.bfloat16 else N.DTYPE_F32, N.ATTN_APPEND_APART)
+            hit = self._launches[ts] = (counts, streams, C.addressof(streams), n, need, tail)
         return hit
 
     def _workspace(self, need: int) -> Tensor:

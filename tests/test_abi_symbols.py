@@ -46,6 +46,9 @@ def test_binding_constants_match_header():
     assert (defs["LBM_LAYOUT_TWO_STREAM"], defs["LBM_LAYOUT_FRAME_PAGES"]) == (N.LAYOUT_TWO_STREAM, N.LAYOUT_FRAME_PAGES)
     # struct sizes: plain int32 fields, no padding
     assert C.sizeof(N.CacheGeom) == 9 * 4 and C.sizeof(N.StepOp) == 8 * 4 and C.sizeof(N.AttnStream) == 5 * 4
+    # lbm_attn_call: ten pointers, a size, a float and seven ints without holes
+    assert N.ATTN_CALL_HEAD.size == 11 * 8 + 4 and len(N.attn_call_tail(0, 1, 2, 3, 4, 5, 6)) == 7 * 4
+    assert (defs["LBM_ATTN_OWN_ROWS"], defs["LBM_ATTN_APPEND_APART"]) == (N.ATTN_OWN_ROWS, N.ATTN_APPEND_APART)
 
 
 def test_host_side_argument_checks_need_no_gpu():
