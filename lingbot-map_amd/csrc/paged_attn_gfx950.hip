@@ -1544,12 +1544,7 @@ __global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32 a) {
 namespace {
 constexpr int kDecQ = 8;         // query rows per stream this path takes
 constexpr int kDecBatch = 8;     // tokens a row group has in flight
-constexpr int kDecOneBatch = 11; // the same where one workgroup takes everything, 16 (head_dim 128) or 32 row groups:
-                                 // a step loads its batch whether the tokens are there or not, so a short list
-                                 // wants few and a long one few trips.  us a launch at head_dim 128, 16 heads, for
-                                 // 6 / 8 / 11 / 20: 64 tokens 3.7 / 4.2 / 4.5 / 6.4, 150 5.8 / 6.6 / 5.4 / 7.1, 300 8.1 / 8.3 /
-                                 // 7.5 / 7.6, 512 10.4 / 10.2 / 9.7 / 11.3; means over 13 lengths from 16 to 512 tokens 6.8 /
-                                 // 7.0 / 6.9 / 8.3, at head_dim 64 5.0 / 5.3 / 5.5 / 6.8
+constexpr int kDecOneBatch = 11; // the most where one workgroup takes everything, 16 (head_dim 128) or 32 row groups
 constexpr int kDecChunk = 256;   // tokens per chunk, as long as that makes at most kDecMaxChunks
 constexpr int kDecMaxChunks = 64;
 constexpr int kDecOneTokens = 512;
@@ -2177,8 +2172,23 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
         if (!carries) d.append_rows = nullptr;
         else *appended = true;
         const dim3 grid(1, num_heads, sch.n_streams * max_q), block(kDecOneWaves * 64);
-        if (head_dim == 64) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<64, kDecOneWaves, kDecOneBatch, true>), grid, block, 0, stream, d);
-        else hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<128, kDecOneWaves, kDecOneBatch, true>), grid, block, 0, stream, d);
+        // As few trips as batches of eleven need, and batches no longer than so many trips need: a step loads its
+        // batch whether the tokens are there or not, 0.13 us for 16 rows of 128 floats at a CU's 64 bytes per cycle.
+        // us a launch, 16 heads, batches of eleven and these: head_dim 128, 16 tokens 4.3, 2.8; 64 4.3, 3.1; 100 4.3, 4.0;
+        // 200 6.2, 5.7; head_dim 64, 100 tokens 4.2, 3.1; 400 6.2, 5.5.  (Ten: no better than eleven.)
+        const int groups = kDecOneWaves * 256 / head_dim, trips = (most + kDecOneBatch * groups - 1) / (kDecOneBatch * groups);
+        const int batch = trips > 0 ? (most + trips * groups - 1) / (trips * groups) : 1;
+#define LBM_DECODE_ONE(NB)                                                                                                                    \
+  {                                                                                                                                          \
+    if (head_dim == 64) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<64, kDecOneWaves, NB, true>), grid, block, 0, stream, d);               \
+    else hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<128, kDecOneWaves, NB, true>), grid, block, 0, stream, d);                             \
+  }
+        if (batch <= 2) LBM_DECODE_ONE(2)
+        else if (batch <= 4) LBM_DECODE_ONE(4)
+        else if (batch <= 6) LBM_DECODE_ONE(6)
+        else if (batch <= 8) LBM_DECODE_ONE(8)
+        else LBM_DECODE_ONE(kDecOneBatch)
+#undef LBM_DECODE_ONE
         return lbm_check_launch("lbm_attn_f32_decode_kernel<one chunk>");
       }
       const dim3 grid(max_chunks, num_heads, sch.n_streams * max_q), block(kDecChunkWaves * 64);
