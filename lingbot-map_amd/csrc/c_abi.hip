@@ -216,7 +216,7 @@ size_t lbm_attn_workspace_bytes(const lbm_attn_stream* streams, int32_t n_stream
   if (num_heads <= 0 || head_dim <= 0) return 0;
   LbmAttnSchedule sch;
   lbm_attn_schedule(streams, n_streams, num_heads, &sch);
-  return lbm_attn_schedule_bytes(sch, num_heads, head_dim);
+  return lbm_attn_schedule_bytes(sch, num_heads, head_dim, false);
 }
 
 static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, void* out, const void* self_k,
@@ -239,11 +239,11 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
   for (int i = 0; own_rows && i < n_streams; ++i) own_rows = (long long)streams[i].kv_tokens * num_heads * head_dim * 2 < (1LL << 32);
   LbmAttnSchedule sch;
   lbm_attn_schedule(streams, n_streams, num_heads, &sch);
-  const size_t need = lbm_attn_schedule_bytes(sch, num_heads, head_dim);
+  const size_t need = lbm_attn_schedule_bytes(sch, num_heads, head_dim, true);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return lbm_fail(LBM_ERR_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", who, workspace_bytes, need);
   return lbm_launch_attention(q, pool, out, self_k, self_v, kv_rows, live_kv_tokens, sch, num_heads, head_dim,
-                              page_size, dtype, sm_scale, workspace, (hipStream_t)stream, append_rows, append_tokens, append_apart, own_rows);
+                              page_size, dtype, sm_scale, workspace, workspace_bytes, (hipStream_t)stream, append_rows, append_tokens, append_apart, own_rows);
 }
 
 int lbm_attn_run(const void* q, const void* pool, void* out, const void* self_k,
@@ -298,7 +298,7 @@ int lbm_attn_run_static(const void* q, const void* pool, void* out, const void* 
   if (num_heads <= 0 || head_dim <= 0) return lbm_fail(LBM_ERR_INVALID, "lbm_attn_run_static: non-positive size");
   LbmAttnSchedule sch;
   lbm_attn_schedule(streams, n_streams, num_heads, &sch);
-  const size_t need = lbm_attn_schedule_bytes(sch, num_heads, head_dim);
+  const size_t need = lbm_attn_schedule_bytes(sch, num_heads, head_dim, true);
   void* ws = nullptr;
   size_t ws_bytes = 0;
   rc = lbm_static_scratch(&ws, &ws_bytes);

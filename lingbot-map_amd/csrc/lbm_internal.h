@@ -62,7 +62,8 @@ struct LbmAttnSchedule {
 };
 void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_heads,
                        LbmAttnSchedule* out);
-size_t lbm_attn_schedule_bytes(const LbmAttnSchedule& sch, int num_heads, int head_dim);
+// least: what a launch cannot do without; otherwise what it is fastest with
+size_t lbm_attn_schedule_bytes(const LbmAttnSchedule& sch, int num_heads, int head_dim, bool least);
 
 struct AttnArgsF32 {
   const float* q;
@@ -90,7 +91,7 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
                          const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                          const LbmAttnSchedule& sch,
                          int num_heads, int head_dim, int page_size, int dtype, float sm_scale,
-                         void* workspace, hipStream_t stream,
+                         void* workspace, size_t workspace_bytes, hipStream_t stream,
                          const int32_t* append_rows = nullptr, int append_tokens = 0, bool append_apart = false,
                          bool own_rows = false);
 

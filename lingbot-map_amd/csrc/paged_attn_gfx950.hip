@@ -1539,13 +1539,15 @@ __global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32 a) {
 //
 // Up to kDecOneTokens tokens one workgroup of eight wavefronts takes a (stream, head, query row) from
 // start to finish: one launch, which also stores the caller's new rows (lbm_attn_run_append).
-// Beyond that the KV axis is cut into chunks of about 256 tokens, one workgroup of four wavefronts
-// each, which leave partial results for lbm_attn_f32_decode_merge_kernel.
+// Beyond that the KV axis is cut into chunks of 256 down to 64 tokens, one workgroup of four wavefronts
+// each, which leave partial results for lbm_attn_f32_decode_merge_kernel.  Where the chip has workgroups to spare a
+// chunk of 64 tokens is one batch of its eight row groups (head_dim 128): one trip to memory instead of four in a row.
 namespace {
 constexpr int kDecQ = 8;         // query rows per stream this path takes
 constexpr int kDecBatch = 8;     // tokens a row group has in flight
 constexpr int kDecOneBatch = 11; // the most where one workgroup takes everything, 16 (head_dim 128) or 32 row groups
 constexpr int kDecChunk = 256;   // tokens per chunk, as long as that makes at most kDecMaxChunks
+constexpr int kDecFineChunk = 64, kDecFineWgs = 512, kDecFineChunks = 16;   // shorter chunks, within so many workgroups a launch and chunks a row
 constexpr int kDecMaxChunks = 64;
 constexpr int kDecOneTokens = 512;
 constexpr int kDecOneWaves = 8, kDecChunkWaves = 4;
@@ -1756,8 +1758,29 @@ __global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeAr
 
 // Chunks per stream for the few-query path, and the floats of partials they need.  Depends on
 // row and token counts only (never on the dtype), so the workspace query can include it.
-static int lbm_decode_chunks(int kv_tokens) {
+//
+// fine_chunks: chunks of 64 tokens up to so many per row, 0 for none.  As many as leave the launch at two workgroups
+// per CU: beyond that its time is that of the bytes and not of the trips.  No more than sixteen a row, since the
+// merge's time grows with them; but thirty-two for caches of 128 floats a row from 3,072 tokens up, where sixteen would be
+// chunks of nearly 256 again.  us a launch, 16 heads, caches in HBM, chunks of 256 | these: head_dim 128, one row over 500
+// tokens 14.5 | 9.1, 700 14.9 | 10.1, 1,500 16.5 | 12.0, 3,000 18.3 | 16.7, 5,000 25.0 | 22.2; four streams of 1,000
+// 20.4 | 17.9; head_dim 64, 700 11.1 | 9.4, 3,000 13.1 | 12.3, four streams of 1,000 13.9 | 12.8.  (Eight rows of one
+// stream, that is four chunks a row: head_dim 64, 700 tokens 11.4 | 11.8, so not from there.)
+static int lbm_decode_fine_chunks(const LbmAttnSchedule& sch, int num_heads, int head_dim) {
+  long long rows = 0;
+  int most = 0;
+  for (int i = 0; i < sch.n_streams; ++i) {
+    rows += sch.s[i].q_rows;
+    if (sch.s[i].kv_tokens > most) most = sch.s[i].kv_tokens;
+  }
+  if (rows <= 0 || rows * num_heads * 8 > kDecFineWgs) return 0;
+  const int fit = (int)(kDecFineWgs / (rows * num_heads)), cap = head_dim == 128 && most > 12 * kDecChunk ? 2 * kDecFineChunks : kDecFineChunks;
+  return fit < cap ? fit : cap;
+}
+static int lbm_decode_chunks(int kv_tokens, int fine_chunks) {
   int n = (kv_tokens + kDecChunk - 1) / kDecChunk;
+  const int fine = (kv_tokens + kDecFineChunk - 1) / kDecFineChunk, most = fine < fine_chunks ? fine : fine_chunks;
+  if (n < most) n = most;
   return n < 1 ? 1 : (n > kDecMaxChunks ? kDecMaxChunks : n);
 }
 static bool lbm_decode_applies(const LbmAttnSchedule& sch) {
@@ -1765,10 +1788,10 @@ static bool lbm_decode_applies(const LbmAttnSchedule& sch) {
     if (sch.s[i].q_rows > kDecQ) return false;
   return sch.n_streams > 0;
 }
-static size_t lbm_decode_bytes(const LbmAttnSchedule& sch, int num_heads, int head_dim) {
+static size_t lbm_decode_bytes(const LbmAttnSchedule& sch, int num_heads, int head_dim, int fine_chunks) {
   if (!lbm_decode_applies(sch)) return 0;
   size_t rows = 0;
-  for (int i = 0; i < sch.n_streams; ++i) rows += (size_t)lbm_decode_chunks(sch.s[i].kv_tokens) * sch.s[i].q_rows;
+  for (int i = 0; i < sch.n_streams; ++i) rows += (size_t)lbm_decode_chunks(sch.s[i].kv_tokens, fine_chunks) * sch.s[i].q_rows;
   return rows * num_heads * (head_dim + 2) * sizeof(float);
 }
 
@@ -2068,12 +2091,12 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
   sch.part_rows = part;
 }
 
-size_t lbm_attn_schedule_bytes(const LbmAttnSchedule& sch, int num_heads, int head_dim) {
+size_t lbm_attn_schedule_bytes(const LbmAttnSchedule& sch, int num_heads, int head_dim, bool least) {
   // bf16 partial outputs followed by one float log-sum-exp per (row, head); or, when every
   // stream has only a few query rows, the fp32 partials of the few-query path (the query does
   // not know the dtype, so it covers both)
   const size_t split_kv = (size_t)sch.part_rows * num_heads * (head_dim * 2 + 4);
-  const size_t few_q = lbm_decode_bytes(sch, num_heads, head_dim);
+  const size_t few_q = lbm_decode_bytes(sch, num_heads, head_dim, least ? 0 : lbm_decode_fine_chunks(sch, num_heads, head_dim));
   return split_kv > few_q ? split_kv : few_q;
 }
 
@@ -2081,7 +2104,7 @@ namespace {
 int lbm_launch_attention_only(const void* q, const void* pool, void* out, const void* self_k,
                               const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                               const LbmAttnSchedule& sch, int num_heads, int head_dim, int page_size, int dtype,
-                              float sm_scale, void* workspace, hipStream_t stream, const int32_t* append_rows,
+                              float sm_scale, void* workspace, size_t workspace_bytes, hipStream_t stream, const int32_t* append_rows,
                               int append_tokens, bool append_apart, bool own_rows, bool* appended);
 }  // namespace
 
@@ -2095,10 +2118,10 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
                          const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                          const LbmAttnSchedule& sch,
                          int num_heads, int head_dim, int page_size, int dtype, float sm_scale,
-                         void* workspace, hipStream_t stream, const int32_t* append_rows, int append_tokens, bool append_apart, bool own_rows) {
+                         void* workspace, size_t workspace_bytes, hipStream_t stream, const int32_t* append_rows, int append_tokens, bool append_apart, bool own_rows) {
   bool appended = false;
   int rc = lbm_launch_attention_only(q, pool, out, self_k, self_v, kv_rows, live_kv_tokens, sch, num_heads, head_dim,
-                                     page_size, dtype, sm_scale, workspace, stream, append_rows, append_tokens, append_apart, own_rows, &appended);
+                                     page_size, dtype, sm_scale, workspace, workspace_bytes, stream, append_rows, append_tokens, append_apart, own_rows, &appended);
   if (rc != LBM_OK || !append_rows || append_tokens <= 0 || appended) return rc;
   return lbm_launch_append(self_k, self_v, dtype, const_cast<void*>(pool), dtype, append_rows, append_tokens, num_heads,
                            head_dim, page_size, stream);
@@ -2108,7 +2131,7 @@ namespace {
 int lbm_launch_attention_only(const void* q, const void* pool, void* out, const void* self_k,
                               const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                               const LbmAttnSchedule& sch, int num_heads, int head_dim, int page_size, int dtype,
-                              float sm_scale, void* workspace, hipStream_t stream, const int32_t* append_rows,
+                              float sm_scale, void* workspace, size_t workspace_bytes, hipStream_t stream, const int32_t* append_rows,
                               int append_tokens, bool append_apart, bool own_rows, bool* appended) {
   if (head_dim != 64 && !(head_dim == 128 && dtype == LBM_DTYPE_F32))
     return lbm_fail(LBM_ERR_UNSUPPORTED, "attention kernels cover head_dim 64 (bf16, fp32) and 128 (fp32), got %d", head_dim);
@@ -2145,11 +2168,13 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       d.append_rows = append_tokens > 0 ? append_rows : nullptr;
       d.append_tokens = append_tokens;
       int max_chunks = 0, max_q = 0, min_q = kDecQ, part = 0, most = 0;
+      int fine = lbm_decode_fine_chunks(sch, num_heads, head_dim);
+      if (workspace_bytes < lbm_decode_bytes(sch, num_heads, head_dim, fine)) fine = 0;   // a workspace for chunks of 256 serves too
       for (int i = 0; i < LBM_MAX_STREAMS; ++i) {
         d.n_chunks[i] = 0;
         d.part_begin[i] = part;
         if (i < sch.n_streams) {
-          d.n_chunks[i] = lbm_decode_chunks(sch.s[i].kv_tokens);
+          d.n_chunks[i] = lbm_decode_chunks(sch.s[i].kv_tokens, fine);
           part += d.n_chunks[i] * sch.s[i].q_rows;
           if (d.n_chunks[i] > max_chunks) max_chunks = d.n_chunks[i];
           if (sch.s[i].q_rows > max_q) max_q = sch.s[i].q_rows;
@@ -2159,10 +2184,14 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       }
       if (max_q == 0) return LBM_OK;
       d.max_q = max_q;
-      // One workgroup per (stream, head, query row): a launch of 16 heads reads 512 tokens of 128
-      // floats in about the time the second launch of the chunked form takes.  With one query row
-      // per stream and nothing to append beyond those rows it carries the append as well.
-      if (most <= kDecOneTokens) {
+      // One workgroup per (stream, head, query row) for short lists.  Up to two trips to memory it is the faster form
+      // (head_dim 128, 300 tokens: 7.2 us against 9.6 of the chunked form from the last-level cache, 10.6 and 10.8 from
+      // HBM), a third one costs more than a second launch (360 tokens 8.1 and 8.9, 11.7 and 10.0; 500 tokens 9.4 and 8.0,
+      // 14.5 and 9.1); half of a third where fewer chunks fit (four streams, 360 tokens 8.2 and 9.4, 12.7 and 12.6;
+      // 500 tokens 9.4 and 8.6, 15.7 and 12.4), and all of kDecOneTokens where only chunks of 256 do.  With one query
+      // row per stream and nothing to append beyond those rows it carries the append as well.
+      const int groups = kDecOneWaves * 256 / head_dim, trip = kDecOneBatch * groups, trips = (most + trip - 1) / trip;
+      if (most <= kDecOneTokens && (!fine || most <= trip * (fine < kDecFineChunks ? 5 : 4) / 2)) {
         for (int i = 0; i < sch.n_streams; ++i) d.n_chunks[i] = 1;
         unsigned covered = 0;   // rows 0 .. n_streams - 1 of the append, each some stream's query row
         for (int i = 0; i < sch.n_streams; ++i)
@@ -2176,7 +2205,6 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
         // batch whether the tokens are there or not, 0.13 us for 16 rows of 128 floats at a CU's 64 bytes per cycle.
         // us a launch, 16 heads, batches of eleven and these: head_dim 128, 16 tokens 4.3, 2.8; 64 4.3, 3.1; 100 4.3, 4.0;
         // 200 6.2, 5.7; head_dim 64, 100 tokens 4.2, 3.1; 400 6.2, 5.5.  (Ten: no better than eleven.)
-        const int groups = kDecOneWaves * 256 / head_dim, trips = (most + kDecOneBatch * groups - 1) / (kDecOneBatch * groups);
         const int batch = trips > 0 ? (most + trips * groups - 1) / (trips * groups) : 1;
 #define LBM_DECODE_ONE(NB)                                                                                                                    \
   {                                                                                                                                          \
