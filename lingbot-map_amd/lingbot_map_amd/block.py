@@ -610,7 +610,7 @@ class _NativeBlock:
         fc1_w, fc1_sum, fc1_b = FoldedNorm.of(mlp, block.norm2, mlp.fc1)
         proj_w, fc2_w = raw(attn.proj), raw(mlp.fc2)
         ls = [f32(m.gamma) if isinstance(m, LayerScale) else None for m in (block.ls1, block.ls2)]
-        self.hints = (proj_w, fc1_w, fc2_w)
+        self.hints = (tuple(t.data_ptr() for t in (proj_w, fc1_w, fc2_w)), tuple(t.numel() * 2 for t in (proj_w, fc1_w, fc2_w)))
 
         def weights(qkv_w, qkv_b, qkv_sum, eps):
             held = (qkv_w, proj_w, fc1_w, fc2_w, qkv_b, f32(attn.proj.bias), fc1_b, f32(mlp.fc2.bias), qkv_sum, fc1_sum, *ls, *qk)
@@ -626,6 +626,14 @@ class _NativeBlock:
             block.norm1.__dict__["_lbm_folded_qkv_weight"] = w    # where the block before this one finds it (hints)
             self.folded = weights(w, bias, colsum, float(block.norm1.eps))
         self.attn = attn
+
+    def hints_with(self, next_norm):
+        """Addresses and sizes of the weights that the launch behind each of the four GEMMs reads: the block's own
+        and, of ``next_norm``'s block, the folded qkv weights if they are laid out on this device (what no peer has
+        opened must not be read)."""
+        ahead = getattr(next_norm, "_lbm_folded_qkv_weight", None)
+        addr, size = (None, 0) if ahead is None or ahead.device != self.device else (ahead.data_ptr(), ahead.numel() * ahead.element_size())
+        return self.hints[0] + (addr,), self.hints[1] + (size,)
 
     def sizes(self, rows: int):
         """(scratch bytes, column tiles of the row statistics, K-split workspace bytes) for ``rows`` rows."""
@@ -662,13 +670,16 @@ class _NativeBlock:
 
 
 class HipPagedBlock(nn.Module):
-    #: name the next launch's weights in front of every GEMM of a captured frame
-    #: (``lbm_linear_prefetch_hint``: a frame walks through far more weight bytes than the caches hold,
-    #: so a layer would find its own in HBM): proj's in front of the qkv projection, fc1's in front of
-    #: proj, fc2's in front of fc1, the next block's qkv weights in front of fc2.  An eager frame is
-    #: not hinted: each launch's weights are named too late there to be worth the reads.  A switch for
-    #: measurements - results do not depend on it.
+    #: name the next launch's weights in front of every GEMM (``lbm_linear_prefetch_hint``: a frame walks
+    #: through far more weight bytes than the caches hold, so a layer would find its own in HBM): proj's in
+    #: front of the qkv projection, fc1's in front of proj, fc2's in front of fc1, the next block's qkv weights
+    #: in front of fc2.  Captured frames, and eager ones from ``HINT_ROWS`` rows up: a block is one native call,
+    #: so that its launches follow one another (ms per eager frame without and with: 261 rows 3.74, 3.61;
+    #: 566 rows 5.32, 5.16; 1,004 rows 6.87, 6.58; four streams of 1,004 rows 16.1, 15.9), but with fewer rows
+    #: the eager frame waits for the host (86 rows: 3.32, 3.38).  A switch for measurements - results do not
+    #: depend on it.
     PREFETCH_HINTS = os.environ.get("LBM_PREFETCH_HINTS", "1") != "0"
+    HINT_ROWS = 192
 
     def __init__(self, dim: int, num_heads: int, mlp_ratio: float = 4.0, qkv_bias: bool = True,
                  proj_bias: bool = True, ffn_bias: bool = True, drop: float = 0.0, attn_drop: float = 0.0,
@@ -817,10 +828,8 @@ class HipPagedBlock(nn.Module):
             if append is None:
                 return None
         hints = ((None,) * 4, (0,) * 4)
-        if self.PREFETCH_HINTS and torch.cuda.is_current_stream_capturing():
-            named = native.hints + (getattr(next_norm, "_lbm_folded_qkv_weight", None),)
-            hints = (tuple(None if t is None else t.data_ptr() for t in named),
-                     tuple(0 if t is None else t.numel() * t.element_size() for t in named))
+        if self.PREFETCH_HINTS and (rows >= self.HINT_ROWS or torch.cuda.is_current_stream_capturing()):
+            hints = native.hints_with(next_norm)
         call = N.BlockCall(
             x.data_ptr(), a.data_ptr(), stats_ptr, out.data_ptr(), None if stats_out is None else stats_out.data_ptr(),
             scratch.data_ptr(), None if table is None else table.data_ptr(), pool, append, kv_rows, live, streams, ws.data_ptr(),

@@ -180,3 +180,17 @@ def test_stream_table_follows_its_rotary_module():
     check()
     with pytest.raises(AssertionError):
         model.stream_table(1, 42, 70, "cpu", first_frame=64)
+
+
+def test_next_blocks_weights_are_named_on_their_own_device_only():
+    """The addresses in front of a block's GEMMs: its own weights', and the next block's folded qkv weights where they
+    lie on the same device."""
+    from lingbot_map_amd.block import _NativeBlock
+    native = object.__new__(_NativeBlock)      # (laying parameters out needs a GPU; the names do not)
+    native.hints, native.device = ((16, 32, 48), (2, 4, 6)), torch.device("cpu")
+    norm = torch.nn.LayerNorm(64)
+    assert native.hints_with(None) == native.hints_with(norm) == ((16, 32, 48, None), (2, 4, 6, 0))
+    w = norm.__dict__["_lbm_folded_qkv_weight"] = torch.zeros(192, 64, dtype=torch.bfloat16)
+    assert native.hints_with(norm) == ((16, 32, 48, w.data_ptr()), (2, 4, 6, 192 * 64 * 2))
+    norm.__dict__["_lbm_folded_qkv_weight"] = w.to("meta")
+    assert native.hints_with(norm) == ((16, 32, 48, None), (2, 4, 6, 0))
