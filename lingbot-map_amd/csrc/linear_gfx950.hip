@@ -186,17 +186,17 @@ __device__ __forceinline__ void gelu_of(const f32x4 (&x)[C], const unsigned shor
 // to each; an XCD's 32 take consecutive tiles of an order that walks panels of 8 column tiles row
 // by row, i.e. 4 row tiles x 8 column tiles (8 x 4 in a last panel of 4): 12 operand tiles per
 // k-step for the XCD's L2 to hold instead of 17 to 33, which is what sets the latency of the
-// operand loads.
-__device__ __forceinline__ void lbm_tile_of_workgroup(int b, int m_tiles, int n_tiles, int& mt, int& nt) {
+// operand loads.  (Tiles of 64 columns x 64 or 32 rows: panels of kRowsPanel column tiles, for the same reason.)
+__device__ __forceinline__ void lbm_tile_of_workgroup(int b, int m_tiles, int n_tiles, int& mt, int& nt, int panel_width = 8) {
   const int x = b & 7, i = b >> 3;
   const int base = (i >> 5) * 256;
   const int in_round = min(m_tiles * n_tiles - base, 256);
   const int t = base + x * (in_round >> 3) + min(x, in_round & 7) + (i & 31);
-  const int panel_tiles = m_tiles * 8;
+  const int panel_tiles = m_tiles * panel_width;
   const int panel = t / panel_tiles, rem = t - panel * panel_tiles;
-  const int width = min(8, n_tiles - panel * 8);
+  const int width = min(panel_width, n_tiles - panel * panel_width);
   mt = rem / width;
-  nt = panel * 8 + rem - mt * width;
+  nt = panel * panel_width + rem - mt * width;
 }
 
 
@@ -829,7 +829,12 @@ __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int mt, nt;
-  lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt);
+  // Panels of 4 column tiles, not 8: fewer bytes for an XCD's L2 where a launch has few row tiles (us, weights rotating
+  // through 24 layers, M x N x K 261 x 1,024 x 4,096 11.2 -> 10.1, 261 x 1,024 x 1,024 5.2 -> 4.9, 261 x 3,072 x 1,024
+  // 6.4 -> 6.2); 16 row tiles of 64 with slices of K read whole rows of a long K, where 8 x 4 is the smaller set
+  // (1,004 x 1,024 x 4,096, weights in HBM: 18.9, 19.2 with 4).
+  constexpr int kRowsPanel = TM == 64 && KS > 1 ? 8 : 4;
+  lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt, kRowsPanel);
   const int m0 = mt * TM, n0 = nt * 64;
   const int nk = p.K / (2 * kKS);                          // 128-wide steps
 
