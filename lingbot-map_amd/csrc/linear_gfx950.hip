@@ -147,23 +147,29 @@ static __device__ __attribute__((aligned(16))) const unsigned short g_gelu_table
 // share a register from their rounding on: their indices are one packed computation, the two lookups land in
 // the halves of the result, and what lies outside the table is patched afterwards, only by wavefronts
 // that hold such a value - ten vector instructions per element where one value at a time took 21 (fc1 of
-// 8,040 rows 78.0 -> 75.7 us, 4,016 rows 38.9 -> 37.9, 1,004 rows 14.7 -> 14.5; what is left of the 8 us
-// that GELU costs a 256 x 256 tile is the lookups' bank conflicts).
+// 8,040 rows 78.0 -> 75.7 us, 4,016 rows 38.9 -> 37.9, 1,004 rows 14.7 -> 14.5).
+// The index is the entry's byte offset, made without a compare or a select: seven per element (with the column
+// vectors read once per column block: 8,032 rows 78.1 -> 75.7, 4,016 rows 39.3 -> 37.9, 1,004 rows 14.8 -> 14.7).
+// Of the 5 us that GELU then costs a 256 x 256 tile the lookups' bank conflicts are two.  (The table at the bottom of
+// LDS, the offset its whole address: another 0.4 us of a 256-row tile in a loop, but whole frames 0.1 to 0.3 % slower.)
 template <int C>
 __device__ __forceinline__ void gelu_of(const f32x4 (&x)[C], const unsigned short* tab, bf16x4 (&y)[C]) {
-  const u16x2 lo = (unsigned short)(kGeluE0 << 7), hi = (unsigned short)((kGeluE0 << 7) + kGeluHalf - 1);
+  // byte offsets of the table's entries: twice the magnitude's bits, the sign shifted out
+  const u16x2 lo = (unsigned short)(kGeluE0 << 8), hi = (unsigned short)((kGeluE0 << 8) + 2 * (kGeluHalf - 1));
   u16x2 in[2 * C], out[2 * C], beyond = {0, 0};
 #pragma unroll
   for (int i = 0; i < 2 * C; ++i) {
     unsigned pair = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{x[i >> 1][(i & 1) * 2], x[i >> 1][(i & 1) * 2 + 1]}, bf16x2));
     asm("" : "+v"(pair));   // (or the signs are taken from x, one compare and one select each)
     in[i] = __builtin_bit_cast(u16x2, pair);
-    const u16x2 mag = in[i] & (unsigned short)0x7fff;
+    const u16x2 mag = in[i] << (unsigned short)1;
     const u16x2 held = __builtin_elementwise_max(__builtin_elementwise_min(mag, hi), lo);
     beyond |= mag ^ held;
-    const u16x2 neg = __builtin_bit_cast(u16x2, __builtin_bit_cast(s16x2, in[i]) >> 15);
-    const u16x2 at = (held - lo) + (neg & (unsigned short)kGeluHalf);
-    out[i] = u16x2{tab[at[0]], tab[at[1]]};
+    unsigned neg = __builtin_bit_cast(unsigned, in[i] >> (unsigned short)15);
+    asm("" : "+v"(neg));    // (or they are: 0 or 1, to multiply with)
+    const u16x2 at = __builtin_bit_cast(u16x2, neg) * (unsigned short)(2 * kGeluHalf) + (held - lo);
+    const char* const bytes = (const char*)tab;
+    out[i] = u16x2{*(const unsigned short*)(bytes + at[0]), *(const unsigned short*)(bytes + at[1])};
   }
   if (__builtin_amdgcn_ballot_w64(__builtin_bit_cast(unsigned, beyond) != 0u)) {
     // outside the table: v / 2 below it, v or v * 0 above it (see kGeluE0)
@@ -1320,30 +1326,35 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   // In registers: the folded LayerNorm's scale and correction, + bias, round (the linear's
   // output), GELU, round; then the tile goes through LDS and leaves as whole rows.
   unsigned short* stage = (unsigned short*)lds_raw;
+  f32x2 row_f[RB];
 #pragma unroll
-  for (int b = 0; b < RB; ++b) {
-    const int row = wm + b * 32 + n32;
-    f32x2 row_f = {1.f, 0.f};
-    if (LNA) row_f = *(const f32x2*)&ln_rows[2 * row];
+  for (int b = 0; b < RB; ++b) row_f[b] = LNA ? *(const f32x2*)&ln_rows[2 * (wm + b * 32 + n32)] : f32x2{1.f, 0.f};
 #pragma unroll
-    for (int a = 0; a < CB; ++a) {
+  for (int a = 0; a < CB; ++a) {
+    f32x4 bias4[4], colsum4[4];   // (read once for all row blocks)
+#pragma unroll
+    for (int c4 = 0; c4 < 4; ++c4) {
+      const int col = wn + a * 32 + c4 * 8 + g * 4;
+      bias4[c4] = *(const f32x4*)&colvec[0][col];
+      if (LNA) colsum4[c4] = *(const f32x4*)&colvec[1][col];
+    }
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
       f32x4 x[4];
       bf16x4 y[4];
 #pragma unroll
       for (int c4 = 0; c4 < 4; ++c4) {
-        const int col = wn + a * 32 + c4 * 8 + g * 4;
-        const f32x4 bias4 = *(const f32x4*)&colvec[0][col], colsum4 = *(const f32x4*)&colvec[1][col];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float lin = acc[a][b][c4 * 4 + e];
-          if (LNA) lin = __builtin_fmaf(lin, row_f[0], row_f[1] * colsum4[e]);
-          x[c4][e] = lin + bias4[e];
+          if (LNA) lin = __builtin_fmaf(lin, row_f[b][0], row_f[b][1] * colsum4[c4][e]);
+          x[c4][e] = lin + bias4[c4][e];
         }
         y[c4] = __builtin_convertvector(x[c4], bf16x4);
       }
       if (EPI == LBM_LINEAR_BIAS_GELU) gelu_of<4>(x, gelu_tab, y);
 #pragma unroll
-      for (int c4 = 0; c4 < 4; ++c4) *(bf16x4*)&stage[row * kBCStride + wn + a * 32 + c4 * 8 + g * 4] = y[c4];
+      for (int c4 = 0; c4 < 4; ++c4) *(bf16x4*)&stage[(wm + b * 32 + n32) * kBCStride + wn + a * 32 + c4 * 8 + g * 4] = y[c4];
     }
   }
   __syncthreads();
