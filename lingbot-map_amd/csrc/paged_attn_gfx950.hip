@@ -1537,7 +1537,7 @@ __global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32 a) {
 // nothing crosses lanes inside the loop but the D/4-lane sum of a dot product (DPP) and there is no
 // barrier in it; the groups meet through LDS once, at the end.
 //
-// Up to kDecOneTokens tokens one workgroup of eight wavefronts takes a (stream, head, query row) from
+// Up to kDecOneTokens tokens one to four workgroups of eight wavefronts take a (stream, head, query row) from
 // start to finish: one launch, which also stores the caller's new rows (lbm_attn_run_append).
 // Beyond that the KV axis is cut into chunks of 256 down to 64 tokens, one workgroup of four wavefronts
 // each, which leave partial results for lbm_attn_f32_decode_merge_kernel.  Where the chip has workgroups to spare a
@@ -1581,16 +1581,26 @@ __device__ __forceinline__ float row_group_sum(float v) {
 }
 
 // grid: x = chunk of the KV axis, y = head, z = stream * max_q + query row.  ONE: the only chunk of
-// its stream - the result goes to `out`; otherwise a partial.
-template <int D, int NW, int NB, bool ONE>
+// its stream - the result goes to `out`; otherwise a partial.  VS: so many workgroups share a row, each with all of
+// K and D / VS dimensions of V (z: one behind the others' rows, so that they meet in an XCD's L2) - the same sums for
+// every output, from fewer bytes through a CU, which is what bounds a launch of few rows (a token of 128 floats is
+// 1,024 bytes for one workgroup, 640 for each of four).  us, 16 heads, caches in HBM, VS 1, 2, 4: head_dim 128, 100
+// tokens 4.9, 4.5, 4.4; 200 8.6, 7.4, 7.0; 300 10.6, 9.2, 8.2; four streams of 300 11.7, 10.1, 9.0; eight of them 12.5,
+// 12.0, 13.6 (two workgroups per CU); head_dim 64, 300 tokens 6.8, 6.2, 5.8.
+template <int D, int NW, int NB, bool ONE, int VS = 1>
 __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs a) {
   constexpr int LPR = D / 4;         // lanes per K/V row, 16 bytes each
   constexpr int RPW = 64 / LPR;      // row groups of a wavefront
   constexpr int G = NW * RPW;        // row groups of the workgroup
-  __shared__ __attribute__((aligned(16))) float red_o[NW][D];
+  constexpr int DV = D / VS, VE = 4 / VS;   // dimensions of V: the workgroup's, a lane's
+  typedef __attribute__((ext_vector_type(VE))) float vec;
+  static_assert(ONE || VS == 1, "partials hold whole rows");
+  __shared__ __attribute__((aligned(16))) float red_o[NW][DV];
   __shared__ float red_m[NW], red_l[NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int b = blockIdx.z / a.max_q, qi = blockIdx.z % a.max_q, head = blockIdx.y, chunk = blockIdx.x;
+  const int rows_of_launch = VS == 1 ? 0 : a.f.n_streams * a.max_q, vs = VS == 1 ? 0 : blockIdx.z / rows_of_launch;
+  const int z = blockIdx.z - vs * rows_of_launch;
+  const int b = z / a.max_q, qi = z % a.max_q, head = blockIdx.y, chunk = blockIdx.x;
   lbm_attn_stream sp = a.f.s[b];
   if (chunk >= a.n_chunks[b] || qi >= sp.q_rows) return;
   if (a.f.live_kv_tokens) sp.kv_tokens = max(a.f.live_kv_tokens[sp.live_at], 0);
@@ -1601,10 +1611,11 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
   const int grp = wave * RPW + lane / LPR, ln = lane % LPR;
 
   const f32x4 q4 = *(const f32x4*)(a.f.q + ((size_t)(sp.q_begin + qi) * H + head) * D + 4 * ln) * a.f.scale_log2;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  vec acc = {};
   float m = -INFINITY, l = 0.f;
   const int32_t* rows = a.f.kv_rows + sp.kv_row_begin;
   const size_t head_off = (size_t)head * D + 4 * ln, v_off = (size_t)a.f.page_size * row_elems;
+  const size_t v_head_off = (size_t)head * D + vs * DV + VE * ln;
   // tokens past the end of the piece re-read its last token (weight 0): no load sits
   // inside a conditional block
   int e[NB];
@@ -1614,13 +1625,14 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
   };
   if (t_begin < t_end) entries(t_begin);
   for (int t0 = t_begin; t0 < t_end; t0 += NB * G) {
-    f32x4 k[NB], v[NB];
+    f32x4 k[NB];
+    vec v[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       // negative entries name rows of the caller's own K/V
-      const size_t off = (size_t)(e[j] ^ (e[j] >> 31)) * row_elems + head_off;
-      k[j] = *(const f32x4*)((e[j] < 0 ? a.f.self_k : a.f.pool) + off);
-      v[j] = *(const f32x4*)((e[j] < 0 ? a.f.self_v : a.f.pool + v_off) + off);
+      const size_t off = (size_t)(e[j] ^ (e[j] >> 31)) * row_elems;
+      k[j] = *(const f32x4*)((e[j] < 0 ? a.f.self_k : a.f.pool) + off + head_off);
+      v[j] = *(const vec*)((e[j] < 0 ? a.f.self_v : a.f.pool + v_off) + off + v_head_off);
     }
     if (t0 + NB * G < t_end) entries(t0 + NB * G);
     float s[NB], mx = m;
@@ -1629,7 +1641,7 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
       s[j] = row_group_sum<LPR>(k[j][0] * q4[0] + k[j][1] * q4[1] + k[j][2] * q4[2] + k[j][3] * q4[3]);
       if (t0 + j * G + grp >= t_end) {
         s[j] = -INFINITY;
-        v[j] = f32x4{0.f, 0.f, 0.f, 0.f};   // (the last token's values may be infinite: 0 x inf)
+        v[j] = vec{};   // (the last token's values may be infinite: 0 x inf)
       }
       mx = fmaxf(mx, s[j]);
     }
@@ -1653,17 +1665,17 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
     const float mt = fmaxf(m, m1), ref = mt > -INFINITY ? mt : 0.f;
     const float w0 = __builtin_amdgcn_exp2f(m - ref), w1 = __builtin_amdgcn_exp2f(m1 - ref);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = acc[i] * w0 + __shfl_xor(acc[i], step) * w1;
+    for (int i = 0; i < VE; ++i) acc[i] = acc[i] * w0 + __shfl_xor(acc[i], step) * w1;
     l = l * w0 + l1 * w1;
     m = mt;
   }
-  if (lane < LPR) *(f32x4*)&red_o[wave][4 * ln] = acc;
+  if (lane < LPR) *(vec*)&red_o[wave][VE * ln] = acc;
   if (lane == 0) {
     red_m[wave] = m;
     red_l[wave] = l;
   }
   __syncthreads();     // (also: every wavefront has read what it needs of the pool)
-  if (tid < D) {
+  if (tid < DV) {
     float mx = red_m[0];
 #pragma unroll
     for (int w = 1; w < NW; ++w) mx = fmaxf(mx, red_m[w]);
@@ -1676,7 +1688,7 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
       o += red_o[w][tid] * wgt;
     }
     if (ONE) {
-      a.f.out[((size_t)(sp.q_begin + qi) * H + head) * D + tid] = lt > 0.f ? o / lt : 0.f;   // no token: zeros
+      a.f.out[((size_t)(sp.q_begin + qi) * H + head) * D + vs * DV + tid] = lt > 0.f ? o / lt : 0.f;   // no token: zeros
     } else {
       float* pp = a.part + (((size_t)a.part_begin[b] + (size_t)chunk * sp.q_rows + qi) * H + head) * (D + 2);
       pp[tid] = o;
@@ -1685,9 +1697,10 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
         pp[D + 1] = lt;
       }
     }
-  } else if (ONE && a.append_rows && tid < 2 * D) {
-    // this (stream, head)'s share of the append: one query row per stream (lbm_launch_decode checks)
-    const int t = sp.q_begin, row = a.append_rows[t], d = tid - D;
+  } else if (ONE && a.append_rows && tid < 2 * DV) {
+    // this (stream, head)'s share of the append: one query row per stream (the launch checks; and where several
+    // workgroups read a row of K, that no table names the row stored here)
+    const int t = sp.q_begin, row = a.append_rows[t], d = vs * DV + tid - DV;
     if (row >= 0) {
       float* dst = const_cast<float*>(a.f.pool) + (size_t)row * row_elems + (size_t)head * D + d;
       const size_t src = ((size_t)t * H + head) * D + d;
@@ -2184,14 +2197,14 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       }
       if (max_q == 0) return LBM_OK;
       d.max_q = max_q;
-      // One workgroup per (stream, head, query row) for short lists.  Up to two trips to memory it is the faster form
-      // (head_dim 128, 300 tokens: 7.2 us against 9.6 of the chunked form from the last-level cache, 10.6 and 10.8 from
-      // HBM), a third one costs more than a second launch (360 tokens 8.1 and 8.9, 11.7 and 10.0; 500 tokens 9.4 and 8.0,
-      // 14.5 and 9.1); half of a third where fewer chunks fit (four streams, 360 tokens 8.2 and 9.4, 12.7 and 12.6;
-      // 500 tokens 9.4 and 8.6, 15.7 and 12.4), and all of kDecOneTokens where only chunks of 256 do.  With one query
-      // row per stream and nothing to append beyond those rows it carries the append as well.
+      // One launch for short lists.  Up to two and a half trips to memory it is the faster form (us, one row of 16 heads
+      // of 128, from the last-level cache and from HBM, against the chunked form: 300 tokens 7.0 and 8.2, 9.6 and 10.8;
+      // 360 tokens 7.6 and 9.0, 8.9 and 9.9; 440 tokens 9.2 and 10.4, 9.1 and 10.3), beyond that it costs more than a
+      // second launch (500 tokens 9.2 and 10.7, 8.0 and 9.0) unless fewer chunks fit (four streams, 500 tokens 10.0 and
+      // 11.9, 11.1 and 12.4).  With one query row per stream and nothing to append beyond those rows it carries the
+      // append as well.
       const int groups = kDecOneWaves * 256 / head_dim, trip = kDecOneBatch * groups, trips = (most + trip - 1) / trip;
-      if (most <= kDecOneTokens && (!fine || most <= trip * (fine < kDecFineChunks ? 5 : 4) / 2)) {
+      if (most <= kDecOneTokens && (fine < kDecFineChunks || most <= trip * 5 / 2)) {
         for (int i = 0; i < sch.n_streams; ++i) d.n_chunks[i] = 1;
         unsigned covered = 0;   // rows 0 .. n_streams - 1 of the append, each some stream's query row
         for (int i = 0; i < sch.n_streams; ++i)
@@ -2200,16 +2213,26 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
                              covered == (1u << append_tokens) - 1u;
         if (!carries) d.append_rows = nullptr;
         else *appended = true;
-        const dim3 grid(1, num_heads, sch.n_streams * max_q), block(kDecOneWaves * 64);
+        // A row to four or two workgroups where that leaves one per CU, not for the shortest lists (16 tokens of 64
+        // floats 2.75, 2.83), and not where a row to append may be one that another workgroup still has to read.
+        const long long rows = (long long)num_heads * sch.n_streams * max_q;
+        const int shares = (d.append_rows && !append_apart) || most <= 32 ? 1 : rows * 4 <= 256 ? 4 : rows * 2 <= 256 ? 2 : 1;
+        const dim3 grid(1, num_heads, sch.n_streams * max_q * shares), block(kDecOneWaves * 64);
         // As few trips as batches of eleven need, and batches no longer than so many trips need: a step loads its
         // batch whether the tokens are there or not, 0.13 us for 16 rows of 128 floats at a CU's 64 bytes per cycle.
         // us a launch, 16 heads, batches of eleven and these: head_dim 128, 16 tokens 4.3, 2.8; 64 4.3, 3.1; 100 4.3, 4.0;
         // 200 6.2, 5.7; head_dim 64, 100 tokens 4.2, 3.1; 400 6.2, 5.5.  (Ten: no better than eleven.)
         const int batch = trips > 0 ? (most + trips * groups - 1) / (trips * groups) : 1;
+#define LBM_DECODE_ONE_VS(NB, VS)                                                                                                              \
+  {                                                                                                                                          \
+    if (head_dim == 64) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<64, kDecOneWaves, NB, true, VS>), grid, block, 0, stream, d);           \
+    else hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<128, kDecOneWaves, NB, true, VS>), grid, block, 0, stream, d);                         \
+  }
 #define LBM_DECODE_ONE(NB)                                                                                                                    \
   {                                                                                                                                          \
-    if (head_dim == 64) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<64, kDecOneWaves, NB, true>), grid, block, 0, stream, d);               \
-    else hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<128, kDecOneWaves, NB, true>), grid, block, 0, stream, d);                             \
+    if (shares == 4) LBM_DECODE_ONE_VS(NB, 4)                                                                                                 \
+    else if (shares == 2) LBM_DECODE_ONE_VS(NB, 2)                                                                                             \
+    else LBM_DECODE_ONE_VS(NB, 1)                                                                                                             \
   }
         if (batch <= 2) LBM_DECODE_ONE(2)
         else if (batch <= 4) LBM_DECODE_ONE(4)
@@ -2217,6 +2240,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
         else if (batch <= 8) LBM_DECODE_ONE(8)
         else LBM_DECODE_ONE(kDecOneBatch)
 #undef LBM_DECODE_ONE
+#undef LBM_DECODE_ONE_VS
         return lbm_check_launch("lbm_attn_f32_decode_kernel<one chunk>");
       }
       const dim3 grid(max_chunks, num_heads, sch.n_streams * max_q), block(kDecChunkWaves * 64);
