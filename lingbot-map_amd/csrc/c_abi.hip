@@ -215,7 +215,7 @@ size_t lbm_attn_workspace_bytes(const lbm_attn_stream* streams, int32_t n_stream
   if (lbm_check_attn_streams(streams, n_streams, "lbm_attn_workspace_bytes") != LBM_OK) return 0;
   if (num_heads <= 0 || head_dim <= 0) return 0;
   LbmAttnSchedule sch;
-  lbm_attn_schedule(streams, n_streams, num_heads, &sch);
+  lbm_attn_schedule(streams, n_streams, num_heads, &sch, true);   // (what lbm_block_run needs covers the others)
   return lbm_attn_schedule_bytes(sch, num_heads, head_dim, false);
 }
 
@@ -225,7 +225,7 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
                              int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
                              void* workspace, size_t workspace_bytes, void* stream,
                              const int32_t* append_rows = nullptr, int32_t append_tokens = 0, bool append_apart = false,
-                             bool own_rows = false) {
+                             bool own_rows = false, bool fixed_order = false) {
   int rc = lbm_check_attn_streams(streams, n_streams, who);
   if (rc != LBM_OK) return rc;
   if (!q || !pool || !out || !kv_rows) return lbm_fail(LBM_ERR_INVALID, "%s: null q, pool, out or kv_rows", who);
@@ -238,7 +238,7 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
   // (rows are addressed by 32-bit byte offsets from the stream's first)
   for (int i = 0; own_rows && i < n_streams; ++i) own_rows = (long long)streams[i].kv_tokens * num_heads * head_dim * 2 < (1LL << 32);
   LbmAttnSchedule sch;
-  lbm_attn_schedule(streams, n_streams, num_heads, &sch);
+  lbm_attn_schedule(streams, n_streams, num_heads, &sch, fixed_order);
   const size_t need = lbm_attn_schedule_bytes(sch, num_heads, head_dim, true);
   if (need > 0 && (!workspace || workspace_bytes < need))
     return lbm_fail(LBM_ERR_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", who, workspace_bytes, need);
@@ -297,7 +297,7 @@ int lbm_attn_run_static(const void* q, const void* pool, void* out, const void* 
   if (rc != LBM_OK) return rc;
   if (num_heads <= 0 || head_dim <= 0) return lbm_fail(LBM_ERR_INVALID, "lbm_attn_run_static: non-positive size");
   LbmAttnSchedule sch;
-  lbm_attn_schedule(streams, n_streams, num_heads, &sch);
+  lbm_attn_schedule(streams, n_streams, num_heads, &sch, false);
   const size_t need = lbm_attn_schedule_bytes(sch, num_heads, head_dim, true);
   void* ws = nullptr;
   size_t ws_bytes = 0;
@@ -357,7 +357,7 @@ int lbm_block_run(const lbm_block_weights* w, const lbm_block_call* c, void* str
     rc = lbm_attn_run_impl("lbm_block_run", q, c->pool ? c->pool : k, heads, c->keep_kv ? k : nullptr, c->keep_kv ? v : nullptr,
                            c->kv_rows, c->live_kv_tokens, c->streams, c->n_streams, w->num_heads, 64, c->page_size, LBM_DTYPE_BF16,
                            0.f, c->attn_workspace, c->attn_workspace_bytes, stream, nullptr, 0, false,
-                           c->own_rows && c->keep_kv && !c->live_kv_tokens);
+                           c->own_rows && c->keep_kv && !c->live_kv_tokens, true);
     if (rc != LBM_OK) return rc;
   }
   if (c->hints[1]) lbm_set_prefetch_hint(c->hints[1], c->hint_bytes[1]);

@@ -57,11 +57,15 @@ struct LbmAttnSchedule {
   int32_t n_streams;
   int32_t total_wgs;
   int32_t small;       // query rows per workgroup of the in-workgroup split kernel (no partial results), 0: the split-KV kernel
+  bool fixed_order;    // no rotation of a stream's pieces either (lbm_attn_schedule)
   int64_t part_rows;   // rows of partial results over all streams (0 when nothing is split)
   LbmAttnStreamPlan s[LBM_MAX_STREAMS];
 };
+// fixed_order: the sums of a stream keep the order that the fixed estimates give them, whatever the fitted costs say.
+// lbm_block_run asks for it: 24 blocks make the last bits of an attention into 0.2 % of the last block's K and V, single
+// values up to 7 %, and a model's results must not move with a schedule.  Needs at least the workspace of the other.
 void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_heads,
-                       LbmAttnSchedule* out);
+                       LbmAttnSchedule* out, bool fixed_order);
 // least: what a launch cannot do without; otherwise what it is fastest with
 size_t lbm_attn_schedule_bytes(const LbmAttnSchedule& sch, int num_heads, int head_dim, bool least);
 

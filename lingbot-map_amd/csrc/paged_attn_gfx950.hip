@@ -1930,10 +1930,11 @@ double price_small(const int* nt, int n_streams, int num_heads, int rows, const 
 }  // namespace
 
 void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_heads,
-                       LbmAttnSchedule* out) {
+                       LbmAttnSchedule* out, bool fixed_order) {
   LbmAttnSchedule& sch = *out;
   sch = LbmAttnSchedule{};
   sch.n_streams = n_streams;
+  sch.fixed_order = fixed_order;
   int qt[LBM_MAX_STREAMS], nt[LBM_MAX_STREAMS], q_rows[LBM_MAX_STREAMS];
   long long work = 0;
   int max_nt = 0;
@@ -1951,7 +1952,7 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
   // several streams would take the CUs rounds of such workgroups.
   bool small_ok = n_streams > 0;
   for (int i = 0; i < n_streams; ++i) small_ok = small_ok && streams[i].kv_tokens <= kSmMaxKv;
-  const bool one_cache = n_streams == 1 && streams[0].kv_tokens != streams[0].q_rows && streams[0].kv_tokens <= kSmMaxCacheKv;
+  const bool one_cache = !fixed_order && n_streams == 1 && streams[0].kv_tokens != streams[0].q_rows && streams[0].kv_tokens <= kSmMaxCacheKv;
   int found = -1;
   for (int j = 0; j < kMemos && found < 0; ++j) {
     const ScheduleKey& m = g_schedules[j];
@@ -2299,7 +2300,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       return lbm_check_launch("lbm_attn_bf16_d64_small_kernel<own rows>");
     }
     bool turn = false;   // (the kernel decides per stream, by the live count)
-    for (int i = 0; i < sch.n_streams; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);
+    for (int i = 0; i < sch.n_streams && !sch.fixed_order; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);
     const dim3 grid(blocks), block(kSmThreads);
     if (sch.small == 64 && turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, true>), grid, block, 0, stream, a);
     else if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false>), grid, block, 0, stream, a);
