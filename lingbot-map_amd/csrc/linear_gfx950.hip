@@ -819,8 +819,8 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
 // slice behind the other, and add them in slice order at the end: the bits of several workgroups that
 // meet in memory, without the meeting (5 us of an fc2 launch).
 // us per launch, weights rotating through 24 layers, before (128 x 64 tiles) and after: M x N x K 81 x 3,072 x
-// 1,024 with the producer 9.4 -> 6.3, 261 rows 10.1 -> 7.7; 261 x 1,024 x 1,024 8.1 -> 5.2, 1,004 rows 8.4 -> 6.6;
-// 261 x 1,024 x 4,096 12.3 -> 11.2, 512 rows 14.6 -> 11.9, 1,004 rows 18.1 -> 15.5.  (Six stages instead of four: no
+// 1,024 with the producer 9.4 -> 6.1, 261 rows 10.1 -> 7.6; 261 x 1,024 x 1,024 8.1 -> 4.9, 1,004 rows 8.4 -> 6.4;
+// 261 x 1,024 x 4,096 12.3 -> 10.1, 512 rows 14.6 -> 11.4, 1,004 rows 18.1 -> 15.3.  (Six stages instead of four: no
 // faster.  What the last are bound by is L2: 256 CUs x 87 bytes per ns against 92 of a bare copy of such rows.)
 template <int EPI, int TM, int KS = 1, int ROPE = 0, bool NORM = false, bool LNA = false>
 __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_kernel(LinearArgs p) {
