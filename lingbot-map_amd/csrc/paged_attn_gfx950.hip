@@ -2031,11 +2031,12 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
     // with 80-1,374 rows 11 change over, 0.83 of their time in the mean and none slower.  us per block of a streamed
     // frame, 24 blocks, pair and this kernel: 400 x 3,600 25.1, 19.4; 261 x 3,393 21.9, 18.5; 261 x 4,437 23.2, 21.9;
     // 800 x 4,800 31.4, 29.5; 1,004 x 5,020 33.8, 34.4;
-    // 120 x 3,000 17.3, 17.8.  Several streams' launches are priced less well and stay.
+    // 120 x 3,000 17.3, 17.8.  Up to 256 rows, where no SIMD has two of the pair's wavefronts at work, only where they see the pair
+    // behind (209 x 2,976 20.6, 19.9; 209 x 3,500 21.5, 22.4).  Several streams' launches are priced less well and stay.
     if (!memo.small && one_cache) {
       const double pair_us = price_candidate(qt, nt, n_streams, num_heads, (int)best_tps, q_rows, cand_splits, false);
       const double us32 = price_small(nt, n_streams, num_heads, 32, q_rows), us64 = price_small(nt, n_streams, num_heads, 64, q_rows);
-      if ((us32 < us64 ? us32 : us64) < 1.08 * pair_us) memo.small = us32 < us64 ? 32 : 64;
+      if ((us32 < us64 ? us32 : us64) < (2 * q_rows[0] <= kQTile ? 0.96 : 1.08) * pair_us) memo.small = us32 < us64 ? 32 : 64;
     }
     memo.n_streams = n_streams;
     memo.num_heads = num_heads;
