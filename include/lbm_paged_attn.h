@@ -24,7 +24,7 @@
 extern "C" {
 #endif
 
-#define LBM_ABI_VERSION 11
+#define LBM_ABI_VERSION 12
 
 #define LBM_OK 0
 #define LBM_ERR_INVALID 1     /* bad argument (null pointer, negative size, bad enum)      */
@@ -319,9 +319,16 @@ int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k,
  *   LBM_ATTN_APPEND_APART  kv_rows names no row of append_rows, as the plans of lbm_tables_step with
  *                          LBM_OP_PLAN_NEWEST_SELF do: launches that merge nothing carry the append as well, by
  *                          workgroups of their own
- * Same results with and without the flags. */
+ *   LBM_ATTN_FIXED_ORDER   (ABI 12) the bf16 sums of a stream are added in the order that its token counts and fixed
+ *                          estimates give them, as lbm_block_run does.  Without it the fastest kernel and the fastest
+ *                          order are taken, which a later version may choose otherwise: one call's results differ by
+ *                          the rounding of bf16, but 24 blocks one behind the other make the last bits of an attention
+ *                          into 0.2 % of the last block's K and V.  Needs no more than lbm_attn_workspace_bytes; fp32
+ *                          calls are the same either way
+ * Same results with and without the first two flags. */
 #define LBM_ATTN_OWN_ROWS 1
 #define LBM_ATTN_APPEND_APART 2
+#define LBM_ATTN_FIXED_ORDER 4
 typedef struct lbm_attn_call {
   const void* q;
   void* pool;
@@ -338,8 +345,8 @@ int lbm_attn_run_call(const lbm_attn_call* call, void* stream);
 
 /* A whole transformer block of the streaming model in one call (ABI 10): qkv projection + producer,
  * attention, proj + LayerScale + residual, fc1 + GELU, fc2 + LayerScale + residual
- * (lingbot_map/layers/block.py:245-285), i.e. lbm_qkv_linear_prepare_norm, lbm_attn_run (or
- * lbm_attn_run_live) and three lbm_linear_norm launches in order, with the same results; what it
+ * (lingbot_map/layers/block.py:245-285), i.e. lbm_qkv_linear_prepare_norm, lbm_attn_run_call with
+ * LBM_ATTN_FIXED_ORDER and three lbm_linear_norm launches in order, with the same results; what it
  * saves is the host's work between them.  bf16, head_dim 64, dim = 64 num_heads. */
 typedef struct lbm_block_weights {
   const void *qkv_w, *proj_w, *fc1_w, *fc2_w;    /* nn.Linear weights, bf16: [3 dim, dim], [dim, dim], [hidden, dim], [dim, hidden] */

@@ -215,7 +215,7 @@ size_t lbm_attn_workspace_bytes(const lbm_attn_stream* streams, int32_t n_stream
   if (lbm_check_attn_streams(streams, n_streams, "lbm_attn_workspace_bytes") != LBM_OK) return 0;
   if (num_heads <= 0 || head_dim <= 0) return 0;
   LbmAttnSchedule sch;
-  lbm_attn_schedule(streams, n_streams, num_heads, &sch, true);   // (what lbm_block_run needs covers the others)
+  lbm_attn_schedule(streams, n_streams, num_heads, &sch, true);   // (what a fixed order needs covers the others)
   return lbm_attn_schedule_bytes(sch, num_heads, head_dim, false);
 }
 
@@ -275,7 +275,8 @@ int lbm_attn_run_call(const lbm_attn_call* c, void* stream) {
   return lbm_attn_run_impl("lbm_attn_run_call", c->q, c->pool, c->out, c->self_k, c->self_v, c->kv_rows, c->live_kv_tokens, c->streams,
                            c->n_streams, c->num_heads, c->head_dim, c->page_size, c->dtype, c->sm_scale, c->workspace,
                            c->workspace_bytes, stream, c->append_rows, c->append_rows ? c->append_tokens : 0,
-                           (c->flags & LBM_ATTN_APPEND_APART) != 0, (c->flags & LBM_ATTN_OWN_ROWS) && c->self_k && !c->live_kv_tokens);
+                           (c->flags & LBM_ATTN_APPEND_APART) != 0, (c->flags & LBM_ATTN_OWN_ROWS) && c->self_k && !c->live_kv_tokens,
+                           (c->flags & LBM_ATTN_FIXED_ORDER) != 0);
 }
 
 int lbm_attn_run_live(const void* q, const void* pool, void* out, const void* self_k,

@@ -24,7 +24,7 @@ HDR = {"frame_count": 0, "n_anchor": 1, "win_head": 2, "win_count": 3, "n_free_p
        "n_free_special": 5, "n_special_pages": 6, "special_tokens": 7, "n_memory": 8,
        "n_memory_pages": 9, "error": 10, "plan_kv_tokens": 11, "plan_n_pages": 12}
 HDR_WORDS = 16
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 
 # Scratch memory that the package keeps per device (the K-split workspace of the GEMM, the
@@ -68,7 +68,7 @@ class AttnStream(C.Structure):
 # call (nine addresses, 0 for none, the workspace's address and size, the softmax scale) and what a plan's calls
 # have in common (``attn_call_tail``).  0.5 us a call; eighteen arguments one by one take the binding 2.7.
 ATTN_CALL_HEAD = struct.Struct("10PNf")
-ATTN_OWN_ROWS, ATTN_APPEND_APART = 1, 2
+ATTN_OWN_ROWS, ATTN_APPEND_APART, ATTN_FIXED_ORDER = 1, 2, 4
 
 
 def attn_call_tail(append_tokens: int, n_streams: int, num_heads: int, head_dim: int, page_size: int, dtype: int, flags: int) -> bytes:

@@ -194,7 +194,7 @@ class HipAggregatorStream(nn.Module):
                 sliding_window=list(windows) if isinstance(windows, (list, tuple)) else windows,
                 max_total_frames=self.max_frame_num + 100, force_fp32=self.kv_cache_force_fp32,
                 page_size=self.page_size, layout=self.layout, num_streams=self.num_streams,
-                device_token_counts=self.device_token_counts)
+                device_token_counts=self.device_token_counts, fixed_order=True)
         return self.kv_cache_manager
 
     def clean_kv_cache(self) -> None:

@@ -21,6 +21,10 @@ Extensions beyond the reference signature (all keyword-only, defaults = referenc
 ``device_token_counts`` the attention kernels read each stream's visible-token count from the
                      device tables instead of the launch arguments, so that a frame's launches
                      stay identical while the trajectory memory grows (HIP-graph replay)
+``fixed_order``      ``step`` and ``compute_attention`` add a stream's bf16 sums in the order that
+                     ``step_qkv`` and a block's native call always keep (``LBM_ATTN_FIXED_ORDER``): for a
+                     model whose blocks call them, through which the last bits of an attention grow.
+                     Without it they take the order that is fastest for one call
 
 With shared tables block 0 leads, as the reference's ``plan()`` at ``block_idx == 0`` does
 (flashinfer_cache.py:385-414): table operations run when ``block_idx == 0`` and the other
@@ -78,6 +82,7 @@ class HipPagedKVCacheManager:
         num_streams: int = 1,
         per_block_tables: bool = False,
         device_token_counts: bool = False,
+        fixed_order: bool = False,
     ):
         device = torch.device(device)
         if device.type != "cuda":
@@ -115,6 +120,7 @@ class HipPagedKVCacheManager:
         self.num_streams = num_streams
         self.per_block_tables = per_block_tables
         self.device_token_counts = bool(device_token_counts)
+        self.fixed_order = bool(fixed_order)
         self.force_fp32 = force_fp32
         if force_fp32:  # flashinfer_cache.py:121-127
             self.dtype = torch.float32
@@ -190,8 +196,8 @@ class HipPagedKVCacheManager:
         self._n_appends: List[int] = [0] * num_blocks    # appends ever made per block (rollbacks do not count down)
         # what the launches of one plan have in common, kept per table set until the plan's token
         # counts change: (counts, stream descriptors, their address, streams with tokens, workspace
-        # bytes, the tail of the attention call's record)
-        self._launches = [((), None, 0, 0, 0, b"") for _ in range(self._n_sets)]
+        # bytes, the tail of the attention call's record, the same with a fixed order of sums)
+        self._launches = [((), None, 0, 0, 0, b"", b"") for _ in range(self._n_sets)]
         self._sm_scale = 1.0 / math.sqrt(head_dim)
         self._frame_shape = torch.Size((num_streams * tokens_per_frame, num_heads, head_dim))
         # a step's operations, with the fields that never change filled in
@@ -708,7 +714,8 @@ class HipPagedKVCacheManager:
 
     def _attend_planned(self, block_idx: int, q: Tensor, self_k: Optional[Tensor], self_v: Optional[Tensor],
                         q_prescaled: bool = False, append_rows: Optional[int] = None) -> Tensor:
-        """``q_prescaled``: q already carries 1 / sqrt(D) and log2(e) (``step_qkv``'s producer).
+        """``q_prescaled``: q already carries 1 / sqrt(D) and log2(e) (``step_qkv``'s producer, whose caller is
+        a block of a model: the order of sums is fixed).
         ``append_rows``: the address of the rows ``self_k`` / ``self_v`` are also stored in, row t in
         pool row ``append_rows[t]``: pages of this frame, which its plan names by the caller's rows
         (``LBM_ATTN_APPEND_APART``)."""
@@ -727,7 +734,7 @@ class HipPagedKVCacheManager:
                 self_k, self_v = self_k.to(self.dtype), self_v.to(self.dtype)
             self_k, self_v = self_k.contiguous(), self_v.contiguous()
             k_ptr, v_ptr = self_k.data_ptr(), self_v.data_ptr()
-        _, _, streams, n, need, tail = self._launch_plan(ts)
+        _, _, streams, n, need, tail, tail_fixed = self._launch_plan(ts)
         if n < self.num_streams:
             out.zero_()
         if n == 0:
@@ -738,7 +745,8 @@ class HipPagedKVCacheManager:
         live = self._live_counts_ptr(ts) if self.device_token_counts and append_rows is None else 0
         N.check(N.lib.lbm_attn_run_call(N.ATTN_CALL_HEAD.pack(
             qc.data_ptr(), self.kv_caches[block_idx].data_ptr(), out.data_ptr(), k_ptr, v_ptr, self._kv_rows_ptr(ts), live,
-            append_rows or 0, streams, ws.data_ptr(), ws.numel(), 0.0 if q_prescaled else self._sm_scale) + tail, self._stream_handle()))
+            append_rows or 0, streams, ws.data_ptr(), ws.numel(), 0.0 if q_prescaled else self._sm_scale)
+            + (tail_fixed if q_prescaled or self.fixed_order else tail), self._stream_handle()))
         return out
 
     def _launch_plan(self, ts: int):
@@ -753,9 +761,10 @@ class HipPagedKVCacheManager:
                     streams[n] = N.AttnStream(b * T, T, b * self._rows_cap, kv, b * self._table_words)
                     n += 1
             need = int(N.lib.lbm_attn_workspace_bytes(streams, n, self.num_heads, self.head_dim)) if n else 0
-            tail = N.attn_call_tail(self._frame_shape[0], n, self.num_heads, self.head_dim, self.page_size,
-                                    N.DTYPE_BF16 if self.dtype == torch.bfloat16 else N.DTYPE_F32, N.ATTN_APPEND_APART)
-            hit = self._launches[ts] = (counts, streams, C.addressof(streams), n, need, tail)
+            tail, tail_fixed = (N.attn_call_tail(self._frame_shape[0], n, self.num_heads, self.head_dim, self.page_size,
+                                                 N.DTYPE_BF16 if self.dtype == torch.bfloat16 else N.DTYPE_F32, flags)
+                                for flags in (N.ATTN_APPEND_APART, N.ATTN_APPEND_APART | N.ATTN_FIXED_ORDER))
+            hit = self._launches[ts] = (counts, streams, C.addressof(streams), n, need, tail, tail_fixed)
         return hit
 
     def _workspace(self, need: int) -> Tensor:

@@ -49,6 +49,7 @@ def test_binding_constants_match_header():
     # lbm_attn_call: ten pointers, a size, a float and seven ints without holes
     assert N.ATTN_CALL_HEAD.size == 11 * 8 + 4 and len(N.attn_call_tail(0, 1, 2, 3, 4, 5, 6)) == 7 * 4
     assert (defs["LBM_ATTN_OWN_ROWS"], defs["LBM_ATTN_APPEND_APART"]) == (N.ATTN_OWN_ROWS, N.ATTN_APPEND_APART)
+    assert defs["LBM_ATTN_FIXED_ORDER"] == N.ATTN_FIXED_ORDER
 
 
 def test_host_side_argument_checks_need_no_gpu():

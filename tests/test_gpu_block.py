@@ -665,3 +665,57 @@ def test_anchor_pass_with_folded_norms_is_no_farther_from_float64(spread):
             x = x + b.ls2.gamma.double() * lin(F.gelu(lin(ln(x, b.norm2), b.mlp.fc1)), b.mlp.fc2)
     err = {native: (run(native)[0] - x).norm().item() for native in (True, False)}
     assert err[True] <= 1.01 * err[False], err
+
+
+@pytest.mark.parametrize("rows,kv", [(261, 2349), (261, 4437), (90, 90)])
+def test_block_as_one_call_equals_its_parts(rows, kv):
+    """``lbm_block_run`` against the launches that its declaration names, bit for bit: the attention over a cache is
+    the flagged call, whose order of sums is fixed."""
+    import ctypes as C
+    from lingbot_map_amd import _native as N
+    dev, H, hidden, S = torch.device("cuda:0"), 16, 2048, 16
+    dim = 64 * H
+    g = torch.Generator(device=dev).manual_seed(rows + kv)
+    rand = lambda *shape, s=1.0: (torch.randn(*shape, generator=g, device=dev) * s)
+    bf = lambda t: t.to(torch.bfloat16)
+    x, a = bf(rand(rows, dim)), bf(rand(rows, dim))
+    ws = {n: bf(rand(*shape, s=shape[1] ** -0.5)) for n, shape in (("qkv", (3 * dim, dim)), ("proj", (dim, dim)), ("fc1", (hidden, dim)), ("fc2", (dim, hidden)))}
+    fc1_sum, ls = ws["fc1"].float().sum(1).contiguous(), rand(dim, s=0.1)
+    pages = -(-kv // S)
+    pool = bf(rand(pages, 2, S, H, 64))
+    t = torch.arange(kv, dtype=torch.int32, device=dev)
+    table = (t // S * 2 * S + t % S).to(torch.int32).contiguous()
+    append = table[-rows:].contiguous()
+    arr = (N.AttnStream * 1)(N.AttnStream(0, rows, 0, kv, 0))
+    need = int(N.lib.lbm_attn_workspace_bytes(arr, 1, H, 64))
+    attn_ws, split_bytes = torch.empty(max(need, 16), dtype=torch.uint8, device=dev), int(N.lib.lbm_linear_workspace_bytes(rows, dim, hidden, N.LINEAR_BIAS_RESIDUAL))
+    split = torch.zeros(max(split_bytes, 16), dtype=torch.uint8, device=dev)
+    scale, tiles = N.q_scale_log2(0.125), int(N.lib.lbm_linear_stats_tiles(rows, dim))
+    st = N.stream_handle(dev)
+    p = lambda t: t.data_ptr()
+
+    one, pool_one = torch.empty_like(x), pool.clone()
+    scratch = torch.empty(int(N.lib.lbm_block_scratch_bytes(rows, H, hidden)), dtype=torch.uint8, device=dev)
+    weights = N.BlockWeights(p(ws["qkv"]), p(ws["proj"]), p(ws["fc1"]), p(ws["fc2"]), None, None, None, None, None, p(fc1_sum), p(ls), p(ls),
+                             None, None, None, None, 0.0, 1e-6, 1e-5, H, hidden)
+    call = N.BlockCall(p(x), p(a), None, p(one), None, p(scratch), None, p(pool_one), p(append), p(table), None, C.addressof(arr),
+                       p(attn_ws), p(split), scratch.numel(), attn_ws.numel(), split_bytes, scale, rows, 0, 0, False, 1, S,
+                       (None,) * 4, (0,) * 4, 0)
+    N.check(N.lib.lbm_block_run(weights, call, st))
+
+    q, heads, x1, parts, pool_parts = (torch.empty_like(t) for t in (x, x, x, x, pool))
+    pool_parts.copy_(pool)
+    mid, stats = torch.empty(rows, hidden, dtype=torch.bfloat16, device=dev), torch.empty(rows, tiles, 2, device=dev)
+    N.check(N.lib.lbm_qkv_linear_prepare_norm(p(a), None, p(ws["qkv"]), None, rows, dim, None, None, None, None, 1e-5, scale, None, 0, p(q),
+                                              None, None, p(pool_parts), p(append), H, 64, S, st))
+    N.check(N.lib.lbm_attn_run_call(
+        N.ATTN_CALL_HEAD.pack(p(q), p(pool_parts), p(heads), 0, 0, p(table), 0, 0, C.addressof(arr), p(attn_ws), attn_ws.numel(), 0.0)
+        + N.attn_call_tail(0, 1, H, 64, S, N.DTYPE_BF16, N.ATTN_FIXED_ORDER), st))
+    N.check(N.lib.lbm_linear_norm(p(heads), None, p(ws["proj"]), None, p(ls), p(x), p(x1), p(stats), rows, dim, dim,
+                                  N.LINEAR_BIAS_RESIDUAL, None, 0, st))
+    N.check(N.lib.lbm_linear_norm(p(x1), N.RowNorm(p(stats), p(fc1_sum), tiles, 1e-6), p(ws["fc1"]), None, None, None, p(mid), None,
+                                  rows, hidden, dim, N.LINEAR_BIAS_GELU, None, 0, st))
+    N.check(N.lib.lbm_linear_norm(p(mid), None, p(ws["fc2"]), None, p(ls), p(x1), p(parts), None, rows, dim, hidden,
+                                  N.LINEAR_BIAS_RESIDUAL, p(split), split_bytes, st))
+    torch.cuda.synchronize()
+    assert torch.isfinite(one.float()).all() and torch.equal(pool_one, pool_parts) and torch.equal(one, parts)

@@ -388,3 +388,43 @@ def test_step_refuses_flags_for_another_number_of_streams(flags, block):
     assert [m.build_visible_page_table(0, s) for s in range(2)] == tables
     m.step(block, *qkv, keyframe=(True, True))
     m.check_device_errors()
+
+
+@pytest.mark.parametrize("frames", [9, 17])
+def test_blocks_and_fixed_order_managers_add_in_the_order_of_the_native_call(frames):
+    """261 rows over 2,349 and 4,437 cached tokens, where one call alone is summed in another order: ``step_qkv``, and
+    ``step`` and ``compute_attention`` of a ``fixed_order`` manager, give the bits of the flagged attention call over
+    their plan's row table (which are ``lbm_block_run``'s: test_block_as_one_call_equals_its_parts)."""
+    import ctypes as C
+    from lingbot_map_amd import HipPagedKVCacheManager, _native as N
+    dev, T, H, D = torch.device("cuda:0"), 261, 16, 64
+    torch.manual_seed(frames)
+    fused, split, plain = (HipPagedKVCacheManager(1, frames + 16, T, H, D, torch.bfloat16, dev, num_special_tokens=5, scale_frames=1,
+                                                  sliding_window=frames - 1, max_total_frames=64, page_size=16, layout="frame_pages",
+                                                  fixed_order=fixed) for fixed in (False, True, True))
+    for _ in range(frames):
+        qkv = torch.randn(T, 3 * H * D, device=dev).to(torch.bfloat16)
+        q, k, v = (t.contiguous() for t in qkv.view(T, 3, H, D).unbind(1))
+        a = fused.step_qkv(0, qkv)
+        b = split.step(0, q, k, v)
+        plain.append_frame(0, k, v)
+        plain.evict_frames(0, 1, frames - 1)
+        c = plain.compute_attention(0, q)
+    kv = frames * T
+    assert [m._plan_tokens[0][0] for m in (fused, split, plain)] == [kv] * 3
+
+    def flagged(m, q, scale, k, v):
+        arr = (N.AttnStream * 1)(N.AttnStream(0, T, 0, kv, 0))
+        ws = torch.empty(max(int(N.lib.lbm_attn_workspace_bytes(arr, 1, H, D)), 16), dtype=torch.uint8, device=dev)
+        out = torch.full_like(q, float("nan"))
+        N.check(N.lib.lbm_attn_run_call(N.ATTN_CALL_HEAD.pack(
+            q.data_ptr(), m.kv_caches[0].data_ptr(), out.data_ptr(), k.data_ptr(), v.data_ptr(), m._kv_rows.data_ptr(), 0, 0, C.addressof(arr),
+            ws.data_ptr(), ws.numel(), scale) + N.attn_call_tail(0, 1, H, D, 16, N.DTYPE_BF16, N.ATTN_FIXED_ORDER), N.stream_handle(dev)))
+        return out
+
+    scaled = torch.empty_like(q)
+    N.check(N.lib.lbm_qkv_prepare(qkv.data_ptr(), N.DTYPE_BF16, None, None, None, None, 1e-5, N.q_scale_log2(0.125), None, 0, scaled.data_ptr(),
+                                  None, None, N.DTYPE_BF16, None, None, T, H, D, 16, N.stream_handle(dev)))
+    assert torch.equal(a, flagged(fused, scaled, 0.0, k, v))
+    assert torch.equal(b, flagged(split, q, 0.125, k, v))
+    assert torch.equal(c, flagged(plain, q, 0.125, k, v)) and torch.equal(b, c)
