@@ -2295,13 +2295,14 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       blocks += (unsigned)(((long long)append_tokens * num_heads * 8 + kSmThreads - 1) / kSmThreads);
       *appended = true;
     }
-    if (own_rows) {
+    bool turn = false;   // (the kernel decides per stream, by the live count)
+    for (int i = 0; i < sch.n_streams && !sch.fixed_order; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);
+    // (own rows in order change where rows are read from, not the order of the sums: a launch that goes round keeps its table)
+    if (own_rows && !turn) {
       if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false, true>), dim3(blocks), dim3(kSmThreads), 0, stream, a);
       else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, false, true>), dim3(blocks), dim3(kSmThreads), 0, stream, a);
       return lbm_check_launch("lbm_attn_bf16_d64_small_kernel<own rows>");
     }
-    bool turn = false;   // (the kernel decides per stream, by the live count)
-    for (int i = 0; i < sch.n_streams && !sch.fixed_order; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);
     const dim3 grid(blocks), block(kSmThreads);
     if (sch.small == 64 && turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, true>), grid, block, 0, stream, a);
     else if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false>), grid, block, 0, stream, a);
