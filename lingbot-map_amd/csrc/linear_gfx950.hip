@@ -192,7 +192,7 @@ __device__ __forceinline__ void gelu_of(const f32x4 (&x)[C], const unsigned shor
 // to each; an XCD's 32 take consecutive tiles of an order that walks panels of 8 column tiles row
 // by row, i.e. 4 row tiles x 8 column tiles (8 x 4 in a last panel of 4): 12 operand tiles per
 // k-step for the XCD's L2 to hold instead of 17 to 33, which is what sets the latency of the
-// operand loads.  (Tiles of 64 columns x 64 or 32 rows: panels of kRowsPanel column tiles, for the same reason.)
+// operand loads.  (Tiles of 64 columns x 64 or 32 rows: panels of 4 or 8, see there.)
 __device__ __forceinline__ void lbm_tile_of_workgroup(int b, int m_tiles, int n_tiles, int& mt, int& nt, int panel_width = 8) {
   const int x = b & 7, i = b >> 3;
   const int base = (i >> 5) * 256;
@@ -842,10 +842,13 @@ __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_
   int mt, nt;
   // Panels of 4 column tiles, not 8: fewer bytes for an XCD's L2 where a launch has few row tiles (us, weights rotating
   // through 24 layers, M x N x K 261 x 1,024 x 4,096 11.2 -> 10.1, 261 x 1,024 x 1,024 5.2 -> 4.9, 261 x 3,072 x 1,024
-  // 6.4 -> 6.2); 16 row tiles of 64 with slices of K read whole rows of a long K, where 8 x 4 is the smaller set
-  // (1,004 x 1,024 x 4,096, weights in HBM: 18.9, 19.2 with 4).
-  constexpr int kRowsPanel = TM == 64 && KS > 1 ? 8 : 4;
-  lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt, kRowsPanel);
+  // 6.4 -> 6.2).  64-row tiles whose K is long or whose rows are many are the exception: there
+  // panels of 8 keep a row of a with two XCDs instead of four (us, M x N x K, weights in HBM, panels of 4 and 8:
+  // 513 x 1,024 x 4,096 15.7, 15.8, 566 19.6, 19.5, 700 20.3, 19.9, 900 16.6, 16.6, 1,004 19.6, 19.3, at 9 to 16 row tiles, and from
+  // the last-level cache the same to 1 %; 1,004 x 896 x 3,584 17.9, 17.5; but 673 x 768 x 3,072 11.4, 11.8, 1,280 14.3, 14.4;
+  // 900 x 640 x 2,560 10.7, 11.1; 1,100 x 512 x 2,048 8.6, 9.0, 1,700 8.8, 9.1, 1,800 9.4, 9.2, 2,048 10.0, 9.5).
+  if (TM == 64 && KS > 1 && (p.K > 3072 || p.m_tiles >= 28)) lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt, 8);
+  else lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt, 4);
   const int m0 = mt * TM, n0 = nt * 64;
   const int nk = p.K / (2 * kKS);                          // 128-wide steps
 

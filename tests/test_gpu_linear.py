@@ -555,6 +555,27 @@ def test_few_rows_are_exact_on_small_integers(M):
                     assert torch.equal(out[:M], want[epi]), (K, Nn, epi, with_ws)
 
 
+@pytest.mark.parametrize("M,K,Nn", [(450, 4096, 1024), (513, 4096, 1024), (1004, 4096, 1024), (700, 3072, 768), (700, 3584, 896),
+                                    (1728, 2048, 512), (1729, 2048, 512), (2000, 2048, 448), (300, 2048, 320)])
+def test_every_tile_of_a_panel_is_computed_once(M, K, Nn):
+    """Tiles dealt in panels of 4 and of 8 column tiles, whole and narrower last panels, on either side of the lines
+    between them, K in slices: sums of whole numbers are exact, so a tile left out or taken for another shows."""
+    N = _native()
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(M + Nn)
+    a, w = (torch.randint(-1, 2, s, generator=g, device=dev).to(torch.bfloat16) for s in ((M, K), (Nn, K)))
+    res = torch.randint(-8, 9, (M, Nn), generator=g, device=dev).to(torch.bfloat16)
+    need = int(N.lib.lbm_linear_workspace_bytes(M, Nn, K, N.LINEAR_BIAS_RESIDUAL))
+    assert need > 0
+    ws = torch.zeros(need, dtype=torch.uint8, device=dev)
+    out = torch.full((M, Nn), float("nan"), dtype=torch.bfloat16, device=dev)
+    N.check(N.lib.lbm_linear_norm(ptr(a), None, ptr(w), None, None, ptr(res), ptr(out), None, M, Nn, K, N.LINEAR_BIAS_RESIDUAL,
+                                  ptr(ws), need, None))
+    torch.cuda.synchronize()
+    lin = (a.float().cpu() @ w.float().cpu().T).to(torch.bfloat16)       # (sums below 2^24: exact in any order)
+    assert torch.equal(out.cpu(), (res.float().cpu() + lin.float()).to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("M,H", [(2, 1), (33, 3), (64, 2), (100, 5)])
 def test_few_rows_with_the_producer_as_the_epilogue(M, H):
     """The producer on the 64- and 32-row tiles: as on the others, bit-equal to the two separate launches."""
