@@ -2027,12 +2027,14 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
     }
     // One stream's attention to a cache: no encoder makes such a launch (theirs attend to their own rows), so the
     // fitted costs may give it to the short-KV kernel, up to 4,864 tokens and where they see the pair less than 8 %
-    // ahead: they underrate the pair by 23 % and this kernel by 17 % where K/V come from HBM.  Of 16 random launches
-    // with 80-1,374 rows 11 change over, 0.83 of their time in the mean and none slower.  us per block of a streamed
-    // frame, 24 blocks, pair and this kernel: 400 x 3,600 25.1, 19.4; 261 x 3,393 21.9, 18.5; 261 x 4,437 23.2, 21.9;
-    // 800 x 4,800 31.4, 29.5; 1,004 x 5,020 33.8, 34.4;
-    // 120 x 3,000 17.3, 17.8.  Up to 256 rows, where no SIMD has two of the pair's wavefronts at work, only where they see the pair
-    // behind (209 x 2,976 20.6, 19.9; 209 x 3,500 21.5, 22.4).  Several streams' launches are priced less well and stay.
+    // ahead, up to 256 rows, where no SIMD has two of the pair's wavefronts at work, 4 % behind.  The costs were fitted to
+    // K/V that caches hold and underrate both kernels from HBM, by more the longer the list; the two lines and the limit
+    // are where the measured crossing (133 launches, 86-1,374 rows over 1,700-4,800 tokens, 8 to 16 heads, K/V from HBM)
+    // leaves no launch slower: 63 change over, at 0.68 to 0.94 of the
+    // pair's time, 0.84 in the mean; of the 70 that stay 27 would take 0.92.  us, 16 heads, pair and this kernel: 209 x
+    // 2,976 19.1, 16.8; 261 x 4,437 23.1, 21.3; 420 x 4,800 26.8, 23.6; 1,004 x 4,800 32.2, 30.3; left to the pair: 209 x
+    // 3,500 19.6, 19.1; 256 x 4,437 21.1, 22.1; 1,004 x 5,700 35.2, 35.1; 1,200 x 4,800 37.3, 50.5.  Several streams'
+    // launches are priced less well and stay.
     if (!memo.small && one_cache) {
       const double pair_us = price_candidate(qt, nt, n_streams, num_heads, (int)best_tps, q_rows, cand_splits, false);
       const double us32 = price_small(nt, n_streams, num_heads, 32, q_rows), us64 = price_small(nt, n_streams, num_heads, 64, q_rows);
