@@ -246,8 +246,10 @@ int32_t lbm_linear_stats_tiles(int32_t M, int32_t N);
  * activations and / or out_stats (NULL = none; residual epilogue only) written.
  * workspace (NULL = none): device memory of at least lbm_linear_workspace_bytes(M, N, K, epilogue)
  * bytes with which a launch with few tiles and a long K (fc2 of one frame: K = 4096) sums K in two
- * or four slices that it adds in a fixed order, so results do not depend on timing: up to K = 4096 within a
- * workgroup, beyond with several workgroups per tile that meet in the workspace.  The first 512 bytes
+ * or four slices that it adds in a fixed order, so results do not depend on timing.  Several workgroups per
+ * tile meet in the workspace, or, up to K = 4096 in slices of whole 256-wide steps, one workgroup adds all
+ * slices of a tile: then the query is the 512 bytes of counters, nothing is written, and a workspace of that
+ * size only says that slices are wanted (without one, or with a smaller one, K is one sum).  The first 512 bytes
  * of the workspace hold one counter per tile, for every shape: the caller zero-fills the workspace
  * once, every launch leaves the counters at zero, and launches of different shapes may share it.  Launches that overlap in time on one GPU need
  * workspaces of their own, and with a workspace the residual may not alias out. */

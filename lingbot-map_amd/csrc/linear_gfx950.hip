@@ -1508,6 +1508,9 @@ size_t lbm_linear_workspace_for(int M, int N, int K, int epilogue) {
   const int tn = lbm_linear_tiles(p);
   const int s = lbm_linear_splits(p, epilogue);
   if (s == 1) return 0;
+  // (one workgroup for all slices of a tile: nothing is parked, the workspace only says that slices are wanted)
+  LinearArgs rows = p;
+  if (lbm_linear_rows_tiles(rows, tn, s)) return kSplitCounterBytes;
   return kSplitCounterBytes + (size_t)p.m_tiles * p.n_tiles * s * kGM * tn * 4;
 }
 
@@ -1582,7 +1585,9 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
   }
   const bool wide = lbm_linear_tiles(p) == 128;
   const int splits = workspace && workspace_bytes >= lbm_linear_workspace_for(M, N, K, epilogue) ? lbm_linear_splits(p, epilogue) : 1;
-  if (splits > 1 && residual == out)   // a workgroup that is not the tile's last would see the other's store
+  // (where several workgroups share a tile, one that is not its last would see the other's store; one workgroup per tile
+  // would not, but what a call with a workspace accepts does not depend on which of the two its sizes give)
+  if (splits > 1 && residual == out)
     return lbm_fail(LBM_ERR_INVALID, "lbm_linear_norm: with a workspace the residual may not alias out");
   if (const int tm = lbm_linear_rows_tiles(p, wide ? 128 : 64, splits)) {
     const dim3 grid_r((unsigned)(p.m_tiles * p.n_tiles)), block_r(lbm_rows_threads(tm));

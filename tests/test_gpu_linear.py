@@ -412,10 +412,11 @@ def test_layernorm_folded_into_the_qkv_projection_and_producer(M):
         assert (a0 - a1).abs().mean().item() <= 2.0 ** -9 * a0.abs().mean().item() + 1e-3
 
 
-@pytest.mark.parametrize("M,K,Nn", [(1004, 4096, 1024), (200, 4096, 256), (130, 2048, 64)])
+@pytest.mark.parametrize("M,K,Nn", [(1004, 4096, 1024), (200, 4096, 256), (130, 2048, 64), (1004, 2304, 1024)])
 def test_residual_epilogue_with_k_split_over_workgroups(M, K, Nn):
-    """With a workspace, launches with few tiles and a long K put several workgroups on a tile; the
-    one that finishes last sums the slices in a fixed order.  Against the CPU arithmetic (same bars
+    """With a workspace, launches with few tiles and a long K sum it in slices: one workgroup per tile in the first
+    three, which leave the workspace alone, several in the last (slices of an odd number of steps), of
+    which the one that finishes last sums the slices in a fixed order.  Against the CPU arithmetic (same bars
     as the one-workgroup kernel), three launches in a row on one workspace (the counters go back to
     zero by themselves) giving the same bits, statistics included."""
     N = _native()
@@ -427,6 +428,7 @@ def test_residual_epilogue_with_k_split_over_workgroups(M, K, Nn):
     need = N.lib.lbm_linear_workspace_bytes(M, Nn, K, N.LINEAR_BIAS_RESIDUAL)
     assert need > 0 and N.lib.lbm_linear_workspace_bytes(M, Nn, K, N.LINEAR_BIAS) == 0
     assert N.lib.lbm_linear_workspace_bytes(1004, 1024, 1024, N.LINEAR_BIAS_RESIDUAL) == 0      # proj: K too short to split
+    assert (need == 512) == (K in (4096, 2048))
     ws = torch.zeros(need, dtype=torch.uint8, device=dev)
     tiles = N.lib.lbm_linear_stats_tiles(M, Nn)
     ad, wd, bd, gd, rd = a.to(dev), w.to(dev), bias.float().to(dev), gamma.float().to(dev), res.to(dev)
@@ -440,6 +442,7 @@ def test_residual_epilogue_with_k_split_over_workgroups(M, K, Nn):
         outs.append((out.cpu(), stats.cpu()))
     n_tiles = ((M + 127) // 128) * tiles
     assert ws[:4 * n_tiles].view(torch.int32).abs().sum().item() == 0            # counters back at zero
+    assert bool(ws.any()) == (need > 512)
     scale = torch.maximum(res.float().abs(), (ref.float() - res.float()).abs())
     check(outs[0][0], ref, scale=scale, bar=2.0 ** -6)
     for o, st in outs[1:]:
@@ -449,7 +452,7 @@ def test_residual_epilogue_with_k_split_over_workgroups(M, K, Nn):
     # a workspace that is too small: the launch runs unsplit; the residual aliasing the output is refused with a workspace
     out = torch.full((M, Nn), float("nan"), dtype=torch.bfloat16, device=dev)
     N.check(N.lib.lbm_linear_norm(ptr(ad), None, ptr(wd), ptr(bd), ptr(gd), ptr(rd), ptr(out), None, M, Nn, K,
-                                  N.LINEAR_BIAS_RESIDUAL, ptr(ws), 1024, None))
+                                  N.LINEAR_BIAS_RESIDUAL, ptr(ws), need - 1, None))
     torch.cuda.synchronize()
     check(out.cpu(), ref, scale=scale, bar=2.0 ** -6)
     assert N.lib.lbm_linear_norm(ptr(ad), None, ptr(wd), ptr(bd), ptr(gd), ptr(rd), ptr(rd), None, M, Nn, K,
@@ -496,12 +499,12 @@ def test_prefetch_hint_changes_no_result(M, K, Nn, epilogue):
         assert torch.equal(outs[0], outs[1]) and torch.isfinite(outs[0].float()).all()
 
 
-def test_k_split_launches_of_two_shapes_share_one_workspace():
+@pytest.mark.parametrize("shapes", [((100, 4096, 256), (900, 4096, 1024))])
+def test_k_split_launches_of_two_shapes_share_one_workspace(shapes):
     """A shape with few tiles, then one with more: the second shape's counters must not lie where the
     first one parked its partial tiles."""
     N = _native()
     dev = torch.device("cuda:0")
-    shapes = [(100, 4096, 256), (900, 4096, 1024)]
     need = [N.lib.lbm_linear_workspace_bytes(M, Nn, K, N.LINEAR_BIAS_RESIDUAL) for M, K, Nn in shapes]
     ws = torch.zeros(max(need), dtype=torch.uint8, device=dev)
     for M, K, Nn in shapes:
