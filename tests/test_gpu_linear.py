@@ -412,10 +412,11 @@ def test_layernorm_folded_into_the_qkv_projection_and_producer(M):
         assert (a0 - a1).abs().mean().item() <= 2.0 ** -9 * a0.abs().mean().item() + 1e-3
 
 
-@pytest.mark.parametrize("M,K,Nn", [(1004, 4096, 1024), (200, 4096, 256), (130, 2048, 64), (1004, 2304, 1024)])
+@pytest.mark.parametrize("M,K,Nn", [(1004, 4096, 1024), (200, 4096, 256), (130, 2048, 64),
+                                    (1004, 2304, 1024), (200, 2304, 256), (512, 6144, 768), (81, 8192, 1024)])
 def test_residual_epilogue_with_k_split_over_workgroups(M, K, Nn):
     """With a workspace, launches with few tiles and a long K sum it in slices: one workgroup per tile in the first
-    three, which leave the workspace alone, several in the last (slices of an odd number of steps), of
+    three, which leave the workspace alone, several in the others (K above 4,096, or slices of an odd number of steps), of
     which the one that finishes last sums the slices in a fixed order.  Against the CPU arithmetic (same bars
     as the one-workgroup kernel), three launches in a row on one workspace (the counters go back to
     zero by themselves) giving the same bits, statistics included."""
@@ -460,7 +461,7 @@ def test_residual_epilogue_with_k_split_over_workgroups(M, K, Nn):
 
 
 @pytest.mark.parametrize("M,K,Nn,epilogue", [(1004, 1024, 3072, "bias"), (1004, 4096, 1024, "residual"), (70, 128, 64, "gelu"),
-                                             (4016, 1024, 4096, "gelu"), (1004, 1024, 1024, "residual")])
+                                             (4016, 1024, 4096, "gelu"), (1004, 1024, 1024, "residual"), (81, 8192, 1024, "residual")])
 def test_prefetch_hint_changes_no_result(M, K, Nn, epilogue):
     """lbm_linear_prefetch_hint: the launch that consumes a hint reads the named memory besides its
     own work - whole buffers, buffers that end inside a 128-byte line, a single line, one shorter
@@ -499,7 +500,8 @@ def test_prefetch_hint_changes_no_result(M, K, Nn, epilogue):
         assert torch.equal(outs[0], outs[1]) and torch.isfinite(outs[0].float()).all()
 
 
-@pytest.mark.parametrize("shapes", [((100, 4096, 256), (900, 4096, 1024))])
+@pytest.mark.parametrize("shapes", [((100, 4096, 256), (900, 4096, 1024)), ((100, 8192, 256), (900, 2304, 1024)),
+                                    ((900, 2304, 1024), (100, 4096, 256), (100, 8192, 256))])
 def test_k_split_launches_of_two_shapes_share_one_workspace(shapes):
     """A shape with few tiles, then one with more: the second shape's counters must not lie where the
     first one parked its partial tiles."""
