@@ -15,6 +15,9 @@ from typing import Callable, Sequence
 import torch
 from torch import Tensor
 
+from .block import _split_workspaces
+from .dense import _workspace as _dense_workspaces
+
 
 class GraphedFrame:
     """``frame_fn(*inputs) -> Tensor`` runs one streamed frame of every stream through all blocks
@@ -55,6 +58,10 @@ class GraphedFrame:
             self.graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(self.graph), torch.no_grad():
                 self._output = frame_fn(*self._inputs)
+            # The captured launches hold the addresses of the scratch memory they were captured with.  The manager and
+            # the package replace theirs when a later call needs more (another size of frame, a longer cache), so
+            # the graph keeps what it was given.
+            self._scratch = (manager.workspace_buffer, *_dense_workspaces.values(), *_split_workspaces.values())
         finally:
             manager._skip_append = skip_before
         if not self.read_only:

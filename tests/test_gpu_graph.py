@@ -250,3 +250,41 @@ def test_pipelined_aggregator_equals_eager_aggregator():
     for x, y in zip(a.kv_cache_manager.kv_caches, b.kv_cache_manager.kv_caches):
         assert torch.equal(x, y)
     b.kv_cache_manager.check_device_errors()
+
+
+def test_replays_keep_the_scratch_memory_they_were_captured_with():
+    """The manager and the package replace their scratch memory when a later call needs more.  A graph's launches still
+    write to what they were captured with: tensors allocated afterwards stay as they are, and the replay equals the
+    eager frame."""
+    from lingbot_map_amd import GraphedFrame, HipPagedKVCacheManager, block, dense, dense_attention
+    dev = torch.device("cuda:0")
+    torch.manual_seed(3)
+    T, H, window = 300, 16, 17
+    mk = lambda: HipPagedKVCacheManager(1, window + 18, 4 * T, H, 64, torch.bfloat16, dev, num_special_tokens=5, scale_frames=1,
+                                        sliding_window=window, max_total_frames=64, page_size=16, layout="frame_pages")
+    eager, graphed = mk(), mk()
+
+    def frame_on(m):
+        def frame(q, k, v):      # (over the cache partial results are merged)
+            return m.step(0, dense_attention(q, k, v, num_streams=1), k, v, cross_frame_special=False)
+        return frame
+
+    xs = [[torch.randn(4 * T, H, 64, device=dev).to(torch.bfloat16) for _ in range(3)] for _ in range(3)]
+    for i in range(window + 2):
+        frame_on(eager)(*xs[i % 3]); frame_on(graphed)(*xs[i % 3])
+    block._split_workspace(dev, 4096)
+    g = GraphedFrame(graphed, frame_on(graphed), xs[0], cross_frame_special=False)
+    lane = (dev, 0)
+    sizes = [graphed.workspace_buffer.numel(), dense._workspace[lane].numel(), block._split_workspaces[lane].numel()]
+    assert graphed._launches[0][4] > 0
+    graphed._workspace(2 * sizes[0])
+    dense._workspace.pop(lane)
+    dense.dense_plan(8, 1, H, 64, dev)
+    block._split_workspace(dev, 2 * sizes[2])
+    torch.cuda.synchronize()
+    later = [torch.full((n,), 7, dtype=torch.uint8, device=dev) for n in sizes for _ in range(3)]
+    for x in xs:
+        want, got = frame_on(eager)(*x), g(*x)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+    assert all((t == 7).all() for t in later)
