@@ -796,8 +796,12 @@ constexpr int kSmThreads = kSmWaves * 64;
 constexpr int kSmMaxKv = 4096;
 constexpr int kSmMaxCacheKv = 4864;   // the same for one stream that attends to more than its own rows (lbm_attn_schedule)
 constexpr int kSmPiece = 32;     // KV tokens per step of a wavefront
-// KV tokens of a launch's longest stream beyond which its workgroups begin at different pieces (lbm_attn_bf16_d64_small_kernel's
-// TURN): 261 rows over 1,305 tokens 9.9 us in order, 10.1 so; 86 over 1,500 13.3, 11.6; 300 over 900 and 2,100 17.3, 16.7.
+// KV tokens of a launch's longest stream beyond which the launch's workgroups begin at different pieces, those of its shorter
+// streams too (lbm_attn_bf16_d64_small_kernel's TURN): 261 rows over 1,305 tokens 9.9 us in order, 10.1 so; 86 over 1,500
+// 13.3, 11.6; 300 over 900 and 2,100 17.3, 16.7.  The shorter streams of such a launch in order instead (16 heads, K/V in
+// HBM, all streams | the long ones only): 261 rows over 783 and 2,088 15.8 | 16.5, over 900 and 2,100 16.7 | 17.5, 330 over
+// three times 990 and 1,980 24.5 | 25.4, but 201 over 804, 1,005 and 1,608 15.9 | 15.6, 261 over 261, 522, 1,305 and 2,349
+// 20.2 | 19.7, 389 over 1,167 and 1,945 17.0 | 16.8.
 constexpr int kSmTurnKv = 1408;
 constexpr int kSmOStride = 68;   // floats per row of a partial output parked in LDS (4-bank shift per row)
 constexpr int kSmPieceBytes = kSmPiece * 64 * 2;                                 // K (or V) rows of a piece, unpadded
@@ -850,7 +854,7 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
   const int n_pieces = (kv_tokens + kSmPiece - 1) / kSmPiece;
   const int pps = (n_pieces + kSmWaves - 1) / kSmWaves;
   const int p0 = wave * pps, p1 = min(p0 + pps, n_pieces);   // this wavefront's pieces (possibly none)
-  // Where in its pieces it begins.  Over a cache the workgroups of a head, which start together, each begin at
+  // Where in its pieces it begins (TURN: the launch's longest stream decided that).  Over a cache the workgroups of a head, which start together, each begin at
   // another place and go round: all at the same one, they would ask HBM for the same two pieces per wavefront,
   // a quarter of what it takes to keep it busy, and wait for them together.  A ragged last piece stays the last
   // (it is masked there).  Attention to a stream's own rows, just written, keeps the order: an encoder's
@@ -2297,7 +2301,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       blocks += (unsigned)(((long long)append_tokens * num_heads * 8 + kSmThreads - 1) / kSmThreads);
       *appended = true;
     }
-    bool turn = false;   // (the kernel decides per stream, by the live count)
+    bool turn = false;   // (for all streams over a cache; the kernel leaves out those with up to two pieces per wavefront, by the live count)
     for (int i = 0; i < sch.n_streams && !sch.fixed_order; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);
     // (own rows in order change where rows are read from, not the order of the sums: a launch that goes round keeps its table)
     if (own_rows && !turn) {
