@@ -269,8 +269,8 @@ size_t lbm_linear_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t epilo
  * lbm_linear, lbm_linear_norm, lbm_qkv_linear_prepare or lbm_qkv_linear_prepare_norm call of the
  * calling host thread then also reads one dword of every 128-byte line of [next_read, next_read +
  * bytes) while it computes (one wavefront per workgroup that does nothing else), which leaves
- * the lines in the memory-side cache.  The hint is consumed by that one call (launches on
- * 256-row tiles ignore it); results are the same with and without it.  The memory must be
+ * the lines in the memory-side cache.  The hint is consumed by that one call (launches on tiles of
+ * 256 columns, whatever their rows, drop it); results are the same with and without it.  The memory must be
  * readable device memory for as long as that launch can run, replays of a captured graph
  * included.  bytes below 128 or next_read = NULL withdraws a pending hint. */
 int lbm_linear_prefetch_hint(const void* next_read, size_t bytes);
@@ -319,10 +319,14 @@ int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k,
  *   LBM_ATTN_OWN_ROWS      entry kv_row_begin + t of kv_rows is -1 - (kv_row_begin + t) for every token t of every
  *                          stream: launches that split no KV rely on it instead of reading the table
  *   LBM_ATTN_APPEND_APART  kv_rows names no row of append_rows, as the plans of lbm_tables_step with
- *                          LBM_OP_PLAN_NEWEST_SELF do: launches that merge nothing carry the append as well, by
- *                          workgroups of their own
- *   LBM_ATTN_FIXED_ORDER   (ABI 12) the bf16 sums of a stream are added in the order that its token counts and fixed
- *                          estimates give them, as lbm_block_run does.  Without it the fastest kernel and the fastest
+ *                          LBM_OP_PLAN_NEWEST_SELF do: the short-KV kernel and the fp32 kernel of head_dim 64, which
+ *                          merge nothing, then carry the append by workgroups of their own, and a row of the few-query
+ *                          kernel may go to several workgroups.  (With or without it, launches that merge partial
+ *                          results carry the append, and so does a few-query launch of one query row per stream that
+ *                          appends those rows; the others, that is a split-KV launch that splits nothing and the fp32
+ *                          kernel of head_dim 128, are followed by a launch of lbm_kv_append's)
+ *   LBM_ATTN_FIXED_ORDER   (ABI 12) the bf16 sums are added in the order that lbm_block_run keeps, which the call's row
+ *                          and token counts and head count decide.  Without it the fastest kernel and the fastest
  *                          order are taken, which a later version may choose otherwise: one call's results differ by
  *                          the rounding of bf16, but 24 blocks one behind the other make the last bits of an attention
  *                          into 0.2 % of the last block's K and V.  Needs no more than lbm_attn_workspace_bytes; fp32

@@ -61,7 +61,7 @@ struct LbmAttnSchedule {
   int64_t part_rows;   // rows of partial results over all streams (0 when nothing is split)
   LbmAttnStreamPlan s[LBM_MAX_STREAMS];
 };
-// fixed_order: the sums of a stream keep the order that the fixed estimates give them, whatever the fitted costs say.
+// fixed_order: neither the schedule's rule for one stream's cache nor workgroups that begin at different pieces.
 // lbm_block_run and calls with LBM_ATTN_FIXED_ORDER ask for it: 24 blocks make the last bits of an attention into 0.2 % of the
 // last block's K and V, single values up to 7 %, and a model's results must not move with a schedule.  Needs at least the workspace of the other.
 void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_heads,

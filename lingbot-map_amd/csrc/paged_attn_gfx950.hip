@@ -2132,8 +2132,8 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
 // append_rows (lbm_attn_run_append): rows of self_k / self_v that are stored in the pool after the
 // attention has read it - inside the launch that merges the split-KV partials when the schedule has
 // one, by lbm_kv_append_kernel behind the attention otherwise.  append_apart: the row tables name none of
-// them, so nobody minds when they are stored, and a launch that merges nothing carries them as well, by
-// workgroups of its own behind the others (a streamed frame of 261 rows over 2,349 tokens, us per block: 19.2 with
+// them, so nobody minds when they are stored, and the short-KV and the fp32 head_dim 64 kernel, which merge nothing, carry
+// them as well, by workgroups of their own behind the others (a streamed frame of 261 rows over 2,349 tokens, us per block: 19.2 with
 // a launch for the append, 16.3 without; fp32, 1,004 rows: 3 us a frame).
 int lbm_launch_attention(const void* q, const void* pool, void* out, const void* self_k,
                          const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
