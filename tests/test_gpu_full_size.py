@@ -230,8 +230,8 @@ def test_frame_blocks_of_several_streams_at_full_size(n_streams):
 @pytest.mark.parametrize("n_streams", [1, 2])
 def test_lookahead_replay_at_full_width(n_streams):
     """The look-ahead replay (next frame's encoder beside the present frame's blocks) at the real
-    widths - 1,004 tokens per frame, dim 1,024, MLP 4,096, so that fc2 splits K over workgroups in
-    both branches (each on the workspace of its own scratch lane) and the launches of the two
+    widths - 1,004 tokens per frame, dim 1,024, MLP 4,096, so that fc2 sums K in slices in
+    both branches (within a workgroup: neither writes to its lane's workspace) and the launches of the two
     branches share the CUs - against the plain replay of a twin model: bit-equal outputs, frame by
     frame, and equal pools."""
     from lingbot_map_amd import GraphedAggregator, HipAggregatorStream, PipelinedAggregator

@@ -215,20 +215,24 @@ def test_graphed_aggregator_equals_eager_aggregator():
     mb.check_device_errors()
 
 
-def test_pipelined_aggregator_equals_eager_aggregator():
+@pytest.mark.parametrize("mlp_ratio", [4.0, 18.0])
+def test_pipelined_aggregator_equals_eager_aggregator(mlp_ratio):
     """The next frame's image encoder as a second branch of the graph that takes the present frame
     through its frame and global blocks: the outputs are those of the eager aggregator bit for
     bit, one call later; keyframes and read-only frames mixed, two ragged streams, an encoder
-    with blocks of its own (whose fc2 splits K, so both branches use a K-split workspace)."""
-    from lingbot_map_amd import HipAggregatorStream, PipelinedAggregator, set_skip_append
+    with blocks of its own.  At an MLP ratio of 18 fc2 has a K of 2,304, which workgroups share in slices of nine steps:
+    both branches park partial sums, each in the workspace of its own scratch lane."""
+    from lingbot_map_amd import HipAggregatorStream, PipelinedAggregator, block, set_skip_append
     dev = torch.device("cuda:0")
     torch.manual_seed(11)
-    kw = dict(img_size=56, patch_size=14, embed_dim=128, depth=2, num_heads=2, init_values=0.5, patch_embed="vit",
+    kw = dict(img_size=56, patch_size=14, embed_dim=128, depth=2, num_heads=2, init_values=0.5, patch_embed="vit", mlp_ratio=mlp_ratio,
               encoder_depth=2, enable_3d_rope=True, max_frame_num=64, kv_cache_sliding_window=[2, 3], kv_cache_scale_frames=1,
               kv_cache_cross_frame_special=False, use_scale_token=False, page_size=4, layout="frame_pages", num_streams=2)
     a = HipAggregatorStream(**kw).to(dev, torch.bfloat16).eval()
     b = HipAggregatorStream(**kw).to(dev, torch.bfloat16).eval()
     b.load_state_dict(a.state_dict())
+    for ws in block._split_workspaces.values():
+        ws[512:].zero_()                         # (behind the counters: the partial sums of earlier launches)
     g = torch.Generator(device=dev).manual_seed(12)
     imgs = [torch.rand(2, 1, 3, 42, 56, generator=g, device=dev).to(torch.bfloat16) for _ in range(5)]
     with torch.no_grad():
@@ -250,6 +254,10 @@ def test_pipelined_aggregator_equals_eager_aggregator():
     for x, y in zip(a.kv_cache_manager.kv_caches, b.kv_cache_manager.kv_caches):
         assert torch.equal(x, y)
     b.kv_cache_manager.check_device_errors()
+    for lane in (0, 1):
+        ws = block._split_workspaces.get((dev, lane))
+        parked = ws is not None and bool(ws[512:].any())
+        assert parked == (mlp_ratio == 18.0) and (ws is None or not ws[:512].any()), lane
 
 
 def test_replays_keep_the_scratch_memory_they_were_captured_with():
