@@ -107,14 +107,14 @@ struct LinearArgs {
   // [M][N >> stats_shift][2], or null
   float* stats_out;
   int stats_shift;               // 6 or 7; 6 where the tiles have 64 columns
-  // K summed in k_splits slices.  SPLITK kernels: k_splits workgroups share a tile, each over its own slice.  Every one
+  // memory the launch after this one will read (lbm_linear_prefetch_hint): one wavefront per workgroup of
+  // the kernels that have one beside the computing and loading ones (touch_lines) asks for it
+  const char* touch;
+  unsigned touch_lines;          // 128-byte lines
+  // SPLITK kernels: K summed in k_splits slices by as many workgroups per tile.  Every one
   // parks its fp32 partial tile in `split_part` and takes a ticket from the tile's counter; the
   // one that draws the last ticket sums the partials in slice order (the same sum whoever is
   // last) and runs the epilogue.  Counters start at zero and are left at zero.
-  // memory the launch after this one will read (lbm_linear_prefetch_hint): one wavefront per workgroup of
-  // lbm_linear_bf16_kernel ask for it
-  const char* touch;
-  unsigned touch_lines;          // 128-byte lines
   int k_splits;
   unsigned* split_counters;      // [m_tiles * n_tiles]
   float* split_part;             // [m_tiles * n_tiles][k_splits][8 waves][NT * 16][64 lanes]
@@ -1487,7 +1487,7 @@ int lbm_set_row_norm(LinearArgs& p, const lbm_row_norm* ln, const char* who) {
 
 namespace {
 // K slices per tile: as many as still leave every workgroup eight k-steps and fit one round of
-// the 256 CUs (fc2 of one frame: 128 tiles x 2); the residual epilogue only
+// the 256 CUs (fc2 of one frame: 128 tiles of 128 x 64, two slices); the residual epilogue only
 int lbm_linear_splits(const LinearArgs& p, int epilogue) {
   if (epilogue != LBM_LINEAR_BIAS_RESIDUAL) return 1;
   const int tiles = p.m_tiles * p.n_tiles, nk = p.K / kGK;

@@ -1779,7 +1779,8 @@ __global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeAr
 // fine_chunks: chunks of 64 tokens up to so many per row, 0 for none.  As many as leave the launch at two workgroups
 // per CU: beyond that its time is that of the bytes and not of the trips.  No more than sixteen a row, since the
 // merge's time grows with them; but thirty-two for caches of 128 floats a row from 3,072 tokens up, where sixteen would be
-// chunks of nearly 256 again.  us a launch, 16 heads, caches in HBM, chunks of 256 | these: head_dim 128, one row over 500
+// chunks of nearly 256 again.  (Beyond 8,192 tokens, or 4,096 of 64 floats, chunks of 256 are the more and decide,
+// whole workgroups per CU or not.)  us a launch, 16 heads, caches in HBM, chunks of 256 | these: head_dim 128, one row over 500
 // tokens 14.5 | 9.1, 700 14.9 | 10.1, 1,500 16.5 | 12.0, 3,000 18.3 | 16.7, 5,000 25.0 | 22.2; four streams of 1,000
 // 20.4 | 17.9; head_dim 64, 700 11.1 | 9.4, 3,000 13.1 | 12.3, four streams of 1,000 13.9 | 12.8.  (Eight rows of one
 // stream, that is four chunks a row: head_dim 64, 700 tokens 11.4 | 11.8, so not from there.)
