@@ -235,6 +235,8 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
   if (live_kv_tokens)
     for (int i = 0; i < n_streams; ++i)
       if (streams[i].live_at < 0) return lbm_fail(LBM_ERR_INVALID, "%s: stream %d has a negative live_at", who, i);
+  // (q travels to LDS directly on the way without a table, 16 bytes a lane; elsewhere it is loaded, from any address)
+  own_rows = own_rows && ((uintptr_t)q & 15) == 0;
   // (rows are addressed by 32-bit byte offsets from the stream's first)
   for (int i = 0; own_rows && i < n_streams; ++i) own_rows = (long long)streams[i].kv_tokens * num_heads * head_dim * 2 < (1LL << 32);
   LbmAttnSchedule sch;
