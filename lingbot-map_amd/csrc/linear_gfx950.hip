@@ -351,11 +351,11 @@ __device__ __forceinline__ unsigned short* produced_rows(const LinearArgs& p, in
 __device__ __forceinline__ void store_produced(const LinearArgs& p, unsigned short* plain, bf16x8 o8, int which, int token, int head, int c8, int pool_row) {
   const int H = p.num_heads;
   const long long nhd = ((long long)token * H + head) * 64 + c8 * 8;
-  if (plain) *(bf16x8*)(plain + nhd) = o8;
+  if (plain) lbm_store_through(plain + nhd, __builtin_bit_cast(u32x4, o8));
   if (which > 0 && pool_row >= 0) {
     const long long row_elems = (long long)H * 64;
     const long long d = (long long)pool_row * row_elems + (which == 2 ? (long long)p.page_size * row_elems : 0) + head * 64 + c8 * 8;
-    *(bf16x8*)(p.pool + d) = o8;
+    lbm_store_through(p.pool + d, __builtin_bit_cast(u32x4, o8));
   }
 }
 
@@ -806,7 +806,7 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
     if (row < p.M) {
       unsigned short* dst = p.out + (size_t)row * p.N + n0 + c;
       if (EPI == LBM_LINEAR_BIAS_RESIDUAL) v = add_rows(res_v[j], v);
-      *(u32x4*)dst = v;
+      lbm_store_through(dst, v);
     }
     if (EPI == LBM_LINEAR_BIAS_RESIDUAL && p.stats_out) store_row_stats(p, v, row, n0 + c, TN == 64 ? 6 : p.stats_shift, tid);
   }
@@ -1041,7 +1041,7 @@ __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_
     return;
   }
   if (EPI == LBM_LINEAR_BIAS_RESIDUAL) v = add_rows(res, v);
-  if (row < p.M) *(u32x4*)(p.out + (size_t)row * p.N + n0 + c8 * 8) = v;
+  if (row < p.M) lbm_store_through(p.out + (size_t)row * p.N + n0 + c8 * 8, v);
   if (EPI == LBM_LINEAR_BIAS_RESIDUAL && p.stats_out) store_row_stats(p, v, row, n0 + c8 * 8, 6, tid);
 }
 
@@ -1391,7 +1391,7 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   for (int j = 0; j < kPasses; ++j) {
     const int r = j * kRowsPerPass + pr, row = m0 + r;
     const u32x2 lo = *(const u32x2*)&stage[r * kBCStride + pc], hi = *(const u32x2*)&stage[r * kBCStride + pc + 4];
-    if (row < p.M) *(u32x4*)(p.out + (size_t)row * p.N + n0 + pc) = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    if (row < p.M) lbm_store_through(p.out + (size_t)row * p.N + n0 + pc, u32x4{lo[0], lo[1], hi[0], hi[1]});
   }
 }
 

@@ -52,6 +52,7 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(8))) float f32x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(8))) short s16x8;
 
@@ -755,7 +756,7 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
       const int row = k * 8 + (lane >> 3);
       const u32x4 v = *(const u32x4*)&stage[row * kKStride + (lane & 7) * 8];
       const int r = q_row0 + qb * 32 + row;
-      if (r < sp.q_rows) *(u32x4*)(dst + ((dst_row0 + r) * H + head) * 64 + (lane & 7) * 8) = v;
+      if (r < sp.q_rows) lbm_store_through(dst + ((dst_row0 + r) * H + head) * 64 + (lane & 7) * 8, v);
     }
     const int r = q_row0 + qb * 32 + n32;
     if (!direct && g == 0 && r < sp.q_rows)
@@ -1192,8 +1193,11 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
     const int r = q_row0 + row;
     if (r < sp.q_rows) {
       unsigned short* dst = a.out + ((size_t)(sp.q_begin + r) * H + head) * 64 + d0;
+      u32x2 y[QB];
 #pragma unroll
-      for (int j = 0; j < QB; ++j) *(bf16x4*)(dst + 4 * j) = __builtin_convertvector(acc[j] * inv, bf16x4);
+      for (int j = 0; j < QB; ++j) y[j] = __builtin_bit_cast(u32x2, __builtin_convertvector(acc[j] * inv, bf16x4));
+      if (QB == 2) lbm_store_through(dst, u32x4{y[0][0], y[0][1], y[QB - 1][0], y[QB - 1][1]});
+      else lbm_store_through(dst, y[0]);
     }
   }
 }
@@ -1296,7 +1300,7 @@ __global__ __launch_bounds__(256) void lbm_attn_combine_bf16_kernel(AttnArgs a) 
   unsigned short* op = a.out + ((size_t)(sp.q_begin + r) * H + h) * 64 + d8 * 8;
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] *= inv;
-  *(bf16x8*)op = __builtin_convertvector(acc, bf16x8);
+  lbm_store_through(op, __builtin_bit_cast(u32x4, __builtin_convertvector(acc, bf16x8)));
 }
 
 // ---------------------------------------------------------------------------- fp32, head_dim 128
