@@ -107,10 +107,10 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
 // aggregator frame of 1,004 rows 6.65 -> 6.49 ms, four streams 16.15 -> 15.90, eight anchor frames 24.7 -> 24.2.  Not for
 // scattered 4- and 8-byte results (log-sum-exps, row statistics): those the L2 collects into lines, and past it the
 // attention of four streams takes 1 % longer.
-// (s_nop: the registers of a 16-byte store may not be written by the very next instruction, which the compiler does not
-// see for inline asm)
+// (s_nop 1: two wait states before a vector instruction may write the registers that a 16-byte store still reads, which the
+// compiler sees to behind its own stores and cannot behind inline asm)
 __device__ __forceinline__ void lbm_store_through(void* dst, __attribute__((ext_vector_type(4))) unsigned int v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" : : "v"(dst), "v"(v) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(dst), "v"(v) : "memory");
 }
 __device__ __forceinline__ void lbm_store_through(void* dst, __attribute__((ext_vector_type(2))) unsigned int v) {
   asm volatile("global_store_dwordx2 %0, %1, off sc1" : : "v"(dst), "v"(v) : "memory");
