@@ -1207,8 +1207,11 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
 //
 // Up to NJ splits (n <= NJ): all 2 NJ loads - the log-sum-exps and the partial rows - are issued
 // before the first use of any of them, one round trip of memory latency instead of three.  NJ is
-// the next of 2, 4, 8 above the split count, so that a launch with two splits (several streams'
-// frame blocks) does not load its last split seven times over.
+// the next of 2, 4, 8, 16 above the split count, so that a launch with two splits (several streams'
+// frame blocks) does not load its last split seven times over.  More than sixteen, few rows of few heads over a long list,
+// go in batches of sixteen.  Bound by trips to memory there; us a launch, batches of 8 log-sum-exps and 4 rows from nine
+// splits on, and these: 261 rows x 16 heads x 14 splits 5.6, 4.0; 261 x 8 x 26 8.0, 5.9; 520 x 4 x 30 8.5, 6.3; 65 x 1 x
+// 64 13.9, 9.0.
 template <int NJ>
 __device__ __forceinline__ void lbm_combine_upto(const float* lse, const unsigned short* po, long long split_stride, int n,
                                                  float& wsum, f32x8& acc) {
@@ -1264,29 +1267,31 @@ __global__ __launch_bounds__(256) void lbm_attn_combine_bf16_kernel(AttnArgs a) 
     lbm_combine_upto<4>(lse, po, split_stride, n, wsum, acc);
   } else if (n <= 8) {
     lbm_combine_upto<8>(lse, po, split_stride, n, wsum, acc);
+  } else if (n <= 16) {
+    lbm_combine_upto<16>(lse, po, split_stride, n, wsum, acc);
   } else {
     // loads are issued in batches (the split count is a run-time value, a plain loop would
     // wait for each load in turn)
     float mx = -INFINITY;
-    for (int s0 = 0; s0 < n; s0 += 8) {
-      float t[8];
+    for (int s0 = 0; s0 < n; s0 += 16) {
+      float t[16];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) t[j] = lse[min(s0 + j, n - 1) * split_stride];
+      for (int j = 0; j < 16; ++j) t[j] = lse[min(s0 + j, n - 1) * split_stride];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) mx = fmaxf(mx, t[j]);
+      for (int j = 0; j < 16; ++j) mx = fmaxf(mx, t[j]);
     }
     if (mx == -INFINITY) mx = 0.f;
-    for (int s0 = 0; s0 < n; s0 += 4) {
-      float t[4];
-      bf16x8 v[4];
+    for (int s0 = 0; s0 < n; s0 += 16) {
+      float t[16];
+      bf16x8 v[16];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < 16; ++j) {
         const long long s = min(s0 + j, n - 1);
         t[j] = lse[s * split_stride];
         v[j] = *(const bf16x8*)(po + s * split_stride * 64);
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < 16; ++j) {
         const float w = s0 + j < n ? __builtin_amdgcn_exp2f(t[j] - mx) : 0.f;
         const f32x8 vf = __builtin_convertvector(v[j], f32x8);
         wsum += w;
