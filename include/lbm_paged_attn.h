@@ -319,12 +319,12 @@ int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k,
  *   LBM_ATTN_OWN_ROWS      entry kv_row_begin + t of kv_rows is -1 - (kv_row_begin + t) for every token t of every
  *                          stream: launches that split no KV rely on it instead of reading the table
  *   LBM_ATTN_APPEND_APART  kv_rows names no row of append_rows, as the plans of lbm_tables_step with
- *                          LBM_OP_PLAN_NEWEST_SELF do: the short-KV kernel and the fp32 kernel of head_dim 64, which
- *                          merge nothing, then carry the append by workgroups of their own, and a row of the few-query
- *                          kernel may go to several workgroups.  (With or without it, launches that merge partial
- *                          results carry the append, and so does a few-query launch of one query row per stream that
- *                          appends those rows; the others, that is a split-KV launch that splits nothing and the fp32
- *                          kernel of head_dim 128, are followed by a launch of lbm_kv_append's)
+ *                          LBM_OP_PLAN_NEWEST_SELF do: the bf16 kernels and the fp32 kernel of head_dim 64 then carry
+ *                          the append by workgroups of their own, and a row of the few-query kernel may go to several
+ *                          workgroups.  (With or without it, few-query launches that merge partial results carry the
+ *                          append, and so does one of one query row per stream that appends those rows; without it
+ *                          the launch that merges a split-KV attention does; the others are followed by a launch of
+ *                          lbm_kv_append's)
  *   LBM_ATTN_FIXED_ORDER   (ABI 12) the bf16 sums are added in the order that lbm_block_run keeps, which the call's row
  *                          and token counts and head count decide.  Without it the fastest kernel and the fastest
  *                          order are taken, which a later version may choose otherwise: one call's results differ by

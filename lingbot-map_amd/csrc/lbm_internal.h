@@ -115,20 +115,38 @@ __device__ __forceinline__ void lbm_store_through(void* dst, __attribute__((ext_
 __device__ __forceinline__ void lbm_store_through(void* dst, __attribute__((ext_vector_type(2))) unsigned int v) {
   asm volatile("global_store_dwordx2 %0, %1, off sc1" : : "v"(dst), "v"(v) : "memory");
 }
-// The append as workgroups of an attention launch: workgroup `wg` of those behind the attention's copies one 16-byte
-// piece of a K row and of the matching V row per thread (row_pieces: 16-byte pieces per row).
+// The append as workgroups of an attention launch: workgroup `wg` of those behind the attention's copies N 16-byte
+// pieces of a K row and of the matching V row per thread (row_pieces: 16-byte pieces per row).
+template <int N = 1>
 __device__ __forceinline__ void lbm_append_pieces(const void* k, const void* v, void* pool, const int32_t* append_rows,
                                                   int append_tokens, int row_pieces, int page_size, int wg, int threads) {
   typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
-  const long long idx = (long long)wg * threads + threadIdx.x;
-  if (idx >= (long long)append_tokens * row_pieces) return;
-  const int t = (int)(idx / row_pieces), piece = (int)(idx % row_pieces);
-  const int row = append_rows[t];
-  if (row < 0) return;
-  const u32x4 kk = ((const u32x4*)k)[idx], vv = ((const u32x4*)v)[idx];
-  u32x4* dst = (u32x4*)pool + (long long)row * row_pieces + piece;
-  lbm_store_through(dst, kk);
-  lbm_store_through(dst + (long long)page_size * row_pieces, vv);
+  // (the workgroup's first piece is uniform; from there 32 bits are enough)
+  const long long base = (long long)wg * N * threads, left = (long long)append_tokens * row_pieces - base;
+  const int t0 = (int)(base / row_pieces);
+  const unsigned at0 = (unsigned)(base - (long long)t0 * row_pieces) + threadIdx.x;
+  if ((long long)threadIdx.x >= left) return;
+  u32x4 kk[N], vv[N];
+  int row[N];
+  unsigned piece[N];
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const bool there = (long long)(threadIdx.x + j * threads) < left;   // past the end: the thread's first once more, not stored
+    const unsigned at = at0 + (there ? (unsigned)(j * threads) : 0u), t = at / (unsigned)row_pieces;
+    piece[j] = at - t * (unsigned)row_pieces;
+    const long long idx = (long long)t0 * row_pieces + at;
+    row[j] = append_rows[t0 + (int)t];
+    if (!there) row[j] = -1;
+    kk[j] = ((const u32x4*)k)[idx];
+    vv[j] = ((const u32x4*)v)[idx];
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    if (row[j] < 0) continue;
+    u32x4* dst = (u32x4*)pool + (long long)row[j] * row_pieces + piece[j];
+    lbm_store_through(dst, kk[j]);
+    lbm_store_through(dst + (long long)page_size * row_pieces, vv[j]);
+  }
 }
 #endif
 

@@ -68,6 +68,8 @@ constexpr int kRingRow = 64;            // bf16 per row of a K/V tile in the LDS
 constexpr int kKStride = 72;            // bf16 per row of a padded patch (Q, output transpose): 144 B, b128 reads hit 64 distinct banks
 constexpr float kHeadroom = 11.0f;      // the softmax reference is set this far above the row maxima (log2 units)
 
+constexpr int kAppendPieces = 4;        // 16-byte pieces of K and of V per thread of a workgroup that appends
+
 struct AttnCore {
   const unsigned short* q;
   const unsigned short* pool;
@@ -81,8 +83,8 @@ struct AttnCore {
   int num_heads;
   int page_size;
   float scale_log2;
-  // the append carried by the merging launch, or by workgroups of the short-KV kernel's launch behind those of
-  // the attention: row t of self_k / self_v to pool row append_rows[t]
+  // the append carried by workgroups behind those of the attention, or by the merging launch: row t of
+  // self_k / self_v to pool row append_rows[t]
   const int32_t* append_rows;
   int append_tokens;
   int combine_blocks;      // blocks (per stream) of that launch that merge; those beyond them append
@@ -769,6 +771,11 @@ __device__ __noinline__ void lbm_attn_split_safe(AttnCore a, LbmAttnStreamPlan s
 }  // namespace
 
 __global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_kernel(AttnArgs a) {
+  if ((int)blockIdx.x >= a.sch.total_wgs) {
+    lbm_append_pieces<kAppendPieces>(a.self_k, a.self_v, const_cast<unsigned short*>(a.pool), a.append_rows, a.append_tokens,
+                                     a.num_heads * 8, a.page_size, (int)blockIdx.x - a.sch.total_wgs, kThreads);
+    return;
+  }
   int b = 0;   // which stream's work is this workgroup
   for (int i = 1; i < a.sch.n_streams; ++i)
     if ((int)blockIdx.x >= a.sch.s[i].wg_begin) b = i;
@@ -2142,8 +2149,8 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
 // append_rows (lbm_attn_run_append): rows of self_k / self_v that are stored in the pool after the
 // attention has read it - inside the launch that merges the split-KV partials when the schedule has
 // one, by lbm_kv_append_kernel behind the attention otherwise.  append_apart: the row tables name none of
-// them, so nobody minds when they are stored, and the short-KV and the fp32 head_dim 64 kernel, which merge nothing, carry
-// them as well, by workgroups of their own behind the others (a streamed frame of 261 rows over 2,349 tokens, us per block: 19.2 with
+// them, so nobody minds when they are stored, and the bf16 kernels and the fp32 head_dim 64 kernel carry
+// them by workgroups of their own behind the others (a streamed frame of 261 rows over 2,349 tokens, us per block: 19.2 with
 // a launch for the append, 16.3 without; fp32, 1,004 rows: 3 us a frame).
 int lbm_launch_attention(const void* q, const void* pool, void* out, const void* self_k,
                          const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
@@ -2326,7 +2333,17 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
     else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, false>), grid, block, 0, stream, a);
     return lbm_check_launch("lbm_attn_bf16_d64_small_kernel");
   }
-  hipLaunchKernelGGL(lbm_attn_bf16_d64_kernel, dim3(sch.total_wgs), dim3(kThreads), 0, stream, a);
+  // The append by workgroups behind the attention's: they run where CUs are done early (the last split of a list has fewer
+  // tiles), and the launch that merges does not wait for them.  us a block, both builds' kernels: 1,004 rows over 17,068
+  // tokens 71.6 + 6.6 for the merge and the append, 72.0 + 5.8; four streams of 1,004 rows 207.5 + 16.3, 209.3 + 11.7.
+  unsigned wgs = (unsigned)sch.total_wgs;
+  if (append_apart && append_rows && append_tokens > 0) {
+    a.append_rows = append_rows;
+    a.append_tokens = append_tokens;
+    wgs += (unsigned)(((long long)append_tokens * num_heads * 8 + kThreads * kAppendPieces - 1) / (kThreads * kAppendPieces));
+    *appended = true;
+  }
+  hipLaunchKernelGGL(lbm_attn_bf16_d64_kernel, dim3(wgs), dim3(kThreads), 0, stream, a);
   int rc = lbm_check_launch("lbm_attn_bf16_d64_kernel");
   if (rc != LBM_OK) return rc;
   if (sch.part_rows > 0) {
@@ -2336,7 +2353,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
     const long long threads = (long long)max_rows * num_heads * 8;
     unsigned blocks = (unsigned)((threads + 255) / 256);
     a.combine_blocks = (int)blocks;
-    if (append_rows && append_tokens > 0) {
+    if (append_rows && append_tokens > 0 && !*appended) {
       a.append_rows = append_rows;
       a.append_tokens = append_tokens;
       blocks += (unsigned)(((long long)append_tokens * num_heads * 8 + 255) / 256);
