@@ -192,7 +192,7 @@ __device__ __forceinline__ void gelu_of(const f32x4 (&x)[C], const unsigned shor
 // to each; an XCD's 32 take consecutive tiles of an order that walks panels of 8 column tiles row
 // by row, i.e. 4 row tiles x 8 column tiles (8 x 4 in a last panel of 4): 12 operand tiles per
 // k-step for the XCD's L2 to hold instead of 17 to 33, which is what sets the latency of the
-// operand loads.  (Tiles of 64 columns x 64 or 32 rows: panels of 4 or 8, see there.)
+// operand loads.  (Tiles of 64 columns x 32, 64 or 96 rows: panels of 4 or 8, see there.)
 __device__ __forceinline__ void lbm_tile_of_workgroup(int b, int m_tiles, int n_tiles, int& mt, int& nt, int panel_width = 8) {
   const int x = b & 7, i = b >> 3;
   const int base = (i >> 5) * 256;
@@ -813,7 +813,7 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
 }
 
 // ---------------------------------------------------------------------------- few rows
-// The same product on tiles of 64 columns x 64 or 32 rows, for launches whose 128-row tiles would leave CUs idle
+// The same product on tiles of 64 columns x 32, 64 or 96 rows, for launches whose 128-row tiles would leave CUs idle
 // (a small image's 261 rows into 1,024 columns: 48 of 256) or share a tile between workgroups that meet in memory.
 // Bound by the fill: a step moves (TM + 64) x 128 bytes through a CU's 64 bytes per cycle for TM x 64 x 64
 // multiplications, a half to a quarter of that time on the matrix pipe, so what counts is how many CUs share the
@@ -823,6 +823,11 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
 // for before the loop.  KS: the launches that sum K in slices (LinearArgs::k_splits) keep KS pairs of sums, one
 // slice behind the other, and add them in slice order at the end: the bits of several workgroups that
 // meet in memory, without the meeting (5 us of an fc2 launch).
+// 96 rows: where 64-row tiles are more than one round of the CUs and 128-row tiles, at 192 rows a step to load instead of
+// 160, are one: 257-384 rows x 4,096 columns, 321-480 x 3,072, 1,025-1,536 x 1,024.  (Three stages, not four: 40 KB each.)  us
+// per launch on tiles of 128 and of 96 rows: 261 x 4,096 x 1,024 + GELU 8.4, 7.5, 384 rows 8.9, 7.9; 330 x 3,072 x 1,024
+// with the producer 9.2, 8.4, 480 rows 9.9, 9.0; 1,200 x 1,024 x 1,024 7.8, 7.0, x 4,096 19.1, 17.8; 1,536 x 1,024 x 4,096
+// 19.8, 19.6; 1,500 x 768 x 3,072 16.3, 14.3.
 // us per launch, weights rotating through 24 layers, before (128 x 64 tiles) and after: M x N x K 81 x 3,072 x
 // 1,024 with the producer 9.4 -> 6.1, 261 rows 10.1 -> 7.6; 261 x 1,024 x 1,024 8.1 -> 4.9, 1,004 rows 8.4 -> 6.4;
 // 261 x 1,024 x 4,096 12.3 -> 10.1, 512 rows 14.6 -> 11.4, 1,004 rows 18.1 -> 15.3.  (Six stages instead of four: no
@@ -832,7 +837,7 @@ __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_
   constexpr int kWaves = TM / 32 * 4;                      // computing wavefronts: (TM / 32) x 2 blocks of 32 x 32, two halves of K each
   constexpr int kHalf = (TM + 64) * kKS;                   // elements of one 64-wide half of a stage: rows of a, then of w
   constexpr int kStage = 2 * kHalf;
-  constexpr int kStages = 4;
+  constexpr int kStages = TM == 96 ? 3 : 4;
   __shared__ __attribute__((aligned(1024))) unsigned short ops[kStages * kStage];
   __shared__ __attribute__((aligned(16))) unsigned short gelu_tab[EPI == LBM_LINEAR_BIAS_GELU ? kGeluEntries : 8];
   __shared__ __attribute__((aligned(8))) float ln_rows[LNA ? TM * 2 : 2];                   // per row: rstd, -mean * rstd
@@ -885,8 +890,8 @@ __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_
       if (i < nk) load_step(i);
     for (int s = -1; s < nk - 1; ++s) {   // the barrier at the top of step s publishes the rows of step s + 1
       const int behind = nk - 2 - s;      // steps that may be in flight behind those
-      if (behind >= 2) LBM_DMA_WAIT(2 * kLoads);
-      else if (behind == 1) LBM_DMA_WAIT(kLoads);
+      if (kStages > 3 && behind >= 2) LBM_DMA_WAIT(2 * kLoads);
+      else if (behind >= 1) LBM_DMA_WAIT(kLoads);
       else LBM_DMA_WAIT(0);
       __builtin_amdgcn_s_barrier();
       if (s + kStages < nk) load_step(s + kStages);
@@ -1410,7 +1415,7 @@ int lbm_linear_tiles(LinearArgs& p) {
   p.stats_shift = p.N % 128 == 0 && tiles >= 160 ? 7 : 6;
   return tn;
 }
-// 64 or 32 rows per tile of 64 columns in the place of 128 x tn tiles where they need fewer rounds of the CUs x
+// 32, 64 or 96 rows per tile of 64 columns in the place of 128 x tn tiles where they need fewer rounds of the CUs x
 // bytes per step (the fill is what bounds either), or 0; sets the row tiles.  With K summed in slices one workgroup
 // walks them all: up to K = 4,096 that is the faster way (M x N x K 31 x 1,024 x 4,096: 10.5 -> 10.4 us,
 // 1,004 rows 17.3 -> 15.6), from there on several workgroups are (512 x 768 x 6,144: 15.4 against 16.2; 81 x
@@ -1420,7 +1425,8 @@ int lbm_linear_rows_tiles(LinearArgs& p, int tn, int splits) {
   const int nt = p.N / 64;
   int best = 0;
   long long best_cost = ((long long)p.m_tiles * nt + 255) / 256 * (128 + 64);
-  for (int tm : {64, 32}) {
+  for (int tm : {64, 32, 96}) {
+    if (tm == 96 && splits > 1) continue;   // (K is sliced where 64 rows are one round)
     const long long cost = ((long long)((p.M + tm - 1) / tm) * nt + 255) / 256 * (tm + 64);
     if (cost < best_cost) best = tm, best_cost = cost;
   }
@@ -1593,7 +1599,8 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
     const dim3 grid_r((unsigned)(p.m_tiles * p.n_tiles)), block_r(lbm_rows_threads(tm));
 #define LBM_ROWS_LAUNCH(E, S, L)                                                                                                \
   {                                                                                                                             \
-    if (tm == 64) hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<E, 64, S, 0, false, L>), grid_r, block_r, 0, stream, p);       \
+    if (S == 1 && tm == 96) hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<E, 96, 1, 0, false, L>), grid_r, block_r, 0, stream, p); \
+    else if (tm == 64) hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<E, 64, S, 0, false, L>), grid_r, block_r, 0, stream, p);       \
     else hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<E, 32, S, 0, false, L>), grid_r, block_r, 0, stream, p);                \
   }
     if (epilogue == LBM_LINEAR_BIAS && lna) LBM_ROWS_LAUNCH(LBM_LINEAR_BIAS, 1, true)
@@ -1700,7 +1707,7 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
   }
 #define LBM_QKV_ROWS(R, NRM)                                                       \
   {                                                                                \
-    if (tm == 64) LBM_QKV_ROWS_T(64, R, NRM) else LBM_QKV_ROWS_T(32, R, NRM)       \
+    if (tm == 96) LBM_QKV_ROWS_T(96, R, NRM) else if (tm == 64) LBM_QKV_ROWS_T(64, R, NRM) else LBM_QKV_ROWS_T(32, R, NRM) \
   }
     if (rope == 0 && !norm) LBM_QKV_ROWS(0, false)
     else if (rope == 0) LBM_QKV_ROWS(0, true)

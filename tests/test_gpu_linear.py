@@ -605,3 +605,33 @@ def test_qkv_projection_with_the_producer_on_tiles_of_128_rows():
     for norm in (False, True):
         for rope in ("none", "interleaved", "half_split"):
             test_qkv_projection_with_the_producer_as_its_epilogue(1950, 16, 256, norm, rope)
+
+
+@pytest.mark.parametrize("M,Nn,epilogue", [(257, 4096, "bias"), (288, 4096, "gelu"), (289, 4096, "bias"), (384, 4096, "gelu"), (321, 3072, "bias"),
+                                           (480, 3072, "bias"), (1025, 1024, "residual"), (1200, 1024, "residual"), (1536, 1024, "residual")])
+def test_tiles_of_96_rows_change_no_bit(M, Nn, epilogue):
+    """The ends of the ranges that run on tiles of 96 rows, one to eight steps of K (fewer than the ring has stages, and odd
+    ones): every element is the same sum in the same order on the 128-row tiles of a launch of more rows.  Rows past M stay."""
+    N = _native()
+    dev = torch.device("cuda:0")
+    epi = {"bias": N.LINEAR_BIAS, "gelu": N.LINEAR_BIAS_GELU, "residual": N.LINEAR_BIAS_RESIDUAL}[epilogue]
+    more = M + (900 if Nn == 1024 else 350)
+    for K in (128, 256, 384, 1024):
+        a, w, bias, g = _inputs(more, K, Nn, seed=K + M)
+        res = torch.randn(more, Nn, generator=g).to(torch.bfloat16).to(dev)
+        a, w, bias = a.to(dev), w.to(dev), bias.float().to(dev)
+        outs = []
+        for rows in (M, more):
+            out = torch.full((rows + 1, Nn), 7.0, dtype=torch.bfloat16, device=dev)
+            N.check(N.lib.lbm_linear(ptr(a), ptr(w), ptr(bias), None, ptr(res) if epilogue == "residual" else None, ptr(out), rows, Nn, K, epi, None))
+            torch.cuda.synchronize()
+            assert (out[rows] == 7.0).all()
+            outs.append(out)
+        assert torch.equal(outs[0][:M], outs[1][:M]), K
+
+
+@pytest.mark.parametrize("M", [321, 385, 480])
+def test_tiles_of_96_rows_with_the_producer_as_the_epilogue(M):
+    for norm in (False, True):
+        for rope in ("none", "interleaved", "half_split"):
+            test_qkv_projection_with_the_producer_as_its_epilogue(M, 16, 256, norm, rope)
