@@ -5,10 +5,12 @@ from __future__ import annotations
 
 import contextlib
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 import struct
 
-from .build import LIB_PATH
+from .build import HOST_PATH, LIB_PATH
 
 OK, ERR_INVALID, ERR_UNSUPPORTED, ERR_WORKSPACE, ERR_HIP = 0, 1, 2, 3, 4
 DTYPE_BF16, DTYPE_F32 = 0, 1
@@ -163,6 +165,20 @@ def _load():
 
 
 lib = _load()
+
+
+def _load_host():
+    """The extension module of the attention calls' host side (``csrc/host_calls.cpp``)."""
+    if not os.path.exists(HOST_PATH):
+        raise RuntimeError(f"{HOST_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'`")
+    import torch  # noqa: F401  (its libraries first)
+    loader = importlib.machinery.ExtensionFileLoader("lbm_host", HOST_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("lbm_host", loader))
+    loader.exec_module(module)
+    return module
+
+
+host = _load_host()
 
 
 class LbmError(RuntimeError):

@@ -200,6 +200,7 @@ class HipPagedKVCacheManager:
         self._launches = [((), None, 0, 0, 0, b"", b"") for _ in range(self._n_sets)]
         self._sm_scale = 1.0 / math.sqrt(head_dim)
         self._frame_shape = torch.Size((num_streams * tokens_per_frame, num_heads, head_dim))
+        self._fit = (*self._frame_shape, self.dtype == torch.float32)     # what rows_fit compares a frame's rows with
         # a step's operations, with the fields that never change filled in
         self._step_ops = self._ops([{} for _ in range(num_streams)])
         self.reset()
@@ -512,7 +513,8 @@ class HipPagedKVCacheManager:
         the others attend to the cache plus their own K/V and leave it untouched.  On the
         leading block all table work (allocate, evict, visible rows) is one launch."""
         shape, dtype = self._frame_shape, self.dtype
-        if not (k.dtype == dtype == v.dtype and k.shape == shape == v.shape and k.is_contiguous() and v.is_contiguous()):
+        fit = N.host.rows_fit(q, k, v, *self._fit)
+        if not fit and not (k.dtype == dtype == v.dtype and k.shape == shape == v.shape and k.is_contiguous() and v.is_contiguous()):
             k, v = self._check_frame("k", k), self._check_frame("v", v)
             if v.dtype != k.dtype:
                 v = v.to(k.dtype)
@@ -523,12 +525,12 @@ class HipPagedKVCacheManager:
             # them, in one call
             self.frame_count[block_idx] += 1
             self._n_appends[block_idx] += 1
-            return self._attend_planned(block_idx, q, k, v, append_rows=self._append_rows_ptr(ts))
+            return self._attend_planned(block_idx, q, k, v, append_rows=self._append_rows_ptr(ts), fit=fit)
         if stores:
             self._scatter(block_idx, self._append_rows[ts], k, v)
             self.frame_count[block_idx] += 1
             self._n_appends[block_idx] += 1
-        return self._attend_planned(block_idx, q, k if reads_own else None, v if reads_own else None)
+        return self._attend_planned(block_idx, q, k if reads_own else None, v if reads_own else None, fit=fit and reads_own)
 
     def step_qkv(self, block_idx: int, qkv: Optional[Tensor], q_norm=None, k_norm=None, rope_cs: Optional[Tensor] = None,
                  norm_eps: float = 1e-5, keyframe: Optional[Sequence[bool]] = None,
@@ -713,8 +715,8 @@ class HipPagedKVCacheManager:
         return ts, stores, True in tail
 
     def _attend_planned(self, block_idx: int, q: Tensor, self_k: Optional[Tensor], self_v: Optional[Tensor],
-                        q_prescaled: bool = False, append_rows: Optional[int] = None) -> Tensor:
-        """``q_prescaled``: q already carries 1 / sqrt(D) and log2(e) (``step_qkv``'s producer, whose caller is
+                        q_prescaled: bool = False, append_rows: Optional[int] = None, fit: bool = False) -> Tensor:
+        """``fit``: q, self_k and self_v are the frame's rows as the kernels take them (``rows_fit``).  ``q_prescaled``: q already carries 1 / sqrt(D) and log2(e) (``step_qkv``'s producer, whose caller is
         a block of a model: the order of sums is fixed).
         ``append_rows``: the address of the rows ``self_k`` / ``self_v`` are also stored in, row t in
         pool row ``append_rows[t]``: pages of this frame, which its plan names by the caller's rows
@@ -723,6 +725,16 @@ class HipPagedKVCacheManager:
         if self._newest_self[ts] and append_rows is None:
             raise RuntimeError("this frame's row table names its newest frame by the caller's K/V rows (step() led "
                                "the frame): every block of the frame takes it through step()")
+        if fit:
+            _, _, streams, n, need, tail, tail_fixed = self._launch_plan(ts)
+            if n == self.num_streams:
+                out = N.host.attend(q, self_k, self_v, self.kv_caches[block_idx], self._kv_rows_ptr(ts),
+                                    self._live_counts_ptr(ts) if self.device_token_counts and append_rows is None else 0, append_rows or 0,
+                                    streams, self._workspace(need), 0.0 if q_prescaled else self._sm_scale,
+                                    tail_fixed if q_prescaled or self.fixed_order else tail)
+                if out.__class__ is int:
+                    N.check(out)
+                return out
         assert q.shape == self._frame_shape, f"q: expected {list(self._frame_shape)}, got {tuple(q.shape)}"
         qc = q if q.dtype == self.dtype else q.to(self.dtype)
         if not qc.is_contiguous():
