@@ -1557,7 +1557,7 @@ __global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32 a) {
 // nothing crosses lanes inside the loop but the D/4-lane sum of a dot product (DPP) and there is no
 // barrier in it; the groups meet through LDS once, at the end.
 //
-// Up to kDecOneTokens tokens one to four workgroups of eight wavefronts take a (stream, head, query row) from
+// Up to kDecOneTokens tokens one to four workgroups of eight or sixteen wavefronts take a (stream, head, query row) from
 // start to finish: one launch, which also stores the caller's new rows (lbm_attn_run_append).
 // Beyond that the KV axis is cut into chunks of 256 down to 64 tokens, one workgroup of four wavefronts
 // each, which leave partial results for lbm_attn_f32_decode_merge_kernel.  Where the chip has workgroups to spare a
@@ -1565,7 +1565,7 @@ __global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32 a) {
 namespace {
 constexpr int kDecQ = 8;         // query rows per stream this path takes
 constexpr int kDecBatch = 8;     // tokens a row group has in flight
-constexpr int kDecOneBatch = 11; // the most where one workgroup takes everything, 16 (head_dim 128) or 32 row groups
+constexpr int kDecOneBatch = 11; // the most where one workgroup takes everything, 16 or 32 (head_dim 128), 32 or 64 row groups
 constexpr int kDecChunk = 256;   // tokens per chunk, as long as that makes at most kDecMaxChunks
 constexpr int kDecFineChunk = 64, kDecFineWgs = 512, kDecFineChunks = 16;   // shorter chunks, within so many workgroups a launch and chunks a row
 constexpr int kDecMaxChunks = 64;
@@ -1700,13 +1700,17 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
 #pragma unroll
     for (int w = 1; w < NW; ++w) mx = fmaxf(mx, red_m[w]);
     const float ref = mx > -INFINITY ? mx : 0.f;
-    float o = 0.f, lt = 0.f;
+    // (sixteen wavefronts' in four sums of four: the longer chain's rounding would show)
+    constexpr int kSums = NW == 16 ? 4 : 1;
+    float os[kSums] = {}, ls[kSums] = {};
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       const float wgt = __builtin_amdgcn_exp2f(red_m[w] - ref);
-      lt += red_l[w] * wgt;
-      o += red_o[w][tid] * wgt;
+      ls[w % kSums] += red_l[w] * wgt;
+      os[w % kSums] += red_o[w][tid] * wgt;
     }
+    const float o = kSums == 1 ? os[0] : (os[0] + os[kSums / 2]) + (os[1 % kSums] + os[kSums - 1]);
+    const float lt = kSums == 1 ? ls[0] : (ls[0] + ls[kSums / 2]) + (ls[1 % kSums] + ls[kSums - 1]);
     if (ONE) {
       a.f.out[((size_t)(sp.q_begin + qi) * H + head) * D + vs * DV + tid] = lt > 0.f ? o / lt : 0.f;   // no token: zeros
     } else {
@@ -2228,7 +2232,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
       // second launch (500 tokens 9.2 and 10.7, 8.0 and 9.0) unless fewer chunks fit (four streams, 500 tokens 10.0 and
       // 11.9, 11.1 and 12.4).  With one query row per stream and nothing to append beyond those rows it carries the
       // append as well.
-      const int groups = kDecOneWaves * 256 / head_dim, trip = kDecOneBatch * groups, trips = (most + trip - 1) / trip;
+      const int few = kDecOneWaves * 256 / head_dim, trip = kDecOneBatch * few;   // row groups of eight wavefronts, their tokens in flight
       if (most <= kDecOneTokens && (fine < kDecFineChunks || most <= trip * 5 / 2)) {
         for (int i = 0; i < sch.n_streams; ++i) d.n_chunks[i] = 1;
         unsigned covered = 0;   // rows 0 .. n_streams - 1 of the append, each some stream's query row
@@ -2242,28 +2246,36 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
         // floats 2.75, 2.83), and not where a row to append may be one that another workgroup still has to read.
         const long long rows = (long long)num_heads * sch.n_streams * max_q;
         const int shares = (d.append_rows && !append_apart) || most <= 32 ? 1 : rows * 4 <= 256 ? 4 : rows * 2 <= 256 ? 2 : 1;
-        const dim3 grid(1, num_heads, sch.n_streams * max_q * shares), block(kDecOneWaves * 64);
+        // Sixteen wavefronts, each group with half as many tokens, where eight would make more than one trip (16 heads, K/V
+        // from HBM, rows of a page each, us with eight and with sixteen: head_dim 128, 150 tokens 5.2, 5.3; 200 6.2, 5.8; 300
+        // 7.2, 6.8; 440 9.4, 8.5; four streams of 300 8.5, 8.0, of 440 10.9, 10.0; head_dim 64, 300 tokens 5.1, 5.2; 400 6.0, 5.7).
+        const bool many = most > trip;
+        const int trips = many ? (most + 2 * trip - 1) / (2 * trip) : 1, groups = many ? 2 * few : few;
+        const dim3 grid(1, num_heads, sch.n_streams * max_q * shares), block((many ? 2 : 1) * kDecOneWaves * 64);
         // As few trips as batches of eleven need, and batches no longer than so many trips need: a step loads its
         // batch whether the tokens are there or not, 0.13 us for 16 rows of 128 floats at a CU's 64 bytes per cycle.
-        // us a launch, 16 heads, batches of eleven and these: head_dim 128, 16 tokens 4.3, 2.8; 64 4.3, 3.1; 100 4.3, 4.0;
+        // us a launch, 16 heads, eight wavefronts, batches of eleven and these: head_dim 128, 16 tokens 4.3, 2.8; 64 4.3, 3.1; 100 4.3, 4.0;
         // 200 6.2, 5.7; head_dim 64, 100 tokens 4.2, 3.1; 400 6.2, 5.5.  (Ten: no better than eleven.)
-        const int batch = trips > 0 ? (most + trips * groups - 1) / (trips * groups) : 1;
-#define LBM_DECODE_ONE_VS(NB, VS)                                                                                                              \
+        const int batch = (most + trips * groups - 1) / (trips * groups);
+#define LBM_DECODE_ONE_VS(NW, NB, VS)                                                                                                          \
   {                                                                                                                                          \
-    if (head_dim == 64) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<64, kDecOneWaves, NB, true, VS>), grid, block, 0, stream, d);           \
-    else hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<128, kDecOneWaves, NB, true, VS>), grid, block, 0, stream, d);                         \
+    if (head_dim == 64) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<64, NW, NB, true, VS>), grid, block, 0, stream, d);                     \
+    else hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<128, NW, NB, true, VS>), grid, block, 0, stream, d);                                   \
   }
-#define LBM_DECODE_ONE(NB)                                                                                                                    \
+#define LBM_DECODE_ONE(NW, NB)                                                                                                                \
   {                                                                                                                                          \
-    if (shares == 4) LBM_DECODE_ONE_VS(NB, 4)                                                                                                 \
-    else if (shares == 2) LBM_DECODE_ONE_VS(NB, 2)                                                                                             \
-    else LBM_DECODE_ONE_VS(NB, 1)                                                                                                             \
+    if (shares == 4) LBM_DECODE_ONE_VS(NW, NB, 4)                                                                                             \
+    else if (shares == 2) LBM_DECODE_ONE_VS(NW, NB, 2)                                                                                         \
+    else LBM_DECODE_ONE_VS(NW, NB, 1)                                                                                                         \
   }
-        if (batch <= 2) LBM_DECODE_ONE(2)
-        else if (batch <= 4) LBM_DECODE_ONE(4)
-        else if (batch <= 6) LBM_DECODE_ONE(6)
-        else if (batch <= 8) LBM_DECODE_ONE(8)
-        else LBM_DECODE_ONE(kDecOneBatch)
+        if (many && batch <= 6) LBM_DECODE_ONE(2 * kDecOneWaves, 6)        // (more than half a trip of sixteen)
+        else if (many && batch <= 8) LBM_DECODE_ONE(2 * kDecOneWaves, 8)
+        else if (many) LBM_DECODE_ONE(2 * kDecOneWaves, kDecOneBatch)
+        else if (batch <= 2) LBM_DECODE_ONE(kDecOneWaves, 2)
+        else if (batch <= 4) LBM_DECODE_ONE(kDecOneWaves, 4)
+        else if (batch <= 6) LBM_DECODE_ONE(kDecOneWaves, 6)
+        else if (batch <= 8) LBM_DECODE_ONE(kDecOneWaves, 8)
+        else LBM_DECODE_ONE(kDecOneWaves, kDecOneBatch)
 #undef LBM_DECODE_ONE
 #undef LBM_DECODE_ONE_VS
         return lbm_check_launch("lbm_attn_f32_decode_kernel<one chunk>");
