@@ -141,21 +141,42 @@ __shared__ __attribute__((aligned(16))) unsigned short lds_q[kWaves][kQPerWave *
 // (it takes the 130 bytes it needs, not the whole argument block with its sixteen stream plans:
 // what is passed by value sizes the kernel's scratch frame)
 __device__ __noinline__ void lbm_attn_split_safe(AttnCore a, LbmAttnStreamPlan sp);
+__device__ __noinline__ void lbm_attn_pair_safe(AttnCore a, LbmAttnStreamPlan sp);
+
+// LDS of the same with both splits of 256 query rows in one workgroup (PAIR below): a ring per split, and patches that
+// the two wavefronts of the same 64 rows share.
+__shared__ __attribute__((aligned(1024))) unsigned short lds_pair_k[2][kStages][kKvTile * kRingRow];
+__shared__ __attribute__((aligned(1024))) unsigned short lds_pair_v[2][kStages][kKvTile * kRingRow];
+__shared__ __attribute__((aligned(16))) unsigned short lds_pair_q[kWaves / 2][kQPerWave * kKStride];
+__shared__ float lds_pair_lse[kWaves][32];   // log-sum-exps of the 32 rows that the other wavefront merges
 
 // One workgroup's share of the split-KV attention: 512 query rows of one head over one run of
 // KV tiles, start to finish.  SAFE = false is the common path (no softmax reference, range
 // check at the end); when the check fails it writes nothing, hands the workgroup to the
 // repeat pass and ends the program there, so that nothing of the common path is live across
 // the call.  SAFE = true is the repeat with a reference that follows the row maxima.
-template <bool SAFE>
+//
+// PAIR: launches whose streams attend to their own rows in order in two splits each (several streams' frame and encoder
+// blocks).  Wavefronts 0-3 take 256 query rows over the first split, 4-7 the same rows over the second, each group from a
+// ring of its own, and the two meet through LDS where the partial results of other launches go through memory to a second
+// kernel: rounded to bf16 and weighted as there, the same bits.  As many workgroups as 512 rows x two splits make, or
+// fewer; a group stages a tile by itself, twice the bytes into LDS per product, of which there were few (DMA of 32 KB per
+// 2,300 cycles).
+template <bool SAFE, bool PAIR>
 __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnStreamPlan& sp) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n32 = lane & 31, g = lane >> 5;
+  constexpr int kRowWaves = PAIR ? kWaves / 2 : kWaves;      // wavefronts with query rows of their own
+  constexpr int kPieces = kWaves / kRowWaves;                // 16-byte pieces of a tile's K (and V) rows per thread
+  const int group = PAIR ? wave / kRowWaves : 0, rw = PAIR ? wave % kRowWaves : wave;
+  unsigned short (*const ring_k)[kKvTile * kRingRow] = PAIR ? lds_pair_k[group] : lds_k;
+  unsigned short (*const ring_v)[kKvTile * kRingRow] = PAIR ? lds_pair_v[group] : lds_v;
+  unsigned short* const patch = PAIR ? lds_pair_q[rw] : lds_q[wave];
 
   // ---- which piece of this stream's work is this workgroup
   const int H = a.num_heads;
   const int local = (int)blockIdx.x - sp.wg_begin;
-  const int n_hs = H * sp.n_splits;
+  const int n_hs = PAIR ? H : H * sp.n_splits;
   int qt, hs;
   if ((n_hs & 7) == 0) {
     // Workgroups are dealt to the 8 XCDs round-robin: keep the query tiles that share one
@@ -168,11 +189,11 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
     hs = local / sp.n_qtiles;
   }
   if (local >= sp.n_qtiles * n_hs) return;  // padding between streams
-  const int head = hs % H, split = hs / H;
+  const int head = PAIR ? hs : hs % H, split = PAIR ? group : hs / H;
   // With device-side token counts the split count stays the host's choice (it fixes the grid
   // and the workspace layout) and the tiles are dealt to the splits from the live count.
-  const int kv_tokens = a.live_kv_tokens ? a.live_kv_tokens[sp.live_at] : sp.kv_tokens;
-  if (kv_tokens <= 0 && sp.n_splits == 1) {
+  const int kv_tokens = !PAIR && a.live_kv_tokens ? a.live_kv_tokens[sp.live_at] : sp.kv_tokens;
+  if (!PAIR && kv_tokens <= 0 && sp.n_splits == 1) {
     // nothing visible: the reference returns zeros (lingbot_map/layers/flashinfer_cache.py:368-370)
     for (int k = 0; k < kQPerWave / 8; ++k) {
       const int r = qt * kQTile + wave * kQPerWave + k * 8 + (lane >> 3);
@@ -182,10 +203,11 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
     return;
   }
   const int n_tiles = (max(kv_tokens, 0) + kKvTile - 1) / kKvTile;
-  const int tiles_per_split = a.live_kv_tokens ? max((n_tiles + sp.n_splits - 1) / sp.n_splits, 1) : sp.tiles_per_split;
+  const int tiles_per_split = !PAIR && a.live_kv_tokens ? max((n_tiles + sp.n_splits - 1) / sp.n_splits, 1) : sp.tiles_per_split;
   const int t0 = split * tiles_per_split;
   const int t1 = min(t0 + tiles_per_split, n_tiles);  // an empty split (t1 <= t0) contributes weight 0
   const int n = t1 - t0;
+  const int n_most = PAIR ? max(min(tiles_per_split, n_tiles), 0) : n;   // tiles of the longer of the workgroup's splits, the first
   const unsigned row_bytes = (unsigned)H * 128u;
 
   // ---- tile staging: each thread moves one 16-byte piece of a K row and of a V row per tile,
@@ -201,7 +223,7 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
   // barrier that publishes a tile.  M0 is declared clobbered, so the compiler keeps nothing of
   // its own in it across a load.
   // Rows past the last token re-read the last token (finite data; the softmax masks them).
-  const int ld_r = tid >> 3;
+  const int ld_r = (PAIR ? tid % (kRowWaves * 64) : tid) >> 3;
   const int ld_ck = ((lane & 7) ^ ((ld_r >> 1) & 7)) * 8, ld_cv = ((lane & 7) ^ (((ld_r >> 1) & 1) * 4)) * 8;
   const char* pool_k = (const char*)(a.pool + (size_t)head * 64 + ld_ck);
   const char* pool_v = (const char*)(a.pool + (size_t)head * 64 + ld_cv) + (size_t)a.page_size * row_bytes;
@@ -211,17 +233,24 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
   const int last_token = max(kv_tokens - 1, 0);
   // Tiles past the end of this split re-read its last tile: the data lands in ring stages
   // nobody reads any more, and the code stays free of branches.
-  auto row_entry = [&](int t) -> int { return rows[min(max(min(t, t1 - 1), 0) * kKvTile + ld_r, last_token)]; };
+  // PAIR: token t is row kv_row_begin + t of the caller's K/V, no table; the "entry" of a tile is its first token.
+  auto row_entry = [&](int t) -> int {
+    const int first = max(min(t, t1 - 1), 0) * kKvTile;
+    return PAIR ? first : rows[min(first + ld_r, last_token)];
+  };
   auto dma = [&](int e, const char* pool_base, const char* own_base, const unsigned short* lds_tile) {
-    // negative entries name rows of the caller's own K/V (read-only tail of a non-keyframe)
-    const char* base = e < 0 ? own_base : pool_base;
-    const unsigned r = (unsigned)(e ^ (e >> 31));
-    const char* src = base + (unsigned long long)r * row_bytes;
-    const unsigned m0v = (unsigned)(size_t)(__attribute__((address_space(3))) const void*)(lds_tile + wave * (8 * kRingRow));
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
-                 :
-                 : "v"(src), "s"(__builtin_amdgcn_readfirstlane(m0v))
-                 : "memory", "m0");
+#pragma unroll
+    for (int k = 0; k < kPieces; ++k) {
+      // negative entries name rows of the caller's own K/V (read-only tail of a non-keyframe)
+      const char* base = PAIR || e < 0 ? own_base : pool_base;
+      const unsigned r = PAIR ? (unsigned)(sp.kv_row_begin + min(e + ld_r + k * (kKvTile / kPieces), last_token)) : (unsigned)(e ^ (e >> 31));
+      const char* src = base + (unsigned long long)r * row_bytes;
+      const unsigned m0v = (unsigned)(size_t)(__attribute__((address_space(3))) const void*)(lds_tile + (k * kRowWaves + rw) * (8 * kRingRow));
+      asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+                   :
+                   : "v"(src), "s"(__builtin_amdgcn_readfirstlane(m0v))
+                   : "memory", "m0");
+    }
   };
 #define LBM_DMA_LANDED() __builtin_amdgcn_s_waitcnt(0x0F70)   /* vmcnt(0); expcnt and lgkmcnt untouched */
 
@@ -230,9 +259,9 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
   // Q rows below travel at the same time.
   const int e_t0 = row_entry(t0), e_t1 = row_entry(t0 + 1);
   int ek = row_entry(t0 + 2), ev = e_t1;   // entries of the loads of the first iteration
-  dma(e_t0, pool_k, own_k, lds_k[0]);
-  dma(e_t1, pool_k, own_k, lds_k[1]);
-  dma(e_t0, pool_v, own_v, lds_v[0]);
+  dma(e_t0, pool_k, own_k, ring_k[0]);
+  dma(e_t1, pool_k, own_k, ring_k[1]);
+  dma(e_t0, pool_v, own_v, ring_v[0]);
 
   // ---- Q fragments (B operand of S^T = K Q^T): lane holds q row n32, d = ks*16 + g*8 .. +8.
   // Each wavefront reads its 64 query rows as whole 128-byte rows (eight lanes per row), parks
@@ -242,22 +271,22 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
   // when the producer already multiplied q by them before its own rounding and the caller
   // passed sm_scale = 0), so the MFMA result is already the exponent of 2.
   bf16x8 qf[2][4];
-  const int q_row0 = qt * kQTile + wave * kQPerWave;
+  const int q_row0 = (qt * kRowWaves + rw) * kQPerWave;
   {
-    unsigned short* patch = lds_q[wave];
-    u32x4 raw[kQPerWave / 8];
+    constexpr int kRaw = kQPerWave / 8 / kPieces;            // (PAIR: half of them, the other group's wavefront the rest)
+    u32x4 raw[kRaw];
 #pragma unroll
-    for (int k = 0; k < kQPerWave / 8; ++k) {
+    for (int k = 0; k < kRaw; ++k) {
       // rows past the stream's last query row re-read that row: their results are never stored,
       // and eight unconditional loads go out back to back (a load inside a conditional block
       // ends up with a wait for everything in flight behind it)
-      const int r = max(min(q_row0 + k * 8 + (lane >> 3), sp.q_rows - 1), 0);
+      const int r = max(min(q_row0 + (group * kRaw + k) * 8 + (lane >> 3), sp.q_rows - 1), 0);
       raw[k] = *(const u32x4*)(a.q + ((size_t)(sp.q_begin + r) * H + head) * 64 + (lane & 7) * 8);
     }
 #pragma unroll
-    for (int k = 0; k < kQPerWave / 8; ++k)
-      *(u32x4*)&patch[(k * 8 + (lane >> 3)) * kKStride + (lane & 7) * 8] = raw[k];
-    __syncthreads();   // (a wavefront only reads its own patch; the barrier orders its lanes' writes and reads)
+    for (int k = 0; k < kRaw; ++k)
+      *(u32x4*)&patch[((group * kRaw + k) * 8 + (lane >> 3)) * kKStride + (lane & 7) * 8] = raw[k];
+    __syncthreads();   // (a wavefront only reads its own patch, PAIR: the two that share it; the barrier orders writes and reads)
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
@@ -307,9 +336,9 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
     const int row = ks * 16 + 4 * g + ((lane & 15) >> 2);
     const int col = (db * 32 + ((lane >> 4) & 1) * 16 + (lane & 3) * 4) ^ (((lane >> 3) & 1) * 32);
     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (s16x4 __attribute__((address_space(3)))*)&lds_v[st][row * kRingRow + col]);
+        (s16x4 __attribute__((address_space(3)))*)&ring_v[st][row * kRingRow + col]);
     const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (s16x4 __attribute__((address_space(3)))*)&lds_v[st][(row + 8) * kRingRow + col]);
+        (s16x4 __attribute__((address_space(3)))*)&ring_v[st][(row + 8) * kRingRow + col]);
     s16x8 both;
     both[0] = lo[0]; both[1] = lo[1]; both[2] = lo[2]; both[3] = lo[3];
     both[4] = hi[0]; both[5] = hi[1]; both[6] = hi[2]; both[7] = hi[3];
@@ -337,7 +366,7 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const bf16x8 ka = __builtin_bit_cast(
-          bf16x8, *(const u32x4*)&lds_k[st][(h * 32 + n32) * kRingRow + ((ks * 2 + g) ^ ((n32 >> 1) & 7)) * 8]);
+          bf16x8, *(const u32x4*)&ring_k[st][(h * 32 + n32) * kRingRow + ((ks * 2 + g) ^ ((n32 >> 1) & 7)) * 8]);
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb)
         sd[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, qf[qb][ks], sd[qb], 0, 0, 0);
@@ -463,7 +492,7 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
     if ((j) == 1) va[1] = v_frag(st_pv, ks_pv, 1);                                               \
     if ((j) == 10 || (j) == 12 || (j) == 14 || (j) == 16)                                        \
       ka[((j) - 10) >> 1] = __builtin_bit_cast(                                                  \
-          bf16x8, *(const u32x4*)&lds_k[st_qk][((h_qk) * 32 + n32) * kRingRow + (((((j) - 10) >> 1) * 2 + g) ^ ((n32 >> 1) & 7)) * 8]); \
+          bf16x8, *(const u32x4*)&ring_k[st_qk][((h_qk) * 32 + n32) * kRingRow + (((((j) - 10) >> 1) * 2 + g) ^ ((n32 >> 1) & 7)) * 8]); \
     if ((j) == 17) vnext[0] = v_frag(st_vn, ks_vn, 0);                                           \
     if ((j) == 18) vnext[1] = v_frag(st_vn, ks_vn, 1);                                           \
     hook(j)                                                                                      \
@@ -523,7 +552,7 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
     if ((j) == 1) va[1] = v_frag(st_pv, ks_pv, 1);                                               \
     if ((j) == 8 || (j) == 10 || (j) == 12 || (j) == 14)                                         \
       ka[((j) - 8) >> 1] = __builtin_bit_cast(                                                   \
-          bf16x8, *(const u32x4*)&lds_k[st_qk][((h_qk) * 32 + n32) * kRingRow + (((((j) - 8) >> 1) * 2 + g) ^ ((n32 >> 1) & 7)) * 8]); \
+          bf16x8, *(const u32x4*)&ring_k[st_qk][((h_qk) * 32 + n32) * kRingRow + (((((j) - 8) >> 1) * 2 + g) ^ ((n32 >> 1) & 7)) * 8]); \
     if ((j) == 16) vnext[0] = v_frag(st_vn, ks_vn, 0);                                           \
     if ((j) == 17) vnext[1] = v_frag(st_vn, ks_vn, 1);                                           \
     hook(j)                                                                                      \
@@ -571,7 +600,9 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
 
     // ---- prologue: K(0), K(1), V(0) are on their way into the ring; the V stage the first PV
     // reads is zeroed
-    *(u32x4*)&lds_v[2][tid * 8] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int k = 0; k < kPieces; ++k)
+      *(u32x4*)&ring_v[2][(k * kRowWaves * 64 + (PAIR ? tid % (kRowWaves * 64) : tid)) * 8] = u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
@@ -605,8 +636,8 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
     // entry fetched for K now serves V in the next iteration.
 #define LBM_NO_HOOK(j)
 #define LBM_STAGING_HOOK(j)                                                          \
-    if ((j) == 1) dma(ek, pool_k, own_k, lds_k[st_k2]);                              \
-    if ((j) == 2) dma(ev, pool_v, own_v, lds_v[st_v1]);                              \
+    if ((j) == 1) dma(ek, pool_k, own_k, ring_k[st_k2]);                              \
+    if ((j) == 2) dma(ev, pool_v, own_v, ring_v[st_v1]);                              \
     if ((j) == 3) {                                                                  \
       ev = ek;                                                                       \
       ek = row_entry(t + 3);                                                         \
@@ -647,7 +678,7 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
     // wavefront it shares the SIMD with.
     if (q_row0 >= sp.q_rows) {
       for (; i < n; ++i)
-        LBM_TILE_ITERATION(, dma(ek, pool_k, own_k, lds_k[st_k2]); dma(ev, pool_v, own_v, lds_v[st_v1]); ev = ek; ek = row_entry(t + 3);, )
+        LBM_TILE_ITERATION(, dma(ek, pool_k, own_k, ring_k[st_k2]); dma(ev, pool_v, own_v, ring_v[st_v1]); ev = ek; ek = row_entry(t + 3);, )
     }
     // half 0 of tile i: softmax(sA) -> pA | PV(tile i-1, half 1) with pB | QK(tile i, half 1) -> sB
     // half 1 of tile i: softmax(sB) -> pB | PV(tile i, half 0) with pA | QK(tile i+1, half 0) -> sA
@@ -682,6 +713,7 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
 #undef LBM_TILE_ITERATION
 #undef LBM_STAGING_HOOK
 #undef LBM_NO_HOOK
+    for (; PAIR && i < n_most; ++i) __syncthreads();   // (the other group's last tiles)
     // PV and row sums of the last half: pB with half 1 of V(n-1), first k-step already in vnext
     {
       pv_step(vnext, pB, 0);
@@ -716,7 +748,8 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
       }
     }
     if (!safe && __builtin_amdgcn_readfirstlane(__syncthreads_or(bad))) {
-      lbm_attn_split_safe(a, sp);
+      if (PAIR) lbm_attn_pair_safe(a, sp);
+      else lbm_attn_split_safe(a, sp);
       __builtin_amdgcn_endpgm();
     }
   }
@@ -731,10 +764,77 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
   // rows); written straight out that is 32 scattered 8-byte stores per instruction.  Each
   // wavefront instead transposes its rows through its Q patch (idle since the prologue) and
   // stores whole 128-byte rows, eight lanes per row.
-  unsigned short* stage = lds_q[wave];
-  const bool direct = sp.n_splits == 1;
+  unsigned short* const stage = patch;
+  const bool direct = PAIR || sp.n_splits == 1;
   unsigned short* dst = direct ? a.out : a.part_o;
   const size_t dst_row0 = direct ? (size_t)sp.q_begin : (size_t)sp.part_begin + (size_t)split * sp.q_rows;
+  if (PAIR) {
+    // A wavefront leaves one block of 32 rows of its partial result to the other group's wavefront of the same rows and
+    // merges the other block: group 0 the first, group 1 the second.  Both partial results as lbm_attn_combine_bf16_kernel
+    // finds them - normalised, bf16 - and its sums, in the order of the splits.  A lane reads what the same lane of the
+    // other wavefront wrote.
+    float lse[2], inv[2];
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      const float sum_lo = lacc[qb][0], sum_hi = lacc[qb][1];
+      const float l_lo = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (lane & 15), __builtin_bit_cast(int, sum_lo)));
+      const float l_hi = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * (lane & 15), __builtin_bit_cast(int, sum_hi)));
+      const float l_tot = (n32 & 16) ? l_hi : l_lo;
+      inv[qb] = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+      lse[qb] = m_run[qb] + __builtin_amdgcn_logf(l_tot);
+    }
+    auto partial = [&](int qb, int db, int c4) -> bf16x4 {
+      f32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = o[qb][db][c4 * 4 + e] * inv[qb];
+      return __builtin_convertvector(w, bf16x4);
+    };
+    auto at = [&](int qb, int db, int c4) { return (bf16x4*)&stage[(qb * 32 + n32) * kKStride + db * 32 + c4 * 8 + g * 4]; };
+    auto leave = [&](auto block) {
+      constexpr int others = decltype(block)::value;
+#pragma unroll
+      for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int c4 = 0; c4 < 4; ++c4) *at(others, db, c4) = partial(others, db, c4);
+      if (g == 0) lds_pair_lse[wave][n32] = lse[others];
+    };
+    auto merge = [&](auto block) {
+      constexpr int mine = decltype(block)::value;   // (and the split that this wavefront summed)
+      const float theirs = lds_pair_lse[wave ^ kRowWaves][n32];
+      const float first = mine == 0 ? lse[mine] : theirs, second = mine == 0 ? theirs : lse[mine];
+      float mx = fmaxf(first, second);
+      if (mx == -INFINITY) mx = 0.f;
+      const float w0 = __builtin_amdgcn_exp2f(first - mx), w1 = __builtin_amdgcn_exp2f(second - mx), wsum = w0 + w1;
+      const float norm = wsum > 0.f ? 1.0f / wsum : 0.f;
+#pragma unroll
+      for (int db = 0; db < 2; ++db)
+#pragma unroll
+        for (int c4 = 0; c4 < 4; ++c4) {
+          const f32x4 x = __builtin_convertvector(partial(mine, db, c4), f32x4), y = __builtin_convertvector(*at(mine, db, c4), f32x4);
+          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            acc[e] += w0 * (mine == 0 ? x[e] : y[e]);
+            acc[e] += w1 * (mine == 0 ? y[e] : x[e]);
+            acc[e] *= norm;
+          }
+          *at(mine, db, c4) = __builtin_convertvector(acc, bf16x4);
+        }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int row = mine * 32 + k * 8 + (lane >> 3);
+        const u32x4 v = *(const u32x4*)&stage[row * kKStride + (lane & 7) * 8];
+        const int r = q_row0 + row;
+        if (r < sp.q_rows) lbm_store_through(dst + ((dst_row0 + r) * H + head) * 64 + (lane & 7) * 8, v);
+      }
+    };
+    if (group == 0) leave(std::integral_constant<int, 1>{});
+    else leave(std::integral_constant<int, 0>{});
+    __syncthreads();
+    if (group == 0) merge(std::integral_constant<int, 0>{});
+    else merge(std::integral_constant<int, 1>{});
+    return;
+  }
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
     // the row sum of query n32 of this block sits in lane n32 % 16, element n32 / 16
@@ -766,7 +866,8 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
   }
 }
 
-__device__ __noinline__ void lbm_attn_split_safe(AttnCore a, LbmAttnStreamPlan sp) { lbm_attn_split<true>(a, sp); }
+__device__ __noinline__ void lbm_attn_split_safe(AttnCore a, LbmAttnStreamPlan sp) { lbm_attn_split<true, false>(a, sp); }
+__device__ __noinline__ void lbm_attn_pair_safe(AttnCore a, LbmAttnStreamPlan sp) { lbm_attn_split<true, true>(a, sp); }
 
 }  // namespace
 
@@ -780,7 +881,16 @@ __global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_kernel(AttnArgs
   for (int i = 1; i < a.sch.n_streams; ++i)
     if ((int)blockIdx.x >= a.sch.s[i].wg_begin) b = i;
   const LbmAttnStreamPlan sp = a.sch.s[b];
-  lbm_attn_split<false>(a, sp);
+  lbm_attn_split<false, false>(a, sp);
+}
+
+// (its sch: n_qtiles and workgroups in tiles of 256 query rows, see the launch)
+__global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_pair_kernel(AttnArgs a) {
+  int b = 0;
+  for (int i = 1; i < a.sch.n_streams; ++i)
+    if ((int)blockIdx.x >= a.sch.s[i].wg_begin) b = i;
+  const LbmAttnStreamPlan sp = a.sch.s[b];
+  lbm_attn_split<false, true>(a, sp);
 }
 
 // ---------------------------------------------------------------------------- bf16, short KV
@@ -2344,6 +2454,25 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
     else if (turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, true>), grid, block, 0, stream, a);
     else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, false>), grid, block, 0, stream, a);
     return lbm_check_launch("lbm_attn_bf16_d64_small_kernel");
+  }
+  // Own rows in order, two splits per stream: both in one workgroup, no launch to merge (lbm_attn_split's PAIR).  us, two
+  // kernels and this one: 16 heads, four streams of 833 rows 28.7, 18.8, of 1,004 32.0, 22.3, of 3,000 154, 140, of 5,000
+  // 383, 361; 2 x 2,000 43.9, 34.9; 1 x 4,096 68.8, 61.0; four streams of 513 rows over 4,609 60.4, 56.1.  Up to 256 rows,
+  // which leave it half as many workgroups and those with half a load each, the two kernels stay: eight streams of 40 rows
+  // over 4,097 45.8, 54.6; 12 heads, 255 rows over 4,223 44.5, 51.9.
+  bool pair = own_rows && !live_kv_tokens && append_tokens <= 0;
+  for (int i = 0; i < sch.n_streams; ++i) pair = pair && sch.s[i].n_splits == 2 && 2 * sch.s[i].q_rows > kQTile;
+  if (pair) {
+    int wg = 0;
+    for (int i = 0; i < sch.n_streams; ++i) {
+      LbmAttnStreamPlan& p = a.sch.s[i];
+      p.n_qtiles = (p.q_rows + kQTile / 2 - 1) / (kQTile / 2);
+      wg = (wg + 7) & ~7;   // (a stream's first workgroup on XCD 0, as in the schedule)
+      p.wg_begin = wg;
+      wg += p.n_qtiles * num_heads;
+    }
+    hipLaunchKernelGGL(lbm_attn_bf16_d64_pair_kernel, dim3((unsigned)wg), dim3(kThreads), 0, stream, a);
+    return lbm_check_launch("lbm_attn_bf16_d64_pair_kernel");
   }
   // The append by workgroups behind the attention's: they run where CUs are done early (the last split of a list has fewer
   // tiles), and the launch that merges does not wait for them.  us a block, both builds' kernels: 1,004 rows over 17,068
