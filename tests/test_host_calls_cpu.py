@@ -17,3 +17,15 @@ def test_attend_refuses_what_was_not_recognised():
     t = torch.zeros(8, 2, 64)
     with pytest.raises(TypeError):
         N.host.attend(t, t, t, t, 0, 0, 0, 0, t, 1.0, b"")
+
+
+def test_the_extension_module_has_no_thread_locals():
+    """A thread-local that nobody touches, in the library loaded last, slows down every other one of the process (glibc up
+    to 2.38): no PT_TLS (7) among the module's program headers (64-bit ELF: their offset, size and number at 32, 54 and 56)."""
+    import struct
+    from lingbot_map_amd.build import HOST_PATH
+    with open(HOST_PATH, "rb") as f:
+        elf = f.read()
+    assert elf[:5] == b"\x7fELF\x02"
+    at, (size, count) = struct.unpack_from("<Q", elf, 32)[0], struct.unpack_from("<HH", elf, 54)
+    assert count > 0 and all(struct.unpack_from("<I", elf, at + i * size)[0] != 7 for i in range(count))
