@@ -46,6 +46,7 @@ namespace {
 
 constexpr int kWaves = 8, kThreads = kWaves * 64;
 constexpr int kRows = 64;               // query rows per workgroup
+constexpr int kAppendPieces = 4;        // 16-byte pieces of K and of V per thread of a workgroup that appends
 constexpr int kTile = 32;               // KV tokens per tile
 constexpr int kTileBytes = kTile * 64 * 4;
 constexpr int kQPlane = kRows * 64;     // bf16 of a Q plane: unpadded rows, chunk c of row r at c ^ ((r >> 1) & 7)
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n32 = lane & 31, g = lane >> 5;
   if (APPEND && (int)blockIdx.x >= a.wg_begin[LBM_MAX_STREAMS]) {
-    lbm_append_pieces(a.self_k, a.self_v, const_cast<float*>(a.pool), a.append_rows, a.append_tokens, a.num_heads * 16, a.page_size,
+    lbm_append_pieces<kAppendPieces>(a.self_k, a.self_v, const_cast<float*>(a.pool), a.append_rows, a.append_tokens, a.num_heads * 16, a.page_size,
                       (int)blockIdx.x - a.wg_begin[LBM_MAX_STREAMS], kThreads);
     return;
   }
@@ -431,7 +432,7 @@ int lbm_launch_attn_f32_d64(AttnArgsF32& a, hipStream_t stream) {
   }
   a.wg_begin[LBM_MAX_STREAMS] = wg;
   if (wg == 0) return LBM_OK;
-  wg += (int)(((long long)a.append_tokens * a.num_heads * 16 + kThreads - 1) / kThreads);
+  wg += (int)(((long long)a.append_tokens * a.num_heads * 16 + kThreads * kAppendPieces - 1) / (kThreads * kAppendPieces));
   if (a.append_tokens > 0) hipLaunchKernelGGL(lbm_attn_f32_d64_kernel<true>, dim3(wg), dim3(kThreads), 0, stream, a);
   else hipLaunchKernelGGL(lbm_attn_f32_d64_kernel<false>, dim3(wg), dim3(kThreads), 0, stream, a);
   return lbm_check_launch("lbm_attn_f32_d64_kernel");
