@@ -317,7 +317,7 @@ int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k,
 /* An attention call as one record (ABI 11): lbm_attn_run, or lbm_attn_run_live with live_kv_tokens, or
  * lbm_attn_run_append with append_rows (not both), and what only a record's flags say:
  *   LBM_ATTN_OWN_ROWS      entry kv_row_begin + t of kv_rows is -1 - (kv_row_begin + t) for every token t of every
- *                          stream: launches that split no KV rely on it instead of reading the table
+ *                          stream: launches that split KV in at most two pieces rely on it instead of reading the table
  *   LBM_ATTN_APPEND_APART  kv_rows names no row of append_rows, as the plans of lbm_tables_step with
  *                          LBM_OP_PLAN_NEWEST_SELF do: the bf16 kernels and the fp32 kernel of head_dim 64 then carry
  *                          the append by workgroups of their own, and a row of the few-query kernel may go to several
@@ -331,7 +331,8 @@ int lbm_attn_run_append(const void* q, void* pool, void* out, const void* new_k,
  *                          the rounding of bf16, but 24 blocks one behind the other make the last bits of an attention
  *                          into 0.2 % of the last block's K and V.  Needs no more than lbm_attn_workspace_bytes; fp32
  *                          calls are the same either way
- * Same results with and without the first two flags. */
+ * Same results with and without the first two flags (bf16 own rows in two splits: up to bf16's rounding where scores leave
+ * the range that needs no softmax reference, about +-100 in log2 units). */
 #define LBM_ATTN_OWN_ROWS 1
 #define LBM_ATTN_APPEND_APART 2
 #define LBM_ATTN_FIXED_ORDER 4

@@ -162,7 +162,9 @@ __shared__ float lds_pair_lse[kWaves][32];   // log-sum-exps of the 32 rows that
 // kernel: rounded to bf16 and weighted as there, the same bits.  As many workgroups as 512 rows x two splits make, or
 // fewer; a group stages a tile by itself, twice the bytes into LDS per product, of which there were few (DMA of 32 KB per
 // 2,300 cycles).
-template <bool SAFE, bool PAIR>
+// OWN (and PAIR): token t of a stream is row kv_row_begin + t of the caller's K/V, addressed without the row table.  (The
+// repeat pass of a launch that is not PAIR reads the table, which says the same.)
+template <bool SAFE, bool PAIR, bool OWN = PAIR>
 __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnStreamPlan& sp) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n32 = lane & 31, g = lane >> 5;
@@ -192,7 +194,7 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
   const int head = PAIR ? hs : hs % H, split = PAIR ? group : hs / H;
   // With device-side token counts the split count stays the host's choice (it fixes the grid
   // and the workspace layout) and the tiles are dealt to the splits from the live count.
-  const int kv_tokens = !PAIR && a.live_kv_tokens ? a.live_kv_tokens[sp.live_at] : sp.kv_tokens;
+  const int kv_tokens = !OWN && a.live_kv_tokens ? a.live_kv_tokens[sp.live_at] : sp.kv_tokens;
   if (!PAIR && kv_tokens <= 0 && sp.n_splits == 1) {
     // nothing visible: the reference returns zeros (lingbot_map/layers/flashinfer_cache.py:368-370)
     for (int k = 0; k < kQPerWave / 8; ++k) {
@@ -203,7 +205,7 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
     return;
   }
   const int n_tiles = (max(kv_tokens, 0) + kKvTile - 1) / kKvTile;
-  const int tiles_per_split = !PAIR && a.live_kv_tokens ? max((n_tiles + sp.n_splits - 1) / sp.n_splits, 1) : sp.tiles_per_split;
+  const int tiles_per_split = !OWN && a.live_kv_tokens ? max((n_tiles + sp.n_splits - 1) / sp.n_splits, 1) : sp.tiles_per_split;
   const int t0 = split * tiles_per_split;
   const int t1 = min(t0 + tiles_per_split, n_tiles);  // an empty split (t1 <= t0) contributes weight 0
   const int n = t1 - t0;
@@ -233,17 +235,17 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
   const int last_token = max(kv_tokens - 1, 0);
   // Tiles past the end of this split re-read its last tile: the data lands in ring stages
   // nobody reads any more, and the code stays free of branches.
-  // PAIR: token t is row kv_row_begin + t of the caller's K/V, no table; the "entry" of a tile is its first token.
+  // OWN: the "entry" of a tile is its first token.
   auto row_entry = [&](int t) -> int {
     const int first = max(min(t, t1 - 1), 0) * kKvTile;
-    return PAIR ? first : rows[min(first + ld_r, last_token)];
+    return OWN ? first : rows[min(first + ld_r, last_token)];
   };
   auto dma = [&](int e, const char* pool_base, const char* own_base, const unsigned short* lds_tile) {
 #pragma unroll
     for (int k = 0; k < kPieces; ++k) {
       // negative entries name rows of the caller's own K/V (read-only tail of a non-keyframe)
-      const char* base = PAIR || e < 0 ? own_base : pool_base;
-      const unsigned r = PAIR ? (unsigned)(sp.kv_row_begin + min(e + ld_r + k * (kKvTile / kPieces), last_token)) : (unsigned)(e ^ (e >> 31));
+      const char* base = OWN || e < 0 ? own_base : pool_base;
+      const unsigned r = OWN ? (unsigned)(sp.kv_row_begin + min(e + ld_r + k * (kKvTile / kPieces), last_token)) : (unsigned)(e ^ (e >> 31));
       const char* src = base + (unsigned long long)r * row_bytes;
       const unsigned m0v = (unsigned)(size_t)(__attribute__((address_space(3))) const void*)(lds_tile + (k * kRowWaves + rw) * (8 * kRingRow));
       asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
@@ -882,6 +884,14 @@ __global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_kernel(AttnArgs
     if ((int)blockIdx.x >= a.sch.s[i].wg_begin) b = i;
   const LbmAttnStreamPlan sp = a.sch.s[b];
   lbm_attn_split<false, false>(a, sp);
+}
+
+__global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_own_kernel(AttnArgs a) {
+  int b = 0;
+  for (int i = 1; i < a.sch.n_streams; ++i)
+    if ((int)blockIdx.x >= a.sch.s[i].wg_begin) b = i;
+  const LbmAttnStreamPlan sp = a.sch.s[b];
+  lbm_attn_split<false, false, true>(a, sp);
 }
 
 // (its sch: n_qtiles and workgroups in tiles of 256 query rows, see the launch)
@@ -2473,6 +2483,14 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
     }
     hipLaunchKernelGGL(lbm_attn_bf16_d64_pair_kernel, dim3((unsigned)wg), dim3(kThreads), 0, stream, a);
     return lbm_check_launch("lbm_attn_bf16_d64_pair_kernel");
+  }
+  // The same in one split.  us, with the table and without, 16 heads: 6 streams of 600 rows 21.6, 20.7; 8 x 1,004
+  // 39.7, 38.7; 3 x 1,500 61.7, 58.3; 16 x 100 over 4,097 76.1, 71.6.
+  bool whole = own_rows && !live_kv_tokens && append_tokens <= 0;
+  for (int i = 0; i < sch.n_streams; ++i) whole = whole && sch.s[i].n_splits == 1;
+  if (whole) {
+    hipLaunchKernelGGL(lbm_attn_bf16_d64_own_kernel, dim3((unsigned)sch.total_wgs), dim3(kThreads), 0, stream, a);
+    return lbm_check_launch("lbm_attn_bf16_d64_own_kernel");
   }
   // The append by workgroups behind the attention's: they run where CUs are done early (the last split of a list has fewer
   // tiles), and the launch that merges does not wait for them.  us a block, both builds' kernels: 1,004 rows over 17,068
