@@ -18,6 +18,7 @@ LAYOUT_TWO_STREAM, LAYOUT_FRAME_PAGES = 0, 1
 ROPE_INTERLEAVED, ROPE_HALF_SPLIT = 0, 1
 LINEAR_BIAS, LINEAR_BIAS_GELU, LINEAR_BIAS_RESIDUAL = 0, 1, 2
 MAX_STREAMS = 16
+MAX_GROUPS = 32
 STATIC_SCRATCH_MIB = 64
 OP_RESET, OP_ROLLBACK, OP_APPEND, OP_EVICT, OP_PLAN, OP_PLAN_NEWEST_SELF = 1, 2, 4, 8, 16, 32
 TERR_NAMES = {1: "patch page pool exhausted", 2: "special page pool exhausted", 4: "window ring full",
@@ -26,7 +27,7 @@ HDR = {"frame_count": 0, "n_anchor": 1, "win_head": 2, "win_count": 3, "n_free_p
        "n_free_special": 5, "n_special_pages": 6, "special_tokens": 7, "n_memory": 8,
        "n_memory_pages": 9, "error": 10, "plan_kv_tokens": 11, "plan_n_pages": 12}
 HDR_WORDS = 16
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 
 # Scratch memory that the package keeps per device (the K-split workspace of the GEMM, the
@@ -102,7 +103,8 @@ class BlockCall(C.Structure):
 
 SYMBOLS = ("lbm_abi_version", "lbm_last_error", "lbm_tables_words", "lbm_tables_step",
            "lbm_rows_from_pages", "lbm_kv_append", "lbm_qkv_prepare", "lbm_residual_norm", "lbm_linear", "lbm_linear_norm", "lbm_linear_stats_tiles", "lbm_linear_workspace_bytes", "lbm_linear_prefetch_hint", "lbm_qkv_linear_prepare", "lbm_qkv_linear_prepare_norm", "lbm_attn_workspace_bytes", "lbm_attn_run", "lbm_attn_run_append", "lbm_attn_run_live", "lbm_attn_run_call",
-           "lbm_attn_run_static", "lbm_block_scratch_bytes", "lbm_block_run")
+           "lbm_attn_run_static", "lbm_block_scratch_bytes", "lbm_block_run",
+           "lbm_group_outputs", "lbm_stream_table", "lbm_normalise_images")
 
 
 def _load():
@@ -159,6 +161,12 @@ def _load():
     lib.lbm_block_scratch_bytes.argtypes = [i32, i32, i32]
     lib.lbm_block_run.restype = C.c_int
     lib.lbm_block_run.argtypes = [p(BlockWeights), p(BlockCall), vp]
+    lib.lbm_group_outputs.restype = C.c_int
+    lib.lbm_group_outputs.argtypes = [p(vp), p(vp), i32, C.c_int64, C.c_int64, vp]
+    lib.lbm_stream_table.restype = C.c_int
+    lib.lbm_stream_table.argtypes = [vp, vp, C.c_int64, vp, i32, i32, i32, vp]
+    lib.lbm_normalise_images.restype = C.c_int
+    lib.lbm_normalise_images.argtypes = [vp, vp, vp, vp, i32, C.c_int64, C.c_int64, vp]
     if lib.lbm_abi_version() != ABI_VERSION:
         raise RuntimeError(f"{LIB_PATH}: ABI version {lib.lbm_abi_version()}, binding expects {ABI_VERSION}")
     return lib

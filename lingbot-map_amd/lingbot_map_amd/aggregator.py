@@ -22,6 +22,7 @@ pre-processing; or any module that returns ``[B * S, patches, C]``).
 """
 from __future__ import annotations
 
+import ctypes as C
 from typing import List, Optional, Sequence, Tuple, Union
 
 import torch
@@ -30,8 +31,39 @@ from torch import Tensor, nn
 from .block import (HipPagedBlock, PositionGetter, RotaryPositionEmbedding2D, RotaryPositionEmbedding3D)
 from .manager import HipPagedKVCacheManager
 
+from . import _native as N
+
 _RESNET_MEAN = (0.485, 0.456, 0.406)
 _RESNET_STD = (0.229, 0.224, 0.225)
+
+
+def _plain(*tensors: Tensor) -> bool:
+    """Whether a kernel may take the place of torch operations on ``tensors``: contiguous GPU tensors of no subclass and
+    under no transform, and nobody who follows the operations (autograd in either direction, a trace)."""
+    return not (torch.is_grad_enabled() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0) and all(
+        type(t) in (Tensor, nn.Parameter) and t.is_cuda and t.is_contiguous()
+        and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
+
+
+def _group_outputs(pairs: List[Tuple[Tensor, Tensor]], stacked: bool = False) -> Union[List[Tensor], Tensor]:
+    """``torch.cat([f, g], dim=-1)`` of every pair, ``[B, S, P, C]`` each (base.py:600-604), in one launch for up to
+    ``N.MAX_GROUPS`` pairs; ``stacked``: as one tensor ``[pairs, B, S, P, 2C]``."""
+    parts = [t for pair in pairs for t in pair]
+    first = parts[0] if parts else None
+    if not (parts and _plain(*parts) and all(t.shape == first.shape and t.dtype == first.dtype and t.device == first.device
+                                             and t.data_ptr() % 16 == 0 for t in parts)
+            and 0 < first.numel() * first.element_size() < 1 << 34 and first.shape[-1] * first.element_size() % 16 == 0):
+        outs = [torch.cat(pair, dim=-1) for pair in pairs]
+        return torch.stack(outs) if stacked else outs
+    shape = (*first.shape[:-1], 2 * first.shape[-1])
+    whole = first.new_empty(len(pairs), *shape) if stacked else None
+    outs = list(whole.unbind(0)) if stacked else [first.new_empty(shape) for _ in pairs]
+    for i in range(0, len(pairs), N.MAX_GROUPS):
+        o, t = outs[i:i + N.MAX_GROUPS], parts[2 * i:2 * (i + N.MAX_GROUPS)]
+        N.check(N.lib.lbm_group_outputs((C.c_void_p * len(t))(*[x.data_ptr() for x in t]), (C.c_void_p * len(o))(*[x.data_ptr() for x in o]),
+                                        len(o), first.numel() // first.shape[-1], first.shape[-1] * first.element_size(),
+                                        N.stream_ptr(first.device)))
+    return whole if stacked else outs
 
 
 class PatchConv(nn.Module):
@@ -59,7 +91,7 @@ class PatchTrunk(nn.Module):
         self.norm = nn.LayerNorm(embed_dim)
 
     def forward(self, images: Tensor) -> Tensor:
-        x = self.conv(images)
+        x = self.conv(images).contiguous()      # (once: the first block and its norm1 both ask for it)
         normed = None
         for i, blk in enumerate(self.blocks):   # each block hands the next one its norm1 (or the final norm)
             nxt = self.blocks[i + 1].norm1 if i + 1 < len(self.blocks) else self.norm
@@ -239,14 +271,26 @@ class HipAggregatorStream(nn.Module):
             raise ValueError(f"Expected 3 input channels, got {c_in}")
         if B != self.num_streams:
             raise ValueError(f"images carry {B} streams, the aggregator was built for {self.num_streams}")
-        images = (images - self._resnet_mean.to(images.dtype)) / self._resnet_std.to(images.dtype)
-        patches = self.patch_embed(images.view(B * S, c_in, H, W))
+        patches = self.patch_embed(self._normalised(images).view(B * S, c_in, H, W))
         if isinstance(patches, dict):
             patches = patches["x_norm_patchtokens"]
         C = patches.shape[-1]
         special = self._prepare_special_tokens(B, S, C, num_frame_for_scale).to(patches.dtype)
         tokens = torch.cat([special, patches], dim=1)
         return tokens, B, S, tokens.shape[1], C
+
+    def _normalised(self, images: Tensor) -> Tensor:
+        """(images - mean) / std (base.py:345)."""
+        mean, std = self._resnet_mean.to(images.dtype), self._resnet_std.to(images.dtype)
+        H, W = images.shape[-2:]
+        if (images.dtype in (torch.bfloat16, torch.float32) and _plain(images, mean, std) and images.device == mean.device == std.device
+                and H * W % 4 == 0 and images.data_ptr() % 16 == 0 and 0 < images.numel() < 1 << 32):
+            out = torch.empty_like(images)
+            N.check(N.lib.lbm_normalise_images(
+                images.data_ptr(), mean.data_ptr(), std.data_ptr(), out.data_ptr(),
+                N.DTYPE_BF16 if images.dtype == torch.bfloat16 else N.DTYPE_F32, images.numel() // (3 * H * W), H * W, N.stream_ptr(images.device)))
+            return out
+        return (images - mean) / std
 
     def _get_positions(self, frames: int, H: int, W: int, device) -> Optional[Tensor]:
         """(y, x) of every token, ``[frames, P, 2]``: specials at (0, 0), patches on the grid
@@ -277,30 +321,51 @@ class HipAggregatorStream(nn.Module):
             return rope(ppf=frames, pph=H, ppw=W, patch_start_idx=self.num_special_tokens, device=device, f_start=f0, f_end=f0 + frames)
         assert 0 <= f0 and f0 + frames <= rope.max_seq_len, \
             f"frames [{f0}, {f0 + frames}) outside the {rope.max_seq_len} positions of the table"
-        version = lambda t: 0 if t.is_inference() else t._version
-        key = (frames, H, W, str(device), self.num_special_tokens, version(rope.inv_freq), version(rope.pair_axis))
-        hit = self.__dict__.get("_table_base")
-        if hit is None or hit[0] != key or hit[1] is not rope.inv_freq or hit[2] is not rope.pair_axis:
-            # the angles of a call that starts at frame 0, and what every frame later adds to them:
-            # one launch per call instead of writing down a frame's coordinates again
-            coords = rope.coordinates(frames, H, W, self.num_special_tokens, device)
-            later = torch.where(rope.pair_axis == 0, rope.inv_freq, torch.zeros_like(rope.inv_freq)).to(device)
-            angles = rope.angles(coords)
-            hit = self.__dict__["_table_base"] = (key, rope.inv_freq, rope.pair_axis, angles, later, torch.ones_like(angles))
-        _, _, _, angles, later, ones = hit
+        angles, later, ones = self._table_base(frames, H, W, device)
         return torch.polar(ones, torch.add(angles, later, alpha=f0))[None, None]
+
+    def _table_base(self, frames: int, rows: int, cols: int, device) -> Tuple[Tensor, Tensor, Tensor]:
+        """The angles of a call that starts at frame 0, what every frame later adds to them, and ones: kept, so that a call
+        does not write down a frame's coordinates again."""
+        rope = self.rope3d
+        version = lambda t: 0 if t.is_inference() else t._version
+        key = (frames, rows, cols, str(device), self.num_special_tokens, version(rope.inv_freq), version(rope.pair_axis))
+        hit = self.__dict__.get("_table_base_cache")
+        if hit is None or hit[0] != key or hit[1] is not rope.inv_freq or hit[2] is not rope.pair_axis:
+            coords = rope.coordinates(frames, rows, cols, self.num_special_tokens, device)
+            later = torch.where(rope.pair_axis == 0, rope.inv_freq, torch.zeros_like(rope.inv_freq)).to(device, torch.float64)   # (a bf16 model's are bf16)
+            angles = rope.angles(coords).contiguous()     # (its indexing leaves the pairs outermost)
+            hit = self.__dict__["_table_base_cache"] = (key, rope.inv_freq, rope.pair_axis, angles, later, torch.ones_like(angles))
+        return hit[3:]
+
+    def _stream_table64(self, frames: int, H: int, W: int, device, streams: int) -> Tensor:
+        """``stream_table`` as the blocks read it: complex64, one copy per stream, ``[streams, 1, frames * P, D / 2]``."""
+        rope, f0 = self.rope3d, self.total_frames_processed
+        if (type(rope) is RotaryPositionEmbedding3D and type(self).stream_table is HipAggregatorStream.stream_table
+                and torch.device(device).type == "cuda" and 0 <= f0 and f0 + frames <= rope.max_seq_len):
+            angles, later, _ = self._table_base(frames, H // self.patch_size, W // self.patch_size, device)
+            if _plain(angles, later) and angles.dtype == later.dtype == torch.float64 and angles.device == later.device and angles.numel():
+                table = torch.empty(streams, 1, *angles.shape, dtype=torch.complex64, device=angles.device)
+                N.check(N.lib.lbm_stream_table(angles.data_ptr(), later.data_ptr(), f0, table.data_ptr(), angles.shape[0],
+                                               angles.shape[1], streams, N.stream_ptr(angles.device)))
+                return table
+        table = self.stream_table(frames, H, W, device)
+        if table.is_complex() and table.dim() == 4:
+            table = table.to(torch.complex64).expand(streams, -1, -1, -1).contiguous()
+        return table
 
     def forward(self, images: Tensor, selected_idx: Optional[List[int]] = None,
                 num_frame_for_scale: Optional[int] = None, sliding_window_size: Optional[int] = None,
                 num_frame_per_block: int = 1, *, pos3d: Optional[Tensor] = None,
-                tokens: Optional[Tensor] = None) -> Tuple[List[Tensor], int]:
+                tokens: Optional[Tensor] = None, stacked: bool = False) -> Tuple[Union[List[Tensor], Tensor], int]:
         """``images`` ``[streams, S, 3, H, W]`` in [0, 1]; ``S`` is 1 in streaming (more only for
         the anchor pass of a single stream).  Returns the groups' outputs ``[streams, S, P, 2C]``
         (all groups, or those in ``selected_idx``) and the index of the first patch token.
         ``pos3d``: the global blocks' rotary table of this call, for a caller that keeps the frame
         index itself (graph replay); the stream's frame counter is then left alone.
         ``tokens``: what ``_embed_images`` returned for these images, ``[streams * S, P, C]``, for
-        a caller that ran the image encoder ahead of time; ``images`` then only gives the sizes."""
+        a caller that ran the image encoder ahead of time; ``images`` then only gives the sizes.
+        ``stacked``: the groups' outputs as one tensor ``[groups, streams, S, P, 2C]``."""
         H, W = images.shape[-2:]
         if tokens is None:
             tokens, B, S, P, C = self._embed_images(images, num_frame_for_scale)
@@ -310,7 +375,7 @@ class HipAggregatorStream(nn.Module):
         manager = self._get_manager(tokens.device, tokens.dtype, P)
         scale_frames = self.num_frame_for_scale if num_frame_for_scale is None else num_frame_for_scale
         frame_idx = global_idx = 0
-        outputs: List[Tensor] = []
+        chosen: List[Tuple[Tensor, Tensor]] = []
         # the blocks in the order they run: each one's last residual kernel also applies the norm1
         # of the block after it, so only the first block of a call launches a LayerNorm of its own
         order = [blocks[i] for g in range(self.aa_block_num) for kind, blocks in
@@ -344,10 +409,13 @@ class HipAggregatorStream(nn.Module):
                     first_group = global_idx < self.aa_block_size
                     if self.rope3d is not None:     # frame index = frames streamed so far (stream.py:464-478)
                         if first_group:
-                            table = pos3d if pos3d is not None else self.stream_table(S, H, W, tokens.device)
-                            if table.is_complex() and table.dim() == 4:
-                                # one complex64 entry per token and stream: the blocks take it as it is
-                                table = table.to(torch.complex64).expand(B, -1, -1, -1).contiguous()
+                            # one complex64 entry per token and stream: the blocks take it as it is
+                            if pos3d is None:
+                                table = self._stream_table64(S, H, W, tokens.device, B)
+                            elif pos3d.is_complex() and pos3d.dim() == 4:
+                                table = pos3d.to(torch.complex64).expand(B, -1, -1, -1).contiguous()
+                            else:
+                                table = pos3d
                             self._cached_pos3d = table
                         pos_g = self._cached_pos3d
                     else:
@@ -364,9 +432,14 @@ class HipAggregatorStream(nn.Module):
                     if first_group and pos3d is None and not getattr(manager, "_skip_append", False):
                         self.total_frames_processed += S
             if selected_idx is None or group in selected_idx:
-                for f, g in zip(frame_out, global_out):
-                    outputs.append(torch.cat([f, g], dim=-1))
-        return outputs, self.patch_start_idx
+                chosen += zip(frame_out, global_out)
+        return _group_outputs(chosen, stacked), self.patch_start_idx
+
+
+def _graph_table(model: HipAggregatorStream, hw: Tuple[int, int], device) -> Tensor:
+    """The rotary table of the model's next frame as a graph's input: float32 ``[1, 1, P, D / 2, 2]``."""
+    with torch.no_grad():
+        return torch.view_as_real(model._stream_table64(1, hw[0], hw[1], device, 1).to(torch.complex64)).contiguous()
 
 
 class GraphedAggregator:
@@ -391,8 +464,7 @@ class GraphedAggregator:
 
         def frame_fn(images: Tensor, table: Optional[Tensor] = None) -> Tensor:
             pos3d = torch.view_as_complex(table) if table is not None else None
-            outs, _ = model(images, selected_idx=selected_idx, pos3d=pos3d)
-            return torch.stack(outs)
+            return model(images, selected_idx=selected_idx, pos3d=pos3d, stacked=True)[0]
 
         inputs = [example_images]
         if model.rope3d is not None:
@@ -401,8 +473,7 @@ class GraphedAggregator:
                                     model.kv_cache_camera_only)
 
     def _table(self, device) -> Tensor:
-        t = self.model.stream_table(1, self._hw[0], self._hw[1], device)
-        return torch.view_as_real(t.to(torch.complex64)).contiguous()
+        return _graph_table(self.model, self._hw, device)
 
     def __call__(self, images: Tensor, keyframe: bool = True) -> Tensor:
         assert tuple(images.shape[-2:]) == self._hw, "the graphs were captured for another image size"
@@ -447,8 +518,7 @@ class PipelinedAggregator:
             with torch.cuda.stream(self._side), N.scratch_lane(1):
                 self._next.copy_(model._embed_images(images_next)[0])
             pos3d = torch.view_as_complex(table) if table is not None else None
-            outs, _ = model(images_next, selected_idx=selected_idx, pos3d=pos3d, tokens=current)
-            out = torch.stack(outs)
+            out = model(images_next, selected_idx=selected_idx, pos3d=pos3d, tokens=current, stacked=True)[0]
             main.wait_stream(self._side)          # join
             return out
 
@@ -459,8 +529,7 @@ class PipelinedAggregator:
                                     model.kv_cache_camera_only)
 
     def _table(self, device) -> Tensor:
-        t = self.model.stream_table(1, self._hw[0], self._hw[1], device)
-        return torch.view_as_real(t.to(torch.complex64)).contiguous()
+        return _graph_table(self.model, self._hw, device)
 
     @torch.no_grad()
     def prime(self, images: Tensor) -> None:

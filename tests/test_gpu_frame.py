@@ -1,0 +1,75 @@
+"""The kernels around the blocks of a frame against the torch operations they stand for, bit for bit."""
+import ctypes as C
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def ptr(t):
+    return C.c_void_p(t.data_ptr())
+
+
+@pytest.mark.parametrize("pairs,shape,dtype", [(1, (1, 1, 1, 8), torch.bfloat16), (4, (1, 1, 261, 1024), torch.bfloat16),
+                                               (3, (2, 1, 37, 768), torch.float32), (33, (1, 2, 5, 24), torch.bfloat16), (2, (1, 1, 9, 12), torch.bfloat16)])
+def test_group_outputs(pairs, shape, dtype):
+    """One pair, more than one launch takes, last workgroups that are nearly empty, rows that are no whole pieces (left to
+    torch), and one tensor for all."""
+    from lingbot_map_amd.aggregator import _group_outputs
+    parts = [(torch.randn(shape, device="cuda").to(dtype), torch.randn(shape, device="cuda").to(dtype)) for _ in range(pairs)]
+    want = [torch.cat(p, dim=-1) for p in parts]
+    with torch.no_grad():
+        got, whole = _group_outputs(parts), _group_outputs(parts, stacked=True)
+        apart = _group_outputs([(f.transpose(1, 2), g.transpose(1, 2)) for f, g in parts])
+    assert len(got) == pairs and all(torch.equal(a, b) and a._base is None for a, b in zip(got, want))
+    assert torch.equal(whole, torch.stack(want))
+    assert all(torch.equal(a, torch.cat((f.transpose(1, 2), g.transpose(1, 2)), dim=-1)) for a, (f, g) in zip(apart, parts))
+    f, g = (t.clone().requires_grad_() for t in parts[0])      # somebody differentiates: torch's own operations
+    _group_outputs([(f, g)])[0].float().sum().backward()
+    assert (f.grad == 1).all() and (g.grad == 1).all()
+
+
+@pytest.mark.parametrize("frames,rows,cols,streams", [(1, 16, 16, 1), (1, 27, 37, 4), (8, 3, 5, 1)])
+@pytest.mark.parametrize("f0", [0, 1, 9_999])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_stream_table(frames, rows, cols, streams, f0, dtype):
+    """The blocks' table against the public one in float64, at the stream's first frames and far into it."""
+    from lingbot_map_amd import HipAggregatorStream
+    from lingbot_map_amd.aggregator import _plain
+    model = HipAggregatorStream(embed_dim=128, depth=2, num_heads=2, enable_3d_rope=True, max_frame_num=10_100, num_streams=streams).cuda().to(dtype)
+    model.total_frames_processed = f0
+    with torch.no_grad():
+        want = model.stream_table(frames, 14 * rows, 14 * cols, "cuda:0").to(torch.complex64).expand(streams, -1, -1, -1)
+        got = model._stream_table64(frames, 14 * rows, 14 * cols, "cuda:0", streams)
+        base = model._table_base(frames, rows, cols, "cuda:0")
+        assert _plain(*base) and all(t.dtype == torch.float64 for t in base)      # (the kernel's path is the one that ran)
+    assert got.shape == want.shape and got.is_contiguous() and torch.equal(torch.view_as_real(got), torch.view_as_real(want.contiguous()))
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 3, 14, 14), (2, 3, 3, 28, 42), (1, 1, 3, 378, 518), (1, 1, 3, 7, 9)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_normalised_images(shape, dtype):
+    from lingbot_map_amd import HipAggregatorStream
+    model = HipAggregatorStream(embed_dim=128, depth=2, num_heads=2).cuda().to(dtype)
+    images = torch.rand(shape, device="cuda").to(dtype)
+    images[0, 0, 0, 0, :3] = torch.tensor([float("inf"), float("-inf"), 0.0])
+    with torch.no_grad():
+        want = (images - model._resnet_mean.to(dtype)) / model._resnet_std.to(dtype)
+        assert torch.equal(model._normalised(images), want)
+        wide = torch.rand(*shape[:-1], 2 * shape[-1], device="cuda").to(dtype)[..., ::2]     # strided: torch's own operations
+        assert torch.equal(model._normalised(wide), (wide - model._resnet_mean.to(dtype)) / model._resnet_std.to(dtype))
+
+
+def test_refusals():
+    from lingbot_map_amd import _native as N
+    t = torch.zeros(64, device="cuda")
+    two, one = (C.c_void_p * 2)(t.data_ptr(), t.data_ptr()), (C.c_void_p * 1)(t.data_ptr())
+    off = (C.c_void_p * 1)(t.data_ptr() + 4)
+    bad = lambda *a: N.lib.lbm_group_outputs(*a, None) == N.ERR_INVALID
+    assert bad(None, one, 1, 1, 16) and bad(two, None, 1, 1, 16) and bad(two, off, 1, 1, 16) and bad(two, one, 0, 1, 16)
+    assert bad(two, one, N.MAX_GROUPS + 1, 1, 16) and bad(two, one, 1, 0, 16) and bad(two, one, 1, 1, 24) and bad(two, one, 1, 1 << 31, 32)
+    bad = lambda *a: N.lib.lbm_stream_table(*a, None) == N.ERR_INVALID
+    assert bad(None, ptr(t), 0, ptr(t), 1, 1, 1) and bad(ptr(t), ptr(t), 0, ptr(t), 0, 1, 1) and bad(ptr(t), ptr(t), 0, ptr(t), 1 << 16, 1 << 15, 1)
+    bad = lambda *a: N.lib.lbm_normalise_images(*a, None) == N.ERR_INVALID
+    assert bad(ptr(t), ptr(t), ptr(t), None, 0, 1, 4) and bad(ptr(t), ptr(t), ptr(t), ptr(t), 7, 1, 4) and bad(ptr(t), ptr(t), ptr(t), ptr(t), 0, 1, 6)
