@@ -212,6 +212,67 @@ LBM_HD void lbm_phase_evict(int32_t* st, const lbm_cache_geom& g, const LbmTable
 }
 
 // ---------------------------------------------------------------------------- plan
+// n (1 to 4) consecutive entries of a row table: first, first + step, ...; whole fours as one store (a table's entries are
+// aligned to 4 bytes and no more, which is what the store needs).
+LBM_HD void lbm_put_rows(int32_t* dst, int first, int step, int n) {
+#ifdef __HIP_DEVICE_COMPILE__
+  typedef int32_t four __attribute__((ext_vector_type(4), aligned(4)));
+  if (n == 4) {
+    *(four*)dst = four{first, first + step, first + 2 * step, first + 3 * step};
+    return;
+  }
+#endif
+  for (int j = 0; j < n; ++j) dst[j] = first + j * step;
+}
+
+// The rows of the cached frames.  A thread owns runs of RUN token slots, u, u + nthr, ... of every frame (consecutive
+// lanes write consecutive runs; RUN divides the page size).  Frames of fewer runs than there are threads are dealt to
+// groups of `runs` threads, group i taking frames i, i + groups, ...: one thread would otherwise walk all frames of a
+// one-token-per-frame cache by itself (10,000 frames: 1.4 ms).  Eight frames at a time so that their page-id loads are in
+// flight together (no division per token, no load waiting on the previous frame's store).
+template <int RUN>
+LBM_HD void lbm_plan_frames(int32_t* out, const int32_t* st, int S, int shift, const LbmTablesLayout& L, const LbmHdr& h,
+                            const lbm_step_op& op, bool newest_self, int limit, int tid, int nthr) {
+  const int32_t* anchor = st + L.off_anchor;
+  const int32_t* win = st + L.off_window;
+  const int nfr = h.na + h.wc, runs = lbm_ceil_div(L.tpf, RUN);
+  const int groups = runs < nthr ? nthr / runs : 1;
+  const int my_group = groups > 1 ? tid / runs : 0;
+  const int u_first = groups > 1 ? (my_group < groups ? tid % runs : runs) : tid;
+  for (int u = u_first; u < runs; u += groups > 1 ? runs : nthr) {
+    const int t = u * RUN, n_run = RUN == 1 || L.tpf - t >= RUN ? RUN : L.tpf - t;
+    const int pg = shift >= 0 ? t >> shift : t / S;
+    const int slot = t - pg * S;
+    for (int f0 = my_group; f0 < nfr; f0 += 8 * groups) {
+      int32_t page[8];
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+#endif
+      for (int k = 0; k < 8; ++k) {
+        const int f = f0 + k * groups < nfr ? f0 + k * groups : nfr - 1;
+        int r = h.wh + f - h.na;                     // ring slot of window frame f - na
+        if (r >= L.ring_frames) r -= L.ring_frames;  // wh < ring_frames and at most ring_frames window frames
+        const int32_t* pages = f < h.na ? anchor + f * L.ppf : win + r * L.ppf;
+        page[k] = pages[pg];
+      }
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+#endif
+      for (int k = 0; k < 8; ++k) {
+        const int f = f0 + k * groups;
+        const int i = f * L.tpf + t;
+        const bool own = newest_self && f == nfr - 1;
+        if (RUN == 1) {
+          if (f < nfr && i < limit) out[i] = own ? -1 - (op.q_begin + t) : page[k] * 2 * S + slot;
+        } else if (f < nfr && i < limit) {
+          lbm_put_rows(out + i, own ? -1 - (op.q_begin + t) : page[k] * 2 * S + slot, own ? -1 : 1,
+                       n_run < limit - i ? n_run : limit - i);
+        }
+      }
+    }
+  }
+}
+
 // build_visible_page_table + compute_last_page_len (flashinfer_cache.py:438-470) with a
 // valid length per page, plus the dense row table the attention kernel gathers through.
 // Never writes more row entries than the host says the table holds (op.expect_kv_tokens, or the
@@ -242,41 +303,11 @@ LBM_HD void lbm_phase_plan(int32_t* st, const lbm_cache_geom& g, const LbmTables
     // token t of a page list sits in page t / S, slot t % S; page sizes are powers of two in
     // every configuration but one (page = patches per frame), so the common case is a shift
     const int shift = (S & (S - 1)) == 0 ? __builtin_ctz((unsigned)S) : -1;
-    // A thread owns token slots t, t + nthr, ... of every frame (consecutive lanes write
-    // consecutive rows).  Frames with fewer tokens than there are threads are dealt to groups of tpf
-    // threads, group i taking frames i, i + groups, ...: one thread would otherwise walk all frames of
-    // a one-token-per-frame cache by itself (10,000 frames: 1.4 ms).  Eight frames at a time so that
-    // their page-id loads are in flight together (no division per token, no load waiting on the
-    // previous frame's store).
-    const int groups = L.tpf < nthr ? nthr / L.tpf : 1;
-    const int my_group = groups > 1 ? tid / L.tpf : 0;
-    const int t_first = groups > 1 ? (my_group < groups ? tid % L.tpf : L.tpf) : tid;
-    for (int t = t_first; t < L.tpf; t += groups > 1 ? L.tpf : nthr) {
-      const int pg = shift >= 0 ? t >> shift : t / S;
-      const int slot = t - pg * S;
-      for (int f0 = my_group; f0 < nfr; f0 += 8 * groups) {
-        int32_t page[8];
-#ifdef __HIP_DEVICE_COMPILE__
-#pragma unroll
-#endif
-        for (int k = 0; k < 8; ++k) {
-          const int f = f0 + k * groups < nfr ? f0 + k * groups : nfr - 1;
-          int r = h.wh + f - h.na;                     // ring slot of window frame f - na
-          if (r >= L.ring_frames) r -= L.ring_frames;  // wh < ring_frames and at most ring_frames window frames
-          const int32_t* pages = f < h.na ? anchor + f * L.ppf : win + r * L.ppf;
-          page[k] = pages[pg];
-        }
-#ifdef __HIP_DEVICE_COMPILE__
-#pragma unroll
-#endif
-        for (int k = 0; k < 8; ++k) {
-          const int f = f0 + k * groups;
-          const int i = f * L.tpf + t;
-          if (f < nfr && i < limit)
-            out[i] = (newest_self && f == nfr - 1) ? -1 - (op.q_begin + t) : page[k] * 2 * S + slot;
-        }
-      }
-    }
+    // Four rows at a time where pages hold whole fours: a page id, its addresses and its compares serve four rows (one
+    // workgroup, us a step: 17 frames of 1,004 tokens 12.7, 8.8; frames of one token have nothing to share, 10,000 of them
+    // 7.8, 9.3).
+    if ((S & 3) == 0 && L.tpf >= 4) lbm_plan_frames<4>(out, st, S, shift, L, h, op, newest_self, limit, tid, nthr);
+    else lbm_plan_frames<1>(out, st, S, shift, L, h, op, newest_self, limit, tid, nthr);
     if (two) {
       for (int c = tid; c < h.stc; c += nthr) {
         const int pg = shift >= 0 ? c >> shift : c / S;

@@ -310,6 +310,34 @@ def test_step_that_appends_inside_the_attention_call(T, H, streams, dtype):
         a._attend_planned(1, q, None, None)
 
 
+@pytest.mark.parametrize("T,page", [(3, 4), (4, 4), (5, 4), (7, 12), (10, 6), (129, 16), (1003, 16), (1005, 8)])
+@pytest.mark.parametrize("own", [False, True])
+def test_row_table_four_rows_at_a_time(T, page, own):
+    """Row tables on either side of the form that writes runs of four: frames of fewer than four tokens, last runs of one
+    to four, pages of whole fours and not, frames that begin at any entry; ``own``: the newest frame named by the caller's rows."""
+    from lingbot_map_amd import HipPagedKVCacheManager
+    from oracle.page_policy import PagePolicy
+    window, frames = 9, 14
+    m = HipPagedKVCacheManager(1, window + 17, T, 2, 64, torch.bfloat16, torch.device("cuda:0"), num_special_tokens=2, scale_frames=1,
+                               sliding_window=window, max_total_frames=frames + 8, page_size=page, layout="frame_pages")
+    m.fuse_append = own
+    pol = PagePolicy(T, 2, page, 1, window, frames + 8, layout="frame_pages")
+    x = torch.zeros(T, 2, 64, dtype=torch.bfloat16, device="cuda")
+    for i in range(frames):
+        pol.append_frame()
+        pol.evict_frames(1, window)
+        m.step(0, x, x, x, keyframe=[True])
+        rows = []
+        for p, n in zip(pol.build_visible_page_table(), pol.build_visible_page_lens()):
+            rows += [p * 2 * page + s for s in range(n)]
+        n_frames = min(pol.frame_count, 1 + window)
+        if own:
+            rows[(n_frames - 1) * T:n_frames * T] = [-1 - t for t in range(T)]
+        assert m._plan_tokens[0][0] == len(rows)
+        assert torch.equal(m._kv_rows[0][:len(rows)].cpu(), torch.tensor(rows, dtype=torch.int32)), i
+    assert m.device_header()["error"] == 0
+
+
 @pytest.mark.parametrize("T,special,window,frames", [(1, 0, 3000, 3100), (37, 5, 200, 900), (300, 5, 20, 1200), (1004, 5, 26, 30)])
 def test_row_table_of_short_frames_and_long_plans(T, special, window, frames):
     """Row tables whose frames have fewer tokens than a workgroup has threads, and plans long enough to
