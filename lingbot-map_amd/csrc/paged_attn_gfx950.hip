@@ -1857,7 +1857,9 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
 // one 128-thread workgroup per (stream, query row, head): merge the chunks' partials (and, grid
 // z beyond the streams, store the caller's new rows: the chunks' kernel has read the pool).  Thread
 // c reads chunk c's maximum and sum (all chunks at once), the weights go through LDS, then
-// thread d sums the weighted outputs with several loads in flight.
+// thread d sums the weighted outputs.  Bound by trips to memory: the first 32 chunks' outputs are asked for beside the
+// maxima, before a weight is known, the others' together (40 chunks of 128 floats: six trips as batches of eight behind
+// the weights, two so: 4.2 us, 4.0).
 template <int D>
 __global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeArgs a) {
   static_assert(kDecMaxChunks <= 128 && D <= 128, "one thread per chunk, one per head dimension");
@@ -1880,11 +1882,13 @@ __global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeAr
   const int H = a.f.num_heads, nc = a.n_chunks[b];
   const size_t stride = (size_t)sp.q_rows * H * (D + 2);      // from one chunk's partial to the next
   const float* base = a.part + (((size_t)a.part_begin[b] + qi) * H + head) * (D + 2);
-  float m_c = -INFINITY, l_c = 0.f;
-  if (tid < nc) {
-    m_c = base[tid * stride + D];
-    l_c = base[tid * stride + D + 1];
-  }
+  constexpr int kBatch = 32;
+  static_assert(kDecMaxChunks <= 2 * kBatch, "two batches hold every chunk");
+  const int d = min(tid, D - 1), c_own = min(tid, nc - 1);      // (loads outside of conditional blocks: they go out together)
+  float x[kBatch], m_c = base[c_own * stride + D], l_c = base[c_own * stride + D + 1];
+#pragma unroll
+  for (int j = 0; j < kBatch; ++j) x[j] = base[min(j, nc - 1) * stride + d];
+  if (tid >= nc) m_c = -INFINITY, l_c = 0.f;
   float m = m_c;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
@@ -1901,15 +1905,16 @@ __global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeAr
   l = red[1][0] + red[1][1];
   if (tid >= D) return;
   float o = 0.f;
-  int c = 0;
-  for (; c + 8 <= nc; c += 8) {
-    float x[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = base[(c + j) * stride + tid];
+  for (int j = 0; j < kBatch; ++j)
+    if (j < nc) o += x[j] * w[j];
+  if (nc > kBatch) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o += x[j] * w[c + j];
+    for (int j = 0; j < kBatch; ++j) x[j] = base[min(kBatch + j, nc - 1) * stride + tid];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j)
+      if (kBatch + j < nc) o += x[j] * w[kBatch + j];
   }
-  for (; c < nc; ++c) o += base[c * stride + tid] * w[c];
   a.f.out[((size_t)(sp.q_begin + qi) * H + head) * D + tid] = l > 0.f ? o / l : 0.f;
 }
 
