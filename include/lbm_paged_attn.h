@@ -478,12 +478,12 @@ int lbm_attn_run_static(const void* q, const void* pool, void* out, const void* 
  *
  * lbm_group_outputs: out[g][row] = parts[2 g][row] followed by parts[2 g + 1][row], for n_groups groups of `rows` rows of
  * row_bytes (a multiple of 16; all pointers 16-byte aligned) - the concatenation of a frame block's and a global block's
- * tokens (aggregator/base.py:500, stream.py:529) for all groups at once.  `parts` and `out` are host memory, read before
+ * tokens (aggregator/base.py:600-604) for all groups at once.  `parts` and `out` are host memory, read before
  * the call returns; no output overlaps a part or another output.
  * lbm_stream_table: out[s][t][j] = (cos, sin)(angles[t][j] + first * later[j]) as float32 for every stream s: the rotary
  * table of the frames that begin at stream index `first` (stream.py:273-295), computed in float64.
  * lbm_normalise_images: (x - mean[c]) / std[c] for n_images x 3 planes of `plane` values (a multiple of 4), rounded to
- * the type of images, mean, std and out after each operation (aggregator/base.py:600-604). */
+ * the type of images, mean, std and out after each operation (aggregator/base.py:335-395). */
 #define LBM_MAX_GROUPS 32
 int lbm_group_outputs(const void* const* parts, void* const* out, int32_t n_groups, int64_t rows, int64_t row_bytes, void* stream);
 int lbm_stream_table(const double* angles, const double* later, int64_t first, float* out, int32_t tokens, int32_t pairs,

@@ -280,7 +280,7 @@ class HipAggregatorStream(nn.Module):
         return tokens, B, S, tokens.shape[1], C
 
     def _normalised(self, images: Tensor) -> Tensor:
-        """(images - mean) / std (base.py:345)."""
+        """(images - mean) / std (base.py:335-395)."""
         mean, std = self._resnet_mean.to(images.dtype), self._resnet_std.to(images.dtype)
         H, W = images.shape[-2:]
         if (images.dtype in (torch.bfloat16, torch.float32) and _plain(images, mean, std) and images.device == mean.device == std.device
