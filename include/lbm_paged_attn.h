@@ -483,13 +483,16 @@ int lbm_attn_run_static(const void* q, const void* pool, void* out, const void* 
  * lbm_stream_table: out[s][t][j] = (cos, sin)(angles[t][j] + first * later[j]) as float32 for every stream s: the rotary
  * table of the frames that begin at stream index `first` (stream.py:273-295), computed in float64.
  * lbm_normalise_images: (x - mean[c]) / std[c] for n_images x 3 planes of `plane` values (a multiple of 4), rounded to
- * the type of images, mean, std and out after each operation (aggregator/base.py:335-395). */
+ * the type of images, mean, std and out after each operation (aggregator/base.py:335-395).
+ * lbm_patch_tokens: out[n][p][c] = conv[n][c][p] + bias[c] in bf16, the sum rounded once: the bias of the patch convolution
+ * (base.py:190-197) and its patches as rows; channels a multiple of 64, out 16-byte aligned. */
 #define LBM_MAX_GROUPS 32
 int lbm_group_outputs(const void* const* parts, void* const* out, int32_t n_groups, int64_t rows, int64_t row_bytes, void* stream);
 int lbm_stream_table(const double* angles, const double* later, int64_t first, float* out, int32_t tokens, int32_t pairs,
                      int32_t n_streams, void* stream);
 int lbm_normalise_images(const void* images, const void* mean, const void* std, void* out, int32_t dtype, int64_t n_images,
                          int64_t plane, void* stream);
+int lbm_patch_tokens(const void* conv, const void* bias, void* out, int32_t n_images, int32_t channels, int32_t patches, void* stream);
 
 #ifdef __cplusplus
 }

@@ -75,6 +75,36 @@ __global__ __launch_bounds__(kThreads) void lbm_normalise_images_kernel(const vo
   }
 }
 
+// ---------------------------------------------------------------------------- patch tokens
+// out[n][p][c] = conv[n][c][p] + bias[c] in bf16: the patch convolution's bias and its channels last.  64 channels x 64
+// patches per workgroup through LDS: patches lie side by side on the way in (of any number, so 2 bytes a lane, 128 a
+// wavefront's load), channels on the way out (16 bytes a lane).  us, 999 patches of 1,024 channels: torch's sum and copy
+// 15.9, this @.
+__global__ __launch_bounds__(kThreads) void lbm_patch_tokens_kernel(const unsigned short* conv, const __bf16* bias, unsigned short* out,
+                                                                    int patches, int channels) {
+  constexpr int kTile = 64, kStride = kTile + 8, kEach = kTile * kTile / kThreads;
+  __shared__ __attribute__((aligned(16))) unsigned short tile[kTile * kStride];   // [patch][channel]
+  const int tid = threadIdx.x, p0 = blockIdx.x * kTile, c0 = blockIdx.y * kTile;
+  const unsigned short* src = conv + ((size_t)blockIdx.z * channels + c0) * patches;
+  const int p = tid & 63, last = patches - 1 - p0;
+  unsigned short v[kEach];
+#pragma unroll
+  for (int j = 0; j < kEach; ++j) v[j] = src[(size_t)(j * (kThreads / 64) + (tid >> 6)) * patches + p0 + min(p, last)];
+#pragma unroll
+  for (int j = 0; j < kEach; ++j) {
+    const int c = j * (kThreads / 64) + (tid >> 6);
+    const __bf16 sum = (__bf16)((float)__builtin_bit_cast(__bf16, v[j]) + (float)bias[c0 + c]);
+    tile[p * kStride + c] = __builtin_bit_cast(unsigned short, sum);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kTile * kTile / 8 / kThreads; ++j) {
+    const int r = j * (kThreads / 8) + (tid >> 3), c = (tid & 7) * 8;
+    if (p0 + r < patches)
+      lbm_store_through(out + ((size_t)blockIdx.z * patches + p0 + r) * channels + c0 + c, *(const u32x4*)&tile[r * kStride + c]);
+  }
+}
+
 bool aligned(const void* p, size_t to) { return ((uintptr_t)p & (to - 1)) == 0; }
 unsigned blocks_for(unsigned long long n, unsigned per_block) { return (unsigned)((n + per_block - 1) / per_block); }
 }  // namespace
@@ -124,4 +154,14 @@ extern "C" int lbm_normalise_images(const void* images, const void* mean, const 
   if (dtype == LBM_DTYPE_BF16) hipLaunchKernelGGL(lbm_normalise_images_kernel<true>, grid, block, 0, (hipStream_t)stream, images, mean, std, out, quads, plane_quads);
   else hipLaunchKernelGGL(lbm_normalise_images_kernel<false>, grid, block, 0, (hipStream_t)stream, images, mean, std, out, quads, plane_quads);
   return lbm_check_launch("lbm_normalise_images_kernel");
+}
+
+extern "C" int lbm_patch_tokens(const void* conv, const void* bias, void* out, int32_t n_images, int32_t channels, int32_t patches, void* stream) {
+  if (!conv || !bias || !out) return lbm_fail(LBM_ERR_INVALID, "lbm_patch_tokens: null argument");
+  if (n_images < 1 || n_images > 65535 || channels < 64 || channels % 64 || channels > 64 * 65535 || patches < 1)
+    return lbm_fail(LBM_ERR_INVALID, "lbm_patch_tokens: %d images of %d channels (a multiple of 64) x %d patches", n_images, channels, patches);
+  if (!aligned(conv, 2) || !aligned(bias, 2) || !aligned(out, 16)) return lbm_fail(LBM_ERR_INVALID, "lbm_patch_tokens: alignment");
+  hipLaunchKernelGGL(lbm_patch_tokens_kernel, dim3(blocks_for(patches, 64), channels / 64, n_images), dim3(kThreads), 0, (hipStream_t)stream,
+                     (const unsigned short*)conv, (const __bf16*)bias, (unsigned short*)out, patches, channels);
+  return lbm_check_launch("lbm_patch_tokens_kernel");
 }

@@ -104,7 +104,7 @@ class BlockCall(C.Structure):
 SYMBOLS = ("lbm_abi_version", "lbm_last_error", "lbm_tables_words", "lbm_tables_step",
            "lbm_rows_from_pages", "lbm_kv_append", "lbm_qkv_prepare", "lbm_residual_norm", "lbm_linear", "lbm_linear_norm", "lbm_linear_stats_tiles", "lbm_linear_workspace_bytes", "lbm_linear_prefetch_hint", "lbm_qkv_linear_prepare", "lbm_qkv_linear_prepare_norm", "lbm_attn_workspace_bytes", "lbm_attn_run", "lbm_attn_run_append", "lbm_attn_run_live", "lbm_attn_run_call",
            "lbm_attn_run_static", "lbm_block_scratch_bytes", "lbm_block_run",
-           "lbm_group_outputs", "lbm_stream_table", "lbm_normalise_images")
+           "lbm_group_outputs", "lbm_stream_table", "lbm_normalise_images", "lbm_patch_tokens")
 
 
 def _load():
@@ -167,6 +167,8 @@ def _load():
     lib.lbm_stream_table.argtypes = [vp, vp, C.c_int64, vp, i32, i32, i32, vp]
     lib.lbm_normalise_images.restype = C.c_int
     lib.lbm_normalise_images.argtypes = [vp, vp, vp, vp, i32, C.c_int64, C.c_int64, vp]
+    lib.lbm_patch_tokens.restype = C.c_int
+    lib.lbm_patch_tokens.argtypes = [vp, vp, vp, i32, i32, i32, vp]
     if lib.lbm_abi_version() != ABI_VERSION:
         raise RuntimeError(f"{LIB_PATH}: ABI version {lib.lbm_abi_version()}, binding expects {ABI_VERSION}")
     return lib

@@ -61,6 +61,24 @@ def test_normalised_images(shape, dtype):
         assert torch.equal(model._normalised(wide), (wide - model._resnet_mean.to(dtype)) / model._resnet_std.to(dtype))
 
 
+@pytest.mark.parametrize("n,rows,cols,channels", [(1, 1, 1, 64), (1, 9, 9, 1024), (2, 8, 8, 768), (3, 13, 5, 128), (1, 27, 37, 1024)])
+def test_patch_tokens(n, rows, cols, channels):
+    """One patch, one short and one more than whole tiles, against the module's own operations."""
+    from lingbot_map_amd.aggregator import PatchConv
+    conv = PatchConv(14, channels).cuda().to(torch.bfloat16)
+    images = torch.randn(n, 3, 14 * rows, 14 * cols, device="cuda").to(torch.bfloat16)
+    want = conv.proj(images).flatten(2).transpose(1, 2)
+    with torch.no_grad():
+        got = conv(images)
+        assert got.is_contiguous() and torch.equal(got, want)
+        seen = []
+        handle = conv.proj.register_forward_hook(lambda m, a, o: seen.append(o.shape))
+        assert torch.equal(conv(images), want) and len(seen) == 1      # somebody listens to the convolution
+        handle.remove()
+    conv(images).float().sum().backward()
+    assert conv.proj.bias.grad is not None
+
+
 def test_refusals():
     from lingbot_map_amd import _native as N
     t = torch.zeros(64, device="cuda")
@@ -71,5 +89,8 @@ def test_refusals():
     assert bad(two, one, N.MAX_GROUPS + 1, 1, 16) and bad(two, one, 1, 0, 16) and bad(two, one, 1, 1, 24) and bad(two, one, 1, 1 << 31, 32)
     bad = lambda *a: N.lib.lbm_stream_table(*a, None) == N.ERR_INVALID
     assert bad(None, ptr(t), 0, ptr(t), 1, 1, 1) and bad(ptr(t), ptr(t), 0, ptr(t), 0, 1, 1) and bad(ptr(t), ptr(t), 0, ptr(t), 1 << 16, 1 << 15, 1)
+    bad = lambda *a: N.lib.lbm_patch_tokens(*a, None) == N.ERR_INVALID
+    assert bad(None, ptr(t), ptr(t), 1, 64, 1) and bad(ptr(t), ptr(t), ptr(t), 0, 64, 1) and bad(ptr(t), ptr(t), ptr(t), 1, 60, 1)
+    assert bad(ptr(t), ptr(t), ptr(t), 1, 64, 0) and bad(ptr(t), ptr(t), C.c_void_p(t.data_ptr() + 2), 1, 64, 1)
     bad = lambda *a: N.lib.lbm_normalise_images(*a, None) == N.ERR_INVALID
     assert bad(ptr(t), ptr(t), ptr(t), None, 0, 1, 4) and bad(ptr(t), ptr(t), ptr(t), ptr(t), 7, 1, 4) and bad(ptr(t), ptr(t), ptr(t), ptr(t), 0, 1, 6)
