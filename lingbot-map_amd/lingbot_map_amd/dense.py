@@ -18,7 +18,7 @@ from . import _native as N
 
 _plans: Dict[tuple, tuple] = {}          # (rows, streams, H, D, device) -> (row table, stream descriptors, workspace bytes)
 _tails: Dict[tuple, bytes] = {}          # (streams, H, D, dtype) -> what the calls of such a plan have in common
-_calls: Dict[tuple, tuple] = {}          # frames_key of a call -> its plan as attend() takes it (addresses of what _plans owns)
+_calls: Dict[tuple, tuple] = {}          # frames_key of a call -> its plan as attend() takes it, and what its addresses belong to
 _workspace: Dict[object, Tensor] = {}
 
 
@@ -64,8 +64,8 @@ def dense_attention(q: Tensor, k: Tensor, v: Tensor, num_streams: int = 1, q_pre
             rows, H, D = key[:3]
             kv_rows, streams, _ = dense_plan(rows, num_streams, H, D, q.device)
             call = _calls[key] = (kv_rows.data_ptr(), C.addressof(streams), max(_plans[(rows, num_streams, H, D, q.device)][2], 16), q.device,
-                                  1.0 / math.sqrt(D), _tail(num_streams, H, D, q.dtype))
-        rows_at, streams_at, need, device, scale, tail = call
+                                  1.0 / math.sqrt(D), _tail(num_streams, H, D, q.dtype), (kv_rows, streams))
+        rows_at, streams_at, need, device, scale, tail, _ = call
         ws = _workspace.get((device, N.current_scratch_lane()))
         if ws is None or ws.numel() < need:
             ws = dense_plan(key[0], num_streams, key[1], key[2], device)[2]
