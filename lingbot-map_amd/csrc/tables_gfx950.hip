@@ -9,6 +9,9 @@
 
 struct LbmStepOps { lbm_step_op s[LBM_MAX_STREAMS]; };
 
+// RUN: lbm_rows_at_a_time.  A kernel for each: with both forms of the plan in one, steps of the one-row form take longer
+// (10,000 frames of one token 7.2 us apart, 7.4 in one; 2,000 5.7, 5.8).
+template <int RUN>
 __global__ __launch_bounds__(1024) void lbm_tables_kernel(
     int32_t* __restrict__ tables, lbm_cache_geom g, LbmStepOps ops, int32_t* append_rows,
     int32_t* kv_rows, int32_t* page_ids, int32_t* page_lens) {
@@ -43,7 +46,7 @@ __global__ __launch_bounds__(1024) void lbm_tables_kernel(
     lbm_phase_evict(st, g, L, op.sliding_window, op.keep_tokens, tid, nthr, h);
     __syncthreads();
   }
-  if (op.ops & LBM_OP_PLAN) lbm_phase_plan(st, g, L, op, kv_rows, page_ids, page_lens, tid, nthr, h);
+  if (op.ops & LBM_OP_PLAN) lbm_phase_plan<RUN>(st, g, L, op, kv_rows, page_ids, page_lens, tid, nthr, h);
   if (tid == 0) lbm_hdr_store(st, h);
 }
 
@@ -117,16 +120,16 @@ int lbm_launch_tables(int32_t* tables, const lbm_cache_geom& g, int n_streams,
   constexpr int kRowsPerGroup = 4096, kSplitRows = 24576, kMostGroups = 64;
   const int groups = most_rows <= kRowsPerGroup ? 1 : (most_rows + kRowsPerGroup - 1) / kRowsPerGroup;
   const bool wide = groups > 1 && (!changes || most_rows > kSplitRows);
+  const auto kernel = lbm_rows_at_a_time(g) == 4 ? lbm_tables_kernel<4> : lbm_tables_kernel<1>;
   if (changes || !wide) {
     if (wide)
       for (int i = 0; i < n_streams; ++i) o.s[i].ops &= ~kPlanBits;
-    hipLaunchKernelGGL(lbm_tables_kernel, dim3(n_streams), dim3(1024), 0, stream, tables, g, o, append_rows, kv_rows,
-                       page_ids, page_lens);
+    hipLaunchKernelGGL(kernel, dim3(n_streams), dim3(1024), 0, stream, tables, g, o, append_rows, kv_rows, page_ids, page_lens);
     const int rc = lbm_check_launch("lbm_tables_kernel");
     if (rc != LBM_OK || !wide) return rc;
   }
   // (append_rows was written by the launch in front, if it was asked for and there was one)
-  hipLaunchKernelGGL(lbm_tables_kernel, dim3(n_streams, groups < kMostGroups ? groups : kMostGroups), dim3(1024), 0, stream,
+  hipLaunchKernelGGL(kernel, dim3(n_streams, groups < kMostGroups ? groups : kMostGroups), dim3(1024), 0, stream,
                      tables, g, plan, changes ? nullptr : append_rows, kv_rows, page_ids, page_lens);
   return lbm_check_launch("lbm_tables_kernel");
 }

@@ -225,17 +225,54 @@ LBM_HD void lbm_put_rows(int32_t* dst, int first, int step, int n) {
   for (int j = 0; j < n; ++j) dst[j] = first + j * step;
 }
 
+// RUN token slots from t on (n_run of them; slot `slot` of page `pg` on) of frames my_group, my_group + groups, ...: BATCH
+// frames at a time, so that their page-id loads are in flight together (no division per token, no load waiting on the
+// previous frame's store).
+template <int RUN, int BATCH>
+LBM_HD void lbm_plan_run(int32_t* out, const int32_t* anchor, const int32_t* win, int S, const LbmTablesLayout& L, const LbmHdr& h,
+                         int q_begin, bool newest_self, int limit, int t, int n_run, int pg, int slot, int my_group, int groups) {
+  const int nfr = h.na + h.wc;
+  for (int f0 = my_group; f0 < nfr; f0 += BATCH * groups) {
+    int32_t page[BATCH];
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+#endif
+    for (int k = 0; k < BATCH; ++k) {
+      const int f = f0 + k * groups < nfr ? f0 + k * groups : nfr - 1;
+      int r = h.wh + f - h.na;                     // ring slot of window frame f - na
+      if (r >= L.ring_frames) r -= L.ring_frames;  // wh < ring_frames and at most ring_frames window frames
+      const int32_t* pages = f < h.na ? anchor + f * L.ppf : win + r * L.ppf;
+      page[k] = pages[pg];
+    }
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+#endif
+    for (int k = 0; k < BATCH; ++k) {
+      const int f = f0 + k * groups;
+      const int i = f * L.tpf + t;
+      const bool own = newest_self && f == nfr - 1;
+      if (RUN == 1) {
+        if (f < nfr && i < limit) out[i] = own ? -1 - (q_begin + t) : page[k] * 2 * S + slot;
+      } else if (f < nfr && i < limit) {
+        lbm_put_rows(out + i, own ? -1 - (q_begin + t) : page[k] * 2 * S + slot, own ? -1 : 1,
+                     n_run < limit - i ? n_run : limit - i);
+      }
+    }
+  }
+}
+
 // The rows of the cached frames.  A thread owns runs of RUN token slots, u, u + nthr, ... of every frame (consecutive
 // lanes write consecutive runs; RUN divides the page size).  Frames of fewer runs than there are threads are dealt to
 // groups of `runs` threads, group i taking frames i, i + groups, ...: one thread would otherwise walk all frames of a
-// one-token-per-frame cache by itself (10,000 frames: 1.4 ms).  Eight frames at a time so that their page-id loads are in
-// flight together (no division per token, no load waiting on the previous frame's store).
+// one-token-per-frame cache by itself (10,000 frames: 1.4 ms).  Eight frames at a time; two where four-row runs leave a
+// thread no more, since a frame that is not there costs its addresses and compares all the same (one workgroup, us a step
+// with eight and with two: 197 tokens x 17 frames 6.1, 5.2; 261 x 17 6.0, 5.1; 1,004 x 5 6.4, 5.5).
 template <int RUN>
 LBM_HD void lbm_plan_frames(int32_t* out, const int32_t* st, int S, int shift, const LbmTablesLayout& L, const LbmHdr& h,
                             const lbm_step_op& op, bool newest_self, int limit, int tid, int nthr) {
   const int32_t* anchor = st + L.off_anchor;
   const int32_t* win = st + L.off_window;
-  const int nfr = h.na + h.wc, runs = lbm_ceil_div(L.tpf, RUN);
+  const int runs = lbm_ceil_div(L.tpf, RUN);
   const int groups = runs < nthr ? nthr / runs : 1;
   const int my_group = groups > 1 ? tid / runs : 0;
   const int u_first = groups > 1 ? (my_group < groups ? tid % runs : runs) : tid;
@@ -243,35 +280,17 @@ LBM_HD void lbm_plan_frames(int32_t* out, const int32_t* st, int S, int shift, c
     const int t = u * RUN, n_run = RUN == 1 || L.tpf - t >= RUN ? RUN : L.tpf - t;
     const int pg = shift >= 0 ? t >> shift : t / S;
     const int slot = t - pg * S;
-    for (int f0 = my_group; f0 < nfr; f0 += 8 * groups) {
-      int32_t page[8];
-#ifdef __HIP_DEVICE_COMPILE__
-#pragma unroll
-#endif
-      for (int k = 0; k < 8; ++k) {
-        const int f = f0 + k * groups < nfr ? f0 + k * groups : nfr - 1;
-        int r = h.wh + f - h.na;                     // ring slot of window frame f - na
-        if (r >= L.ring_frames) r -= L.ring_frames;  // wh < ring_frames and at most ring_frames window frames
-        const int32_t* pages = f < h.na ? anchor + f * L.ppf : win + r * L.ppf;
-        page[k] = pages[pg];
-      }
-#ifdef __HIP_DEVICE_COMPILE__
-#pragma unroll
-#endif
-      for (int k = 0; k < 8; ++k) {
-        const int f = f0 + k * groups;
-        const int i = f * L.tpf + t;
-        const bool own = newest_self && f == nfr - 1;
-        if (RUN == 1) {
-          if (f < nfr && i < limit) out[i] = own ? -1 - (op.q_begin + t) : page[k] * 2 * S + slot;
-        } else if (f < nfr && i < limit) {
-          lbm_put_rows(out + i, own ? -1 - (op.q_begin + t) : page[k] * 2 * S + slot, own ? -1 : 1,
-                       n_run < limit - i ? n_run : limit - i);
-        }
-      }
-    }
+    if (RUN > 1 && h.na + h.wc <= 2 * groups)
+      lbm_plan_run<RUN, 2>(out, anchor, win, S, L, h, op.q_begin, newest_self, limit, t, n_run, pg, slot, my_group, groups);
+    else
+      lbm_plan_run<RUN, 8>(out, anchor, win, S, L, h, op.q_begin, newest_self, limit, t, n_run, pg, slot, my_group, groups);
   }
 }
+
+// Four rows at a time where pages hold whole fours: a page id, its addresses and its compares serve four rows.  Frames of
+// one token have nothing to share.  One workgroup, us a step with one row and with four: 17 frames of 1,004 tokens 9.5, 7.2,
+// 21 frames 9.9, 7.4; 261 x 17 5.6, 5.1; 65 x 17 5.3, 4.7; 5 x 101 4.6, 4.7; 4 x 17 4.4, 4.5; 10,000 x 1 7.8, 9.3.
+LBM_HD int lbm_rows_at_a_time(const lbm_cache_geom& g) { return (g.page_size & 3) == 0 && lbm_tables_layout(g).tpf >= 4 ? 4 : 1; }
 
 // build_visible_page_table + compute_last_page_len (flashinfer_cache.py:438-470) with a
 // valid length per page, plus the dense row table the attention kernel gathers through.
@@ -279,6 +298,8 @@ LBM_HD void lbm_plan_frames(int32_t* out, const int32_t* st, int S, int shift, c
 // capacity it gives instead) and publishes a count within that bound, so a host/device
 // disagreement cannot make the attention kernel read outside the table (it sets
 // LBM_TERR_KV_COUNT instead).
+// RUN: rows that a thread writes at a time, as lbm_rows_at_a_time says (0: asked here).
+template <int RUN = 0>
 LBM_HD void lbm_phase_plan(int32_t* st, const lbm_cache_geom& g, const LbmTablesLayout& L,
                            const lbm_step_op& op, int32_t* kv_rows, int32_t* page_ids,
                            int32_t* page_lens, int tid, int nthr, LbmHdr& h) {
@@ -303,10 +324,7 @@ LBM_HD void lbm_phase_plan(int32_t* st, const lbm_cache_geom& g, const LbmTables
     // token t of a page list sits in page t / S, slot t % S; page sizes are powers of two in
     // every configuration but one (page = patches per frame), so the common case is a shift
     const int shift = (S & (S - 1)) == 0 ? __builtin_ctz((unsigned)S) : -1;
-    // Four rows at a time where pages hold whole fours: a page id, its addresses and its compares serve four rows (one
-    // workgroup, us a step: 17 frames of 1,004 tokens 12.7, 8.8; frames of one token have nothing to share, 10,000 of them
-    // 7.8, 9.3).
-    if ((S & 3) == 0 && L.tpf >= 4) lbm_plan_frames<4>(out, st, S, shift, L, h, op, newest_self, limit, tid, nthr);
+    if (RUN == 4 || (RUN == 0 && lbm_rows_at_a_time(g) == 4)) lbm_plan_frames<4>(out, st, S, shift, L, h, op, newest_self, limit, tid, nthr);
     else lbm_plan_frames<1>(out, st, S, shift, L, h, op, newest_self, limit, tid, nthr);
     if (two) {
       for (int c = tid; c < h.stc; c += nthr) {

@@ -31,3 +31,16 @@ extern "C" int lbm_tables_step_host(int32_t* tables, const lbm_cache_geom* geom,
 extern "C" long long lbm_tables_words_host(const lbm_cache_geom* geom) {
   return lbm_geom_valid(*geom) ? lbm_tables_layout(*geom).words : 0;
 }
+
+// The plan phase alone as the workgroup's threads run it, one after the other.
+extern "C" int lbm_tables_plan_host(int32_t* tables, const lbm_cache_geom* geom, const lbm_step_op* op, int32_t* kv_rows, int32_t threads) {
+  if (!lbm_geom_valid(*geom)) return LBM_ERR_INVALID;
+  const LbmTablesLayout L = lbm_tables_layout(*geom);
+  int err = 0;
+  for (int t = 0; t < threads; ++t) {
+    LbmHdr h = lbm_hdr_load(tables);
+    lbm_phase_plan(tables, *geom, L, *op, kv_rows, nullptr, nullptr, t, threads, h);
+    err |= h.err;
+  }
+  return err;
+}

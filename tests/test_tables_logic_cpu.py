@@ -241,3 +241,27 @@ def test_plan_with_the_newest_frame_named_by_the_callers_rows(host_lib, page_siz
             want[first: first + T] = -1 - (b * T + np.arange(T))
             assert flagged.kv_rows[lo: lo + visible[b]].tolist() == want.tolist()
             assert flagged.hdr(b)[10] == 0
+
+
+@pytest.mark.parametrize("T,threads,frames", [(9, 64, (1, 2, 41, 42, 43)), (37, 64, (11, 12, 13, 40)), (260, 64, (2, 3, 9)), (37, 128, (24, 25)),
+                                              (4, 64, (2, 129)), (3, 64, (5, 40)), (1004, 1024, (8, 9)), (197, 1024, (40, 41))])
+@pytest.mark.parametrize("page_size", [16, 3])
+@pytest.mark.parametrize("own", [False, True])
+def test_plan_dealt_to_the_threads_of_workgroups(host_lib, T, threads, frames, page_size, own):
+    """The rows that all threads of a workgroup write, against the oracle's, on either side of the frame counts from which a
+    thread takes eight frames at a time instead of two (2 x the groups of ``ceil(T / 4)`` threads that fit), four rows and
+    one at a time, last runs of 1, 2, 3 and 4 rows; nothing is written behind the rows that the host expects."""
+    for nfr in frames:
+        pol = PagePolicy(T, 1, page_size, 1, nfr - 1, max_total_frames=nfr + 6, layout=LAYOUT_FRAME_PAGES)
+        ht = HostTables(host_lib, pol, max_total_frames=nfr + 6)
+        for _ in range(nfr + 3):       # (the window's ring has gone round)
+            pol.append_frame(); pol.evict_frames(1, nfr - 1, cross_frame_special=False)
+            ht.step([{"ops": OP_APPEND | OP_EVICT, "sliding_window": nfr - 1, "keep_tokens": 0}], append=True)
+        want = oracle_rows(pol)
+        if own:
+            want[(nfr - 1) * T:] = [-1 - (7 + t) for t in range(T)]
+        op = Op(ops=OP_PLAN | (32 if own else 0), q_begin=7, expect_kv_tokens=len(want))
+        got = np.full(len(want) + 8, -9999, dtype=np.int32)
+        p = lambda a: a.ctypes.data_as(C.c_void_p)
+        assert host_lib.lbm_tables_plan_host(p(ht.tables), C.byref(ht.g), C.byref(op), p(got), threads) == 0
+        assert got[:len(want)].tolist() == want and (got[len(want):] == -9999).all(), nfr
