@@ -1854,36 +1854,17 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
   }
 }
 
-// one 128-thread workgroup per (stream, query row, head): merge the chunks' partials (and, grid
-// z beyond the streams, store the caller's new rows: the chunks' kernel has read the pool).  Thread
-// c reads chunk c's maximum and sum (all chunks at once), the weights go through LDS, then
-// thread d sums the weighted outputs.  Bound by trips to memory: the first 32 chunks' outputs are asked for beside the
-// maxima, before a weight is known, the others' together (40 chunks of 128 floats: six trips as batches of eight behind
-// the weights, two so: 4.2 us, 4.0).
-template <int D>
-__global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeArgs a) {
-  static_assert(kDecMaxChunks <= 128 && D <= 128, "one thread per chunk, one per head dimension");
-  __shared__ float w[kDecMaxChunks];
-  __shared__ float red[2][2];
-  const int b = blockIdx.z, head = blockIdx.y, qi = blockIdx.x, tid = threadIdx.x;
-  if (b >= a.f.n_streams) {
-    for (int t = (b - a.f.n_streams) * a.max_q + qi; t < a.append_tokens; t += a.max_q * ((int)gridDim.z - a.f.n_streams)) {
-      const int row = a.append_rows[t];
-      if (row < 0 || tid >= D) continue;
-      const size_t row_elems = (size_t)a.f.num_heads * D, src = (size_t)t * row_elems + (size_t)head * D + tid;
-      float* dst = const_cast<float*>(a.f.pool) + (size_t)row * row_elems + (size_t)head * D + tid;
-      dst[0] = a.f.self_k[src];
-      dst[(size_t)a.f.page_size * row_elems] = a.f.self_v[src];
-    }
-    return;
-  }
-  const lbm_attn_stream sp = a.f.s[b];
-  if (qi >= sp.q_rows) return;
-  const int H = a.f.num_heads, nc = a.n_chunks[b];
-  const size_t stride = (size_t)sp.q_rows * H * (D + 2);      // from one chunk's partial to the next
-  const float* base = a.part + (((size_t)a.part_begin[b] + qi) * H + head) * (D + 2);
-  constexpr int kBatch = 32;
-  static_assert(kDecMaxChunks <= 2 * kBatch, "two batches hold every chunk");
+// One row's merge by the 128 threads of a workgroup.  Thread c reads chunk c's maximum and sum (all chunks at once), the
+// weights go through LDS, then thread d sums the weighted outputs.  Bound by trips to memory: the first kBatch chunks'
+// outputs are asked for beside the maxima, before a weight is known, the others' together (40 chunks of 128 floats: six
+// trips as batches of eight behind the weights 4.2 us, two so 4.0).  kBatch is the next of 8, 16 and 32 above the number of
+// chunks: loads of chunks that are not there cost their issue all the same (us a launch, always 32 and these: 8 chunks 3.9,
+// 3.45, 9 to 16 3.9, 3.6; 32 and more are the same either way).
+constexpr int kDecMergeBatch = 32;
+static_assert(kDecMaxChunks <= 2 * kDecMergeBatch, "two batches hold every chunk");
+template <int D, int kBatch>
+__device__ __forceinline__ void lbm_decode_merge_row(const float* base, size_t stride, int nc, float* out, float* w, float (*red)[2]) {
+  const int tid = threadIdx.x;
   const int d = min(tid, D - 1), c_own = min(tid, nc - 1);      // (loads outside of conditional blocks: they go out together)
   float x[kBatch], m_c = base[c_own * stride + D], l_c = base[c_own * stride + D + 1];
 #pragma unroll
@@ -1908,14 +1889,44 @@ __global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeAr
 #pragma unroll
   for (int j = 0; j < kBatch; ++j)
     if (j < nc) o += x[j] * w[j];
-  if (nc > kBatch) {
+  if (kBatch == kDecMergeBatch && nc > kBatch) {
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) x[j] = base[min(kBatch + j, nc - 1) * stride + tid];
 #pragma unroll
     for (int j = 0; j < kBatch; ++j)
       if (kBatch + j < nc) o += x[j] * w[kBatch + j];
   }
-  a.f.out[((size_t)(sp.q_begin + qi) * H + head) * D + tid] = l > 0.f ? o / l : 0.f;
+  out[tid] = l > 0.f ? o / l : 0.f;
+}
+
+// one 128-thread workgroup per (stream, query row, head) merges the chunks' partials (and, grid z beyond the streams, stores
+// the caller's new rows: the chunks' kernel has read the pool).
+template <int D>
+__global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeArgs a) {
+  static_assert(kDecMaxChunks <= 128 && D <= 128, "one thread per chunk, one per head dimension");
+  __shared__ float w[kDecMaxChunks];
+  __shared__ float red[2][2];
+  const int b = blockIdx.z, head = blockIdx.y, qi = blockIdx.x, tid = threadIdx.x;
+  if (b >= a.f.n_streams) {
+    for (int t = (b - a.f.n_streams) * a.max_q + qi; t < a.append_tokens; t += a.max_q * ((int)gridDim.z - a.f.n_streams)) {
+      const int row = a.append_rows[t];
+      if (row < 0 || tid >= D) continue;
+      const size_t row_elems = (size_t)a.f.num_heads * D, src = (size_t)t * row_elems + (size_t)head * D + tid;
+      float* dst = const_cast<float*>(a.f.pool) + (size_t)row * row_elems + (size_t)head * D + tid;
+      dst[0] = a.f.self_k[src];
+      dst[(size_t)a.f.page_size * row_elems] = a.f.self_v[src];
+    }
+    return;
+  }
+  const lbm_attn_stream sp = a.f.s[b];
+  if (qi >= sp.q_rows) return;
+  const int H = a.f.num_heads, nc = a.n_chunks[b];
+  const size_t stride = (size_t)sp.q_rows * H * (D + 2);      // from one chunk's partial to the next
+  const float* base = a.part + (((size_t)a.part_begin[b] + qi) * H + head) * (D + 2);
+  float* out = a.f.out + ((size_t)(sp.q_begin + qi) * H + head) * D;
+  if (nc <= 8) lbm_decode_merge_row<D, 8>(base, stride, nc, out, w, red);
+  else if (nc <= 16) lbm_decode_merge_row<D, 16>(base, stride, nc, out, w, red);
+  else lbm_decode_merge_row<D, kDecMergeBatch>(base, stride, nc, out, w, red);
 }
 
 // Chunks per stream for the few-query path, and the floats of partials they need.  Depends on
