@@ -78,7 +78,8 @@ class PatchConv(nn.Module):
     def forward(self, images: Tensor) -> Tensor:          # [N, 3, H, W] -> [N, patches, C]
         proj = self.proj
         if (images.dim() == 4 and type(proj) is nn.Conv2d and proj.bias is not None and proj.bias.dtype == proj.weight.dtype == images.dtype == torch.bfloat16
-                and proj.out_channels % 64 == 0 and _plain(images, proj.weight, proj.bias) and images.device == proj.bias.device
+                and proj.bias.shape == proj.weight.shape[:1] and proj.weight.shape[0] % 64 == 0
+                and _plain(images, proj.weight, proj.bias) and images.device == proj.bias.device
                 and not (proj._forward_hooks or proj._forward_pre_hooks or _global_forward_hooks or _global_forward_pre_hooks)):
             # the convolution adds its bias in a launch of its own; here the launch that brings the patches into rows does
             y = proj._conv_forward(images, proj.weight, None)

@@ -79,6 +79,16 @@ def test_patch_tokens(n, rows, cols, channels):
     assert conv.proj.bias.grad is not None
 
 
+@pytest.mark.parametrize("bias,channels", [(1, 64), (63, 64), (128, 64), (64, 128)])
+def test_patch_tokens_with_another_bias(bias, channels):
+    """A bias that is not one value per channel is refused, as the convolution refuses it, and never read by the kernel."""
+    from lingbot_map_amd.aggregator import PatchConv
+    conv = PatchConv(14, channels).cuda().to(torch.bfloat16)
+    conv.proj.bias = torch.nn.Parameter(torch.zeros(bias, device="cuda", dtype=torch.bfloat16))
+    with torch.no_grad(), pytest.raises(RuntimeError):
+        conv(torch.randn(1, 3, 28, 28, device="cuda").to(torch.bfloat16))
+
+
 def test_refusals():
     from lingbot_map_amd import _native as N
     t = torch.zeros(64, device="cuda")
