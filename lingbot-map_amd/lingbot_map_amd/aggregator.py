@@ -297,8 +297,9 @@ class HipAggregatorStream(nn.Module):
         """(images - mean) / std (base.py:335-395)."""
         mean, std = self._resnet_mean.to(images.dtype), self._resnet_std.to(images.dtype)
         H, W = images.shape[-2:]
+        # (the kernel reads one value per colour of either, whatever a replaced buffer would broadcast to)
         if (images.dtype in (torch.bfloat16, torch.float32) and _plain(images, mean, std) and images.device == mean.device == std.device
-                and H * W % 4 == 0 and images.data_ptr() % 16 == 0 and 0 < images.numel() < 1 << 32):
+                and mean.shape == std.shape == (1, 1, 3, 1, 1) and H * W % 4 == 0 and images.data_ptr() % 16 == 0 and 0 < images.numel() < 1 << 32):
             out = torch.empty_like(images)
             N.check(N.lib.lbm_normalise_images(
                 images.data_ptr(), mean.data_ptr(), std.data_ptr(), out.data_ptr(),

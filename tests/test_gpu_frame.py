@@ -61,6 +61,18 @@ def test_normalised_images(shape, dtype):
         assert torch.equal(model._normalised(wide), (wide - model._resnet_mean.to(dtype)) / model._resnet_std.to(dtype))
 
 
+@pytest.mark.parametrize("name", ["_resnet_mean", "_resnet_std"])
+@pytest.mark.parametrize("shape", [(), (1, 1, 1, 1, 1), (1, 1, 1, 14, 1), (1, 1, 1, 3, 1), (3, 1, 1), (2, 1, 3, 1, 1)])
+def test_normalised_images_with_another_mean_or_deviation(name, shape):
+    """Replaced statistics broadcast as torch broadcasts them: one value for all colours, one per row, one set per stream."""
+    from lingbot_map_amd import HipAggregatorStream
+    model = HipAggregatorStream(embed_dim=128, depth=2, num_heads=2).cuda().to(torch.bfloat16)
+    images = torch.rand(2, 1, 3, 14 if shape != (1, 1, 1, 3, 1) else 3, 28, device="cuda").to(torch.bfloat16)
+    setattr(model, name, (0.25 + torch.rand(shape, device="cuda")).to(torch.bfloat16))
+    with torch.no_grad():
+        assert torch.equal(model._normalised(images), (images - model._resnet_mean) / model._resnet_std)
+
+
 @pytest.mark.parametrize("n,rows,cols,channels", [(1, 1, 1, 64), (1, 9, 9, 1024), (2, 8, 8, 768), (3, 13, 5, 128), (1, 27, 37, 1024)])
 def test_patch_tokens(n, rows, cols, channels):
     """One patch, one short and one more than whole tiles, against the module's own operations."""
