@@ -75,21 +75,26 @@ class PatchConv(nn.Module):
         super().__init__()
         self.proj = nn.Conv2d(3, embed_dim, kernel_size=patch_size, stride=patch_size)
 
-    def forward(self, images: Tensor) -> Tensor:          # [N, 3, H, W] -> [N, patches, C]
+    def _bias_with_rows(self, images: Tensor) -> bool:
+        """Whether the launch that brings the patches into rows may add the convolution's bias, in bf16 as the convolution does
+        in a launch of its own."""
         proj = self.proj
-        if (images.dim() == 4 and type(proj) is nn.Conv2d and proj.bias is not None and proj.bias.dtype == proj.weight.dtype == images.dtype == torch.bfloat16
+        return (images.dim() == 4 and 0 < images.shape[0] < 1 << 16 and type(proj) is nn.Conv2d and proj.bias is not None
+                and proj.bias.dtype == proj.weight.dtype == images.dtype == torch.bfloat16
+                and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16)
                 and proj.bias.shape == proj.weight.shape[:1] and proj.weight.shape[0] % 64 == 0
                 and _plain(images, proj.weight, proj.bias) and images.device == proj.bias.device
-                and not (proj._forward_hooks or proj._forward_pre_hooks or _global_forward_hooks or _global_forward_pre_hooks)):
-            # the convolution adds its bias in a launch of its own; here the launch that brings the patches into rows does
-            y = proj._conv_forward(images, proj.weight, None)
-            n, channels, rows, cols = y.shape
-            if y.dtype == torch.bfloat16 and y.is_contiguous() and 0 < n < 1 << 16 and rows * cols > 0:
-                out = torch.empty(n, rows * cols, channels, dtype=y.dtype, device=y.device)
-                N.check(N.lib.lbm_patch_tokens(y.data_ptr(), proj.bias.data_ptr(), out.data_ptr(), n, channels, rows * cols, N.stream_ptr(y.device)))
-                return out
-            return (y + proj.bias.view(-1, 1, 1)).flatten(2).transpose(1, 2)
-        return proj(images).flatten(2).transpose(1, 2)
+                and not (proj._forward_hooks or proj._forward_pre_hooks or _global_forward_hooks or _global_forward_pre_hooks))
+
+    def forward(self, images: Tensor) -> Tensor:          # [N, 3, H, W] -> [N, patches, C]
+        proj = self.proj
+        if not self._bias_with_rows(images):
+            return proj(images).flatten(2).transpose(1, 2)
+        y = proj._conv_forward(images, proj.weight, None).contiguous()
+        n, channels, rows, cols = y.shape
+        out = torch.empty(n, rows * cols, channels, dtype=y.dtype, device=y.device)
+        N.check(N.lib.lbm_patch_tokens(y.data_ptr(), proj.bias.data_ptr(), out.data_ptr(), n, channels, rows * cols, N.stream_ptr(y.device)))
+        return out
 
 
 class PatchTrunk(nn.Module):

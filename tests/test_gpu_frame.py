@@ -101,6 +101,25 @@ def test_patch_tokens_with_another_bias(bias, channels):
         conv(torch.randn(1, 3, 28, 28, device="cuda").to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("autocast", [torch.float16, torch.bfloat16])
+def test_patch_tokens_under_autocast(autocast):
+    """The type that the convolution gives under autocast, and its values."""
+    from lingbot_map_amd.aggregator import PatchConv
+    conv = PatchConv(14, 128).cuda().to(torch.bfloat16)
+    images = torch.randn(2, 3, 42, 28, device="cuda").to(torch.bfloat16)
+    with torch.no_grad(), torch.autocast("cuda", dtype=autocast):
+        want = conv.proj(images).flatten(2).transpose(1, 2)
+        got = conv(images)
+        assert got.dtype == want.dtype == autocast and torch.equal(got, want)
+
+
+def test_patch_tokens_of_no_image():
+    from lingbot_map_amd.aggregator import PatchConv
+    conv = PatchConv(14, 64).cuda().to(torch.bfloat16)
+    with torch.no_grad():
+        assert conv(torch.empty(0, 3, 28, 42, device="cuda", dtype=torch.bfloat16)).shape == (0, 6, 64)
+
+
 def test_refusals():
     from lingbot_map_amd import _native as N
     t = torch.zeros(64, device="cuda")
