@@ -87,7 +87,9 @@ class PatchConv(nn.Module):
                 and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16)
                 and proj.bias.shape == proj.weight.shape[:1] and proj.weight.shape[0] % 64 == 0
                 and _plain(images, proj.weight, proj.bias) and images.device == proj.bias.device
-                and not (proj._forward_hooks or proj._forward_pre_hooks or _global_forward_hooks or _global_forward_pre_hooks))
+                and not (proj._forward_hooks or proj._forward_pre_hooks or _global_forward_hooks or _global_forward_pre_hooks)
+                # (a method wrapped on the instance, or a compiled call)
+                and not ("forward" in proj.__dict__ or "_conv_forward" in proj.__dict__ or proj._compiled_call_impl is not None))
 
     def forward(self, images: Tensor) -> Tensor:          # [N, 3, H, W] -> [N, patches, C]
         proj = self.proj

@@ -113,6 +113,19 @@ def test_patch_tokens_under_autocast(autocast):
         assert got.dtype == want.dtype == autocast and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("name", ["forward", "_conv_forward", "_compiled_call_impl"])
+def test_patch_tokens_with_a_method_of_the_instance(name):
+    """A wrapper set on the convolution itself is what a call of it runs."""
+    from lingbot_map_amd.aggregator import PatchConv
+    conv = PatchConv(14, 64).cuda().to(torch.bfloat16)
+    images = torch.randn(1, 3, 28, 28, device="cuda").to(torch.bfloat16)
+    own = conv.proj.forward if name == "_compiled_call_impl" else getattr(conv.proj, name)
+    with torch.no_grad():
+        plain = conv.proj(images).flatten(2).transpose(1, 2)
+        setattr(conv.proj, name, lambda *args: 2 * own(*args))
+        assert torch.equal(conv(images), 2 * plain)
+
+
 def test_patch_tokens_of_no_image():
     from lingbot_map_amd.aggregator import PatchConv
     conv = PatchConv(14, 64).cuda().to(torch.bfloat16)
