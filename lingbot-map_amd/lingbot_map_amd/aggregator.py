@@ -76,13 +76,14 @@ class PatchConv(nn.Module):
         self.proj = nn.Conv2d(3, embed_dim, kernel_size=patch_size, stride=patch_size)
 
     def _bias_with_rows(self, images: Tensor) -> bool:
-        """Whether the launch that brings the patches into rows may add the convolution's bias, in bf16 as the convolution does
-        in a launch of its own."""
+        """Whether the launch that brings the patches into rows may add the convolution's bias: to sums that are rounded to bf16,
+        as the convolution library does in a launch of its own (torch's own convolution, with the library switched off, adds
+        it before it rounds)."""
         proj = self.proj
         # somebody traces: no question about a proxy's values, no call that is none of torch's
         if type(images) is not Tensor or torch.compiler.is_compiling() or torch.jit.is_tracing():
             return False
-        return (images.dim() == 4 and 0 < images.shape[0] < 1 << 16 and type(proj) is nn.Conv2d and proj.bias is not None
+        return (torch.backends.cudnn.enabled and images.dim() == 4 and 0 < images.shape[0] < 1 << 16 and type(proj) is nn.Conv2d and proj.bias is not None
                 and proj.bias.dtype == proj.weight.dtype == images.dtype == torch.bfloat16
                 and not (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16)
                 and proj.bias.shape == proj.weight.shape[:1] and proj.weight.shape[0] % 64 == 0

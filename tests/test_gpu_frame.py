@@ -126,6 +126,17 @@ def test_patch_tokens_with_a_method_of_the_instance(name):
         assert torch.equal(conv(images), 2 * plain)
 
 
+@pytest.mark.parametrize("n,rows,cols,channels", [(1, 16, 16, 1024), (2, 27, 37, 128)])
+def test_patch_tokens_of_another_convolution(n, rows, cols, channels):
+    """With the convolution library switched off the bits are those of torch's own convolution, which need not round before
+    its bias."""
+    from lingbot_map_amd.aggregator import PatchConv
+    conv = PatchConv(14, channels).cuda().to(torch.bfloat16)
+    images = torch.randn(n, 3, 14 * rows, 14 * cols, device="cuda").to(torch.bfloat16)
+    with torch.no_grad(), torch.backends.cudnn.flags(enabled=False):
+        assert torch.equal(conv(images), conv.proj(images).flatten(2).transpose(1, 2))
+
+
 def test_patch_tokens_of_no_image():
     from lingbot_map_amd.aggregator import PatchConv
     conv = PatchConv(14, 64).cuda().to(torch.bfloat16)
