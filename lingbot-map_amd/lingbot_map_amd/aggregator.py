@@ -368,7 +368,7 @@ class HipAggregatorStream(nn.Module):
         """``stream_table`` as the blocks read it: complex64, one copy per stream, ``[streams, 1, frames * P, D / 2]``."""
         rope, f0 = self.rope3d, self.total_frames_processed
         if (type(rope) is RotaryPositionEmbedding3D and type(self).stream_table is HipAggregatorStream.stream_table
-                and torch.device(device).type == "cuda" and 0 <= f0 and f0 + frames <= rope.max_seq_len):
+                and "stream_table" not in self.__dict__ and torch.device(device).type == "cuda" and 0 <= f0 and f0 + frames <= rope.max_seq_len):
             angles, later, _ = self._table_base(frames, H // self.patch_size, W // self.patch_size, device)
             if _plain(angles, later) and angles.dtype == later.dtype == torch.float64 and angles.device == later.device and angles.numel():
                 table = torch.empty(streams, 1, *angles.shape, dtype=torch.complex64, device=angles.device)

@@ -47,6 +47,19 @@ def test_stream_table(frames, rows, cols, streams, f0, dtype):
     assert got.shape == want.shape and got.is_contiguous() and torch.equal(torch.view_as_real(got), torch.view_as_real(want.contiguous()))
 
 
+def test_stream_table_of_the_instance():
+    """A ``stream_table`` set on the model itself is the one that the blocks and the replayed frames take."""
+    from lingbot_map_amd import HipAggregatorStream
+    from lingbot_map_amd.aggregator import _graph_table
+    model = HipAggregatorStream(embed_dim=128, depth=2, num_heads=2, enable_3d_rope=True, num_streams=2).cuda().to(torch.bfloat16)
+    own = model.stream_table
+    model.stream_table = lambda *args, **kwargs: own(*args, **kwargs).conj()
+    with torch.no_grad():
+        want = own(1, 28, 42, "cuda:0").conj().to(torch.complex64).expand(2, -1, -1, -1)
+        assert torch.equal(torch.view_as_real(model._stream_table64(1, 28, 42, "cuda:0", 2)), torch.view_as_real(want.resolve_conj()))
+        assert torch.equal(_graph_table(model, (28, 42), "cuda:0"), torch.view_as_real(want[:1].resolve_conj()))
+
+
 @pytest.mark.parametrize("shape", [(1, 1, 3, 14, 14), (2, 3, 3, 28, 42), (1, 1, 3, 378, 518), (1, 1, 3, 7, 9)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_normalised_images(shape, dtype):
