@@ -28,6 +28,8 @@ from typing import List, Optional, Sequence, Tuple, Union
 import torch
 from torch import Tensor, nn
 from torch.nn.modules.module import _global_forward_hooks, _global_forward_pre_hooks
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from .block import (HipPagedBlock, PositionGetter, RotaryPositionEmbedding2D, RotaryPositionEmbedding3D)
 from .manager import HipPagedKVCacheManager
@@ -40,8 +42,12 @@ _RESNET_STD = (0.229, 0.224, 0.225)
 
 def _plain(*tensors: Tensor) -> bool:
     """Whether a kernel may take the place of torch operations on ``tensors``: contiguous GPU tensors of no subclass and
-    under no transform, and nobody who follows the operations (autograd in either direction, a trace)."""
-    return not (torch.is_grad_enabled() or torch.jit.is_tracing() or torch.autograd.forward_ad._current_level >= 0) and all(
+    under no transform, and nobody who follows the operations (autograd in either direction, a trace, a mode that counts or
+    records them)."""
+    return not (torch.compiler.is_compiling() or torch.is_grad_enabled() or torch.jit.is_tracing()
+                or torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
+                # (a default device is a mode too, and says nothing about tensors that are there)
+                or (torch._C._len_torch_function_stack() and any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()))) and all(
         type(t) in (Tensor, nn.Parameter) and t.is_cuda and t.is_contiguous()
         and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
 

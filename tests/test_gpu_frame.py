@@ -157,6 +157,66 @@ def test_patch_tokens_of_no_image():
         assert conv(torch.empty(0, 3, 28, 42, device="cuda", dtype=torch.bfloat16)).shape == (0, 6, 64)
 
 
+class _Dispatched(torch.utils._python_dispatch.TorchDispatchMode):
+    def __init__(self, seen):
+        super().__init__()
+        self.seen = seen
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.seen.append(func.overloadpacket.__name__)
+        return func(*args, **(kwargs or {}))
+
+
+class _Called(torch.overrides.TorchFunctionMode):
+    def __init__(self, seen):
+        super().__init__()
+        self.seen = seen
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen.append(func.__name__)
+        return func(*args, **(kwargs or {}))
+
+
+def _native_calls(monkeypatch, *names):
+    """How often each of the library's entry points is called."""
+    from lingbot_map_amd import _native as N
+    count = dict.fromkeys(names, 0)
+    for name in names:
+        def counted(*args, name=name, own=getattr(N.lib, name)):
+            count[name] += 1
+            return own(*args)
+        monkeypatch.setattr(N.lib, name, counted)
+    return count
+
+
+@pytest.mark.parametrize("mode", [_Dispatched, _Called])
+def test_modes_see_the_operations(mode, monkeypatch):
+    """Inside a mode that counts or records torch's operations they are torch's, with the same results; a default device,
+    which is a mode as well, changes nothing."""
+    from lingbot_map_amd import HipAggregatorStream
+    from lingbot_map_amd.aggregator import _group_outputs
+    model = HipAggregatorStream(embed_dim=128, depth=2, num_heads=2, enable_3d_rope=True).cuda().to(torch.bfloat16)
+    images = torch.rand(1, 1, 3, 28, 42, device="cuda").to(torch.bfloat16)
+    f, g = (torch.randn(1, 1, 6, 128, device="cuda").to(torch.bfloat16) for _ in range(2))
+    count = _native_calls(monkeypatch, "lbm_normalise_images", "lbm_patch_tokens", "lbm_group_outputs", "lbm_stream_table")
+
+    def run():
+        return (model._normalised(images), model.patch_embed(images[0]), _group_outputs([(f, g)])[0],
+                torch.view_as_real(model._stream_table64(1, 28, 42, "cuda:0", 1)))
+
+    with torch.no_grad():
+        want = run()
+        assert set(count.values()) == {1}
+        with torch.device("cuda"):
+            again = run()
+        assert set(count.values()) == {2} and all(torch.equal(a, b) for a, b in zip(again, want))
+        seen = []
+        with mode(seen):
+            got = run()
+        assert set(count.values()) == {2} and all(torch.equal(a, b) for a, b in zip(got, want))
+    assert all(any(op in name for name in seen) for op in ("sub", "div", "conv", "cat", "polar")), seen
+
+
 def test_refusals():
     from lingbot_map_amd import _native as N
     t = torch.zeros(64, device="cuda")
