@@ -52,25 +52,93 @@ def _plain(*tensors: Tensor) -> bool:
         and not torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
 
 
-def _group_outputs(pairs: List[Tuple[Tensor, Tensor]], stacked: bool = False) -> Union[List[Tensor], Tensor]:
-    """``torch.cat([f, g], dim=-1)`` of every pair, ``[B, S, P, C]`` each (base.py:600-604), in one launch for up to
-    ``N.MAX_GROUPS`` pairs; ``stacked``: as one tensor ``[pairs, B, S, P, 2C]``."""
-    parts = [t for pair in pairs for t in pair]
+def _one_launch(parts: List[Tensor]) -> bool:
+    """Whether ``lbm_group_outputs`` may concatenate these parts, the two of a group one behind the other."""
     first = parts[0] if parts else None
-    if not (parts and _plain(*parts) and all(t.shape == first.shape and t.dtype == first.dtype and t.device == first.device
-                                             and t.data_ptr() % 16 == 0 for t in parts)
-            and 0 < first.numel() * first.element_size() < 1 << 34 and first.shape[-1] * first.element_size() % 16 == 0):
-        outs = [torch.cat(pair, dim=-1) for pair in pairs]
-        return torch.stack(outs) if stacked else outs
-    shape = (*first.shape[:-1], 2 * first.shape[-1])
-    whole = first.new_empty(len(pairs), *shape) if stacked else None
-    outs = list(whole.unbind(0)) if stacked else [first.new_empty(shape) for _ in pairs]
-    for i in range(0, len(pairs), N.MAX_GROUPS):
+    return bool(parts) and _plain(*parts) and all(t.shape == first.shape and t.dtype == first.dtype and t.device == first.device
+                                                  and t.data_ptr() % 16 == 0 for t in parts) \
+        and 0 < first.numel() * first.element_size() < 1 << 34 and first.shape[-1] * first.element_size() % 16 == 0
+
+
+def _concatenate(parts: List[Tensor], outs: List[Tensor]) -> None:
+    first = parts[0]
+    for i in range(0, len(outs), N.MAX_GROUPS):
         o, t = outs[i:i + N.MAX_GROUPS], parts[2 * i:2 * (i + N.MAX_GROUPS)]
         N.check(N.lib.lbm_group_outputs((C.c_void_p * len(t))(*[x.data_ptr() for x in t]), (C.c_void_p * len(o))(*[x.data_ptr() for x in o]),
                                         len(o), first.numel() // first.shape[-1], first.shape[-1] * first.element_size(),
                                         N.stream_ptr(first.device)))
+
+
+def _group_outputs(pairs: List[Tuple[Tensor, Tensor]], stacked: bool = False) -> Union[List[Tensor], Tensor]:
+    """``torch.cat([f, g], dim=-1)`` of every pair, ``[B, S, P, C]`` each (base.py:600-604), in one launch for up to
+    ``N.MAX_GROUPS`` pairs; ``stacked``: as one tensor ``[pairs, B, S, P, 2C]``."""
+    parts = [t for pair in pairs for t in pair]
+    if not _one_launch(parts):
+        outs = [torch.cat(pair, dim=-1) for pair in pairs]
+        return torch.stack(outs) if stacked else outs
+    shape = (*parts[0].shape[:-1], 2 * parts[0].shape[-1])
+    whole = parts[0].new_empty(len(pairs), *shape) if stacked else None
+    outs = list(whole.unbind(0)) if stacked else [parts[0].new_empty(shape) for _ in pairs]
+    _concatenate(parts, outs)
     return whole if stacked else outs
+
+
+def _only_reads(block: nn.Module) -> bool:
+    """Whether a block leaves the tokens that it is handed as they are: one of this package's, with nobody else's code called
+    on them (a replaced block may work in place)."""
+    own = lambda m: not (m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ or m._compiled_call_impl is not None)
+    return (type(block) is HipPagedBlock and own(block) and type(block.norm1) is nn.LayerNorm and own(block.norm1)
+            and not (_global_forward_hooks or _global_forward_pre_hooks))
+
+
+class _GroupOutputs:
+    """The outputs of a call's chosen groups, in as few launches as a bounded number of bytes of their parts allows: the parts
+    of a frame's four groups of 1,004 tokens are 16 MB, those of 24 groups of eight such frames 790 MB beside results of
+    the same size."""
+    HELD_BYTES = 32 << 20
+
+    def __init__(self, groups: int, stacked: bool) -> None:
+        self.groups, self.stacked = groups, stacked
+        self.held: List[Tuple[Tensor, Tensor]] = []
+        self.handed_on = False                  # the tokens that the next block is handed are held
+        self.outs: List[Tensor] = []
+        self.whole: Optional[Tensor] = None     # stacked: what the outputs so far are entries of
+
+    def add(self, pairs: List[Tuple[Tensor, Tensor]]) -> None:
+        """One chosen group's."""
+        self.held += pairs
+        self.handed_on = True
+        if sum(t.numel() * t.element_size() for pair in self.held for t in pair) >= self.HELD_BYTES:
+            self.put_together()
+
+    def before(self, block: nn.Module) -> None:
+        """``block`` runs next."""
+        if self.handed_on and self.held and not _only_reads(block):
+            self.put_together()
+        self.handed_on = False
+
+    def put_together(self) -> None:
+        held, self.held = self.held, []
+        if not held:
+            return
+        done, parts = len(self.outs), [t for pair in held for t in pair]
+        if self.stacked and _one_launch(parts) and (done == 0 or self.whole is not None):
+            shape = (*parts[0].shape[:-1], 2 * parts[0].shape[-1])
+            if done == 0:
+                self.whole = parts[0].new_empty(self.groups, *shape)
+            if self.whole.shape[1:] == shape and self.whole.dtype == parts[0].dtype and done + len(held) <= len(self.whole):
+                outs = list(self.whole[done:done + len(held)].unbind(0))
+                _concatenate(parts, outs)
+                self.outs += outs
+                return
+        self.whole = None
+        self.outs += _group_outputs(held)
+
+    def result(self) -> Union[List[Tensor], Tensor]:
+        self.put_together()
+        if not self.stacked:
+            return self.outs
+        return self.whole if self.whole is not None and len(self.outs) == len(self.whole) else torch.stack(self.outs)
 
 
 class PatchConv(nn.Module):
@@ -407,7 +475,8 @@ class HipAggregatorStream(nn.Module):
         manager = self._get_manager(tokens.device, tokens.dtype, P)
         scale_frames = self.num_frame_for_scale if num_frame_for_scale is None else num_frame_for_scale
         frame_idx = global_idx = 0
-        chosen: List[Tuple[Tensor, Tensor]] = []
+        groups = sum(selected_idx is None or g in selected_idx for g in range(self.aa_block_num)) if stacked else 0
+        chosen = _GroupOutputs(groups * self.aa_block_size, stacked)
         # the blocks in the order they run: each one's last residual kernel also applies the norm1
         # of the block after it, so only the first block of a call launches a LayerNorm of its own
         order = [blocks[i] for g in range(self.aa_block_num) for kind, blocks in
@@ -419,6 +488,7 @@ class HipAggregatorStream(nn.Module):
             nonlocal step
             nxt = order[step + 1].norm1 if step + 1 < len(order) else None
             assert order[step] is block
+            chosen.before(block)
             step += 1
             if nxt is None:
                 return block(tokens, normed=normed, **kw), None
@@ -464,8 +534,8 @@ class HipAggregatorStream(nn.Module):
                     if first_group and pos3d is None and not getattr(manager, "_skip_append", False):
                         self.total_frames_processed += S
             if selected_idx is None or group in selected_idx:
-                chosen += zip(frame_out, global_out)
-        return _group_outputs(chosen, stacked), self.patch_start_idx
+                chosen.add(list(zip(frame_out, global_out)))
+        return chosen.result(), self.patch_start_idx
 
 
 def _graph_table(model: HipAggregatorStream, hw: Tuple[int, int], device) -> Tensor:

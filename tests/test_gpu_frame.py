@@ -30,6 +30,45 @@ def test_group_outputs(pairs, shape, dtype):
     assert (f.grad == 1).all() and (g.grad == 1).all()
 
 
+@pytest.mark.parametrize("selected", [None, [0, 2, 3]])
+def test_group_outputs_of_a_call(selected, monkeypatch):
+    """The chosen groups' parts are held up to a number of bytes: one launch for all groups of a small frame, one per group
+    where the bound is passed each time, the same bits, as a list and as one tensor; and where the parts are not held the
+    call's peak is lower by them."""
+    from lingbot_map_amd import HipAggregatorStream
+    from lingbot_map_amd.aggregator import _GroupOutputs
+    torch.manual_seed(1)
+    model = HipAggregatorStream(embed_dim=128, depth=16, num_heads=2, aa_block_size=2, kv_cache_sliding_window=4, kv_cache_scale_frames=1,
+                                page_size=16, layout="frame_pages").cuda().to(torch.bfloat16).eval()
+    images = torch.rand(1, 1, 3, 14 * 9, 14 * 13, device="cuda").to(torch.bfloat16)
+    count = _native_calls(monkeypatch, "lbm_group_outputs")
+    groups = 8 if selected is None else len(selected)
+    results, launches, peaks = [], [], []
+    for held in (1 << 30, 0):
+        monkeypatch.setattr(_GroupOutputs, "HELD_BYTES", held)
+        for stacked in (False, True):
+            model.clean_kv_cache()
+            with torch.no_grad():
+                model(images, selected_idx=selected, stacked=stacked)     # (whatever is kept is there)
+                model.clean_kv_cache()
+                before = count["lbm_group_outputs"]
+                torch.cuda.synchronize()
+                torch.cuda.reset_peak_memory_stats()
+                base = torch.cuda.memory_allocated()
+                out = model(images, selected_idx=selected, stacked=stacked)[0]
+                peaks.append(torch.cuda.max_memory_allocated() - base)
+            assert torch.is_tensor(out) == stacked and len(out) == 2 * groups
+            launches.append(count["lbm_group_outputs"] - before)
+            results.append(list(out))
+            del out
+    assert launches == [1, 1, groups, groups]
+    assert all(torch.equal(a, b) for r in results[1:] for a, b in zip(r, results[0]))
+    part = 2 * 128 * (9 * 13 + 6)
+    # All 4 x groups parts are there at the held call's peak, beside all results.  The other's peak is inside a block, beside its
+    # scratch memory: less than half of them here.  (Of three groups the parts are less than the call's other memory.)
+    assert peaks[0] - peaks[2] >= (2 * groups * part if selected is None else 0), peaks
+
+
 @pytest.mark.parametrize("frames,rows,cols,streams", [(1, 16, 16, 1), (1, 27, 37, 4), (8, 3, 5, 1)])
 @pytest.mark.parametrize("f0", [0, 1, 9_999])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
