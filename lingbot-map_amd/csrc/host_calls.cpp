@@ -110,4 +110,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "lbm_host", nullptr, -1, kMethods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_lbm_host() { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit_lbm_host() {
+  PyObject* module = PyModule_Create(&kModule);
+  // (the layout of lbm_attn_call that attend fills in)
+  if (module && PyModule_AddIntConstant(module, "ABI_VERSION", LBM_ABI_VERSION) != 0) Py_CLEAR(module);
+  return module;
+}

@@ -185,6 +185,8 @@ def _load_host():
     loader = importlib.machinery.ExtensionFileLoader("lbm_host", HOST_PATH)
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader("lbm_host", loader))
     loader.exec_module(module)
+    if getattr(module, "ABI_VERSION", None) != ABI_VERSION:
+        raise RuntimeError(f"{HOST_PATH}: built for ABI version {getattr(module, 'ABI_VERSION', None)}, binding expects {ABI_VERSION}")
     return module
 
 

@@ -46,6 +46,8 @@ def _build_host() -> None:
 
 def build(verbose: bool = False) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
+    if os.path.exists(HOST_PATH):      # (built last: no old one is left beside a new library)
+        os.remove(HOST_PATH)
     cmd = [HIPCC, *FLAGS, "-o", LIB_PATH, *[os.path.join(CSRC, s) for s in SOURCES]]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     out = "\n".join(l for l in proc.stdout.splitlines() if "not a recognized feature" not in l)

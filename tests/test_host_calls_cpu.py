@@ -29,3 +29,31 @@ def test_the_extension_module_has_no_thread_locals():
     assert elf[:5] == b"\x7fELF\x02"
     at, (size, count) = struct.unpack_from("<Q", elf, 32)[0], struct.unpack_from("<HH", elf, 54)
     assert count > 0 and all(struct.unpack_from("<I", elf, at + i * size)[0] != 7 for i in range(count))
+
+
+def test_a_module_of_another_abi_version_is_refused(monkeypatch):
+    import pytest
+    from lingbot_map_amd import _native as N
+    assert N._load_host().ABI_VERSION == N.ABI_VERSION == N.lib.lbm_abi_version()
+    monkeypatch.setattr(N, "ABI_VERSION", N.ABI_VERSION + 1)
+    with pytest.raises(RuntimeError, match="ABI version"):
+        N._load_host()
+
+
+def test_a_build_that_fails_leaves_no_old_module(monkeypatch, tmp_path):
+    import pytest
+    from lingbot_map_amd import build
+    for name, value in (("LIB_DIR", str(tmp_path)), ("LIB_PATH", str(tmp_path / "lib.so")), ("HOST_PATH", str(tmp_path / "host.so"))):
+        monkeypatch.setattr(build, name, value)
+    old = tmp_path / "host.so"
+    old.write_bytes(b"old")
+    monkeypatch.setattr(build, "HIPCC", "false")
+    with pytest.raises(RuntimeError):
+        build.build()
+    assert not old.exists()
+    old.write_bytes(b"old")                        # the library is built, the module is not
+    monkeypatch.setattr(build, "HIPCC", "true")
+    monkeypatch.setenv("CXX", "false")
+    with pytest.raises(RuntimeError):
+        build.build()
+    assert not old.exists()
