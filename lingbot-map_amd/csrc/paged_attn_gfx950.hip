@@ -2393,26 +2393,29 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
         // us a launch, 16 heads, eight wavefronts, batches of eleven and these: head_dim 128, 16 tokens 4.3, 2.8; 64 4.3, 3.1; 100 4.3, 4.0;
         // 200 6.2, 5.7; head_dim 64, 100 tokens 4.2, 3.1; 400 6.2, 5.5.  (Ten: no better than eleven.)
         const int batch = (most + trips * groups - 1) / (trips * groups);
-#define LBM_DECODE_ONE_VS(NW, NB, VS)                                                                                                          \
+#define LBM_DECODE_ONE_VS(D, NW, NB, VS) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<D, NW, NB, true, VS>), grid, block, 0, stream, d);
+#define LBM_DECODE_ONE_D(D, NW, NB)                                                                                                            \
   {                                                                                                                                          \
-    if (head_dim == 64) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<64, NW, NB, true, VS>), grid, block, 0, stream, d);                     \
-    else hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<128, NW, NB, true, VS>), grid, block, 0, stream, d);                                   \
+    if (shares == 4) LBM_DECODE_ONE_VS(D, NW, NB, 4)                                                                                           \
+    else if (shares == 2) LBM_DECODE_ONE_VS(D, NW, NB, 2)                                                                                      \
+    else LBM_DECODE_ONE_VS(D, NW, NB, 1)                                                                                                       \
   }
 #define LBM_DECODE_ONE(NW, NB)                                                                                                                \
   {                                                                                                                                          \
-    if (shares == 4) LBM_DECODE_ONE_VS(NW, NB, 4)                                                                                             \
-    else if (shares == 2) LBM_DECODE_ONE_VS(NW, NB, 2)                                                                                         \
-    else LBM_DECODE_ONE_VS(NW, NB, 1)                                                                                                         \
+    if (head_dim == 64) LBM_DECODE_ONE_D(64, NW, NB)                                                                                           \
+    else LBM_DECODE_ONE_D(128, NW, NB)                                                                                                         \
   }
+        static_assert(kDecOneTokens <= 8 * 2 * kDecOneWaves * 256 / 64, "head_dim 64 needs no longer batches of sixteen wavefronts than eight");
         if (many && batch <= 6) LBM_DECODE_ONE(2 * kDecOneWaves, 6)        // (more than half a trip of sixteen)
         else if (many && batch <= 8) LBM_DECODE_ONE(2 * kDecOneWaves, 8)
-        else if (many) LBM_DECODE_ONE(2 * kDecOneWaves, kDecOneBatch)
+        else if (many) LBM_DECODE_ONE_D(128, 2 * kDecOneWaves, kDecOneBatch)
         else if (batch <= 2) LBM_DECODE_ONE(kDecOneWaves, 2)
         else if (batch <= 4) LBM_DECODE_ONE(kDecOneWaves, 4)
         else if (batch <= 6) LBM_DECODE_ONE(kDecOneWaves, 6)
         else if (batch <= 8) LBM_DECODE_ONE(kDecOneWaves, 8)
         else LBM_DECODE_ONE(kDecOneWaves, kDecOneBatch)
 #undef LBM_DECODE_ONE
+#undef LBM_DECODE_ONE_D
 #undef LBM_DECODE_ONE_VS
         return lbm_check_launch("lbm_attn_f32_decode_kernel<one chunk>");
       }
