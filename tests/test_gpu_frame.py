@@ -11,23 +11,42 @@ def ptr(t):
     return C.c_void_p(t.data_ptr())
 
 
+def _native_calls(monkeypatch, *names):
+    """How often each of the library's entry points is called."""
+    from lingbot_map_amd import _native as N
+    count = dict.fromkeys(names, 0)
+    for name in names:
+        def counted(*args, name=name, own=getattr(N.lib, name)):
+            count[name] += 1
+            return own(*args)
+        monkeypatch.setattr(N.lib, name, counted)
+    return count
+
+
 @pytest.mark.parametrize("pairs,shape,dtype", [(1, (1, 1, 1, 8), torch.bfloat16), (4, (1, 1, 261, 1024), torch.bfloat16),
                                                (3, (2, 1, 37, 768), torch.float32), (33, (1, 2, 5, 24), torch.bfloat16), (2, (1, 1, 9, 12), torch.bfloat16)])
-def test_group_outputs(pairs, shape, dtype):
+def test_group_outputs(pairs, shape, dtype, monkeypatch):
     """One pair, more than one launch takes, last workgroups that are nearly empty, rows that are no whole pieces (left to
     torch), and one tensor for all."""
+    from lingbot_map_amd import _native as N
     from lingbot_map_amd.aggregator import _group_outputs
+    count = _native_calls(monkeypatch, "lbm_group_outputs")
+    launches = -(-pairs // N.MAX_GROUPS) if shape[-1] * torch.finfo(dtype).bits // 8 % 16 == 0 else 0
     parts = [(torch.randn(shape, device="cuda").to(dtype), torch.randn(shape, device="cuda").to(dtype)) for _ in range(pairs)]
     want = [torch.cat(p, dim=-1) for p in parts]
     with torch.no_grad():
         got, whole = _group_outputs(parts), _group_outputs(parts, stacked=True)
+        assert count["lbm_group_outputs"] == 2 * launches
         apart = _group_outputs([(f.transpose(1, 2), g.transpose(1, 2)) for f, g in parts])
     assert len(got) == pairs and all(torch.equal(a, b) and a._base is None for a, b in zip(got, want))
     assert torch.equal(whole, torch.stack(want))
     assert all(torch.equal(a, torch.cat((f.transpose(1, 2), g.transpose(1, 2)), dim=-1)) for a, (f, g) in zip(apart, parts))
+    if shape[1] > 1:
+        assert count["lbm_group_outputs"] == 2 * launches      # (the transposed are not contiguous)
+    before = count["lbm_group_outputs"]
     f, g = (t.clone().requires_grad_() for t in parts[0])      # somebody differentiates: torch's own operations
     _group_outputs([(f, g)])[0].float().sum().backward()
-    assert (f.grad == 1).all() and (g.grad == 1).all()
+    assert count["lbm_group_outputs"] == before and (f.grad == 1).all() and (g.grad == 1).all()
 
 
 @pytest.mark.parametrize("selected", [None, [0, 2, 3]])
@@ -101,16 +120,19 @@ def test_stream_table_of_the_instance():
 
 @pytest.mark.parametrize("shape", [(1, 1, 3, 14, 14), (2, 3, 3, 28, 42), (1, 1, 3, 378, 518), (1, 1, 3, 7, 9)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-def test_normalised_images(shape, dtype):
+def test_normalised_images(shape, dtype, monkeypatch):
+    """The kernel's values where planes are whole fours, torch's where they are not and where images are strided."""
     from lingbot_map_amd import HipAggregatorStream
+    count = _native_calls(monkeypatch, "lbm_normalise_images")
     model = HipAggregatorStream(embed_dim=128, depth=2, num_heads=2).cuda().to(dtype)
     images = torch.rand(shape, device="cuda").to(dtype)
     images[0, 0, 0, 0, :3] = torch.tensor([float("inf"), float("-inf"), 0.0])
     with torch.no_grad():
         want = (images - model._resnet_mean.to(dtype)) / model._resnet_std.to(dtype)
-        assert torch.equal(model._normalised(images), want)
+        assert torch.equal(model._normalised(images), want) and count["lbm_normalise_images"] == (shape[-1] * shape[-2] % 4 == 0)
         wide = torch.rand(*shape[:-1], 2 * shape[-1], device="cuda").to(dtype)[..., ::2]     # strided: torch's own operations
         assert torch.equal(model._normalised(wide), (wide - model._resnet_mean.to(dtype)) / model._resnet_std.to(dtype))
+    assert count["lbm_normalise_images"] == (shape[-1] * shape[-2] % 4 == 0)
 
 
 @pytest.mark.parametrize("name", ["_resnet_mean", "_resnet_std"])
@@ -126,21 +148,22 @@ def test_normalised_images_with_another_mean_or_deviation(name, shape):
 
 
 @pytest.mark.parametrize("n,rows,cols,channels", [(1, 1, 1, 64), (1, 9, 9, 1024), (2, 8, 8, 768), (3, 13, 5, 128), (1, 27, 37, 1024)])
-def test_patch_tokens(n, rows, cols, channels):
+def test_patch_tokens(n, rows, cols, channels, monkeypatch):
     """One patch, one short and one more than whole tiles, against the module's own operations."""
     from lingbot_map_amd.aggregator import PatchConv
     conv = PatchConv(14, channels).cuda().to(torch.bfloat16)
     images = torch.randn(n, 3, 14 * rows, 14 * cols, device="cuda").to(torch.bfloat16)
     want = conv.proj(images).flatten(2).transpose(1, 2)
     with torch.no_grad():
+        count = _native_calls(monkeypatch, "lbm_patch_tokens")
         got = conv(images)
-        assert got.is_contiguous() and torch.equal(got, want)
+        assert got.is_contiguous() and torch.equal(got, want) and count["lbm_patch_tokens"] == 1
         seen = []
         handle = conv.proj.register_forward_hook(lambda m, a, o: seen.append(o.shape))
         assert torch.equal(conv(images), want) and len(seen) == 1      # somebody listens to the convolution
         handle.remove()
     conv(images).float().sum().backward()
-    assert conv.proj.bias.grad is not None
+    assert conv.proj.bias.grad is not None and count["lbm_patch_tokens"] == 1
 
 
 @pytest.mark.parametrize("bias,channels", [(1, 64), (63, 64), (128, 64), (64, 128)])
@@ -214,18 +237,6 @@ class _Called(torch.overrides.TorchFunctionMode):
     def __torch_function__(self, func, types, args=(), kwargs=None):
         self.seen.append(func.__name__)
         return func(*args, **(kwargs or {}))
-
-
-def _native_calls(monkeypatch, *names):
-    """How often each of the library's entry points is called."""
-    from lingbot_map_amd import _native as N
-    count = dict.fromkeys(names, 0)
-    for name in names:
-        def counted(*args, name=name, own=getattr(N.lib, name)):
-            count[name] += 1
-            return own(*args)
-        monkeypatch.setattr(N.lib, name, counted)
-    return count
 
 
 @pytest.mark.parametrize("mode", [_Dispatched, _Called])
