@@ -1,5 +1,5 @@
-// What stands around the blocks of a frame, one launch each: the images' normalisation, the rotary table of the frame's
-// place in the stream, the groups' outputs side by side.  A few MB each, bound by their launches and a trip to memory;
+// What stands around the blocks of a frame, one launch each: the images' normalisation, the patch convolution's bias with its
+// patches as rows, the rotary table of the frame's place in the stream, the groups' outputs side by side.  A few MB each, bound by their launches and a trip to memory;
 // as torch operations they are several launches with whole passes over memory between them.
 #include <hip/hip_runtime.h>
 #include "lbm_internal.h"

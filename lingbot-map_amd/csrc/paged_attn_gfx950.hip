@@ -68,7 +68,11 @@ constexpr int kRingRow = 64;            // bf16 per row of a K/V tile in the LDS
 constexpr int kKStride = 72;            // bf16 per row of a padded patch (Q, output transpose): 144 B, b128 reads hit 64 distinct banks
 constexpr float kHeadroom = 11.0f;      // the softmax reference is set this far above the row maxima (log2 units)
 
-constexpr int kAppendPieces = 4;        // 16-byte pieces of K and of V per thread of a workgroup that appends
+// 16-byte pieces of K and of V per thread of a workgroup that appends, in the split-KV launch.  In the short-KV launch and the
+// merging one it is one: stored past the L2 they take no longer than they did with plain stores (us, plain and these:
+// short-KV 65 rows over 325 tokens 7.0, 6.7, 261 over 4,437 20.9, 20.8, 500 over 2,000 14.8, 14.8; merge 1,004 rows over 17,068
+// 6.3, 6.1, 505 over 8,585 5.7, 5.0).
+constexpr int kAppendPieces = 4;
 
 struct AttnCore {
   const unsigned short* q;
@@ -1859,7 +1863,7 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
 // outputs are asked for beside the maxima, before a weight is known, the others' together (40 chunks of 128 floats: six
 // trips as batches of eight behind the weights 4.2 us, two so 4.0).  kBatch is the next of 8, 16 and 32 above the number of
 // chunks: loads of chunks that are not there cost their issue all the same (us a launch, always 32 and these: 8 chunks 3.9,
-// 3.45, 9 to 16 3.9, 3.6; 32 and more are the same either way).
+// 3.4, 9 to 16 3.9, 3.55; 32 and more are the same either way).
 constexpr int kDecMergeBatch = 32;
 static_assert(kDecMaxChunks <= 2 * kDecMergeBatch, "two batches hold every chunk");
 template <int D, int kBatch>
@@ -2486,9 +2490,10 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
   }
   // Own rows in order, two splits per stream: both in one workgroup, no launch to merge (lbm_attn_split's PAIR).  us, two
   // kernels and this one: 16 heads, four streams of 833 rows 28.7, 18.8, of 1,004 32.0, 22.3, of 3,000 154, 140, of 5,000
-  // 383, 361; 2 x 2,000 43.9, 34.9; 1 x 4,096 68.8, 61.0; four streams of 513 rows over 4,609 60.4, 56.1.  Up to 256 rows,
-  // which leave it half as many workgroups and those with half a load each, the two kernels stay: eight streams of 40 rows
-  // over 4,097 45.8, 54.6; 12 heads, 255 rows over 4,223 44.5, 51.9.
+  // 383, 361; 2 x 2,000 43.9, 34.9; 1 x 4,096 68.8, 61.0; four streams of 513 rows over 4,609 60.4, 56.1; from the line on,
+  // eight streams of 257 rows over 4,097 54.1, 48.8, 12 heads 51.8, 47.8, of 300 52.1, 49.2, of 448 56.8, 50.7; six of 257
+  // 58.8, 54.7; eight of 385 over 1,500 32.2, 25.9.  Up to 256 rows, which leave it half as many workgroups and those with half a
+  // load each, the two kernels stay: eight streams of 40 rows over 4,097 45.8, 54.6; 12 heads, 255 rows over 4,223 44.5, 51.9.
   bool pair = own_rows && !live_kv_tokens && append_tokens <= 0;
   for (int i = 0; i < sch.n_streams; ++i) pair = pair && sch.s[i].n_splits == 2 && 2 * sch.s[i].q_rows > kQTile;
   if (pair) {

@@ -113,10 +113,12 @@ int lbm_launch_tables(int32_t* tables, const lbm_cache_geom& g, int n_streams,
       if (rows > most_rows) most_rows = rows;
     }
   }
-  // Writing the rows is what takes time in a long plan: 0.35 us per 1,000 rows from one workgroup
-  // (24 us at 67,000 rows).  A plan that follows no other operation reads the tables only and
-  // takes one workgroup per 4,096 rows (5 us at 67,000); a step that also changes the tables is
-  // worth a second launch for its plan from about 24,000 rows on (a launch costs 3-4 us).
+  // Writing the rows is what takes time in a long plan.  A plan that follows no other operation reads the tables only and
+  // takes one workgroup per 4,096 rows: 4.5 to 5.2 us from 4,096 rows to 65,000 (per 2,048 rows the same, per 8,192 up to
+  // 0.2 more).  A step that also changes the tables needs a second launch for its plan then.  us, one launch and two: frames
+  // of 1,004 tokens, 25,100 rows 6.9, 8.6, 33,132 7.4, 8.7, 41,164 8.8, 8.7, 65,260 9.9, 8.7; frames of one token, 10,000 rows
+  // 7.4, 7.8, 20,000 9.3, 8.2, 40,000 12.9, 8.2.  The line lies between the two forms': 40,000 rows written four at a time,
+  // 13,000 written one at a time.
   constexpr int kRowsPerGroup = 4096, kSplitRows = 24576, kMostGroups = 64;
   const int groups = most_rows <= kRowsPerGroup ? 1 : (most_rows + kRowsPerGroup - 1) / kRowsPerGroup;
   const bool wide = groups > 1 && (!changes || most_rows > kSplitRows);

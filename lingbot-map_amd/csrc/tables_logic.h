@@ -266,7 +266,7 @@ LBM_HD void lbm_plan_run(int32_t* out, const int32_t* anchor, const int32_t* win
 // groups of `runs` threads, group i taking frames i, i + groups, ...: one thread would otherwise walk all frames of a
 // one-token-per-frame cache by itself (10,000 frames: 1.4 ms).  Eight frames at a time; two where four-row runs leave a
 // thread no more, since a frame that is not there costs its addresses and compares all the same (one workgroup, us a step
-// with eight and with two: 197 tokens x 17 frames 6.1, 5.2; 261 x 17 6.0, 5.1; 1,004 x 5 6.4, 5.5).
+// with eight and with two: 197 tokens x 17 frames 6.1, 5.1; 261 x 17 5.9, 5.0; 1,004 x 5 6.3, 5.3).
 template <int RUN>
 LBM_HD void lbm_plan_frames(int32_t* out, const int32_t* st, int S, int shift, const LbmTablesLayout& L, const LbmHdr& h,
                             const lbm_step_op& op, bool newest_self, int limit, int tid, int nthr) {
@@ -288,8 +288,8 @@ LBM_HD void lbm_plan_frames(int32_t* out, const int32_t* st, int S, int shift, c
 }
 
 // Four rows at a time where pages hold whole fours: a page id, its addresses and its compares serve four rows.  Frames of
-// one token have nothing to share.  One workgroup, us a step with one row and with four: 17 frames of 1,004 tokens 9.5, 7.2,
-// 21 frames 9.9, 7.4; 261 x 17 5.6, 5.1; 65 x 17 5.3, 4.7; 5 x 101 4.6, 4.7; 4 x 17 4.4, 4.5; 10,000 x 1 7.8, 9.3.
+// one token have nothing to share.  One workgroup, us a step with one row and with four: 17 frames of 1,004 tokens 9.5, 7.1,
+// 21 frames 9.9, 7.2; 261 x 17 5.6, 5.0; 65 x 17 5.3, 4.6; 5 x 101 4.6, 4.6; 4 x 17 4.4, 4.5; 10,000 x 1 7.8, 9.3.
 LBM_HD int lbm_rows_at_a_time(const lbm_cache_geom& g) { return (g.page_size & 3) == 0 && lbm_tables_layout(g).tpf >= 4 ? 4 : 1; }
 
 // build_visible_page_table + compute_last_page_len (flashinfer_cache.py:438-470) with a
