@@ -268,9 +268,10 @@ size_t lbm_linear_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t epilo
  * the next one will read - the weights of the layer that follows - names it here: the next
  * lbm_linear, lbm_linear_norm, lbm_qkv_linear_prepare or lbm_qkv_linear_prepare_norm call of the
  * calling host thread then also reads one dword of every 128-byte line of [next_read, next_read +
- * bytes) while it computes (one wavefront per workgroup that does nothing else), which leaves
- * the lines in the memory-side cache.  The hint is consumed by that one call (launches on tiles of
- * 256 columns, whatever their rows, drop it); results are the same with and without it.  The memory must be
+ * bytes) while it computes, which leaves the lines in the memory-side cache: by workgroups of their own
+ * where the launch's last round leaves 32 CUs or more without one, otherwise by one wavefront per workgroup
+ * that does nothing else (launches on tiles of 256 columns have none and drop the hint).  The hint is consumed by that
+ * one call; results are the same with and without it.  The memory must be
  * readable device memory for as long as that launch can run, replays of a captured graph
  * included.  bytes below 128 or next_read = NULL withdraws a pending hint. */
 int lbm_linear_prefetch_hint(const void* next_read, size_t bytes);
@@ -387,7 +388,8 @@ typedef struct lbm_block_call {
   int32_t rows, stats_tiles, rope_layout, keep_kv, n_streams, page_size;
                                /* keep_kv: kv_rows names rows of this call (negative entries);
                                 * n_streams 0: no attention, the caller filled its output */
-  const void* hints[4];        /* lbm_linear_prefetch_hint in front of the four GEMM launches; NULL: none */
+  const void* hints[4];        /* memory to ask for ahead (lbm_linear_prefetch_hint): what proj, fc1, fc2 and the launch behind
+                                * this block read, each asked for by the one launch before it that can do so at least cost; NULL: none */
   size_t hint_bytes[4];
   int32_t own_rows;            /* ABI 11; 1: kv_rows is as LBM_ATTN_OWN_ROWS says (with keep_kv) */
 } lbm_block_call;

@@ -225,7 +225,7 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
                              int32_t head_dim, int32_t page_size, int32_t dtype, float sm_scale,
                              void* workspace, size_t workspace_bytes, void* stream,
                              const int32_t* append_rows = nullptr, int32_t append_tokens = 0, bool append_apart = false,
-                             bool own_rows = false, bool fixed_order = false) {
+                             bool own_rows = false, bool fixed_order = false, const LbmTouch* touch = nullptr) {
   int rc = lbm_check_attn_streams(streams, n_streams, who);
   if (rc != LBM_OK) return rc;
   if (!q || !pool || !out || !kv_rows) return lbm_fail(LBM_ERR_INVALID, "%s: null q, pool, out or kv_rows", who);
@@ -245,7 +245,7 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
   if (need > 0 && (!workspace || workspace_bytes < need))
     return lbm_fail(LBM_ERR_WORKSPACE, "%s: workspace of %zu bytes, %zu needed", who, workspace_bytes, need);
   return lbm_launch_attention(q, pool, out, self_k, self_v, kv_rows, live_kv_tokens, sch, num_heads, head_dim,
-                              page_size, dtype, sm_scale, workspace, workspace_bytes, (hipStream_t)stream, append_rows, append_tokens, append_apart, own_rows);
+                              page_size, dtype, sm_scale, workspace, workspace_bytes, (hipStream_t)stream, append_rows, append_tokens, append_apart, own_rows, touch);
 }
 
 int lbm_attn_run(const void* q, const void* pool, void* out, const void* self_k,
@@ -350,28 +350,69 @@ int lbm_block_run(const lbm_block_weights* w, const lbm_block_call* c, void* str
   const int tiles = lbm_linear_stats_tiles_for(c->rows, (int)dim);
   const lbm_row_norm norm1 = {c->stats, w->qkv_colsum, c->stats_tiles, w->norm1_eps};
   const lbm_row_norm norm2 = {stats1, w->fc1_colsum, tiles, w->norm2_eps};
-  if (c->hints[0]) lbm_set_prefetch_hint(c->hints[0], c->hint_bytes[0]);
+  // Which launch asks for which of the weights ahead (hints[r] is what launch 2 + r reads, the fourth the next block's
+  // first): the nearest of the three before it that can, but rather one of 256-column tiles with idle CUs than one that
+  // would do it by wavefronts beside the computing ones.  Three, since further ahead costs more than it saves once K/V and the
+  // rows of a few streams pass through the memory-side cache in between (ms a frame, three | any before it: two streams of 1,004
+  // rows 8.82 | 9.14, three anchor frames of 666 rows 7.37 | 7.68).  The nearest, since the 64 idle CUs of a qkv launch on 128 x 128
+  // tiles, which L2 binds, take from it what asking for all of them saves (1,004 rows 5.88, by wavefronts in between 5.86);
+  // 256-column tiles leave L2 the time (qkv projection, proj, fc1, fc2 of 2,008 rows: fc1's weights asked for by proj's wavefronts
+  // 66.5 us, by the qkv launch 64.9; of 3,000 rows 87.6, 86.7).
+  int by[4] = {-1, -1, -1, -1};
+  if (c->hints[0] || c->hints[1] || c->hints[2] || c->hints[3]) {
+    bool attends = false;
+    if (c->n_streams > 0 && lbm_check_attn_streams(c->streams, c->n_streams, "lbm_block_run") == LBM_OK) {
+      LbmAttnSchedule sch;
+      lbm_attn_schedule(c->streams, c->n_streams, w->num_heads, &sch, true);
+      attends = lbm_attention_asks(sch);
+    }
+    const bool split = c->split_workspace && c->split_workspace_bytes >= lbm_linear_workspace_for(c->rows, (int)dim, w->hidden, LBM_LINEAR_BIAS_RESIDUAL);
+    const LbmAsks asks[5] = {lbm_linear_asks(c->rows, 3 * (int)dim, (int)dim, 0, w->num_heads, false), attends ? LBM_ASKS_IDLE : LBM_ASKS_NOT,
+                         lbm_linear_asks(c->rows, (int)dim, (int)dim, LBM_LINEAR_BIAS_RESIDUAL, 0, false),
+                         lbm_linear_asks(c->rows, w->hidden, (int)dim, LBM_LINEAR_BIAS_GELU, 0, false),
+                         lbm_linear_asks(c->rows, (int)dim, w->hidden, LBM_LINEAR_BIAS_RESIDUAL, 0, split)};
+    for (int r = 0; r < 4; ++r) {
+      const int first = r > 0 ? r - 1 : 0;
+      for (int l = 1 + r; l >= first && by[r] < 0; --l)
+        if (asks[l] != LBM_ASKS_NOT) by[r] = l;
+      if (by[r] >= 0 && asks[by[r]] == LBM_ASKS_WAVES)
+        for (int l = by[r] - 1; l >= first; --l)
+          if (asks[l] == LBM_ASKS_WIDE_IDLE) {
+            by[r] = l;
+            break;
+          }
+    }
+  }
+  auto hint = [&](int launch) {
+    lbm_set_prefetch_hint(nullptr, 0);
+    for (int r = 0; r < 4; ++r)
+      if (by[r] == launch) lbm_add_prefetch_hint(c->hints[r], c->hint_bytes[r]);
+  };
+  hint(0);
   int rc = lbm_qkv_linear_prepare_norm(c->a, c->stats ? &norm1 : nullptr, w->qkv_w, w->qkv_b, c->rows, (int32_t)dim, w->q_norm_w,
                                        w->q_norm_b, w->k_norm_w, w->k_norm_b, w->qk_eps, c->q_scale, c->rope_cs, c->rope_layout, q,
                                        c->keep_kv ? k : nullptr, c->keep_kv ? v : nullptr, c->pool, c->append_rows, w->num_heads, 64,
                                        c->page_size, stream);
   if (rc != LBM_OK) return rc;
   if (c->n_streams > 0) {
+    hint(1);
+    LbmTouch touch;
+    lbm_take_prefetch_hint(touch);
     rc = lbm_attn_run_impl("lbm_block_run", q, c->pool ? c->pool : k, heads, c->keep_kv ? k : nullptr, c->keep_kv ? v : nullptr,
                            c->kv_rows, c->live_kv_tokens, c->streams, c->n_streams, w->num_heads, 64, c->page_size, LBM_DTYPE_BF16,
                            0.f, c->attn_workspace, c->attn_workspace_bytes, stream, nullptr, 0, false,
-                           c->own_rows && c->keep_kv && !c->live_kv_tokens, true);
+                           c->own_rows && c->keep_kv && !c->live_kv_tokens, true, &touch);
     if (rc != LBM_OK) return rc;
   }
-  if (c->hints[1]) lbm_set_prefetch_hint(c->hints[1], c->hint_bytes[1]);
+  hint(2);
   rc = lbm_linear_norm(heads, nullptr, w->proj_w, w->proj_b, w->ls1, c->x, x1, stats1, c->rows, (int32_t)dim, (int32_t)dim,
                        LBM_LINEAR_BIAS_RESIDUAL, nullptr, 0, stream);
   if (rc != LBM_OK) return rc;
-  if (c->hints[2]) lbm_set_prefetch_hint(c->hints[2], c->hint_bytes[2]);
+  hint(3);
   rc = lbm_linear_norm(x1, &norm2, w->fc1_w, w->fc1_b, nullptr, nullptr, hidden, nullptr, c->rows, w->hidden, (int32_t)dim,
                        LBM_LINEAR_BIAS_GELU, nullptr, 0, stream);
   if (rc != LBM_OK) return rc;
-  if (c->hints[3]) lbm_set_prefetch_hint(c->hints[3], c->hint_bytes[3]);
+  hint(4);
   return lbm_linear_norm(hidden, nullptr, w->fc2_w, w->fc2_b, w->ls2, x1, c->out, c->out_stats, c->rows, (int32_t)dim, w->hidden,
                          LBM_LINEAR_BIAS_RESIDUAL, c->split_workspace, c->split_workspace_bytes, stream);
 }

@@ -6,6 +6,7 @@
 #include <stddef.h>
 #include <stdint.h>
 #include "../../include/lbm_paged_attn.h"
+#include "touch_logic.h"
 
 // Records `msg` as the calling thread's last error and returns `code`.
 int lbm_fail(int code, const char* fmt, ...);
@@ -37,7 +38,17 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
                       const void* residual, void* out, float* out_stats, int M, int N, int K, int epilogue,
                       void* workspace, size_t workspace_bytes, hipStream_t stream);
 int lbm_linear_stats_tiles_for(int M, int N);
-void lbm_set_prefetch_hint(const void* ptr, size_t bytes);
+
+void lbm_set_prefetch_hint(const void* ptr, size_t bytes);   // the calling thread's next launch asks for this alone
+void lbm_add_prefetch_hint(const void* ptr, size_t bytes);   // for this too, up to kTouchRanges ranges
+void lbm_take_prefetch_hint(LbmTouch& t);
+// The grid of a launch of `wgs` workgroups, one a CU: with t.wgs more that ask for t's ranges where its last round leaves
+// kTouchIdle CUs without work (16 or 64: within 0.5 % of a frame for most sizes, but 16 three anchor frames of 666 rows 8 % slower).
+dim3 lbm_touch_grid(LbmTouch& t, unsigned wgs);
+// How lbm_linear_norm (heads 0) or the qkv projection of so many heads would ask for a hint: not at all, by wavefronts beside the
+// computing ones, by workgroups of their own on idle CUs, and that beside tiles of 256 columns
+enum LbmAsks { LBM_ASKS_NOT, LBM_ASKS_WAVES, LBM_ASKS_IDLE, LBM_ASKS_WIDE_IDLE };
+LbmAsks lbm_linear_asks(int M, int N, int K, int epilogue, int heads, bool may_split);
 size_t lbm_linear_workspace_for(int M, int N, int K, int epilogue);
 
 int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, const void* w, const float* bias, int M, int K,
@@ -97,7 +108,9 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
                          int num_heads, int head_dim, int page_size, int dtype, float sm_scale,
                          void* workspace, size_t workspace_bytes, hipStream_t stream,
                          const int32_t* append_rows = nullptr, int append_tokens = 0, bool append_apart = false,
-                         bool own_rows = false);
+                         bool own_rows = false, const LbmTouch* touch = nullptr);
+// whether such a launch has CUs to spare for the workgroups that ask for a hint
+bool lbm_attention_asks(const LbmAttnSchedule& sch);
 
 #ifdef __HIPCC__
 // 16 or 8 bytes stored past the L2 (device scope), for results that whole lines of neighbouring lanes leave.  A kernel ends
@@ -114,6 +127,34 @@ __device__ __forceinline__ void lbm_store_through(void* dst, __attribute__((ext_
 }
 __device__ __forceinline__ void lbm_store_through(void* dst, __attribute__((ext_vector_type(2))) unsigned int v) {
   asm volatile("global_store_dwordx2 %0, %1, off sc1" : : "v"(dst), "v"(v) : "memory");
+}
+// What workgroups with blockIdx.y > 0 do, thread by thread, and, where a kernel has one (`wave`), the wavefront beside the
+// computing ones in a launch without such workgroups.  In a model every launch finds its weights in HBM - a frame walks
+// through 600 MB of them, the caches hold 256 - and the loop's steps of look-ahead cover a trip to the memory-side cache, not
+// that.  A caller that knows which memory launches behind this one will read says so, and these threads read one dword of every
+// 128-byte line of it; the lines have then travelled while the launch computed.  (Plain loads whose results the compiler sees - a load
+// whose result it does not know of could land in a register it has reused - eight in flight per lane.  The kernels call it
+// in one place, behind a branch on a scalar register: called in two, its arguments were loaded in front of the computing
+// path, 0.2 us of every launch.)
+// Workgroups of their own where CUs are idle: a wavefront beside the computing ones takes its CU's vector memory path from
+// them and may end after them, as 48 workgroups' wavefronts with 1,365 lines each did: qkv projection, proj, fc1 and fc2
+// of 86 rows 34.6 us by wavefronts (34.2 without a hint, 25.3 with the weights in the caches), 27.1 by workgroups; 261 rows
+// 33.4 -> 30.9, 566 rows 44.1 -> 41.8.
+__device__ __forceinline__ void lbm_touch(const LbmTouch& t, unsigned threads, bool wave) {
+  const LbmTouchPlace at = lbm_touch_place(t, blockIdx.x, blockIdx.y, gridDim.x, threadIdx.x, threads, wave);
+  if (!at.step) return;
+  const LbmTouchPart part = lbm_touch_part(t, at.xcd, at.xcd_shift);
+  for (unsigned from = at.first; from < part.end; from += 8u * at.step) {
+    unsigned got[8], folded = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const unsigned line = from + (unsigned)j * at.step;
+      got[j] = line < part.end ? *(const __attribute__((address_space(1))) unsigned*)lbm_touch_line(part, line) : 0u;   // (from an integer it would be a flat load)
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) folded ^= got[j];
+    asm volatile("" : : "v"(folded));
+  }
 }
 // The append as workgroups of an attention launch: workgroup `wg` of those behind the attention's copies N 16-byte
 // pieces of a K row and of the matching V row per thread (row_pieces: 16-byte pieces per row).

@@ -107,10 +107,7 @@ struct LinearArgs {
   // [M][N >> stats_shift][2], or null
   float* stats_out;
   int stats_shift;               // 6 or 7; 6 where the tiles have 64 columns
-  // memory the launch after this one will read (lbm_linear_prefetch_hint): one wavefront per workgroup of
-  // the kernels that have one beside the computing and loading ones (touch_lines) asks for it
-  const char* touch;
-  unsigned touch_lines;          // 128-byte lines
+  LbmTouch touch;                // what launches behind this one will read (lbm_linear_prefetch_hint)
   // SPLITK kernels: K summed in k_splits slices by as many workgroups per tile.  Every one
   // parks its fp32 partial tile in `split_part` and takes a ticket from the tile's counter; the
   // one that draws the last ticket sums the partials in slice order (the same sum whoever is
@@ -210,37 +207,6 @@ __device__ __forceinline__ void lbm_tile_of_workgroup(int b, int m_tiles, int n_
 
 // s_waitcnt vmcnt(N), the other counters untouched
 #define LBM_DMA_WAIT(N) __builtin_amdgcn_s_waitcnt(0x0F70 | ((N) & 15) | (((N) >> 4) << 14))
-
-// What a wavefront beside the computing ones does with a prefetch hint (lbm_linear_prefetch_hint).  It holds
-// no operand and joins no barrier (a wavefront that has ended is not waited for).  In a model every launch
-// finds its weights in HBM - a frame walks through far more weight bytes than the caches hold - and the
-// loop's steps of look-ahead do not cover that latency: the same launch takes 0.6 to 5 us longer on weights
-// that no cache holds.  A caller that knows which memory the launch AFTER this one will read says so, and
-// these wavefronts, all workgroups' together, read one dword of every 128-byte line of it: the lines are
-// then in the memory-side cache (or an L2) when that launch starts, having travelled while this one computed.
-// (plain loads whose results the compiler sees - a load whose result it does not know of could
-// land in a register it has reused: eight in flight per lane, their values folded into a word
-// that is stored only under a condition that never holds)
-__device__ __forceinline__ void touch_lines(const LinearArgs& p, int lane) {
-  unsigned folded = 0;
-  // A launch of 128 workgroups or more: an XCD's ask for the eighth of the lines that its own tiles of the next launch
-  // are likely to read (weights by rows, panels of tiles by XCD), which then also waits in its L2 (a frame of 261 rows
-  // 3.58 -> 3.55 ms, of 1,004 rows 6.61 -> 6.58).  The few of a smaller launch share all of them (86 rows 3.36 ms, 3.37
-  // by eighths).
-  const unsigned xcds = gridDim.x >= 128u ? 8u : 1u, xcd = blockIdx.x % xcds, share = (p.touch_lines + xcds - 1u) / xcds;
-  const unsigned end = min(share * (xcd + 1u), p.touch_lines), stride = (gridDim.x - xcd + xcds - 1u) / xcds * 64u;
-  for (unsigned first = share * xcd + blockIdx.x / xcds * 64u + (unsigned)lane; first < end; first += 8u * stride) {
-    unsigned got[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const unsigned line = first + (unsigned)j * stride;
-      got[j] = line < end ? *(const unsigned*)(p.touch + (size_t)line * 128) : 0u;
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) folded ^= got[j];
-  }
-  if (folded == 0x5bd1e995u && p.M < 0) p.out[lane] = (unsigned short)folded;   // (M is never negative)
-}
 
 // LNA: the statistics of a row, held by four neighbouring lanes that take every fourth (mean, M2) partial each;
 // equal-sized partials merge as mean = avg(mean_i), M2 = sum(M2_i) + n_i * sum((mean_i - mean)^2) (Chan et
@@ -428,7 +394,12 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
   const char* a_base = (const char*)(p.a + k_first);
   const char* w_base = (const char*)(p.w + (size_t)n0 * p.K + k_first);
   constexpr bool kLoaders = TN != 256;
-  if (kLoaders && wave >= kGThreads / 64 && wave < kGThreads / 64 + kGLoadWaves) {
+  // (blockIdx.y is a scalar register: nothing is loaded to know)
+  if (blockIdx.y || wave >= kGThreads / 64 + kGLoadWaves) {
+    lbm_touch(p.touch, lbm_linear_threads(TN), true);
+    return;
+  }
+  if (kLoaders && wave >= kGThreads / 64) {
     // A loading wavefront: every second KB - eight rows - of each step's operands.  The rows of a step are waited
     // for before the barrier that the computing wavefronts read them behind, and asked for behind the one that
     // frees their stage.  (M x N x K 1,004 x 3,072 x 1,024: 13.0 us with every wavefront loading its rows between
@@ -466,10 +437,6 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
       __builtin_amdgcn_s_barrier();
       if (s >= 0 && s + kStages < nk) load_step(s + kStages);
     }
-    return;
-  }
-  if (wave >= kGThreads / 64) {   // (a scalar condition: the whole wavefront branches)
-    touch_lines(p, lane);
     return;
   }
   // The loads are written as inline assembly: the compiler would otherwise wait for every
@@ -857,9 +824,10 @@ __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_
   const int m0 = mt * TM, n0 = nt * 64;
   const int nk = p.K / (2 * kKS);                          // 128-wide steps
 
-  if (wave >= kWaves) {
-    if (wave == kWaves + 2) {
-      touch_lines(p, lane);
+  if (blockIdx.y || wave >= kWaves) {
+    // (blockIdx.y is a scalar register: nothing is loaded to know)
+    if (blockIdx.y || wave == kWaves + 2) {
+      lbm_touch(p.touch, lbm_rows_threads(TM), true);
       return;
     }
     // A loading wavefront, as in the kernel above: one 64-wide half of every step, eight whole rows per load.
@@ -1099,6 +1067,11 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   int mt, nt;
   lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt);
   const int m0 = mt * BM, n0 = nt * kBN;
+
+  if (blockIdx.y) {   // (a scalar register: nothing is loaded to know)
+    lbm_touch(p.touch, lbm_big_threads(BM, ROPE), false);
+    return;
+  }
 
   // ---- staging (as in the kernel above: eight 128-byte rows per wavefront and load)
   constexpr int kPassA = BM / 64, kPassW = kBN / 64;
@@ -1528,20 +1501,62 @@ int lbm_linear_stats_tiles_for(int M, int N) {
 }
 
 namespace {
-// what the calling thread's next GEMM launch is to ask for on behalf of the launch after it
-thread_local const char* g_prefetch_hint = nullptr;
-thread_local size_t g_prefetch_hint_bytes = 0;
-void lbm_take_prefetch_hint(LinearArgs& p) {
-  p.touch = g_prefetch_hint;
-  p.touch_lines = (unsigned)(g_prefetch_hint ? g_prefetch_hint_bytes / 128 : 0);
-  g_prefetch_hint = nullptr;
-  g_prefetch_hint_bytes = 0;
-}
+// what the calling thread's next GEMM launch is to ask for on behalf of launches behind it
+thread_local LbmTouch g_prefetch_hint = {};
 }  // namespace
 
 void lbm_set_prefetch_hint(const void* ptr, size_t bytes) {
-  g_prefetch_hint = bytes >= 128 ? (const char*)ptr : nullptr;
-  g_prefetch_hint_bytes = g_prefetch_hint ? bytes : 0;
+  g_prefetch_hint = {};
+  lbm_add_prefetch_hint(ptr, bytes);
+}
+void lbm_add_prefetch_hint(const void* ptr, size_t bytes) {
+  if (!ptr || bytes < 128) return;
+  for (int r = 0; r < kTouchRanges; ++r)
+    if (!g_prefetch_hint.lines[r]) {
+      g_prefetch_hint.at[r] = (const char*)ptr;
+      g_prefetch_hint.lines[r] = (unsigned)(bytes / 128);
+      return;
+    }
+}
+void lbm_take_prefetch_hint(LbmTouch& t) {
+  t = g_prefetch_hint;
+  g_prefetch_hint = {};
+}
+dim3 lbm_touch_grid(LbmTouch& t, unsigned wgs) {
+  const int idle = lbm_idle_cus(wgs);
+  if (!t.lines[0] || idle < kTouchIdle || wgs == 0) return dim3(wgs);
+  t.wgs = (unsigned)idle;
+  return dim3(wgs, 1 + (t.wgs + wgs - 1) / wgs);
+}
+
+namespace {
+// What a launch runs as (and p's tile counts): tiles of `big` rows x 256 columns, of `rows` rows x 64, or of 128 rows x `tn`
+// (x 256: wider); `splits` slices of K.  heads: of the qkv projection, whose tiles must not straddle q | k | v.
+struct LinearForm { int big, rows, tn, splits; bool wider; };
+LinearForm lbm_linear_form(LinearArgs& p, int epilogue, int heads, bool may_split) {
+  LinearForm f = {0, 0, 0, 1, false};
+  const bool qkv = epilogue == kEpiQkvPrepare;
+  // (256 columns: four whole heads each)
+  if (qkv ? (heads & 3) == 0 : epilogue != LBM_LINEAR_BIAS_RESIDUAL) f.big = lbm_linear_big_tiles(p);
+  if (f.big) return f;
+  f.tn = lbm_linear_tiles(p);
+  if (qkv && f.tn == 128 && (heads & 1)) {   // (128 columns: an even number of heads)
+    f.tn = 64;
+    p.n_tiles = p.N / 64;
+  }
+  if (may_split) f.splits = lbm_linear_splits(p, epilogue);
+  f.rows = lbm_linear_rows_tiles(p, f.tn, f.splits);
+  f.wider = !f.rows && !qkv && f.splits == 1 && f.tn == 128 && lbm_linear_wider(p);
+  return f;
+}
+}  // namespace
+
+LbmAsks lbm_linear_asks(int M, int N, int K, int epilogue, int heads, bool may_split) {
+  LinearArgs p = {};
+  p.M = M; p.N = N; p.K = K;
+  const LinearForm f = lbm_linear_form(p, heads ? kEpiQkvPrepare : epilogue, heads, may_split);
+  if ((f.rows || f.splits == 1) && lbm_idle_cus((long long)p.m_tiles * p.n_tiles) >= kTouchIdle) return f.big || f.wider ? LBM_ASKS_WIDE_IDLE : LBM_ASKS_IDLE;
+  return f.big || f.wider ? LBM_ASKS_NOT : LBM_ASKS_WAVES;
 }
 
 int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, const float* bias, const float* gamma,
@@ -1568,13 +1583,14 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
   p.res = (const unsigned short*)residual;
   p.out = (unsigned short*)out;
   p.M = M; p.N = N; p.K = K;
-  lbm_take_prefetch_hint(p);
+  lbm_take_prefetch_hint(p.touch);
   if (int rc = lbm_set_row_norm(p, a_norm, "lbm_linear_norm")) return rc;
   const bool lna = a_norm != nullptr;
   const dim3 block(kGThreads), block_s(lbm_linear_threads(128));
+  const LinearForm f = lbm_linear_form(p, epilogue, 0, workspace && workspace_bytes >= lbm_linear_workspace_for(M, N, K, epilogue));
   if (epilogue == LBM_LINEAR_BIAS || epilogue == LBM_LINEAR_BIAS_GELU) {
-    if (const int bm = lbm_linear_big_tiles(p)) {
-      const dim3 grid_b((unsigned)(p.m_tiles * p.n_tiles));
+    if (const int bm = f.big) {
+      const dim3 grid_b = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles));
 #define LBM_BIG_LAUNCH(E, L)                                                                                         \
       {                                                                                                              \
         if (bm == 256) hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<256, E, 0, false, L>), grid_b, block, 0, stream, p); \
@@ -1589,14 +1605,13 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
       return lbm_check_launch("lbm_linear_bf16_big_kernel");
     }
   }
-  const bool wide = lbm_linear_tiles(p) == 128;
-  const int splits = workspace && workspace_bytes >= lbm_linear_workspace_for(M, N, K, epilogue) ? lbm_linear_splits(p, epilogue) : 1;
+  const int splits = f.splits;
   // (where several workgroups share a tile, one that is not its last would see the other's store; one workgroup per tile
   // would not, but what a call with a workspace accepts does not depend on which of the two its sizes give)
   if (splits > 1 && residual == out)
     return lbm_fail(LBM_ERR_INVALID, "lbm_linear_norm: with a workspace the residual may not alias out");
-  if (const int tm = lbm_linear_rows_tiles(p, wide ? 128 : 64, splits)) {
-    const dim3 grid_r((unsigned)(p.m_tiles * p.n_tiles)), block_r(lbm_rows_threads(tm));
+  if (const int tm = f.rows) {
+    const dim3 grid_r = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles)), block_r(lbm_rows_threads(tm));
 #define LBM_ROWS_LAUNCH(E, S, L)                                                                                                \
   {                                                                                                                             \
     if (S == 1 && tm == 96) hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<E, 96, 1, 0, false, L>), grid_r, block_r, 0, stream, p); \
@@ -1623,8 +1638,8 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
     hipLaunchKernelGGL((lbm_linear_bf16_kernel<LBM_LINEAR_BIAS_RESIDUAL, 64, 0, false, false, true>), grid_s, block_s, 0, stream, p);
     return lbm_check_launch("lbm_linear_bf16_kernel<split K>");
   }
-  const bool wider = wide && lbm_linear_wider(p);
-  const dim3 grid((unsigned)(p.m_tiles * p.n_tiles));
+  const bool wide = f.tn == 128, wider = f.wider;
+  const dim3 grid = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles));
 #define LBM_LINEAR_LAUNCH(E, L)                                                                                  \
   {                                                                                                              \
     if (wider) hipLaunchKernelGGL((lbm_linear_bf16_kernel<E, 256, 0, false, L>), grid, block, 0, stream, p);     \
@@ -1657,7 +1672,7 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
   p.bias = bias;
   p.out = (unsigned short*)q_out;
   p.M = M; p.N = N; p.K = K;
-  lbm_take_prefetch_hint(p);
+  lbm_take_prefetch_hint(p.touch);
   p.q_norm_w = q_norm_w; p.q_norm_b = q_norm_b; p.k_norm_w = k_norm_w; p.k_norm_b = k_norm_b;
   p.rope_cs = rope_cs;
   p.k_out = (unsigned short*)k_out; p.v_out = (unsigned short*)v_out;
@@ -1670,9 +1685,9 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
   const bool lna = a_norm != nullptr;
   const int rope = !rope_cs ? 0 : (rope_layout == LBM_ROPE_INTERLEAVED ? 1 : 2);
   const bool norm = q_norm_w != nullptr;
-  // 256-wide tiles: four whole heads each, so that a tile does not straddle q | k | v
-  if (const int bm = (num_heads & 3) == 0 ? lbm_linear_big_tiles(p) : 0) {
-    const dim3 grid_b((unsigned)(p.m_tiles * p.n_tiles)), block_b(lbm_big_threads(bm, rope));
+  const LinearForm f = lbm_linear_form(p, kEpiQkvPrepare, num_heads, false);
+  if (const int bm = f.big) {
+    const dim3 grid_b = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles)), block_b(lbm_big_threads(bm, rope));
 #define LBM_QKV_BIG_M(BM, R, NRM)                                                                                               \
     {                                                                                                                           \
       if (lna) hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<BM, kEpiQkvPrepare, R, NRM, true>), grid_b, block_b, 0, stream, p);  \
@@ -1692,14 +1707,9 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
 #undef LBM_QKV_BIG_M
     return lbm_check_launch("lbm_linear_bf16_big_kernel<qkv prepare>");
   }
-  // a tile must not straddle q | k | v: 128-wide tiles need an even number of heads
-  bool wide = lbm_linear_tiles(p) == 128;
-  if (wide && (num_heads & 1)) {
-    wide = false;
-    p.n_tiles = N / 64;
-  }
-  if (const int tm = lbm_linear_rows_tiles(p, wide ? 128 : 64, 1)) {
-    const dim3 grid_r((unsigned)(p.m_tiles * p.n_tiles)), block_r(lbm_rows_threads(tm));
+  const bool wide = f.tn == 128;
+  if (const int tm = f.rows) {
+    const dim3 grid_r = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles)), block_r(lbm_rows_threads(tm));
 #define LBM_QKV_ROWS_T(T, R, NRM)                                                                                                       \
   {                                                                                                                                     \
     if (lna) hipLaunchKernelGGL((lbm_linear_bf16_rows_kernel<kEpiQkvPrepare, T, 1, R, NRM, true>), grid_r, block_r, 0, stream, p);       \
@@ -1719,7 +1729,7 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
 #undef LBM_QKV_ROWS_T
     return lbm_check_launch("lbm_linear_bf16_rows_kernel<qkv prepare>");
   }
-  const dim3 grid((unsigned)(p.m_tiles * p.n_tiles)), block(lbm_linear_threads(128));
+  const dim3 grid = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles)), block(lbm_linear_threads(128));
 #define LBM_QKV_LAUNCH_L(R, NRM, L)                                                                                   \
   {                                                                                                                   \
     if (wide) hipLaunchKernelGGL((lbm_linear_bf16_kernel<kEpiQkvPrepare, 128, R, NRM, L>), grid, block, 0, stream, p); \

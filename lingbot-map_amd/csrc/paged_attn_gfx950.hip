@@ -95,6 +95,7 @@ struct AttnCore {
 };
 struct AttnArgs : AttnCore {
   LbmAttnSchedule sch;
+  LbmTouch touch;
 };
 
 // Exchange between lane l and lane l^32.  v_permlane32_swap swaps the upper half of its first
@@ -878,6 +879,10 @@ __device__ __noinline__ void lbm_attn_pair_safe(AttnCore a, LbmAttnStreamPlan sp
 }  // namespace
 
 __global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_kernel(AttnArgs a) {
+  if (__builtin_expect(blockIdx.y, 0)) {
+    lbm_touch(a.touch, kThreads, false);
+    return;
+  }
   if ((int)blockIdx.x >= a.sch.total_wgs) {
     lbm_append_pieces<kAppendPieces>(a.self_k, a.self_v, const_cast<unsigned short*>(a.pool), a.append_rows, a.append_tokens,
                                      a.num_heads * 8, a.page_size, (int)blockIdx.x - a.sch.total_wgs, kThreads);
@@ -960,6 +965,10 @@ __global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(
   // pieces is compiled as divergent control flow)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n32 = lane & 31, g = lane >> 5;
+  if (__builtin_expect(blockIdx.y, 0)) {
+    lbm_touch(a.touch, kSmThreads, false);
+    return;
+  }
   if ((int)blockIdx.x >= a.sch.total_wgs) {
     lbm_append_pieces(a.self_k, a.self_v, const_cast<unsigned short*>(a.pool), a.append_rows, a.append_tokens, a.num_heads * 8, a.page_size,
                       (int)blockIdx.x - a.sch.total_wgs, kSmThreads);
@@ -2282,12 +2291,14 @@ size_t lbm_attn_schedule_bytes(const LbmAttnSchedule& sch, int num_heads, int he
   return split_kv > few_q ? split_kv : few_q;
 }
 
+bool lbm_attention_asks(const LbmAttnSchedule& sch) { return lbm_idle_cus(sch.total_wgs) >= kTouchIdle; }
+
 namespace {
 int lbm_launch_attention_only(const void* q, const void* pool, void* out, const void* self_k,
                               const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                               const LbmAttnSchedule& sch, int num_heads, int head_dim, int page_size, int dtype,
                               float sm_scale, void* workspace, size_t workspace_bytes, hipStream_t stream, const int32_t* append_rows,
-                              int append_tokens, bool append_apart, bool own_rows, bool* appended);
+                              int append_tokens, bool append_apart, bool own_rows, const LbmTouch* touch, bool* appended);
 }  // namespace
 
 // append_rows (lbm_attn_run_append): rows of self_k / self_v that are stored in the pool after the
@@ -2300,10 +2311,10 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
                          const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                          const LbmAttnSchedule& sch,
                          int num_heads, int head_dim, int page_size, int dtype, float sm_scale,
-                         void* workspace, size_t workspace_bytes, hipStream_t stream, const int32_t* append_rows, int append_tokens, bool append_apart, bool own_rows) {
+                         void* workspace, size_t workspace_bytes, hipStream_t stream, const int32_t* append_rows, int append_tokens, bool append_apart, bool own_rows, const LbmTouch* touch) {
   bool appended = false;
   int rc = lbm_launch_attention_only(q, pool, out, self_k, self_v, kv_rows, live_kv_tokens, sch, num_heads, head_dim,
-                                     page_size, dtype, sm_scale, workspace, workspace_bytes, stream, append_rows, append_tokens, append_apart, own_rows, &appended);
+                                     page_size, dtype, sm_scale, workspace, workspace_bytes, stream, append_rows, append_tokens, append_apart, own_rows, touch, &appended);
   if (rc != LBM_OK || !append_rows || append_tokens <= 0 || appended) return rc;
   return lbm_launch_append(self_k, self_v, dtype, const_cast<void*>(pool), dtype, append_rows, append_tokens, num_heads,
                            head_dim, page_size, stream);
@@ -2314,7 +2325,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
                               const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                               const LbmAttnSchedule& sch, int num_heads, int head_dim, int page_size, int dtype,
                               float sm_scale, void* workspace, size_t workspace_bytes, hipStream_t stream, const int32_t* append_rows,
-                              int append_tokens, bool append_apart, bool own_rows, bool* appended) {
+                              int append_tokens, bool append_apart, bool own_rows, const LbmTouch* touch, bool* appended) {
   if (head_dim != 64 && !(head_dim == 128 && dtype == LBM_DTYPE_F32))
     return lbm_fail(LBM_ERR_UNSUPPORTED, "attention kernels cover head_dim 64 (bf16, fp32) and 128 (fp32), got %d", head_dim);
   if (dtype == LBM_DTYPE_F32) {
@@ -2464,6 +2475,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
   a.append_tokens = 0;
   a.combine_blocks = 0x7fffffff;
   a.sch = sch;
+  a.touch = touch ? *touch : LbmTouch{};
   if (sch.total_wgs == 0) return LBM_OK;
   if (sch.small) {
     unsigned blocks = (unsigned)sch.total_wgs;
@@ -2475,13 +2487,13 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
     }
     bool turn = false;   // (for all streams over a cache; the kernel leaves out those with up to two pieces per wavefront, by the live count)
     for (int i = 0; i < sch.n_streams && !sch.fixed_order; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);
+    const dim3 grid = lbm_touch_grid(a.touch, blocks), block(kSmThreads);
     // (own rows in order change where rows are read from, not the order of the sums: a launch that goes round keeps its table)
     if (own_rows && !turn) {
-      if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false, true>), dim3(blocks), dim3(kSmThreads), 0, stream, a);
-      else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, false, true>), dim3(blocks), dim3(kSmThreads), 0, stream, a);
+      if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false, true>), grid, block, 0, stream, a);
+      else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, false, true>), grid, block, 0, stream, a);
       return lbm_check_launch("lbm_attn_bf16_d64_small_kernel<own rows>");
     }
-    const dim3 grid(blocks), block(kSmThreads);
     if (sch.small == 64 && turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, true>), grid, block, 0, stream, a);
     else if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false>), grid, block, 0, stream, a);
     else if (turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, true>), grid, block, 0, stream, a);
@@ -2526,7 +2538,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
     wgs += (unsigned)(((long long)append_tokens * num_heads * 8 + kThreads * kAppendPieces - 1) / (kThreads * kAppendPieces));
     *appended = true;
   }
-  hipLaunchKernelGGL(lbm_attn_bf16_d64_kernel, dim3(wgs), dim3(kThreads), 0, stream, a);
+  hipLaunchKernelGGL(lbm_attn_bf16_d64_kernel, lbm_touch_grid(a.touch, wgs), dim3(kThreads), 0, stream, a);
   int rc = lbm_check_launch("lbm_attn_bf16_d64_kernel");
   if (rc != LBM_OK) return rc;
   if (sch.part_rows > 0) {

@@ -670,16 +670,12 @@ class _NativeBlock:
 
 
 class HipPagedBlock(nn.Module):
-    #: name the next launch's weights in front of every GEMM (``lbm_linear_prefetch_hint``: a frame walks
-    #: through far more weight bytes than the caches hold, so a layer would find its own in HBM): proj's in
-    #: front of the qkv projection, fc1's in front of proj, fc2's in front of fc1, the next block's qkv weights
-    #: in front of fc2.  Captured frames, and eager ones from ``HINT_ROWS`` rows up: a block is one native call,
-    #: so that its launches follow one another (ms per eager frame without and with: 261 rows 3.74, 3.61;
-    #: 566 rows 5.32, 5.16; 1,004 rows 6.87, 6.58; four streams of 1,004 rows 16.1, 15.9), but with fewer rows
-    #: the eager frame waits for the host (86 rows: 3.32, 3.38).  A switch for measurements - results do not
-    #: depend on it.
+    #: name the weights ahead (``lbm_linear_prefetch_hint``: a frame walks through far more weight bytes than the caches
+    #: hold, so a layer would find its own in HBM): proj's, fc1's and fc2's and the next block's qkv weights, which
+    #: ``lbm_block_run`` asks for from launches before theirs.  ms per frame without and with, replayed: 86 rows 3.31,
+    #: 2.78; 261 rows 3.61, 3.22; 1,004 rows 6.74, 6.37; eager, where the frame waits for the host: 187 rows 3.51, 3.22,
+    #: 86 rows 3.26, 3.26.  A switch for measurements - results do not depend on it.
     PREFETCH_HINTS = os.environ.get("LBM_PREFETCH_HINTS", "1") != "0"
-    HINT_ROWS = 192
 
     def __init__(self, dim: int, num_heads: int, mlp_ratio: float = 4.0, qkv_bias: bool = True,
                  proj_bias: bool = True, ffn_bias: bool = True, drop: float = 0.0, attn_drop: float = 0.0,
@@ -828,7 +824,7 @@ class HipPagedBlock(nn.Module):
             if append is None:
                 return None
         hints = ((None,) * 4, (0,) * 4)
-        if self.PREFETCH_HINTS and (rows >= self.HINT_ROWS or torch.cuda.is_current_stream_capturing()):
+        if self.PREFETCH_HINTS:
             hints = native.hints_with(next_norm)
         call = N.BlockCall(
             x.data_ptr(), a.data_ptr(), stats_ptr, out.data_ptr(), None if stats_out is None else stats_out.data_ptr(),

@@ -719,3 +719,27 @@ def test_block_as_one_call_equals_its_parts(rows, kv):
                                   N.LINEAR_BIAS_RESIDUAL, p(split), split_bytes, st))
     torch.cuda.synchronize()
     assert torch.isfinite(one.float()).all() and torch.equal(pool_one, pool_parts) and torch.equal(one, parts)
+
+
+@pytest.mark.parametrize("rows", [20, 261, 600])
+def test_weights_asked_for_ahead_change_no_result(rows, monkeypatch):
+    """A block's launches ask for the weights of those behind them, the attention among them where it leaves CUs idle: a frame
+    block's and a streamed block's results with and without."""
+    from lingbot_map_amd import HipPagedBlock, HipPagedKVCacheManager
+    torch.manual_seed(rows)
+    dev, heads = torch.device("cuda:0"), 16
+    blocks = [HipPagedBlock(64 * heads, heads, init_values=0.1).to(dev, torch.bfloat16).eval() for _ in range(2)]
+    frames = [torch.randn(1, rows, 64 * heads, device=dev).to(torch.bfloat16) for _ in range(3)]
+    got = []
+    for hints in (False, True):
+        monkeypatch.setattr(HipPagedBlock, "PREFETCH_HINTS", hints)
+        m = HipPagedKVCacheManager(1, 20, rows, heads, 64, torch.bfloat16, dev, num_special_tokens=5, scale_frames=1,
+                                   sliding_window=2, max_total_frames=32, page_size=16, layout="frame_pages")
+        outs = []
+        with torch.no_grad():
+            for x in frames:
+                x, normed = blocks[0](x, next_norm=blocks[1].norm1)
+                outs.append(blocks[1](x, kv_cache=m, global_idx=0, num_frames=1, normed=normed))
+        got.append(outs)
+    for a, b in zip(*got):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b)

@@ -500,6 +500,23 @@ def test_prefetch_hint_changes_no_result(M, K, Nn, epilogue):
         assert torch.equal(outs[0], outs[1]) and torch.isfinite(outs[0].float()).all()
 
 
+@pytest.mark.parametrize("M,K,Nn,epilogue", [(1, 128, 64, "bias"), (86, 1024, 1024, "residual"), (261, 1024, 4096, "gelu"), (1004, 1024, 3072, "bias"),
+                                             (2008, 1024, 3072, "bias"), (1200, 1024, 4096, "gelu"), (900, 1024, 1024, "residual")])
+def test_prefetch_hint_by_workgroups_of_their_own(M, K, Nn, epilogue):
+    """Launches whose last round leaves 32 CUs or more idle (tiles of 32 to 256 rows) ask for a hint by further
+    workgroups, up to 255 times as many as their tiles: the results are those without a hint, bit for bit."""
+    N = _native()
+    a, w, bias, g = _inputs(M, K, Nn, seed=M + K + Nn)
+    epi = {"bias": N.LINEAR_BIAS, "gelu": N.LINEAR_BIAS_GELU, "residual": N.LINEAR_BIAS_RESIDUAL}[epilogue]
+    gamma = torch.rand(Nn, generator=g).to(torch.bfloat16) if epilogue == "residual" else None
+    res = torch.randn(M, Nn, generator=g).to(torch.bfloat16) if epilogue == "residual" else None
+    plain = run_linear(a, w, bias, epi, gamma, res)
+    ahead = torch.zeros(4_194_304, dtype=torch.bfloat16, device="cuda:0")
+    for nbytes in (ahead.numel() * 2, 100_100, 1_000, 128):
+        assert N.lib.lbm_linear_prefetch_hint(ptr(ahead), nbytes) == N.OK
+        assert torch.equal(run_linear(a, w, bias, epi, gamma, res), plain), nbytes
+
+
 @pytest.mark.parametrize("shapes", [((100, 4096, 256), (900, 4096, 1024)), ((100, 8192, 256), (900, 2304, 1024)),
                                     ((900, 2304, 1024), (100, 4096, 256), (100, 8192, 256))])
 def test_k_split_launches_of_two_shapes_share_one_workspace(shapes):
