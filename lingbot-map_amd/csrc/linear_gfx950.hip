@@ -45,6 +45,7 @@
 #include <hip/hip_runtime.h>
 #include "lbm_internal.h"
 #include "qkv_math.h"
+#include "tile_logic.h"
 
 #pragma clang fp contract(off)
 
@@ -73,15 +74,17 @@ constexpr int kKS = 64;          // K elements per LDS stage
 constexpr int kStagesG = 4;      // LDS stages: three being loaded while one is multiplied (six stages for the 64-column tile,
                                  // which has the room: slower, 8.4 -> 8.8 us for proj - the longer prologue costs more than the depth gains)
 
-struct LinearArgs {
+// what a workgroup's first loads need, in one line of the scalar cache
+struct LinearOperands {
   const unsigned short* a;       // [M, K]
   const unsigned short* w;       // [N, K]
+  int M, N, K;
+};
+struct LinearArgs : LinearOperands, LbmTiles {
   const float* bias;             // [N] or null
   const float* gamma;            // [N] LayerScale (RESIDUAL only) or null
   const unsigned short* res;     // [M, N] residual (RESIDUAL only)
   unsigned short* out;           // [M, N]
-  int M, N, K;
-  int m_tiles, n_tiles;
   // LBM_LINEAR_QKV_PREPARE: the fused pre-attention producer as the epilogue of the qkv projection
   const float* q_norm_w;         // all four null: no qk-norm
   const float* q_norm_b;
@@ -184,24 +187,6 @@ __device__ __forceinline__ void gelu_of(const f32x4 (&x)[C], const unsigned shor
   for (int c = 0; c < C; ++c)
     y[c] = __builtin_bit_cast(bf16x4, u32x2{__builtin_bit_cast(unsigned, out[2 * c]), __builtin_bit_cast(unsigned, out[2 * c + 1])});
 }
-
-// Workgroup b's tile.  Workgroups are dealt to the 8 XCDs round-robin (b % 8), 32 of a round of 256
-// to each; an XCD's 32 take consecutive tiles of an order that walks panels of 8 column tiles row
-// by row, i.e. 4 row tiles x 8 column tiles (8 x 4 in a last panel of 4): 12 operand tiles per
-// k-step for the XCD's L2 to hold instead of 17 to 33, which is what sets the latency of the
-// operand loads.  (Tiles of 64 columns x 32, 64 or 96 rows: panels of 4 or 8, see there.)
-__device__ __forceinline__ void lbm_tile_of_workgroup(int b, int m_tiles, int n_tiles, int& mt, int& nt, int panel_width = 8) {
-  const int x = b & 7, i = b >> 3;
-  const int base = (i >> 5) * 256;
-  const int in_round = min(m_tiles * n_tiles - base, 256);
-  const int t = base + x * (in_round >> 3) + min(x, in_round & 7) + (i & 31);
-  const int panel_tiles = m_tiles * panel_width;
-  const int panel = t / panel_tiles, rem = t - panel * panel_tiles;
-  const int width = min(panel_width, n_tiles - panel * panel_width);
-  mt = rem / width;
-  nt = panel * panel_width + rem - mt * width;
-}
-
 
 // ---- pieces that the kernels below share
 
@@ -355,7 +340,7 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
   {
     const int n_tiles_all = p.m_tiles * p.n_tiles;
     if (!SPLITK) {
-      lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt);
+      lbm_tile_of_workgroup((int)blockIdx.x, p, mt, nt);
     } else if ((p.n_tiles & 7) == 0) {
       const int x = blockIdx.x & 7;
       int i = blockIdx.x >> 3;
@@ -812,15 +797,7 @@ __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int mt, nt;
-  // Panels of 4 column tiles, not 8: fewer bytes for an XCD's L2 where a launch has few row tiles (us, weights rotating
-  // through 24 layers, M x N x K 261 x 1,024 x 4,096 11.2 -> 10.1, 261 x 1,024 x 1,024 5.2 -> 4.9, 261 x 3,072 x 1,024
-  // 6.4 -> 6.2).  64-row tiles whose K is long or whose rows are many are the exception: there
-  // panels of 8 keep a row of a with two XCDs instead of four (us, M x N x K, weights in HBM, panels of 4 and 8:
-  // 513 x 1,024 x 4,096 15.7, 15.8, 566 19.6, 19.5, 700 20.3, 19.9, 900 16.6, 16.6, 1,004 19.6, 19.3, at 9 to 16 row tiles, and from
-  // the last-level cache the same to 1 %; 1,004 x 896 x 3,584 17.9, 17.5; but 673 x 768 x 3,072 11.4, 11.8, 1,280 14.3, 14.4;
-  // 900 x 640 x 2,560 10.7, 11.1; 1,100 x 512 x 2,048 8.6, 9.0, 1,700 8.8, 9.1, 1,800 9.4, 9.2, 2,048 10.0, 9.5).
-  if (TM == 64 && KS > 1 && (p.K > 3072 || p.m_tiles >= 28)) lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt, 8);
-  else lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt, 4);
+  lbm_tile_of_workgroup((int)blockIdx.x, p, mt, nt);
   const int m0 = mt * TM, n0 = nt * 64;
   const int nk = p.K / (2 * kKS);                          // 128-wide steps
 
@@ -1065,7 +1042,7 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   const int rg = wave % kRowGroups, cg = wave / kRowGroups;
   const int wm = rg * (RB * 32), wn = cg * (CB * 32);       // this wavefront's corner of the tile
   int mt, nt;
-  lbm_tile_of_workgroup((int)blockIdx.x, p.m_tiles, p.n_tiles, mt, nt);
+  lbm_tile_of_workgroup((int)blockIdx.x, p, mt, nt);
   const int m0 = mt * BM, n0 = nt * kBN;
 
   if (blockIdx.y) {   // (a scalar register: nothing is loaded to know)
@@ -1530,6 +1507,19 @@ dim3 lbm_touch_grid(LbmTouch& t, unsigned wgs) {
 }
 
 namespace {
+// Panels of 4 column tiles, not 8: fewer bytes for an XCD's L2 where a launch has few row tiles (us, weights rotating
+// through 24 layers, M x N x K 261 x 1,024 x 4,096 11.2 -> 10.1, 261 x 1,024 x 1,024 5.2 -> 4.9, 261 x 3,072 x 1,024
+// 6.4 -> 6.2).  64-row tiles whose K is long or whose rows are many are the exception: there
+// panels of 8 keep a row of a with two XCDs instead of four (us, M x N x K, weights in HBM, panels of 4 and 8:
+// 513 x 1,024 x 4,096 15.7, 15.8, 566 19.6, 19.5, 700 20.3, 19.9, 900 16.6, 16.6, 1,004 19.6, 19.3, at 9 to 16 row tiles, and from
+// the last-level cache the same to 1 %; 1,004 x 896 x 3,584 17.9, 17.5; but 673 x 768 x 3,072 11.4, 11.8, 1,280 14.3, 14.4;
+// 900 x 640 x 2,560 10.7, 11.1; 1,100 x 512 x 2,048 8.6, 9.0, 1,700 8.8, 9.1, 1,800 9.4, 9.2, 2,048 10.0, 9.5).
+void lbm_linear_panels(LinearArgs& p, int rows, int splits) {
+  lbm_set_panels(p, rows && !(rows == 64 && splits > 1 && (p.K > 3072 || p.m_tiles >= 28)) ? 2 : 3);
+}
+}  // namespace
+
+namespace {
 // What a launch runs as (and p's tile counts): tiles of `big` rows x 256 columns, of `rows` rows x 64, or of 128 rows x `tn`
 // (x 256: wider); `splits` slices of K.  heads: of the qkv projection, whose tiles must not straddle q | k | v.
 struct LinearForm { int big, rows, tn, splits; bool wider; };
@@ -1538,7 +1528,10 @@ LinearForm lbm_linear_form(LinearArgs& p, int epilogue, int heads, bool may_spli
   const bool qkv = epilogue == kEpiQkvPrepare;
   // (256 columns: four whole heads each)
   if (qkv ? (heads & 3) == 0 : epilogue != LBM_LINEAR_BIAS_RESIDUAL) f.big = lbm_linear_big_tiles(p);
-  if (f.big) return f;
+  if (f.big) {
+    lbm_linear_panels(p, 0, 1);
+    return f;
+  }
   f.tn = lbm_linear_tiles(p);
   if (qkv && f.tn == 128 && (heads & 1)) {   // (128 columns: an even number of heads)
     f.tn = 64;
@@ -1547,6 +1540,7 @@ LinearForm lbm_linear_form(LinearArgs& p, int epilogue, int heads, bool may_spli
   if (may_split) f.splits = lbm_linear_splits(p, epilogue);
   f.rows = lbm_linear_rows_tiles(p, f.tn, f.splits);
   f.wider = !f.rows && !qkv && f.splits == 1 && f.tn == 128 && lbm_linear_wider(p);
+  lbm_linear_panels(p, f.rows, f.splits);
   return f;
 }
 }  // namespace
