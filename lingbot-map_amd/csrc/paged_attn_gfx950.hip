@@ -1990,8 +1990,8 @@ static size_t lbm_decode_bytes(const LbmAttnSchedule& sch, int num_heads, int he
 // tile counts per workgroup is priced with the measured costs below by simulating the
 // hand-out (streams with the longest workgroups first), and the cheapest wins.  The result
 // depends on row and tile counts only, and the last few are remembered per thread: a frame's blocks
-// alternate between two or three of them (attention within the frame, over the cache, the encoder's),
-// and pricing one takes the host 15 us with one stream and 40 us with four.
+// alternate between two or three of them (attention within the frame, over the cache, the encoder's), and pricing one
+// takes the host 1 us with one stream and 3 with four.
 namespace {
 // Costs in us, fitted to back-to-back launches at 16 heads x 64 over 100-1,374 query rows and 100-17,000
 // tokens, one to four streams (the choice is within 10 % of the best one measured in 19 of 20).  What a
@@ -2017,28 +2017,49 @@ double small_step_us(int rows, double busy) { return rows == 64 ? 0.88 + 0.30 * 
 
 // `count` workgroups of `us` each
 struct WorkgroupClass { double us; long long count; };
-// When the last of them ends, each handed to the CU (of 256) that frees up first, longest first: a binary
-// heap of finish times.
+// When the last of them ends, each handed to the CU (of 256) that frees up first, longest first.  CUs that free up at the same
+// time are one group: a class takes a whole group or the part of it that it has workgroups for, so there is at
+// most one group more per class.  (Workgroup by workgroup, through a heap of finish times, a launch not seen before took the host 12
+// to 120 us, twice in each frame of a stream that grows, now 1 to 2: five frames of 830 rows from an empty cache 340 -> 135 us,
+// eight of 1,004 rows in fp32 1,182 -> 1,149.)
 double makespan(WorkgroupClass* c, int n) {
   for (int i = 1; i < n; ++i)
     for (int j = i; j > 0 && c[j].us > c[j - 1].us; --j) { const WorkgroupClass t = c[j]; c[j] = c[j - 1]; c[j - 1] = t; }
-  double heap[256];
-  for (int i = 0; i < 256; ++i) heap[i] = 0.0;
+  struct { double at; long long cus; } g[2 * LBM_MAX_STREAMS + 2];   // by time
+  int groups = 1;
+  g[0].at = 0.0;
+  g[0].cus = 256;
   double last = 0.0;
   for (int i = 0; i < n; ++i)
-    for (long long w = 0; w < c[i].count; ++w) {
-      const double t = heap[0] + c[i].us;
-      if (t > last) last = t;
+    for (long long left = c[i].count; left > 0;) {
+      const long long cus = left < g[0].cus ? left : g[0].cus;
+      const double at = g[0].at + c[i].us;
+      if (at > last) last = at;
+      left -= cus;
+      g[0].cus -= cus;
       int k = 0;
-      for (;;) {   // replace the root and sift down
-        int m = 2 * k + 1;
-        if (m >= 256) break;
-        if (m + 1 < 256 && heap[m + 1] < heap[m]) ++m;
-        if (heap[m] >= t) break;
-        heap[k] = heap[m];
-        k = m;
+      if (g[0].cus == 0) {   // its place goes to the groups before the new one's
+        --groups;
+        for (; k < groups && g[k + 1].at < at; ++k) g[k] = g[k + 1];
+        if (k < groups && g[k + 1].at == at) {
+          g[k + 1].cus += cus;
+          for (; k < groups; ++k) g[k] = g[k + 1];
+        } else {
+          g[k].at = at;
+          g[k].cus = cus;
+          ++groups;
+        }
+      } else {
+        for (k = groups; k > 0 && g[k - 1].at > at; --k) g[k] = g[k - 1];
+        if (g[k - 1].at == at) {   // (a workgroup of no time)
+          g[k - 1].cus += cus;
+          for (; k < groups; ++k) g[k] = g[k + 1];
+        } else {
+          g[k].at = at;
+          g[k].cus = cus;
+          ++groups;
+        }
       }
-      heap[k] = t;
     }
   return last;
 }
