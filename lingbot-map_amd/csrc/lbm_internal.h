@@ -6,6 +6,7 @@
 #include <stddef.h>
 #include <stdint.h>
 #include "../../include/lbm_paged_attn.h"
+#include "tile_logic.h"
 #include "touch_logic.h"
 
 // Records `msg` as the calling thread's last error and returns `code`.
@@ -63,6 +64,7 @@ struct LbmAttnStreamPlan {
   int32_t n_qtiles, n_splits, tiles_per_split;
   int32_t wg_begin;    // first workgroup of this stream
   int32_t part_begin;  // first partial-result row (unit: q row of one split) in the workspace
+  uint32_t per_qtiles; // lbm_per(n_qtiles), for the launch
 };
 struct LbmAttnSchedule {
   int32_t n_streams;
@@ -80,7 +82,7 @@ void lbm_attn_schedule(const lbm_attn_stream* streams, int n_streams, int num_he
 // least: what a launch cannot do without; otherwise what it is fastest with
 size_t lbm_attn_schedule_bytes(const LbmAttnSchedule& sch, int num_heads, int head_dim, bool least);
 
-struct AttnArgsF32 {
+struct AttnCoreF32 {
   const float* q;
   const float* pool;
   float* out;
@@ -92,15 +94,20 @@ struct AttnArgsF32 {
   int page_size;
   float scale_log2;
   int n_streams;
-  lbm_attn_stream s[LBM_MAX_STREAMS];
-  int wg_begin[LBM_MAX_STREAMS + 1];
+  unsigned per_heads, per_eighth;   // lbm_per of the heads, and of an eighth of them where that is whole
   // the append carried by workgroups behind the attention's (LBM_ATTN_APPEND_APART; 0 tokens: none): row t of
   // self_k / self_v to pool row append_rows[t]
   const int32_t* append_rows;
   int append_tokens;
 };
+template <int S>   // room for so many streams, 1 or LBM_MAX_STREAMS (as AttnArgs of the bf16 kernels)
+struct AttnArgsF32 : AttnCoreF32 {
+  lbm_attn_stream s[S];
+  int wg_begin[S + 1];     // beyond the streams: more than any workgroup's index
+};
 // fp32 attention at head_dim 64 on bf16 matrix instructions (paged_attn_f32_gfx950.hip)
-int lbm_launch_attn_f32_d64(AttnArgsF32& a, hipStream_t stream);
+template <int S>
+int lbm_launch_attn_f32_d64(AttnArgsF32<S>& a, hipStream_t stream);
 
 int lbm_launch_attention(const void* q, const void* pool, void* out, const void* self_k,
                          const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,

@@ -45,7 +45,6 @@
 #include <hip/hip_runtime.h>
 #include "lbm_internal.h"
 #include "qkv_math.h"
-#include "tile_logic.h"
 
 #pragma clang fp contract(off)
 

@@ -118,28 +118,35 @@ __device__ __forceinline__ void mfma_split(const bf16x8 (&a)[3], const bf16x8 (&
 
 // APPEND: workgroups behind the attention's carry the append; an instance of its own, as asking which a workgroup is costs
 // every launch 0.2 to 0.4 us (400 rows over themselves: 18.3, 18.8)
-template <bool APPEND>
-__global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32 a) {
+template <int S, bool APPEND>
+__global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<S> a) {
   __shared__ __attribute__((aligned(1024))) unsigned char lds[kLdsBytes];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n32 = lane & 31, g = lane >> 5;
-  if (APPEND && (int)blockIdx.x >= a.wg_begin[LBM_MAX_STREAMS]) {
+  // (what the first loads need of the arguments, the first stream's beside the launch's, in one trip,
+  // without integer divisions behind it: 282 own rows of 8 heads 15.1 -> 14.7 us, a block of 148 rows over 740 tokens 26.4 -> 25.6)
+  lbm_attn_stream sp = a.s[0];
+  asm volatile("" : : "s"(a.q), "s"(a.pool), "s"(a.self_k), "s"(a.self_v), "s"(a.kv_rows), "s"(a.live_kv_tokens), "s"(a.num_heads), "s"(a.page_size), "s"(a.scale_log2),
+               "s"(a.n_streams), "s"(a.per_heads), "s"(a.per_eighth), "s"(sp.q_begin), "s"(sp.q_rows), "s"(sp.kv_row_begin), "s"(sp.kv_tokens),
+               "s"(APPEND ? a.wg_begin[S] : 0));
+  if (APPEND && __builtin_expect((int)blockIdx.x >= a.wg_begin[S], 0)) {
     lbm_append_pieces<kAppendPieces>(a.self_k, a.self_v, const_cast<float*>(a.pool), a.append_rows, a.append_tokens, a.num_heads * 16, a.page_size,
-                      (int)blockIdx.x - a.wg_begin[LBM_MAX_STREAMS], kThreads);
+                      (int)blockIdx.x - a.wg_begin[S], kThreads);
     return;
   }
   int b = 0;
-  for (int i = 1; i < a.n_streams; ++i)
-    if ((int)blockIdx.x >= a.wg_begin[i]) b = i;
-  const lbm_attn_stream sp = a.s[b];
+  if (S > 1 && a.n_streams > 1) {
+#pragma unroll
+    for (int i = 1; i < S; ++i) b += (int)((unsigned)(a.wg_begin[i] - 1 - (int)blockIdx.x) >> 31);   // (beyond the streams: more than any workgroup)
+    sp = a.s[b];
+  }
   const int H = a.num_heads, local = (int)blockIdx.x - a.wg_begin[b];
   int head, qt;
   if ((H & 7) == 0) {   // the query blocks of one head on one XCD (blockIdx mod 8): its L2 serves their K/V
-    head = (local >> 3) % (H >> 3) * 8 + (local & 7);
-    qt = (local >> 3) / (H >> 3);
+    qt = lbm_divide(local >> 3, H >> 3, a.per_eighth, head);
+    head = head * 8 + (local & 7);
   } else {
-    head = local % H;
-    qt = local / H;
+    qt = lbm_divide(local, H, a.per_heads, head);
   }
   const int q_row0 = qt * kRows;
   if (q_row0 >= sp.q_rows) return;   // padding between streams (whole workgroups)
@@ -423,17 +430,21 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32 
   }
 }
 
-int lbm_launch_attn_f32_d64(AttnArgsF32& a, hipStream_t stream) {
+template <int S>
+int lbm_launch_attn_f32_d64(AttnArgsF32<S>& a, hipStream_t stream) {
   int wg = 0;
-  for (int i = 0; i < LBM_MAX_STREAMS; ++i) {
+  for (int i = 0; i < S; ++i) {
     if (i < a.n_streams) wg = (wg + 7) & ~7;   // a stream starts on XCD 0, as the kernel's head -> XCD map assumes
     a.wg_begin[i] = wg;
     if (i < a.n_streams) wg += (a.s[i].q_rows + kRows - 1) / kRows * a.num_heads;
   }
-  a.wg_begin[LBM_MAX_STREAMS] = wg;
+  a.wg_begin[S] = wg;
+  for (int i = a.n_streams; i < S; ++i) a.wg_begin[i] = wg;
   if (wg == 0) return LBM_OK;
   wg += (int)(((long long)a.append_tokens * a.num_heads * 16 + kThreads * kAppendPieces - 1) / (kThreads * kAppendPieces));
-  if (a.append_tokens > 0) hipLaunchKernelGGL(lbm_attn_f32_d64_kernel<true>, dim3(wg), dim3(kThreads), 0, stream, a);
-  else hipLaunchKernelGGL(lbm_attn_f32_d64_kernel<false>, dim3(wg), dim3(kThreads), 0, stream, a);
+  if (a.append_tokens > 0) hipLaunchKernelGGL((lbm_attn_f32_d64_kernel<S, true>), dim3(wg), dim3(kThreads), 0, stream, a);
+  else hipLaunchKernelGGL((lbm_attn_f32_d64_kernel<S, false>), dim3(wg), dim3(kThreads), 0, stream, a);
   return lbm_check_launch("lbm_attn_f32_d64_kernel");
 }
+template int lbm_launch_attn_f32_d64<1>(AttnArgsF32<1>&, hipStream_t);
+template int lbm_launch_attn_f32_d64<LBM_MAX_STREAMS>(AttnArgsF32<LBM_MAX_STREAMS>&, hipStream_t);

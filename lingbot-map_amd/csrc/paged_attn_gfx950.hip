@@ -92,11 +92,41 @@ struct AttnCore {
   const int32_t* append_rows;
   int append_tokens;
   int combine_blocks;      // blocks (per stream) of that launch that merge; those beyond them append
+  unsigned per_heads, per_eighth;   // lbm_per of the heads, and of an eighth of them where that is whole
 };
+// S: streams that a launch's arguments have room for, 1 or LBM_MAX_STREAMS.  The runtime copies a launch's arguments on their way to
+// the GPU: 0.4 us of the host for 0.9 KB of them that a launch of one stream does not read (82 and 261 own rows, whose calls wait for
+// the host, 5.6 -> 5.25 and 5.7 -> 5.35 us).
+template <int S>
 struct AttnArgs : AttnCore {
-  LbmAttnSchedule sch;
+  int32_t n_streams, total_wgs;
+  LbmAttnStreamPlan s[S];
+  int32_t first_wg[S];       // s[i].wg_begin, beyond the streams more than any workgroup
   LbmTouch touch;
 };
+
+// The first stream's plan, with everything else that a workgroup's first loads need of the arguments: asked for at once.  A launch
+// finds its arguments in no cache; read where they are used - the workgroup count, the streams', the plan, the live counts'
+// address, q's, k's - they were four to six trips one behind the other, with two integer divisions in between, in front of
+// the first row's request.  us: 1,004 own rows 9.7 -> 9.2, 479 of 12 heads 6.3 -> 5.8, a block of 195 rows over 585 tokens 7.5 -> 6.9, of
+// 261 over 4,437 20.7 -> 20.3, of four streams of 280 rows 23.5 -> 22.9, a read-only frame of 285 rows over 5,455 tokens 26.0 -> 24.9.
+template <int S>
+__device__ __forceinline__ LbmAttnStreamPlan lbm_first_plan(const AttnArgs<S>& a) {
+  const LbmAttnStreamPlan sp = a.s[0];
+  asm volatile("" : : "s"(a.total_wgs), "s"(a.n_streams), "s"(a.num_heads), "s"(a.per_heads), "s"(a.per_eighth), "s"(a.live_kv_tokens), "s"(a.q),
+               "s"(a.self_k), "s"(a.self_v), "s"(a.pool), "s"(a.kv_rows), "s"(a.page_size), "s"(sp.q_begin), "s"(sp.q_rows), "s"(sp.kv_row_begin), "s"(sp.kv_tokens),
+               "s"(sp.n_qtiles), "s"(sp.n_splits), "s"(sp.tiles_per_split), "s"(sp.wg_begin), "s"(sp.per_qtiles));
+  return sp;
+}
+// A workgroup's plan where there are several streams
+template <int S>
+__device__ __forceinline__ void lbm_plan_of_workgroup(const AttnArgs<S>& a, LbmAttnStreamPlan& sp) {
+  if (S == 1 || a.n_streams == 1) return;
+  int b = 0;
+#pragma unroll
+  for (int i = 1; i < S; ++i) b += (int)((unsigned)(a.first_wg[i] - 1 - (int)blockIdx.x) >> 31);   // (no compare: its result would go by way of a vector register)
+  sp = a.s[b];
+}
 
 // Exchange between lane l and lane l^32.  v_permlane32_swap swaps the upper half of its first
 // register with the lower half of its second; fed two copies of x it leaves {x_lo, x_lo} in
@@ -189,14 +219,13 @@ __device__ __forceinline__ void lbm_attn_split(const AttnCore& a, const LbmAttnS
     // Workgroups are dealt to the 8 XCDs round-robin: keep the query tiles that share one
     // (head, split) - hence the same K/V rows - on one XCD so its L2 serves the re-reads.
     const int x = local & 7, i = local >> 3;
-    qt = i % sp.n_qtiles;
-    hs = (i / sp.n_qtiles) * 8 + x;
+    hs = lbm_divide(i, sp.n_qtiles, sp.per_qtiles, qt) * 8 + x;
   } else {
-    qt = local % sp.n_qtiles;
-    hs = local / sp.n_qtiles;
+    hs = lbm_divide(local, sp.n_qtiles, sp.per_qtiles, qt);
   }
   if (local >= sp.n_qtiles * n_hs) return;  // padding between streams
-  const int head = PAIR ? hs : hs % H, split = PAIR ? group : hs / H;
+  int head = hs, split = group;
+  if (!PAIR) split = lbm_divide(hs, H, a.per_heads, head);
   // With device-side token counts the split count stays the host's choice (it fixes the grid
   // and the workspace layout) and the tiles are dealt to the splits from the live count.
   const int kv_tokens = !OWN && a.live_kv_tokens ? a.live_kv_tokens[sp.live_at] : sp.kv_tokens;
@@ -878,37 +907,33 @@ __device__ __noinline__ void lbm_attn_pair_safe(AttnCore a, LbmAttnStreamPlan sp
 
 }  // namespace
 
-__global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_kernel(AttnArgs a) {
-  if (__builtin_expect(blockIdx.y, 0)) {
-    lbm_touch(a.touch, kThreads, false);
+template <int S>
+__global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_kernel(AttnArgs<S> a) {
+  LbmAttnStreamPlan sp = lbm_first_plan(a);
+  if (__builtin_expect((int)blockIdx.x >= a.total_wgs || blockIdx.y, 0)) {
+    if (blockIdx.y)
+      lbm_touch(a.touch, kThreads, false);
+    else
+      lbm_append_pieces<kAppendPieces>(a.self_k, a.self_v, const_cast<unsigned short*>(a.pool), a.append_rows, a.append_tokens,
+                                       a.num_heads * 8, a.page_size, (int)blockIdx.x - a.total_wgs, kThreads);
     return;
   }
-  if ((int)blockIdx.x >= a.sch.total_wgs) {
-    lbm_append_pieces<kAppendPieces>(a.self_k, a.self_v, const_cast<unsigned short*>(a.pool), a.append_rows, a.append_tokens,
-                                     a.num_heads * 8, a.page_size, (int)blockIdx.x - a.sch.total_wgs, kThreads);
-    return;
-  }
-  int b = 0;   // which stream's work is this workgroup
-  for (int i = 1; i < a.sch.n_streams; ++i)
-    if ((int)blockIdx.x >= a.sch.s[i].wg_begin) b = i;
-  const LbmAttnStreamPlan sp = a.sch.s[b];
+  lbm_plan_of_workgroup(a, sp);
   lbm_attn_split<false, false>(a, sp);
 }
 
-__global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_own_kernel(AttnArgs a) {
-  int b = 0;
-  for (int i = 1; i < a.sch.n_streams; ++i)
-    if ((int)blockIdx.x >= a.sch.s[i].wg_begin) b = i;
-  const LbmAttnStreamPlan sp = a.sch.s[b];
+template <int S>
+__global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_own_kernel(AttnArgs<S> a) {
+  LbmAttnStreamPlan sp = lbm_first_plan(a);
+  lbm_plan_of_workgroup(a, sp);
   lbm_attn_split<false, false, true>(a, sp);
 }
 
 // (its sch: n_qtiles and workgroups in tiles of 256 query rows, see the launch)
-__global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_pair_kernel(AttnArgs a) {
-  int b = 0;
-  for (int i = 1; i < a.sch.n_streams; ++i)
-    if ((int)blockIdx.x >= a.sch.s[i].wg_begin) b = i;
-  const LbmAttnStreamPlan sp = a.sch.s[b];
+template <int S>
+__global__ __launch_bounds__(kThreads, 1) void lbm_attn_bf16_d64_pair_kernel(AttnArgs<S> a) {
+  LbmAttnStreamPlan sp = lbm_first_plan(a);
+  lbm_plan_of_workgroup(a, sp);
   lbm_attn_split<false, true>(a, sp);
 }
 
@@ -957,38 +982,34 @@ static_assert(lbm_sm_lds_bytes(64) <= 160 * 1024, "LDS budget of the short-KV ke
 // OWN: token t of a stream is row kv_row_begin + t of the caller's K/V (LBM_ATTN_OWN_ROWS): the rows are asked for
 // at once, without the trip to memory for their table entries and the one through LDS for their addresses (261
 // rows 5.5 -> 5.2 us, 1,004 rows 11.4 -> 10.6, 2,000 rows 29.4 -> 26.3).
-template <int QB, bool TURN, bool OWN = false>
-__global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(AttnArgs a) {
+template <int S, int QB, bool TURN, bool OWN = false>
+__global__ __launch_bounds__(kSmThreads, 1) void lbm_attn_bf16_d64_small_kernel(AttnArgs<S> a) {
   __shared__ __attribute__((aligned(16))) unsigned char lds_raw[lbm_sm_lds_bytes(32 * QB)];
   constexpr int kRows = 32 * QB;
   // (the wavefront index is uniform by construction; said so, or the loop over this wavefront's
   // pieces is compiled as divergent control flow)
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n32 = lane & 31, g = lane >> 5;
-  if (__builtin_expect(blockIdx.y, 0)) {
-    lbm_touch(a.touch, kSmThreads, false);
-    return;
-  }
-  if ((int)blockIdx.x >= a.sch.total_wgs) {
-    lbm_append_pieces(a.self_k, a.self_v, const_cast<unsigned short*>(a.pool), a.append_rows, a.append_tokens, a.num_heads * 8, a.page_size,
-                      (int)blockIdx.x - a.sch.total_wgs, kSmThreads);
-    return;
-  }
   // ---- which (stream, 64 query rows, head)
-  int b = 0;
-  for (int i = 1; i < a.sch.n_streams; ++i)
-    if ((int)blockIdx.x >= a.sch.s[i].wg_begin) b = i;
-  const LbmAttnStreamPlan sp = a.sch.s[b];
+  LbmAttnStreamPlan sp = lbm_first_plan(a);
+  if (__builtin_expect((int)blockIdx.x >= a.total_wgs || blockIdx.y, 0)) {
+    if (blockIdx.y)
+      lbm_touch(a.touch, kSmThreads, false);
+    else
+      lbm_append_pieces(a.self_k, a.self_v, const_cast<unsigned short*>(a.pool), a.append_rows, a.append_tokens, a.num_heads * 8, a.page_size,
+                        (int)blockIdx.x - a.total_wgs, kSmThreads);
+    return;
+  }
+  lbm_plan_of_workgroup(a, sp);
   const int H = a.num_heads;
   const int local = (int)blockIdx.x - sp.wg_begin;
   int q_tile, head;
   if ((H & 7) == 0) {   // the query blocks of one head on one XCD (blockIdx mod 8): its L2 serves their K/V
     const int x = local & 7, i = local >> 3;
-    head = (i % (H >> 3)) * 8 + x;
-    q_tile = i / (H >> 3);
+    q_tile = lbm_divide(i, H >> 3, a.per_eighth, head);
+    head = head * 8 + x;
   } else {
-    head = local % H;
-    q_tile = local / H;
+    q_tile = lbm_divide(local, H, a.per_heads, head);
   }
   if (q_tile >= sp.n_qtiles) return;   // padding between streams (whole workgroups)
   const int kv_tokens = max(a.live_kv_tokens ? a.live_kv_tokens[sp.live_at] : sp.kv_tokens, 0);
@@ -1377,7 +1398,8 @@ __device__ __forceinline__ void lbm_combine_upto(const float* lse, const unsigne
   }
 }
 
-__global__ __launch_bounds__(256) void lbm_attn_combine_bf16_kernel(AttnArgs a) {
+template <int S>
+__global__ __launch_bounds__(256) void lbm_attn_combine_bf16_kernel(AttnArgs<S> a) {
   if ((int)blockIdx.x >= a.combine_blocks) {
     // The append's share of the launch (lbm_attn_run_append): the main kernel has read the pool,
     // the new frames' rows - attended to from the caller's tensors - now go into their pages.
@@ -1386,7 +1408,7 @@ __global__ __launch_bounds__(256) void lbm_attn_combine_bf16_kernel(AttnArgs a) 
                         (int)blockIdx.x - a.combine_blocks, 256);
     return;
   }
-  const LbmAttnStreamPlan sp = a.sch.s[blockIdx.y];
+  const LbmAttnStreamPlan sp = a.s[S == 1 ? 0 : blockIdx.y];
   if (sp.n_splits <= 1) return;
   const int H = a.num_heads;
   const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1441,8 +1463,7 @@ __global__ __launch_bounds__(256) void lbm_attn_combine_bf16_kernel(AttnArgs a) 
     }
   }
   const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
-  const long long r = rh / H, h = rh % H;
-  unsigned short* op = a.out + ((size_t)(sp.q_begin + r) * H + h) * 64 + d8 * 8;
+  unsigned short* op = a.out + ((size_t)sp.q_begin * H + rh) * 64 + d8 * 8;
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] *= inv;
   lbm_store_through(op, __builtin_bit_cast(u32x4, __builtin_convertvector(acc, bf16x8)));
@@ -1484,7 +1505,8 @@ __device__ __forceinline__ float max_over_lane_groups(float x) {
   return fmaxf(a, b);
 }
 
-__global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32 a) {
+template <int S>
+__global__ __launch_bounds__(512) void lbm_attn_f32_kernel(AttnArgsF32<S> a) {
   constexpr int D = 128;
   // NG groups of four waves: wave w of every group owns the same 16 query rows, group j takes
   // KV tiles j, j + NG, ... (NG waves per SIMD, so one wave's softmax, LDS waits and barriers
@@ -1705,12 +1727,15 @@ constexpr int kDecMaxChunks = 64;
 constexpr int kDecOneTokens = 512;
 constexpr int kDecOneWaves = 8, kDecChunkWaves = 4;
 
+template <int S>   // streams that there is room for
 struct DecodeArgs {
-  AttnArgsF32 f;
+  AttnArgsF32<S> f;
   float* part;                           // [sum n_chunks][q_rows][H][D + 2]
-  int n_chunks[LBM_MAX_STREAMS];
-  int part_begin[LBM_MAX_STREAMS];       // in (chunk, query row) units
+  int n_chunks[S];
+  int part_begin[S];                     // in (chunk, query row) units
+  unsigned per_chunks[S];                // lbm_per(n_chunks)
   int max_q;                             // most query rows of any stream
+  unsigned per_max_q;                    // lbm_per(max_q)
   // lbm_attn_run_append: rows of self_k / self_v that go into the pool once it has been read (NULL: none)
   const int32_t* append_rows;
   int append_tokens;
@@ -1740,8 +1765,8 @@ __device__ __forceinline__ float row_group_sum(float v) {
 // 1,024 bytes for one workgroup, 640 for each of four).  us, 16 heads, caches in HBM, VS 1, 2, 4: head_dim 128, 100
 // tokens 4.9, 4.5, 4.4; 200 8.6, 7.4, 7.0; 300 10.6, 9.2, 8.2; four streams of 300 11.7, 10.1, 9.0; eight of them 12.5,
 // 12.0, 13.6 (two workgroups per CU); head_dim 64, 300 tokens 6.8, 6.2, 5.8.
-template <int D, int NW, int NB, bool ONE, int VS = 1>
-__global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs a) {
+template <int S, int D, int NW, int NB, bool ONE, int VS = 1>
+__global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs<S> a) {
   constexpr int LPR = D / 4;         // lanes per K/V row, 16 bytes each
   constexpr int RPW = 64 / LPR;      // row groups of a wavefront
   constexpr int G = NW * RPW;        // row groups of the workgroup
@@ -1751,16 +1776,33 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
   __shared__ __attribute__((aligned(16))) float red_o[NW][DV];
   __shared__ float red_m[NW], red_l[NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int rows_of_launch = VS == 1 ? 0 : a.f.n_streams * a.max_q, vs = VS == 1 ? 0 : blockIdx.z / rows_of_launch;
-  const int z = blockIdx.z - vs * rows_of_launch;
-  const int b = z / a.max_q, qi = z % a.max_q, head = blockIdx.y, chunk = blockIdx.x;
-  lbm_attn_stream sp = a.f.s[b];
-  if (chunk >= a.n_chunks[b] || qi >= sp.q_rows) return;
+  // (what the first loads need of the arguments, the first stream's beside the launch's, in one trip and without divisions behind
+  // it: see lbm_first_plan; sixteen caches of 300 tokens of 128 floats a frame 120 -> 111 us, one of 10,000 37.8 -> 37.2)
+  lbm_attn_stream sp = a.f.s[0];
+  int n_chunks = a.n_chunks[0], part_begin = ONE ? 0 : a.part_begin[0];
+  unsigned per_chunks = ONE ? 0 : a.per_chunks[0];
+  asm volatile("" : : "s"(a.f.q), "s"(a.f.pool), "s"(a.f.self_k), "s"(a.f.self_v), "s"(a.f.kv_rows), "s"(a.f.live_kv_tokens), "s"(a.f.num_heads), "s"(a.f.page_size),
+               "s"(a.f.scale_log2), "s"(a.f.n_streams), "s"(a.max_q), "s"(a.per_max_q), "s"(sp.q_begin), "s"(sp.q_rows), "s"(sp.kv_row_begin), "s"(sp.kv_tokens), "s"(n_chunks),
+               "s"(part_begin), "s"(per_chunks));
+  const int rows_of_launch = VS == 1 ? 0 : a.f.n_streams * a.max_q;
+  int vs = 0, z = blockIdx.z, qi;
+#pragma unroll
+  for (int i = 1; i < VS; ++i)
+    if ((int)blockIdx.z >= i * rows_of_launch) vs = i, z = (int)blockIdx.z - i * rows_of_launch;
+  const int b = lbm_divide(z, a.max_q, a.per_max_q, qi), head = blockIdx.y, chunk = blockIdx.x;
+  if (S > 1 && b > 0) {
+    sp = a.f.s[b];
+    n_chunks = a.n_chunks[b];
+    part_begin = ONE ? 0 : a.part_begin[b];
+    per_chunks = ONE ? 0 : a.per_chunks[b];
+  }
+  if (chunk >= n_chunks || qi >= sp.q_rows) return;
   if (a.f.live_kv_tokens) sp.kv_tokens = max(a.f.live_kv_tokens[sp.live_at], 0);
   const int H = a.f.num_heads;
   const size_t row_elems = (size_t)H * D;
-  const int per = (sp.kv_tokens + a.n_chunks[b] - 1) / a.n_chunks[b];
-  const int t_begin = chunk * per, t_end = min(t_begin + per, sp.kv_tokens);
+  int rest = 0;
+  const int per = ONE ? sp.kv_tokens : lbm_divide(sp.kv_tokens + n_chunks - 1, n_chunks, per_chunks, rest);
+  const int t_begin = ONE ? 0 : chunk * per, t_end = min(t_begin + per, sp.kv_tokens);
   const int grp = wave * RPW + lane / LPR, ln = lane % LPR;
 
   const f32x4 q4 = *(const f32x4*)(a.f.q + ((size_t)(sp.q_begin + qi) * H + head) * D + 4 * ln) * a.f.scale_log2;
@@ -1847,7 +1889,7 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
     if (ONE) {
       a.f.out[((size_t)(sp.q_begin + qi) * H + head) * D + vs * DV + tid] = lt > 0.f ? o / lt : 0.f;   // no token: zeros
     } else {
-      float* pp = a.part + (((size_t)a.part_begin[b] + (size_t)chunk * sp.q_rows + qi) * H + head) * (D + 2);
+      float* pp = a.part + (((size_t)part_begin + (size_t)chunk * sp.q_rows + qi) * H + head) * (D + 2);
       pp[tid] = o;
       if (tid == 0) {
         pp[D] = mx;
@@ -1914,8 +1956,8 @@ __device__ __forceinline__ void lbm_decode_merge_row(const float* base, size_t s
 
 // one 128-thread workgroup per (stream, query row, head) merges the chunks' partials (and, grid z beyond the streams, stores
 // the caller's new rows: the chunks' kernel has read the pool).
-template <int D>
-__global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeArgs a) {
+template <int S, int D>
+__global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeArgs<S> a) {
   static_assert(kDecMaxChunks <= 128 && D <= 128, "one thread per chunk, one per head dimension");
   __shared__ float w[kDecMaxChunks];
   __shared__ float red[2][2];
@@ -1931,11 +1973,11 @@ __global__ __launch_bounds__(128) void lbm_attn_f32_decode_merge_kernel(DecodeAr
     }
     return;
   }
-  const lbm_attn_stream sp = a.f.s[b];
+  const lbm_attn_stream sp = a.f.s[S == 1 ? 0 : b];
   if (qi >= sp.q_rows) return;
-  const int H = a.f.num_heads, nc = a.n_chunks[b];
+  const int H = a.f.num_heads, nc = a.n_chunks[S == 1 ? 0 : b];
   const size_t stride = (size_t)sp.q_rows * H * (D + 2);      // from one chunk's partial to the next
-  const float* base = a.part + (((size_t)a.part_begin[b] + qi) * H + head) * (D + 2);
+  const float* base = a.part + (((size_t)a.part_begin[S == 1 ? 0 : b] + qi) * H + head) * (D + 2);
   float* out = a.f.out + ((size_t)(sp.q_begin + qi) * H + head) * D;
   if (nc <= 8) lbm_decode_merge_row<D, 8>(base, stride, nc, out, w, red);
   else if (nc <= 16) lbm_decode_merge_row<D, 16>(base, stride, nc, out, w, red);
@@ -2342,6 +2384,226 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
 }
 
 namespace {
+template <int S>
+int lbm_launch_f32(const AttnCoreF32& core, const LbmAttnSchedule& sch, int head_dim, void* workspace, size_t workspace_bytes, hipStream_t stream,
+                   const int32_t* append_rows, int append_tokens, bool append_apart, bool* appended) {
+  AttnArgsF32<S> f;
+  static_cast<AttnCoreF32&>(f) = core;
+  int wg = 0;
+  for (int i = 0; i < S; ++i) {
+    f.s[i] = lbm_attn_stream{0, 0, 0, 0, 0};
+    f.wg_begin[i] = wg;
+    if (i < sch.n_streams) {
+      f.s[i] = lbm_attn_stream{sch.s[i].q_begin, sch.s[i].q_rows, sch.s[i].kv_row_begin, sch.s[i].kv_tokens, sch.s[i].live_at};
+      wg += ((sch.s[i].q_rows + kF32Rows - 1) / kF32Rows) * f.num_heads;
+    }
+  }
+  f.wg_begin[S] = wg;
+  if (wg == 0) return LBM_OK;
+  if (lbm_decode_applies(sch)) {
+    DecodeArgs<S> d;
+    d.f = f;
+    d.part = (float*)workspace;
+    d.append_rows = append_tokens > 0 ? append_rows : nullptr;
+    d.append_tokens = append_tokens;
+    int max_chunks = 0, max_q = 0, min_q = kDecQ, part = 0, most = 0;
+    int fine = lbm_decode_fine_chunks(sch, f.num_heads, head_dim);
+    if (workspace_bytes < lbm_decode_bytes(sch, f.num_heads, head_dim, fine)) fine = 0;   // a workspace for chunks of 256 serves too
+    for (int i = 0; i < S; ++i) {
+      d.n_chunks[i] = 0;
+      d.part_begin[i] = part;
+      if (i < sch.n_streams) {
+        d.n_chunks[i] = lbm_decode_chunks(sch.s[i].kv_tokens, fine);
+        part += d.n_chunks[i] * sch.s[i].q_rows;
+        if (d.n_chunks[i] > max_chunks) max_chunks = d.n_chunks[i];
+        if (sch.s[i].q_rows > max_q) max_q = sch.s[i].q_rows;
+        if (sch.s[i].q_rows < min_q) min_q = sch.s[i].q_rows;
+        if (sch.s[i].kv_tokens > most) most = sch.s[i].kv_tokens;
+      }
+    }
+    if (max_q == 0) return LBM_OK;
+    d.max_q = max_q;
+    d.per_max_q = lbm_per(max_q);
+    for (int i = 0; i < sch.n_streams; ++i) d.per_chunks[i] = lbm_per(d.n_chunks[i]);
+    // One launch for short lists.  Up to two and a half trips to memory it is the faster form (us, one row of 16 heads
+    // of 128, from the last-level cache and from HBM, against the chunked form: 300 tokens 7.0 and 8.2, 9.6 and 10.8;
+    // 360 tokens 7.6 and 9.0, 8.9 and 9.9; 440 tokens 9.2 and 10.4, 9.1 and 10.3), beyond that it costs more than a
+    // second launch (500 tokens 9.2 and 10.7, 8.0 and 9.0) unless fewer chunks fit (four streams, 500 tokens 10.0 and
+    // 11.9, 11.1 and 12.4).  With one query row per stream and nothing to append beyond those rows it carries the
+    // append as well.
+    const int few = kDecOneWaves * 256 / head_dim, trip = kDecOneBatch * few;   // row groups of eight wavefronts, their tokens in flight
+    if (most <= kDecOneTokens && (fine < kDecFineChunks || most <= trip * 5 / 2)) {
+      for (int i = 0; i < sch.n_streams; ++i) d.n_chunks[i] = 1;
+      unsigned covered = 0;   // rows 0 .. n_streams - 1 of the append, each some stream's query row
+      for (int i = 0; i < sch.n_streams; ++i)
+        if (sch.s[i].q_begin < LBM_MAX_STREAMS) covered |= 1u << sch.s[i].q_begin;
+      const bool carries = d.append_rows && max_q == 1 && min_q == 1 && append_tokens == sch.n_streams &&
+                           covered == (1u << append_tokens) - 1u;
+      if (!carries) d.append_rows = nullptr;
+      else *appended = true;
+      // A row to four or two workgroups where that leaves one per CU, not for the shortest lists (16 tokens of 64
+      // floats 2.75, 2.83), and not where a row to append may be one that another workgroup still has to read.
+      const long long rows = (long long)f.num_heads * sch.n_streams * max_q;
+      const int shares = (d.append_rows && !append_apart) || most <= 32 ? 1 : rows * 4 <= 256 ? 4 : rows * 2 <= 256 ? 2 : 1;
+      // Sixteen wavefronts, each group with half as many tokens, where eight would make more than one trip (16 heads, K/V
+      // from HBM, rows of a page each, us with eight and with sixteen: head_dim 128, 150 tokens 5.2, 5.3; 200 6.2, 5.8; 300
+      // 7.2, 6.8; 440 9.4, 8.5; four streams of 300 8.5, 8.0, of 440 10.9, 10.0; head_dim 64, 300 tokens 5.1, 5.2; 400 6.0, 5.7).
+      const bool many = most > trip;
+      const int trips = many ? (most + 2 * trip - 1) / (2 * trip) : 1, groups = many ? 2 * few : few;
+      const dim3 grid(1, f.num_heads, sch.n_streams * max_q * shares), block((many ? 2 : 1) * kDecOneWaves * 64);
+      // As few trips as batches of eleven need, and batches no longer than so many trips need: a step loads its
+      // batch whether the tokens are there or not, 0.13 us for 16 rows of 128 floats at a CU's 64 bytes per cycle.
+      // us a launch, 16 heads, eight wavefronts, batches of eleven and these: head_dim 128, 16 tokens 4.3, 2.8; 64 4.3, 3.1; 100 4.3, 4.0;
+      // 200 6.2, 5.7; head_dim 64, 100 tokens 4.2, 3.1; 400 6.2, 5.5.  (Ten: no better than eleven.)
+      const int batch = (most + trips * groups - 1) / (trips * groups);
+#define LBM_DECODE_ONE_VS(D, NW, NB, VS) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<S, D, NW, NB, true, VS>), grid, block, 0, stream, d);
+#define LBM_DECODE_ONE_D(D, NW, NB)                                                                                                            \
+  {                                                                                                                                          \
+  if (shares == 4) LBM_DECODE_ONE_VS(D, NW, NB, 4)                                                                                           \
+  else if (shares == 2) LBM_DECODE_ONE_VS(D, NW, NB, 2)                                                                                      \
+  else LBM_DECODE_ONE_VS(D, NW, NB, 1)                                                                                                       \
+  }
+#define LBM_DECODE_ONE(NW, NB)                                                                                                                \
+  {                                                                                                                                          \
+  if (head_dim == 64) LBM_DECODE_ONE_D(64, NW, NB)                                                                                           \
+  else LBM_DECODE_ONE_D(128, NW, NB)                                                                                                         \
+  }
+      static_assert(kDecOneTokens <= 8 * 2 * kDecOneWaves * 256 / 64, "head_dim 64 needs no longer batches of sixteen wavefronts than eight");
+      if (many && batch <= 6) LBM_DECODE_ONE(2 * kDecOneWaves, 6)        // (more than half a trip of sixteen)
+      else if (many && batch <= 8) LBM_DECODE_ONE(2 * kDecOneWaves, 8)
+      else if (many) LBM_DECODE_ONE_D(128, 2 * kDecOneWaves, kDecOneBatch)
+      else if (batch <= 2) LBM_DECODE_ONE(kDecOneWaves, 2)
+      else if (batch <= 4) LBM_DECODE_ONE(kDecOneWaves, 4)
+      else if (batch <= 6) LBM_DECODE_ONE(kDecOneWaves, 6)
+      else if (batch <= 8) LBM_DECODE_ONE(kDecOneWaves, 8)
+      else LBM_DECODE_ONE(kDecOneWaves, kDecOneBatch)
+#undef LBM_DECODE_ONE
+#undef LBM_DECODE_ONE_D
+#undef LBM_DECODE_ONE_VS
+      return lbm_check_launch("lbm_attn_f32_decode_kernel<one chunk>");
+    }
+    const dim3 grid(max_chunks, f.num_heads, sch.n_streams * max_q), block(kDecChunkWaves * 64);
+    const dim3 mgrid(max_q, f.num_heads, sch.n_streams + (d.append_rows ? (append_tokens + max_q - 1) / max_q : 0));
+    if (d.append_rows) *appended = true;
+    if (head_dim == 64) {
+      hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<S, 64, kDecChunkWaves, kDecBatch, false>), grid, block, 0, stream, d);
+      hipLaunchKernelGGL((lbm_attn_f32_decode_merge_kernel<S, 64>), mgrid, dim3(128), 0, stream, d);
+    } else {
+      hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<S, 128, kDecChunkWaves, kDecBatch, false>), grid, block, 0, stream, d);
+      hipLaunchKernelGGL((lbm_attn_f32_decode_merge_kernel<S, 128>), mgrid, dim3(128), 0, stream, d);
+    }
+    return lbm_check_launch("lbm_attn_f32_decode_kernel");
+  }
+  if (head_dim == 64) {
+    if (append_apart && append_rows && append_tokens > 0) {
+      f.append_rows = append_rows;
+      f.append_tokens = append_tokens;
+      *appended = true;
+    }
+    return lbm_launch_attn_f32_d64(f, stream);
+  }
+  hipLaunchKernelGGL(lbm_attn_f32_kernel<S>, dim3(wg), dim3(512), 0, stream, f);
+  return lbm_check_launch("lbm_attn_f32_kernel");
+}
+
+template <int S>
+int lbm_launch_bf16(const AttnCore& core, const LbmAttnSchedule& sch, hipStream_t stream, const int32_t* append_rows, int append_tokens,
+                    bool append_apart, bool own_rows, const LbmTouch* touch, bool* appended) {
+  AttnArgs<S> a;
+  static_cast<AttnCore&>(a) = core;
+  a.n_streams = sch.n_streams;
+  a.total_wgs = sch.total_wgs;
+  a.touch = touch ? *touch : LbmTouch{};
+  for (int i = 0; i < sch.n_streams; ++i) a.s[i] = sch.s[i];
+  auto streams_by_workgroup = [&]() {
+    for (int i = 0; i < S; ++i) a.first_wg[i] = i < sch.n_streams ? a.s[i].wg_begin : 0x7fffffff;
+    for (int i = 0; i < sch.n_streams; ++i) a.s[i].per_qtiles = lbm_per(a.s[i].n_qtiles);
+  };
+  streams_by_workgroup();
+  if (sch.small) {
+    unsigned blocks = (unsigned)sch.total_wgs;
+    if (append_apart && append_rows && append_tokens > 0) {
+      a.append_rows = append_rows;
+      a.append_tokens = append_tokens;
+      blocks += (unsigned)(((long long)append_tokens * a.num_heads * 8 + kSmThreads - 1) / kSmThreads);
+      *appended = true;
+    }
+    bool turn = false;   // (for all streams over a cache; the kernel leaves out those with up to two pieces per wavefront, by the live count)
+    for (int i = 0; i < sch.n_streams && !sch.fixed_order; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);
+    const dim3 grid = lbm_touch_grid(a.touch, blocks), block(kSmThreads);
+    // (own rows in order change where rows are read from, not the order of the sums: a launch that goes round keeps its table)
+    if (own_rows && !turn) {
+      if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<S, 2, false, true>), grid, block, 0, stream, a);
+      else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<S, 1, false, true>), grid, block, 0, stream, a);
+      return lbm_check_launch("lbm_attn_bf16_d64_small_kernel<own rows>");
+    }
+    if (sch.small == 64 && turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<S, 2, true>), grid, block, 0, stream, a);
+    else if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<S, 2, false>), grid, block, 0, stream, a);
+    else if (turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<S, 1, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<S, 1, false>), grid, block, 0, stream, a);
+    return lbm_check_launch("lbm_attn_bf16_d64_small_kernel");
+  }
+  // Own rows in order, two splits per stream: both in one workgroup, no launch to merge (lbm_attn_split's PAIR).  us, two
+  // kernels and this one: 16 heads, four streams of 833 rows 28.7, 18.8, of 1,004 32.0, 22.3, of 3,000 154, 140, of 5,000
+  // 383, 361; 2 x 2,000 43.9, 34.9; 1 x 4,096 68.8, 61.0; four streams of 513 rows over 4,609 60.4, 56.1; from the line on,
+  // eight streams of 257 rows over 4,097 54.1, 48.8, 12 heads 51.8, 47.8, of 300 52.1, 49.2, of 448 56.8, 50.7; six of 257
+  // 58.8, 54.7; eight of 385 over 1,500 32.2, 25.9.  Up to 256 rows, which leave it half as many workgroups and those with half a
+  // load each, the two kernels stay: eight streams of 40 rows over 4,097 45.8, 54.6; 12 heads, 255 rows over 4,223 44.5, 51.9.
+  bool pair = own_rows && !a.live_kv_tokens && append_tokens <= 0;
+  for (int i = 0; i < sch.n_streams; ++i) pair = pair && sch.s[i].n_splits == 2 && 2 * sch.s[i].q_rows > kQTile;
+  if (pair) {
+    int wg = 0;
+    for (int i = 0; i < sch.n_streams; ++i) {
+      LbmAttnStreamPlan& p = a.s[i];
+      p.n_qtiles = (p.q_rows + kQTile / 2 - 1) / (kQTile / 2);
+      wg = (wg + 7) & ~7;   // (a stream's first workgroup on XCD 0, as in the schedule)
+      p.wg_begin = wg;
+      wg += p.n_qtiles * a.num_heads;
+    }
+    streams_by_workgroup();
+    hipLaunchKernelGGL(lbm_attn_bf16_d64_pair_kernel<S>, dim3((unsigned)wg), dim3(kThreads), 0, stream, a);
+    return lbm_check_launch("lbm_attn_bf16_d64_pair_kernel");
+  }
+  // The same in one split.  us, with the table and without, 16 heads: 6 streams of 600 rows 21.6, 20.7; 8 x 1,004
+  // 39.7, 38.7; 3 x 1,500 61.7, 58.3; 16 x 100 over 4,097 76.1, 71.6.
+  bool whole = own_rows && !a.live_kv_tokens && append_tokens <= 0;
+  for (int i = 0; i < sch.n_streams; ++i) whole = whole && sch.s[i].n_splits == 1;
+  if (whole) {
+    hipLaunchKernelGGL(lbm_attn_bf16_d64_own_kernel<S>, dim3((unsigned)sch.total_wgs), dim3(kThreads), 0, stream, a);
+    return lbm_check_launch("lbm_attn_bf16_d64_own_kernel");
+  }
+  // The append by workgroups behind the attention's: they run where CUs are done early (the last split of a list has fewer
+  // tiles), and the launch that merges does not wait for them.  us a block, both builds' kernels: 1,004 rows over 17,068
+  // tokens 71.6 + 6.6 for the merge and the append, 72.0 + 5.8; four streams of 1,004 rows 207.5 + 16.3, 209.3 + 11.7.
+  unsigned wgs = (unsigned)sch.total_wgs;
+  if (append_apart && append_rows && append_tokens > 0) {
+    a.append_rows = append_rows;
+    a.append_tokens = append_tokens;
+    wgs += (unsigned)(((long long)append_tokens * a.num_heads * 8 + kThreads * kAppendPieces - 1) / (kThreads * kAppendPieces));
+    *appended = true;
+  }
+  hipLaunchKernelGGL(lbm_attn_bf16_d64_kernel<S>, lbm_touch_grid(a.touch, wgs), dim3(kThreads), 0, stream, a);
+  int rc = lbm_check_launch("lbm_attn_bf16_d64_kernel");
+  if (rc != LBM_OK) return rc;
+  if (sch.part_rows > 0) {
+    int max_rows = 0;
+    for (int i = 0; i < sch.n_streams; ++i)
+      if (sch.s[i].n_splits > 1 && sch.s[i].q_rows > max_rows) max_rows = sch.s[i].q_rows;
+    const long long threads = (long long)max_rows * a.num_heads * 8;
+    unsigned blocks = (unsigned)((threads + 255) / 256);
+    a.combine_blocks = (int)blocks;
+    if (append_rows && append_tokens > 0 && !*appended) {
+      a.append_rows = append_rows;
+      a.append_tokens = append_tokens;
+      blocks += (unsigned)(((long long)append_tokens * a.num_heads * 8 + 255) / 256);
+      *appended = true;
+    }
+    hipLaunchKernelGGL(lbm_attn_combine_bf16_kernel<S>, dim3(blocks, sch.n_streams), dim3(256), 0, stream, a);
+    rc = lbm_check_launch("lbm_attn_combine_bf16_kernel");
+  }
+  return rc;
+}
+
 int lbm_launch_attention_only(const void* q, const void* pool, void* out, const void* self_k,
                               const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                               const LbmAttnSchedule& sch, int num_heads, int head_dim, int page_size, int dtype,
@@ -2350,7 +2612,7 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
   if (head_dim != 64 && !(head_dim == 128 && dtype == LBM_DTYPE_F32))
     return lbm_fail(LBM_ERR_UNSUPPORTED, "attention kernels cover head_dim 64 (bf16, fp32) and 128 (fp32), got %d", head_dim);
   if (dtype == LBM_DTYPE_F32) {
-    AttnArgsF32 f;
+    AttnCoreF32 f;
     f.q = (const float*)q;
     f.pool = (const float*)pool;
     f.out = (float*)out;
@@ -2361,125 +2623,17 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
     f.num_heads = num_heads;
     f.page_size = page_size;
     f.scale_log2 = sm_scale == 0.f ? 1.0f : sm_scale * 1.4426950408889634f;   // 0: q already carries scale * log2(e)
+    f.per_heads = lbm_per(num_heads);
+    f.per_eighth = lbm_per(num_heads >> 3);
     f.n_streams = sch.n_streams;
     f.append_rows = nullptr;
     f.append_tokens = 0;
-    int wg = 0;
-    for (int i = 0; i < LBM_MAX_STREAMS; ++i) {
-      f.s[i] = lbm_attn_stream{0, 0, 0, 0, 0};
-      f.wg_begin[i] = wg;
-      if (i < sch.n_streams) {
-        f.s[i] = lbm_attn_stream{sch.s[i].q_begin, sch.s[i].q_rows, sch.s[i].kv_row_begin, sch.s[i].kv_tokens, sch.s[i].live_at};
-        wg += ((sch.s[i].q_rows + kF32Rows - 1) / kF32Rows) * num_heads;
-      }
-    }
-    f.wg_begin[LBM_MAX_STREAMS] = wg;
-    if (wg == 0) return LBM_OK;
-    if (lbm_decode_applies(sch)) {
-      DecodeArgs d;
-      d.f = f;
-      d.part = (float*)workspace;
-      d.append_rows = append_tokens > 0 ? append_rows : nullptr;
-      d.append_tokens = append_tokens;
-      int max_chunks = 0, max_q = 0, min_q = kDecQ, part = 0, most = 0;
-      int fine = lbm_decode_fine_chunks(sch, num_heads, head_dim);
-      if (workspace_bytes < lbm_decode_bytes(sch, num_heads, head_dim, fine)) fine = 0;   // a workspace for chunks of 256 serves too
-      for (int i = 0; i < LBM_MAX_STREAMS; ++i) {
-        d.n_chunks[i] = 0;
-        d.part_begin[i] = part;
-        if (i < sch.n_streams) {
-          d.n_chunks[i] = lbm_decode_chunks(sch.s[i].kv_tokens, fine);
-          part += d.n_chunks[i] * sch.s[i].q_rows;
-          if (d.n_chunks[i] > max_chunks) max_chunks = d.n_chunks[i];
-          if (sch.s[i].q_rows > max_q) max_q = sch.s[i].q_rows;
-          if (sch.s[i].q_rows < min_q) min_q = sch.s[i].q_rows;
-          if (sch.s[i].kv_tokens > most) most = sch.s[i].kv_tokens;
-        }
-      }
-      if (max_q == 0) return LBM_OK;
-      d.max_q = max_q;
-      // One launch for short lists.  Up to two and a half trips to memory it is the faster form (us, one row of 16 heads
-      // of 128, from the last-level cache and from HBM, against the chunked form: 300 tokens 7.0 and 8.2, 9.6 and 10.8;
-      // 360 tokens 7.6 and 9.0, 8.9 and 9.9; 440 tokens 9.2 and 10.4, 9.1 and 10.3), beyond that it costs more than a
-      // second launch (500 tokens 9.2 and 10.7, 8.0 and 9.0) unless fewer chunks fit (four streams, 500 tokens 10.0 and
-      // 11.9, 11.1 and 12.4).  With one query row per stream and nothing to append beyond those rows it carries the
-      // append as well.
-      const int few = kDecOneWaves * 256 / head_dim, trip = kDecOneBatch * few;   // row groups of eight wavefronts, their tokens in flight
-      if (most <= kDecOneTokens && (fine < kDecFineChunks || most <= trip * 5 / 2)) {
-        for (int i = 0; i < sch.n_streams; ++i) d.n_chunks[i] = 1;
-        unsigned covered = 0;   // rows 0 .. n_streams - 1 of the append, each some stream's query row
-        for (int i = 0; i < sch.n_streams; ++i)
-          if (sch.s[i].q_begin < LBM_MAX_STREAMS) covered |= 1u << sch.s[i].q_begin;
-        const bool carries = d.append_rows && max_q == 1 && min_q == 1 && append_tokens == sch.n_streams &&
-                             covered == (1u << append_tokens) - 1u;
-        if (!carries) d.append_rows = nullptr;
-        else *appended = true;
-        // A row to four or two workgroups where that leaves one per CU, not for the shortest lists (16 tokens of 64
-        // floats 2.75, 2.83), and not where a row to append may be one that another workgroup still has to read.
-        const long long rows = (long long)num_heads * sch.n_streams * max_q;
-        const int shares = (d.append_rows && !append_apart) || most <= 32 ? 1 : rows * 4 <= 256 ? 4 : rows * 2 <= 256 ? 2 : 1;
-        // Sixteen wavefronts, each group with half as many tokens, where eight would make more than one trip (16 heads, K/V
-        // from HBM, rows of a page each, us with eight and with sixteen: head_dim 128, 150 tokens 5.2, 5.3; 200 6.2, 5.8; 300
-        // 7.2, 6.8; 440 9.4, 8.5; four streams of 300 8.5, 8.0, of 440 10.9, 10.0; head_dim 64, 300 tokens 5.1, 5.2; 400 6.0, 5.7).
-        const bool many = most > trip;
-        const int trips = many ? (most + 2 * trip - 1) / (2 * trip) : 1, groups = many ? 2 * few : few;
-        const dim3 grid(1, num_heads, sch.n_streams * max_q * shares), block((many ? 2 : 1) * kDecOneWaves * 64);
-        // As few trips as batches of eleven need, and batches no longer than so many trips need: a step loads its
-        // batch whether the tokens are there or not, 0.13 us for 16 rows of 128 floats at a CU's 64 bytes per cycle.
-        // us a launch, 16 heads, eight wavefronts, batches of eleven and these: head_dim 128, 16 tokens 4.3, 2.8; 64 4.3, 3.1; 100 4.3, 4.0;
-        // 200 6.2, 5.7; head_dim 64, 100 tokens 4.2, 3.1; 400 6.2, 5.5.  (Ten: no better than eleven.)
-        const int batch = (most + trips * groups - 1) / (trips * groups);
-#define LBM_DECODE_ONE_VS(D, NW, NB, VS) hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<D, NW, NB, true, VS>), grid, block, 0, stream, d);
-#define LBM_DECODE_ONE_D(D, NW, NB)                                                                                                            \
-  {                                                                                                                                          \
-    if (shares == 4) LBM_DECODE_ONE_VS(D, NW, NB, 4)                                                                                           \
-    else if (shares == 2) LBM_DECODE_ONE_VS(D, NW, NB, 2)                                                                                      \
-    else LBM_DECODE_ONE_VS(D, NW, NB, 1)                                                                                                       \
-  }
-#define LBM_DECODE_ONE(NW, NB)                                                                                                                \
-  {                                                                                                                                          \
-    if (head_dim == 64) LBM_DECODE_ONE_D(64, NW, NB)                                                                                           \
-    else LBM_DECODE_ONE_D(128, NW, NB)                                                                                                         \
-  }
-        static_assert(kDecOneTokens <= 8 * 2 * kDecOneWaves * 256 / 64, "head_dim 64 needs no longer batches of sixteen wavefronts than eight");
-        if (many && batch <= 6) LBM_DECODE_ONE(2 * kDecOneWaves, 6)        // (more than half a trip of sixteen)
-        else if (many && batch <= 8) LBM_DECODE_ONE(2 * kDecOneWaves, 8)
-        else if (many) LBM_DECODE_ONE_D(128, 2 * kDecOneWaves, kDecOneBatch)
-        else if (batch <= 2) LBM_DECODE_ONE(kDecOneWaves, 2)
-        else if (batch <= 4) LBM_DECODE_ONE(kDecOneWaves, 4)
-        else if (batch <= 6) LBM_DECODE_ONE(kDecOneWaves, 6)
-        else if (batch <= 8) LBM_DECODE_ONE(kDecOneWaves, 8)
-        else LBM_DECODE_ONE(kDecOneWaves, kDecOneBatch)
-#undef LBM_DECODE_ONE
-#undef LBM_DECODE_ONE_D
-#undef LBM_DECODE_ONE_VS
-        return lbm_check_launch("lbm_attn_f32_decode_kernel<one chunk>");
-      }
-      const dim3 grid(max_chunks, num_heads, sch.n_streams * max_q), block(kDecChunkWaves * 64);
-      const dim3 mgrid(max_q, num_heads, sch.n_streams + (d.append_rows ? (append_tokens + max_q - 1) / max_q : 0));
-      if (d.append_rows) *appended = true;
-      if (head_dim == 64) {
-        hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<64, kDecChunkWaves, kDecBatch, false>), grid, block, 0, stream, d);
-        hipLaunchKernelGGL(lbm_attn_f32_decode_merge_kernel<64>, mgrid, dim3(128), 0, stream, d);
-      } else {
-        hipLaunchKernelGGL((lbm_attn_f32_decode_kernel<128, kDecChunkWaves, kDecBatch, false>), grid, block, 0, stream, d);
-        hipLaunchKernelGGL(lbm_attn_f32_decode_merge_kernel<128>, mgrid, dim3(128), 0, stream, d);
-      }
-      return lbm_check_launch("lbm_attn_f32_decode_kernel");
-    }
-    if (head_dim == 64) {
-      if (append_apart && append_rows && append_tokens > 0) {
-        f.append_rows = append_rows;
-        f.append_tokens = append_tokens;
-        *appended = true;
-      }
-      return lbm_launch_attn_f32_d64(f, stream);
-    }
-    hipLaunchKernelGGL(lbm_attn_f32_kernel, dim3(wg), dim3(512), 0, stream, f);
-    return lbm_check_launch("lbm_attn_f32_kernel");
+    if (sch.n_streams == 1)
+      return lbm_launch_f32<1>(f, sch, head_dim, workspace, workspace_bytes, stream, append_rows, append_tokens, append_apart, appended);
+    return lbm_launch_f32<LBM_MAX_STREAMS>(f, sch, head_dim, workspace, workspace_bytes, stream, append_rows, append_tokens, append_apart, appended);
   }
   if (dtype != LBM_DTYPE_BF16) return lbm_fail(LBM_ERR_INVALID, "unknown dtype %d", dtype);
-  AttnArgs a;
+  AttnCore a;
   a.q = (const unsigned short*)q;
   a.pool = (const unsigned short*)pool;
   a.out = (unsigned short*)out;
@@ -2495,90 +2649,11 @@ int lbm_launch_attention_only(const void* q, const void* pool, void* out, const 
   a.append_rows = nullptr;
   a.append_tokens = 0;
   a.combine_blocks = 0x7fffffff;
-  a.sch = sch;
-  a.touch = touch ? *touch : LbmTouch{};
+  a.per_heads = lbm_per(num_heads);
+  a.per_eighth = lbm_per(num_heads >> 3);
   if (sch.total_wgs == 0) return LBM_OK;
-  if (sch.small) {
-    unsigned blocks = (unsigned)sch.total_wgs;
-    if (append_apart && append_rows && append_tokens > 0) {
-      a.append_rows = append_rows;
-      a.append_tokens = append_tokens;
-      blocks += (unsigned)(((long long)append_tokens * num_heads * 8 + kSmThreads - 1) / kSmThreads);
-      *appended = true;
-    }
-    bool turn = false;   // (for all streams over a cache; the kernel leaves out those with up to two pieces per wavefront, by the live count)
-    for (int i = 0; i < sch.n_streams && !sch.fixed_order; ++i) turn = turn || (sch.s[i].kv_tokens != sch.s[i].q_rows && sch.s[i].kv_tokens > kSmTurnKv);
-    const dim3 grid = lbm_touch_grid(a.touch, blocks), block(kSmThreads);
-    // (own rows in order change where rows are read from, not the order of the sums: a launch that goes round keeps its table)
-    if (own_rows && !turn) {
-      if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false, true>), grid, block, 0, stream, a);
-      else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, false, true>), grid, block, 0, stream, a);
-      return lbm_check_launch("lbm_attn_bf16_d64_small_kernel<own rows>");
-    }
-    if (sch.small == 64 && turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, true>), grid, block, 0, stream, a);
-    else if (sch.small == 64) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<2, false>), grid, block, 0, stream, a);
-    else if (turn) hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<1, false>), grid, block, 0, stream, a);
-    return lbm_check_launch("lbm_attn_bf16_d64_small_kernel");
-  }
-  // Own rows in order, two splits per stream: both in one workgroup, no launch to merge (lbm_attn_split's PAIR).  us, two
-  // kernels and this one: 16 heads, four streams of 833 rows 28.7, 18.8, of 1,004 32.0, 22.3, of 3,000 154, 140, of 5,000
-  // 383, 361; 2 x 2,000 43.9, 34.9; 1 x 4,096 68.8, 61.0; four streams of 513 rows over 4,609 60.4, 56.1; from the line on,
-  // eight streams of 257 rows over 4,097 54.1, 48.8, 12 heads 51.8, 47.8, of 300 52.1, 49.2, of 448 56.8, 50.7; six of 257
-  // 58.8, 54.7; eight of 385 over 1,500 32.2, 25.9.  Up to 256 rows, which leave it half as many workgroups and those with half a
-  // load each, the two kernels stay: eight streams of 40 rows over 4,097 45.8, 54.6; 12 heads, 255 rows over 4,223 44.5, 51.9.
-  bool pair = own_rows && !live_kv_tokens && append_tokens <= 0;
-  for (int i = 0; i < sch.n_streams; ++i) pair = pair && sch.s[i].n_splits == 2 && 2 * sch.s[i].q_rows > kQTile;
-  if (pair) {
-    int wg = 0;
-    for (int i = 0; i < sch.n_streams; ++i) {
-      LbmAttnStreamPlan& p = a.sch.s[i];
-      p.n_qtiles = (p.q_rows + kQTile / 2 - 1) / (kQTile / 2);
-      wg = (wg + 7) & ~7;   // (a stream's first workgroup on XCD 0, as in the schedule)
-      p.wg_begin = wg;
-      wg += p.n_qtiles * num_heads;
-    }
-    hipLaunchKernelGGL(lbm_attn_bf16_d64_pair_kernel, dim3((unsigned)wg), dim3(kThreads), 0, stream, a);
-    return lbm_check_launch("lbm_attn_bf16_d64_pair_kernel");
-  }
-  // The same in one split.  us, with the table and without, 16 heads: 6 streams of 600 rows 21.6, 20.7; 8 x 1,004
-  // 39.7, 38.7; 3 x 1,500 61.7, 58.3; 16 x 100 over 4,097 76.1, 71.6.
-  bool whole = own_rows && !live_kv_tokens && append_tokens <= 0;
-  for (int i = 0; i < sch.n_streams; ++i) whole = whole && sch.s[i].n_splits == 1;
-  if (whole) {
-    hipLaunchKernelGGL(lbm_attn_bf16_d64_own_kernel, dim3((unsigned)sch.total_wgs), dim3(kThreads), 0, stream, a);
-    return lbm_check_launch("lbm_attn_bf16_d64_own_kernel");
-  }
-  // The append by workgroups behind the attention's: they run where CUs are done early (the last split of a list has fewer
-  // tiles), and the launch that merges does not wait for them.  us a block, both builds' kernels: 1,004 rows over 17,068
-  // tokens 71.6 + 6.6 for the merge and the append, 72.0 + 5.8; four streams of 1,004 rows 207.5 + 16.3, 209.3 + 11.7.
-  unsigned wgs = (unsigned)sch.total_wgs;
-  if (append_apart && append_rows && append_tokens > 0) {
-    a.append_rows = append_rows;
-    a.append_tokens = append_tokens;
-    wgs += (unsigned)(((long long)append_tokens * num_heads * 8 + kThreads * kAppendPieces - 1) / (kThreads * kAppendPieces));
-    *appended = true;
-  }
-  hipLaunchKernelGGL(lbm_attn_bf16_d64_kernel, lbm_touch_grid(a.touch, wgs), dim3(kThreads), 0, stream, a);
-  int rc = lbm_check_launch("lbm_attn_bf16_d64_kernel");
-  if (rc != LBM_OK) return rc;
-  if (sch.part_rows > 0) {
-    int max_rows = 0;
-    for (int i = 0; i < sch.n_streams; ++i)
-      if (sch.s[i].n_splits > 1 && sch.s[i].q_rows > max_rows) max_rows = sch.s[i].q_rows;
-    const long long threads = (long long)max_rows * num_heads * 8;
-    unsigned blocks = (unsigned)((threads + 255) / 256);
-    a.combine_blocks = (int)blocks;
-    if (append_rows && append_tokens > 0 && !*appended) {
-      a.append_rows = append_rows;
-      a.append_tokens = append_tokens;
-      blocks += (unsigned)(((long long)append_tokens * num_heads * 8 + 255) / 256);
-      *appended = true;
-    }
-    hipLaunchKernelGGL(lbm_attn_combine_bf16_kernel, dim3(blocks, sch.n_streams), dim3(256), 0, stream, a);
-    rc = lbm_check_launch("lbm_attn_combine_bf16_kernel");
-  }
-  return rc;
+  if (sch.n_streams == 1) return lbm_launch_bf16<1>(a, sch, stream, append_rows, append_tokens, append_apart, own_rows, touch, appended);
+  return lbm_launch_bf16<LBM_MAX_STREAMS>(a, sch, stream, append_rows, append_tokens, append_apart, own_rows, touch, appended);
 }
 }  // namespace
 

@@ -7,15 +7,16 @@
 #include "tables_logic.h"
 #include "lbm_internal.h"
 
-struct LbmStepOps { lbm_step_op s[LBM_MAX_STREAMS]; };
+template <int S>   // streams that there is room for, 1 or LBM_MAX_STREAMS (arguments that nobody reads are copied all the same: 0.2 us of the host)
+struct LbmStepOps { lbm_step_op s[S]; };
 
 // RUN: lbm_rows_at_a_time.  A kernel for each: with both forms of the plan in one, steps of the one-row form take longer
 // (10,000 frames of one token 7.2 us apart, 7.4 in one; 2,000 5.7, 5.8).
-template <int RUN>
+template <int S, int RUN>
 __global__ __launch_bounds__(1024) void lbm_tables_kernel(
-    int32_t* __restrict__ tables, lbm_cache_geom g, LbmStepOps ops, int32_t* append_rows,
+    int32_t* __restrict__ tables, lbm_cache_geom g, LbmStepOps<S> ops, int32_t* append_rows,
     int32_t* kv_rows, int32_t* page_ids, int32_t* page_lens) {
-  const int b = blockIdx.x;
+  const int b = S == 1 ? 0 : blockIdx.x;
   const lbm_step_op op = ops.s[b];
   // (more than one workgroup per stream only where every stream's operation is a plan alone: the
   // phases in front of it need the barriers below)
@@ -96,11 +97,12 @@ __global__ __launch_bounds__(1024) void lbm_rows_from_pages_kernel(
   for (int i = carry + tid; i < limit; i += nthr) out[i] = 0;
 }
 
-int lbm_launch_tables(int32_t* tables, const lbm_cache_geom& g, int n_streams,
+template <int S>
+static int lbm_launch_tables_of(int32_t* tables, const lbm_cache_geom& g, int n_streams,
                       const lbm_step_op* ops, int32_t* append_rows, int32_t* kv_rows,
                       int32_t* page_ids, int32_t* page_lens, hipStream_t stream) {
-  LbmStepOps o, plan;
-  for (int i = 0; i < LBM_MAX_STREAMS; ++i) o.s[i] = plan.s[i] = lbm_step_op{};
+  LbmStepOps<S> o, plan;
+  for (int i = 0; i < S; ++i) o.s[i] = plan.s[i] = lbm_step_op{};
   constexpr int32_t kPlanBits = LBM_OP_PLAN | LBM_OP_PLAN_NEWEST_SELF;
   bool changes = false;
   int most_rows = 0;
@@ -122,7 +124,7 @@ int lbm_launch_tables(int32_t* tables, const lbm_cache_geom& g, int n_streams,
   constexpr int kRowsPerGroup = 4096, kSplitRows = 24576, kMostGroups = 64;
   const int groups = most_rows <= kRowsPerGroup ? 1 : (most_rows + kRowsPerGroup - 1) / kRowsPerGroup;
   const bool wide = groups > 1 && (!changes || most_rows > kSplitRows);
-  const auto kernel = lbm_rows_at_a_time(g) == 4 ? lbm_tables_kernel<4> : lbm_tables_kernel<1>;
+  const auto kernel = lbm_rows_at_a_time(g) == 4 ? lbm_tables_kernel<S, 4> : lbm_tables_kernel<S, 1>;
   if (changes || !wide) {
     if (wide)
       for (int i = 0; i < n_streams; ++i) o.s[i].ops &= ~kPlanBits;
@@ -134,6 +136,13 @@ int lbm_launch_tables(int32_t* tables, const lbm_cache_geom& g, int n_streams,
   hipLaunchKernelGGL(kernel, dim3(n_streams, groups < kMostGroups ? groups : kMostGroups), dim3(1024), 0, stream,
                      tables, g, plan, changes ? nullptr : append_rows, kv_rows, page_ids, page_lens);
   return lbm_check_launch("lbm_tables_kernel");
+}
+
+int lbm_launch_tables(int32_t* tables, const lbm_cache_geom& g, int n_streams,
+                      const lbm_step_op* ops, int32_t* append_rows, int32_t* kv_rows,
+                      int32_t* page_ids, int32_t* page_lens, hipStream_t stream) {
+  return n_streams == 1 ? lbm_launch_tables_of<1>(tables, g, n_streams, ops, append_rows, kv_rows, page_ids, page_lens, stream)
+                        : lbm_launch_tables_of<LBM_MAX_STREAMS>(tables, g, n_streams, ops, append_rows, kv_rows, page_ids, page_lens, stream);
 }
 
 int lbm_launch_rows_from_pages(const int32_t* page_ids, const int32_t* page_lens,

@@ -9,11 +9,12 @@
 #define LBM_TILE_FN inline
 #endif
 
-// t / d (0 <= t, 0 < d) and the remainder, given per = lbm_per(d): t x per / 2^32 is at most the quotient and less than one below it.
+// t / d (0 <= t, 0 < d) and the remainder, given per = lbm_per(d): t x per / 2^32 is at most the quotient and less than two below
+// it (32-bit division: a call works several out on its way to the launch).
 // On a uniform value the compiler divides by way of a vector reciprocal and back: 40 instructions that wait for one
 // another, in front of a launch's first load.  (qkv projection, proj, fc1 and fc2, two divisions each, and their sizes in one line of
 // the scalar cache: 86 rows 25.3 -> 24.8 us, 261 28.7 -> 28.0, 1,004 43.0 -> 42.3, 2,008 60.5 -> 59.7.)
-LBM_TILE_FN unsigned lbm_per(long long d) { return d > 1 ? (unsigned)((1LL << 32) / d) : 0xffffffffu; }
+LBM_TILE_FN unsigned lbm_per(int d) { return d > 1 ? 0xffffffffu / (unsigned)d : 0xffffffffu; }
 LBM_TILE_FN int lbm_divide(int t, int d, unsigned per, int& rest) {
   int q = (int)(((unsigned long long)(unsigned)t * per) >> 32);
   rest = t - q * d;
@@ -34,7 +35,7 @@ struct LbmTiles {
 LBM_TILE_FN void lbm_set_panels(LbmTiles& p, int panel_shift) {
   p.panel_shift = panel_shift;
   p.last_width = p.n_tiles & ((1 << panel_shift) - 1);
-  p.per_panel = lbm_per((long long)p.m_tiles << panel_shift);
+  p.per_panel = lbm_per(p.m_tiles << panel_shift);
   p.per_last = lbm_per(p.last_width);
 }
 // Workgroup b's tile.  Workgroups are dealt to the 8 XCDs round-robin (b % 8), 32 of a round of 256
