@@ -1400,6 +1400,8 @@ __device__ __forceinline__ void lbm_combine_upto(const float* lse, const unsigne
 
 template <int S>
 __global__ __launch_bounds__(256) void lbm_attn_combine_bf16_kernel(AttnArgs<S> a) {
+  const LbmAttnStreamPlan sp = a.s[S == 1 ? 0 : blockIdx.y];
+  asm volatile("" : : "s"(a.combine_blocks), "s"(a.num_heads), "s"(a.part_lse), "s"(a.part_o), "s"(a.out), "s"(sp.n_splits), "s"(sp.q_rows), "s"(sp.part_begin), "s"(sp.q_begin));   // (in one trip: lbm_first_plan)
   if ((int)blockIdx.x >= a.combine_blocks) {
     // The append's share of the launch (lbm_attn_run_append): the main kernel has read the pool,
     // the new frames' rows - attended to from the caller's tensors - now go into their pages.
@@ -1408,7 +1410,6 @@ __global__ __launch_bounds__(256) void lbm_attn_combine_bf16_kernel(AttnArgs<S> 
                         (int)blockIdx.x - a.combine_blocks, 256);
     return;
   }
-  const LbmAttnStreamPlan sp = a.s[S == 1 ? 0 : blockIdx.y];
   if (sp.n_splits <= 1) return;
   const int H = a.num_heads;
   const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
