@@ -295,7 +295,7 @@ __device__ __forceinline__ void ask_rotary(const LinearArgs& p, int token, int c
     cs[0] = src[0]; cs[1] = src[1]; cs[2] = src[2]; cs[3] = src[3];
   }
 }
-template <int ROPE, bool NORM>
+template <int ROPE, bool NORM, bool READY = false>
 __device__ __forceinline__ bf16x8 produce_row(u32x4 raw, int which, int c8, const lbm_qkv::f32x4 (&w4)[2], const lbm_qkv::f32x4 (&b4)[2],
                                               const lbm_qkv::f32x4 (&cs)[4], float eps, float post) {
   bf16x8 o8 = __builtin_bit_cast(bf16x8, raw);   // v rows leave as they are
@@ -304,7 +304,7 @@ __device__ __forceinline__ bf16x8 produce_row(u32x4 raw, int which, int c8, cons
     float x[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = __builtin_bit_cast(float, (i & 1) ? (raw[i >> 1] & 0xffff0000u) : (raw[i >> 1] << 16));
-    lbm_qkv::norm_rope_unrounded<0, ROPE, NORM>(x, w4, b4, cs, c8, eps, post);
+    lbm_qkv::norm_rope_unrounded<0, ROPE, NORM, READY>(x, w4, b4, cs, c8, eps, post);
 #pragma unroll
     for (int i = 0; i < 8; ++i) o8[i] = (__bf16)x[i];
   }
@@ -1030,10 +1030,10 @@ __global__ __launch_bounds__(lbm_rows_threads(TM), 1) void lbm_linear_bf16_rows_
 constexpr int kBN = 256;
 constexpr int kBCStride = kBN + 4;                          // bf16 per staged output row
 constexpr int lbm_big_stages(int bm) { return bm == 128 ? 3 : 2; }
-// Whether two more wavefronts load, as above: where the others can do with 168 registers, that is with
-// 128 rows, and with 192 unless the store holds rotary entries.
-constexpr bool lbm_big_loaders(int bm, int rope) { return bm == 128 || (bm == 192 && rope == 0); }
-constexpr int lbm_big_threads(int bm, int rope) { return kGThreads + (lbm_big_loaders(bm, rope) ? kGLoadWaves * 64 : 0); }
+// Whether two more wavefronts load, as above: where the others can do with 168 registers, that is with up to 192 rows.
+constexpr bool lbm_big_loaders(int bm) { return bm <= 192; }
+constexpr int lbm_big_norm_rows(int epi, bool norm) { return epi == kEpiQkvPrepare && norm ? 4 : 1; }
+constexpr int lbm_big_threads(int bm) { return kGThreads + (lbm_big_loaders(bm) ? kGLoadWaves * 64 : 0); }
 constexpr int lbm_big_lds_bytes(int bm) {
   const int stages = lbm_big_stages(bm) * (bm + kBN) * kKS * 2;
   return bm * kBCStride * 2 > stages ? bm * kBCStride * 2 : stages;
@@ -1041,7 +1041,7 @@ constexpr int lbm_big_lds_bytes(int bm) {
 static_assert(lbm_big_lds_bytes(256) + kGeluEntries * 2 + 2 * kBN * 4 + 256 * 8 <= 160 * 1024, "LDS budget of the 256 x 256 tile");
 
 template <int BM, int EPI, int ROPE = 0, bool NORM = false, bool LNA = false>
-__global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_big_kernel(LinearArgs p) {
+__global__ __launch_bounds__(lbm_big_threads(BM), 1) void lbm_linear_bf16_big_kernel(LinearArgs p) {
   constexpr int kRowGroups = BM == 256 ? 4 : 2;             // wavefronts along the rows of the tile
   constexpr int kColGroups = 8 / kRowGroups;
   constexpr int RB = BM / 32 / kRowGroups, CB = kBN / 32 / kColGroups;   // 32 x 32 blocks per wavefront: 2 x 4 or 3 x 2
@@ -1051,6 +1051,8 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   __shared__ __attribute__((aligned(16))) unsigned short gelu_tab[EPI == LBM_LINEAR_BIAS_GELU ? kGeluEntries : 8];
   __shared__ __attribute__((aligned(8))) float ln_rows[LNA ? BM * 2 : 2];                   // per row: rstd, -mean * rstd
 
+  __shared__ __attribute__((aligned(16))) float qk_norm[lbm_big_norm_rows(EPI, NORM)][64];           // q's weight and bias, k's
+
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   hold_arguments<EPI, LNA, NORM>(p);
   const int n32 = lane & 31, g = lane >> 5;
@@ -1059,9 +1061,32 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   int mt, nt;
   lbm_tile_of_workgroup((int)blockIdx.x, p, mt, nt);
   const int m0 = mt * BM, n0 = nt * kBN;
+  // The tile's columns in four slots of 64.  Where the producer has work to do, three tiles share four heads of q, k and v so that none
+  // has more than three slots of q and k: q0 q1 k0 v0 | q2 k1 k2 v1 | q3 k3 v2 v3, a digit 4 x (q, k, v) + head for each slot.
+  // The store is bound by the producer's vector instructions, and a launch of one round by its slowest tile: four slots of q
+  // were 187 instructions per eight elements behind the loop, beside tiles of v with none.  Mixed, with a token's
+  // entries rounded once for its slots instead of once for each and, the entries being few now, loading wavefronts on 192 rows too, us of
+  // 16 heads x 1,024, interleaved and half-split entries, before and now: 2,008 rows 19.8, 20.4 -> 17.2, 17.4; 4,016 30.7, 33.1 -> 26.7, 27.0;
+  // 5,000 38.1, 39.9 -> 34.0, 34.1; 8,040 59.8, 65.7 -> 52.1, 53.0.  Without norm and table slots of one kind stay: they leave as
+  // rows of 512 bytes (mixed 2,008 rows 17.4 for 15.6, 8,040 51.2 for 46.2; q, k, v in turn instead of two neighbours where there are two 1 % more).
+  constexpr bool kQkv = EPI == kEpiQkvPrepare, kMixed = kQkv && (ROPE != 0 || NORM);
+  auto slot_of = [&](int j, int& head) {
+    const int group = nt / 3;
+    const int digit = (int)(0xBA7396528410ull >> (4 * (4 * (nt - 3 * group) + j))) & 15;
+    head = 4 * group + (digit & 3);
+    return digit >> 2;
+  };
+  auto slot_col = [&](int j) {
+    int head;
+    const int which = slot_of(j, head);
+    return (which * p.num_heads + head) * 64;
+  };
+  int w_rows[kBN / 64];   // each slot's first row of w, from w_base on
+#pragma unroll
+  for (int j = 0; j < kBN / 64; ++j) w_rows[j] = kMixed ? slot_col(j) : 64 * j;
 
   if (blockIdx.y) {   // (a scalar register: nothing is loaded to know)
-    lbm_touch(p.touch, lbm_big_threads(BM, ROPE), false);
+    lbm_touch(p.touch, lbm_big_threads(BM), false);
     return;
   }
 
@@ -1075,7 +1100,7 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   const unsigned w_off = ((unsigned)ld_r * (unsigned)p.K + sw_c) * 2u;
   const int nk = p.K / kKS;
   const char* a_base = (const char*)p.a;
-  const char* w_base = (const char*)(p.w + (size_t)n0 * p.K);
+  const char* w_base = (const char*)(p.w + (kMixed ? 0 : (size_t)n0 * p.K));
   auto dma_row = [&](const char* base, unsigned voff, const unsigned char* lds_dst) {
     const unsigned m0v = (unsigned)(size_t)(__attribute__((address_space(3))) const void*)lds_dst;
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
@@ -1087,11 +1112,11 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   auto dma_one = [&](int ks, int stage, int j) {
     unsigned char* st = lds_raw + stage * kStageBytes;
     if (j < kPassA) dma_row(a_base + ks * (kKS * 2), a_off[j], st + (64 * j + 8 * wave) * (kKS * 2));
-    else dma_row(w_base + ((size_t)(64 * (j - kPassA)) * p.K + (size_t)ks * kKS) * 2, w_off,
+    else dma_row(w_base + ((size_t)w_rows[j - kPassA] * p.K + (size_t)ks * kKS) * 2, w_off,
                  st + BM * kKS * 2 + (64 * (j - kPassA) + 8 * wave) * (kKS * 2));
   };
   constexpr int kDma = kPassA + kPassW;
-  constexpr bool kLoaders = lbm_big_loaders(BM, ROPE);
+  constexpr bool kLoaders = lbm_big_loaders(BM);
   constexpr int kStages = lbm_big_stages(BM);
   if (kLoaders && wave >= kGThreads / 64) {
     // a loading wavefront: every second KB of a step's operands (as in the kernel above)
@@ -1101,7 +1126,7 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
     unsigned off[kLoads];
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
-      const int row = u < kUnitsA ? min(m0 + 8 * (2 * u + par) + l8, p.M - 1) : 8 * (2 * (u - kUnitsA) + par) + l8;
+      const int row = u < kUnitsA ? min(m0 + 8 * (2 * u + par) + l8, p.M - 1) : w_rows[(u - kUnitsA) / 4] + (8 * (2 * (u - kUnitsA) + par) + l8) % 64;
       off[u] = ((unsigned)row * (unsigned)p.K + chunk) * 2u;
     }
     const unsigned lds_first = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)&lds_raw[0]) + (unsigned)par * 1024u;
@@ -1136,10 +1161,12 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
       if ((tid & 1) + 2 * i < p.ln_tiles) ln_part[i] = *(const f32x2*)(ln_st + 2 * ((tid & 1) + 2 * i));
   }
   // per-column vectors of the tile into LDS (read in the epilogue, many barriers from here)
-  float cv_bias = 0.f, cv_sum = 0.f;
+  float cv_bias = 0.f, cv_sum = 0.f, cv_norm = 0.f;
   if (tid < kBN) {
-    if (p.bias) cv_bias = p.bias[n0 + tid];
-    if (LNA) cv_sum = p.ln_colsum[n0 + tid];
+    const int col = kMixed ? slot_col(wave) + lane : n0 + tid;
+    if (p.bias) cv_bias = p.bias[col];
+    if (LNA) cv_sum = p.ln_colsum[col];
+    if (kQkv && NORM) cv_norm = (wave == 0 ? p.q_norm_w : wave == 1 ? p.q_norm_b : wave == 2 ? p.k_norm_w : p.k_norm_b)[lane];
   }
   if (EPI == LBM_LINEAR_BIAS_GELU && tid < kGeluEntries / 8)
     dma_row((const char*)g_gelu_table, (unsigned)tid * 16u, (const unsigned char*)&gelu_tab[wave * 512]);
@@ -1148,6 +1175,7 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   if (tid < kBN) {
     colvec[0][tid] = cv_bias;
     colvec[1][tid] = cv_sum;
+    if (kQkv && NORM) qk_norm[wave][lane] = cv_norm;
   }
   if (LNA && (tid >> 1) < BM) {
     const int r = tid >> 1, part = tid & 1;
@@ -1192,7 +1220,7 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   const unsigned m0_wave = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds_raw + (unsigned)wave * 1024u);
   unsigned w_offs[kPassW];
 #pragma unroll
-  for (int j = 0; j < kPassW; ++j) w_offs[j] = w_off + (unsigned)(64 * j) * (unsigned)p.K * 2u;
+  for (int j = 0; j < kPassW; ++j) w_offs[j] = w_off + (unsigned)w_rows[j] * (unsigned)p.K * 2u;
   auto dma_at = [&](const char* base, unsigned voff, unsigned m0v) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(m0v) : "memory", "m0");
   };
@@ -1267,38 +1295,20 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
   }
 #undef LBM_SGB
 
-  // ---- epilogue.  What the producer's first passes need from global memory is asked for now and
-  // arrives while the tile is staged.
-  constexpr int kPieces = kBN / 8;                    // 16-byte pieces per row of the tile: 32
-  constexpr int kRowsPerPass = kGThreads / kPieces;   // 16
-  constexpr int kPasses = BM / kRowsPerPass;          // 16 or 12
-  constexpr int kGroup = BM == 128 ? 2 : 4;           // passes whose rotary entries and pool rows travel together
-  const int pr = tid / kPieces, pc = (tid % kPieces) * 8;
+  // ---- epilogue.  A lane of the producer works on the same eight columns of all four slots of a token: one set of rotary entries,
+  // asked for a pass ahead (the first now, it arrives while the tile is staged) and rounded once.
   typedef lbm_qkv::f32x4 qf4;
-  const int H = p.num_heads;
-  const int pq_col = n0 + pc;
-  const int which = EPI == kEpiQkvPrepare ? pq_col / (H * 64) : 0;   // uniform over the workgroup (H * 64 is a multiple of 256)
-  const int ph = (pq_col - which * H * 64) >> 6, c8 = (pq_col & 63) >> 3;
-  qf4 w4[2] = {}, b4[2] = {};
-  qf4 cs4[2][kGroup][4] = {};
-  int pool_row[2][kGroup];
-  auto ask = [&](int grp, qf4 (&cs)[kGroup][4], int (&rows)[kGroup]) {
+  constexpr int kTokenPasses = BM / 64;
+  const int c8 = lane & 7;
+  qf4 cs4[2][4] = {};
+  int pool_row[kTokenPasses];
+  if (kMixed) {
 #pragma unroll
-    for (int j = 0; j < kGroup; ++j) {
-      const int t = min(m0 + (grp * kGroup + j) * kRowsPerPass + pr, p.M - 1);
-      if (which < 2) ask_rotary<ROPE>(p, t, c8, cs[j]);
-      rows[j] = -1;
-      if (which > 0 && p.append_rows) rows[j] = p.append_rows[t];
+    for (int j = 0; j < kTokenPasses; ++j) {
+      const int t = min(m0 + j * 64 + (tid >> 3), p.M - 1);
+      if (j == 0) ask_rotary<ROPE>(p, t, c8, cs4[0]);
+      pool_row[j] = p.append_rows ? p.append_rows[t] : -1;
     }
-  };
-  if (EPI == kEpiQkvPrepare) {
-    if (NORM && which < 2) {
-      const qf4* wp = (const qf4*)((which == 0 ? p.q_norm_w : p.k_norm_w) + c8 * 8);
-      const qf4* bp = (const qf4*)((which == 0 ? p.q_norm_b : p.k_norm_b) + c8 * 8);
-      w4[0] = wp[0]; w4[1] = wp[1];
-      b4[0] = bp[0]; b4[1] = bp[1];
-    }
-    ask(0, cs4[0], pool_row[0]);
   }
   __syncthreads();   // the operand stages are dead: the output tile is staged over them
   // In registers: the folded LayerNorm's scale and correction, + bias, round (the linear's
@@ -1336,32 +1346,79 @@ __global__ __launch_bounds__(lbm_big_threads(BM, ROPE), 1) void lbm_linear_bf16_
     }
   }
   __syncthreads();
-  if (EPI == kEpiQkvPrepare) {
-    // the producer on the staged tile, as in the kernel above; the rotary entries and pool rows of
-    // four passes are asked for while the four before them are worked on
-    unsigned short* const plain = produced_rows(p, which);
-    const float post = which == 0 ? p.q_scale : 1.0f;
-    auto work = [&](int grp, const qf4 (&cs)[kGroup][4], const int (&rows)[kGroup]) {
+  if (kMixed) {
+    // the producer on the staged tile, as in the kernel above
+    qf4 w4[2][2] = {}, b4[2][2] = {};   // q's, k's
+    if (NORM)
 #pragma unroll
-      for (int j = 0; j < kGroup; ++j) {
-        const int r = (grp * kGroup + j) * kRowsPerPass + pr;
-        const u32x2 lo = *(const u32x2*)&stage[r * kBCStride + pc], hi = *(const u32x2*)&stage[r * kBCStride + pc + 4];
-        const bf16x8 o8 = produce_row<ROPE, NORM>(u32x4{lo[0], lo[1], hi[0], hi[1]}, which, c8, w4, b4, cs[j], p.eps, post);
-        if (m0 + r < p.M) store_produced(p, plain, o8, which, m0 + r, ph, c8, rows[j]);
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          w4[i][e] = *(const qf4*)&qk_norm[2 * i][c8 * 8 + 4 * e];
+          b4[i][e] = *(const qf4*)&qk_norm[2 * i + 1][c8 * 8 + 4 * e];
+        }
+#pragma unroll
+    for (int j = 0; j < kTokenPasses; ++j) {
+      const int r = j * 64 + (tid >> 3);
+      if (j + 1 < kTokenPasses) ask_rotary<ROPE>(p, min(m0 + r + 64, p.M - 1), c8, cs4[(j + 1) & 1]);
+      u32x4 raw[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const u32x2 lo = *(const u32x2*)&stage[r * kBCStride + s * 64 + c8 * 8], hi = *(const u32x2*)&stage[r * kBCStride + s * 64 + c8 * 8 + 4];
+        raw[s] = u32x4{lo[0], lo[1], hi[0], hi[1]};
       }
-    };
+      lbm_qkv::ready_rotary<ROPE>(cs4[j & 1], c8);
 #pragma unroll
-    for (int grp = 0; grp < kPasses / kGroup; ++grp) {
-      if (grp + 1 < kPasses / kGroup) ask(grp + 1, cs4[(grp + 1) & 1], pool_row[(grp + 1) & 1]);
-      work(grp, cs4[grp & 1], pool_row[grp & 1]);
+      for (int s = 0; s < 4; ++s) {
+        int head;
+        const int which = slot_of(s, head);
+        bf16x8 o8;
+        if (which == 0) o8 = produce_row<ROPE, NORM, true>(raw[s], 0, c8, w4[0], b4[0], cs4[j & 1], p.eps, p.q_scale);
+        else o8 = produce_row<ROPE, NORM, true>(raw[s], which, c8, w4[1], b4[1], cs4[j & 1], p.eps, 1.0f);
+        if (m0 + r < p.M) store_produced(p, produced_rows(p, which), o8, which, m0 + r, head, c8, pool_row[j]);
+      }
     }
     return;
   }
-#pragma unroll
-  for (int j = 0; j < kPasses; ++j) {
-    const int r = j * kRowsPerPass + pr, row = m0 + r;
+  constexpr int kPieces = kBN / 8;                    // 16-byte pieces per row of the tile: 32
+  constexpr int kRowsPerPass = kGThreads / kPieces;   // 16
+  constexpr int kPasses = BM / kRowsPerPass;          // 16 or 12
+  const int pr = tid / kPieces, pc = (tid % kPieces) * 8;
+  auto piece = [&](int j) {
+    const int r = j * kRowsPerPass + pr;
     const u32x2 lo = *(const u32x2*)&stage[r * kBCStride + pc], hi = *(const u32x2*)&stage[r * kBCStride + pc + 4];
-    if (row < p.M) lbm_store_through(p.out + (size_t)row * p.N + n0 + pc, u32x4{lo[0], lo[1], hi[0], hi[1]});
+    return u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
+  if (!kQkv) {
+#pragma unroll
+    for (int j = 0; j < kPasses; ++j) {
+      const int row = m0 + j * kRowsPerPass + pr;
+      const u32x4 v = piece(j);
+      if (row < p.M) lbm_store_through(p.out + (size_t)row * p.N + n0 + pc, v);
+    }
+    return;
+  }
+  // a producer with nothing to do but q's factor (an encoder's): rows of four heads of one kind
+  const int dim = p.num_heads * 64, which = n0 / dim, col = n0 + pc - which * dim;   // (dim is a multiple of 256)
+  unsigned short* const plain = produced_rows(p, which);
+  if (plain) {
+#pragma unroll
+    for (int j = 0; j < kPasses; ++j) {
+      const int row = m0 + j * kRowsPerPass + pr;
+      u32x4 v = piece(j);
+      const qf4 none[2] = {};
+      if (which == 0) v = __builtin_bit_cast(u32x4, produce_row<0, false>(v, 0, 0, none, none, cs4[0], 0.f, p.q_scale));
+      if (row < p.M) lbm_store_through(plain + (size_t)row * dim + col, v);
+    }
+  }
+  if (which > 0 && p.append_rows) {
+    int to[kPasses];
+#pragma unroll
+    for (int j = 0; j < kPasses; ++j) to[j] = p.append_rows[min(m0 + j * kRowsPerPass + pr, p.M - 1)];
+#pragma unroll
+    for (int j = 0; j < kPasses; ++j)
+      if (m0 + j * kRowsPerPass + pr < p.M)
+        store_produced(p, nullptr, __builtin_bit_cast(bf16x8, piece(j)), which, 0, col >> 6, (col & 63) >> 3, to[j]);
   }
 }
 
@@ -1603,8 +1660,8 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
 #define LBM_BIG_LAUNCH(E, L)                                                                                         \
       {                                                                                                              \
         if (bm == 256) hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<256, E, 0, false, L>), grid_b, block, 0, stream, p); \
-        else if (bm == 192) hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<192, E, 0, false, L>), grid_b, dim3(lbm_big_threads(192, 0)), 0, stream, p);           \
-        else hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<128, E, 0, false, L>), grid_b, dim3(lbm_big_threads(128, 0)), 0, stream, p);           \
+        else if (bm == 192) hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<192, E, 0, false, L>), grid_b, dim3(lbm_big_threads(192)), 0, stream, p);           \
+        else hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<128, E, 0, false, L>), grid_b, dim3(lbm_big_threads(128)), 0, stream, p);           \
       }
       if (epilogue == LBM_LINEAR_BIAS && lna) LBM_BIG_LAUNCH(LBM_LINEAR_BIAS, true)
       else if (epilogue == LBM_LINEAR_BIAS) LBM_BIG_LAUNCH(LBM_LINEAR_BIAS, false)
@@ -1696,7 +1753,7 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
   const bool norm = q_norm_w != nullptr;
   const LinearForm f = lbm_linear_form(p, kEpiQkvPrepare, num_heads, false);
   if (const int bm = f.big) {
-    const dim3 grid_b = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles)), block_b(lbm_big_threads(bm, rope));
+    const dim3 grid_b = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles)), block_b(lbm_big_threads(bm));
 #define LBM_QKV_BIG_M(BM, R, NRM)                                                                                               \
     {                                                                                                                           \
       if (lna) hipLaunchKernelGGL((lbm_linear_bf16_big_kernel<BM, kEpiQkvPrepare, R, NRM, true>), grid_b, block_b, 0, stream, p);  \

@@ -69,18 +69,38 @@ __device__ __forceinline__ void round_bf16_pair(float a, float b, float& ra, flo
   rb = __builtin_bit_cast(float, pk & 0xffff0000u);
 }
 
+// The sine of a half-split pair's element, its sign flipped where the element is of the first 16 (c: its lane of the row's
+// eight): see norm_rope_unrounded.
+__device__ __forceinline__ float flip_sine(float si, int c) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, si) ^ ((c & 2) == 0 ? 0x80000000u : 0u));
+}
+// A lane's rotary entries for bf16 rows (SRC 0 below): rounded, sines with the sign that their product takes
+template <int ROPE>
+__device__ __forceinline__ void ready_rotary(f32x4 (&cs4)[4], int c) {
+#pragma unroll
+  for (int p = 0; p < (ROPE == 0 ? 0 : (ROPE == 1 ? 2 : 4)); ++p)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      float co, si;
+      round_bf16_pair(cs4[p][2 * j], cs4[p][2 * j + 1], co, si);
+      cs4[p][2 * j] = co;
+      cs4[p][2 * j + 1] = ROPE == 2 ? flip_sine(si, c) : si;
+    }
+}
+
 // x: this lane's elements 8 c .. 8 c + 7 of the row (c = lane % 8; the row's 8 lanes are
 // consecutive and aligned, so the shuffles below stay inside it).  SRC 0: bf16 activations
 // (roundings after the LayerNorm, of cos and sin, and after every product and sum), 1: fp32.
 // ROPE 0 none, 1 interleaved pairs (cs4[0..1] = (cos, sin) of this lane's four pairs), 2
 // half-split pairs (cs4[0..3] = (cos, sin) of its eight elements).  w4 / b4: LayerNorm weight
 // and bias of the lane's eight elements.
+// READY: cs4 holds what ready_rotary made of it, once for the heads of a token that a lane works on.
 // post: a factor the row is multiplied by in fp32 BEFORE the rounding that ends its last
 // operation (the rotary sum, else the LayerNorm, else the plain copy), so that a scaled q row
 // is rounded once; 1.0f leaves every result as it was (x * 1.0f is exact).
 // norm_rope_unrounded leaves that last rounding of a bf16 row (SRC 0) to the caller, who makes it
 // with the conversion that packs the row for its store; every rounding before it is made here.
-template <int SRC, int ROPE, bool NORM>
+template <int SRC, int ROPE, bool NORM, bool READY = false>
 __device__ __forceinline__ void norm_rope_unrounded(float (&x)[8], const f32x4 (&w4)[2], const f32x4 (&b4)[2],
                                                     const f32x4 (&cs4)[4], int c, float eps, float post = 1.0f) {
   const float post_norm = ROPE == 0 ? post : 1.0f;
@@ -117,7 +137,7 @@ __device__ __forceinline__ void norm_rope_unrounded(float (&x)[8], const f32x4 (
         float co = q4[2 * j], si = q4[2 * j + 1];
         const float x1 = x[i], x2 = x[i + 1];
         if (SRC == 0) {
-          round_bf16_pair(co, si, co, si);
+          if (!READY) round_bf16_pair(co, si, co, si);
           float cc, ss, sc, cs;
           round_bf16_pair(mul_rn(x1, co), mul_rn(x2, si), cc, ss);
           round_bf16_pair(mul_rn(x1, si), mul_rn(x2, co), sc, cs);
@@ -132,9 +152,8 @@ __device__ __forceinline__ void norm_rope_unrounded(float (&x)[8], const f32x4 (
   } else if (ROPE != 0) {
     // half-split pairs: in each 32-element half, element j < 16 rotates with element j + 16
     // (x * cos + rotate(x) * sin with rotate = (-second, first), rope.py:123-152); the partner
-    // sits two lanes away in the 8-lane group.  a - b is a + (-b) bit for bit, so the lanes of
-    // the first 16 flip the sign of the second product instead of choosing between two results.
-    const unsigned flip = (c & 2) == 0 ? 0x80000000u : 0u;
+    // sits two lanes away in the 8-lane group.  a - b is a + (-b) bit for bit, and b's sign is its sine's,
+    // so the lanes of the first 16 flip the sine instead of choosing between two results.
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       const f32x4 q4 = cs4[p];  // (cos, sin) of two elements
@@ -145,13 +164,12 @@ __device__ __forceinline__ void norm_rope_unrounded(float (&x)[8], const f32x4 (
         const float own = x[i];
         const float other = lane_xor2(own);
         float a0, b0;
-        if (SRC == 0) {
-          round_bf16_pair(co, si, co, si);
-          round_bf16_pair(mul_rn(own, co), mul_rn(other, si), a0, b0);
-        } else {
-          a0 = mul_rn(own, co), b0 = mul_rn(other, si);
+        if (!READY) {
+          if (SRC == 0) round_bf16_pair(co, si, co, si);
+          si = flip_sine(si, c);
         }
-        b0 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, b0) ^ flip);
+        if (SRC == 0) round_bf16_pair(mul_rn(own, co), mul_rn(other, si), a0, b0);
+        else a0 = mul_rn(own, co), b0 = mul_rn(other, si);
         x[i] = mul_rn(add_rn(a0, b0), post);
       }
     }

@@ -243,6 +243,32 @@ def test_qkv_projection_with_the_producer_as_its_epilogue(M, H, K, norm, rope):
     assert bad(ptr(a), ptr(w), None, M, K, None, None, None, None, 1e-5, 1.0, None, 0, ptr(q1), None, None, None, ptr(rows), H, D, S, None)  # rows without pool
 
 
+@pytest.mark.parametrize("norm,rope", [(True, "half_split"), (True, "interleaved"), (False, "half_split"), (True, "none"), (False, "none")])
+@pytest.mark.parametrize("M,H", [(2008, 16), (8321, 4), (3649, 12), (4097, 16), (5377, 12)])
+def test_producer_on_tiles_of_four_heads(M, H, norm, rope):
+    """As above on tiles of 256 columns - q, k and v heads mixed where there is a norm or a table, four of a kind
+    where there is neither - of 128 (2,008 and 8,321 rows), 192 (3,649) and 256 rows (4,097, and 5,377 with one row in the last
+    tile), with a factor on q."""
+    test_qkv_projection_with_the_producer_as_its_epilogue(M, H, 128, norm, rope)
+    N, dev, D, K = _native(), torch.device("cuda:0"), 64, 128
+    g = torch.Generator().manual_seed(M + H)
+    a = torch.randn(M, K, generator=g).to(torch.bfloat16).to(dev)
+    w = (torch.randn(3 * H * D, K, generator=g) / K ** 0.5).to(torch.bfloat16).to(dev)
+    ln = [(1 + 0.2 * torch.randn(D, generator=g)).to(dev) for _ in range(4)] if norm else [None] * 4
+    cs = None if rope == "none" else torch.randn(M, D // 2 if rope == "interleaved" else D, 2, generator=g).to(dev)
+    layout = N.ROPE_INTERLEAVED if rope == "interleaved" else N.ROPE_HALF_SPLIT
+    qkv = torch.empty(M, 3 * H * D, dtype=torch.bfloat16, device=dev)
+    got, want = ([torch.full((M, H, D), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(3)] for _ in range(2))
+    scale = N.q_scale_log2(0.125)
+    N.check(N.lib.lbm_linear(ptr(a), ptr(w), None, None, None, ptr(qkv), M, 3 * H * D, K, N.LINEAR_BIAS, None))
+    N.check(N.lib.lbm_qkv_prepare(ptr(qkv), N.DTYPE_BF16, *[ptr(t) for t in ln], 1e-5, scale, ptr(cs), layout, *[ptr(t) for t in want],
+                                  N.DTYPE_BF16, None, None, M, H, D, 16, None))
+    N.check(N.lib.lbm_qkv_linear_prepare(ptr(a), ptr(w), None, M, K, *[ptr(t) for t in ln], 1e-5, scale, ptr(cs), layout, *[ptr(t) for t in got],
+                                         None, None, H, D, 16, None))
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+
+
 def _row_norm(N, stats, colsum, tiles, eps=1e-5):
     return N.RowNorm(stats.data_ptr(), colsum.data_ptr(), tiles, eps)
 
