@@ -20,8 +20,9 @@
 // 1,004 rows x 16 heads: 1,004 tokens 48 -> 37 us, 8,032 tokens 337 -> 240 us against the fp32 instruction.
 // Infinities have a pass of their own at the end of the kernel.
 //
-// One workgroup = eight wavefronts on 64 query rows of one head.  A wavefront takes every eighth
-// 32-token tile of the KV list, for all 64 rows (so that a value of K or V is split once per 64 rows),
+// One workgroup = eight wavefronts on 64 query rows of one head, or on 32 where those of 64 would leave CUs idle
+// (lbm_f32_row_blocks).  A wavefront takes every eighth
+// 32-token tile of the KV list, for all the rows (so that a value of K or V is split once per 64 rows),
 // from an LDS buffer of its own: nothing is shared inside the loop and there is no barrier in it.  The
 // rows travel global -> LDS directly as fp32 (global_load_lds_dwordx4), the next K tile as soon as this
 // one's fragments are read, the next V tile likewise, so either has half an iteration to land and one
@@ -45,18 +46,17 @@ typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 namespace {
 
 constexpr int kWaves = 8, kThreads = kWaves * 64;
-constexpr int kRows = 64;               // query rows per workgroup
 constexpr int kAppendPieces = 4;        // 16-byte pieces of K and of V per thread of a workgroup that appends
 constexpr int kTile = 32;               // KV tokens per tile
 constexpr int kTileBytes = kTile * 64 * 4;
-constexpr int kQPlane = kRows * 64;     // bf16 of a Q plane: unpadded rows, chunk c of row r at c ^ ((r >> 1) & 7)
 constexpr int kEntryBytes = 256 + kTile * 2 * 8;   // a wavefront's row entries, and the K and V addresses they name
 constexpr int kOffEntries = kWaves * 2 * kTileBytes, kOffQ = kOffEntries + kWaves * kEntryBytes;
 constexpr int kOStride = 68;            // floats per row of a partial output parked in LDS
-constexpr int kMergeBytes = kWaves * (kRows * kOStride + 2 * kRows) * 4;
-constexpr int kLoopBytes = kOffQ + 3 * kQPlane * 2;
-constexpr int kLdsBytes = kLoopBytes > kMergeBytes ? kLoopBytes : kMergeBytes;
-static_assert(kLdsBytes <= 160 * 1024, "LDS of a CU");
+constexpr int lbm_f32_lds_bytes(int rows) {
+  const int merge = kWaves * (rows * kOStride + 2 * rows) * 4, loop = kOffQ + 3 * rows * 64 * 2;
+  return loop > merge ? loop : merge;
+}
+static_assert(lbm_f32_lds_bytes(64) <= 160 * 1024, "LDS of a CU");
 constexpr float kSlack = 8.f;           // a score this far above the reference raises it
 
 // value of the other half-wave's lane beside the own one
@@ -99,15 +99,15 @@ __device__ __forceinline__ void split_rounded(f32x8 x, bf16x8 (&p)[3]) {
   }
 }
 // hi[i] += the leading products of a * b[i] over 16 k's, lo[i] += the seven others, small ones first
-__device__ __forceinline__ void mfma_split(const bf16x8 (&a)[3], const bf16x8 (&b0)[3], const bf16x8 (&b1)[3], f32x16 (&hi)[2], f32x16 (&lo)[2]) {
+template <int QB>
+__device__ __forceinline__ void mfma_split(const bf16x8 (&a)[3], const bf16x8 (&b)[QB][3], f32x16 (&hi)[QB], f32x16 (&lo)[QB]) {
   constexpr int pa[7] = {2, 1, 2, 0, 1, 1, 0}, pb[7] = {1, 2, 0, 2, 1, 0, 1};
 #pragma unroll
-  for (int i = 0; i < 7; ++i) {
-    lo[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[i]], b0[pb[i]], lo[0], 0, 0, 0);
-    lo[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[i]], b1[pb[i]], lo[1], 0, 0, 0);
-  }
-  hi[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b0[0], hi[0], 0, 0, 0);
-  hi[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b1[0], hi[1], 0, 0, 0);
+  for (int i = 0; i < 7; ++i)
+#pragma unroll
+    for (int q = 0; q < QB; ++q) lo[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[pa[i]], b[q][pb[i]], lo[q], 0, 0, 0);
+#pragma unroll
+  for (int q = 0; q < QB; ++q) hi[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[q][0], hi[q], 0, 0, 0);
 }
 
 // loads of this wavefront still allowed in flight (expcnt and lgkmcnt untouched), and LDS reads done
@@ -118,9 +118,12 @@ __device__ __forceinline__ void mfma_split(const bf16x8 (&a)[3], const bf16x8 (&
 
 // APPEND: workgroups behind the attention's carry the append; an instance of its own, as asking which a workgroup is costs
 // every launch 0.2 to 0.4 us (400 rows over themselves: 18.3, 18.8)
-template <int S, bool APPEND>
+// QB: blocks of 32 query rows per workgroup, 2 or 1
+template <int S, bool APPEND, int QB>
 __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<S> a) {
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[kLdsBytes];
+  constexpr int kRows = 32 * QB;
+  constexpr int kQPlane = kRows * 64;     // bf16 of a Q plane: unpadded rows, chunk c of row r at c ^ ((r >> 1) & 7)
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[lbm_f32_lds_bytes(kRows)];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n32 = lane & 31, g = lane >> 5;
   // (what the first loads need of the arguments, the first stream's beside the launch's, in one trip,
@@ -152,8 +155,8 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
   if (q_row0 >= sp.q_rows) return;   // padding between streams (whole workgroups)
   const int kv_tokens = max(a.live_kv_tokens ? a.live_kv_tokens[sp.live_at] : sp.kv_tokens, 0);
   const int n_tiles = (kv_tokens + kTile - 1) / kTile, last_token = max(kv_tokens - 1, 0);
-  const int out_row = tid >> 3, out_d = (tid & 7) * 8;   // this thread's part of the result
-  const bool out_ok = q_row0 + out_row < sp.q_rows;
+  const int out_row = (tid >> 3) % kRows, out_d = (tid & 7) * 8;   // this thread's part of the result
+  const bool out_ok = q_row0 + out_row < sp.q_rows && tid < kRows * 8;
   float* out = a.out + ((size_t)(sp.q_begin + q_row0 + out_row) * H + head) * 64 + out_d;
   if (n_tiles == 0) {   // nothing visible: zeros (lingbot_map/layers/flashinfer_cache.py:368-370)
     if (out_ok) ((f32x4*)out)[0] = ((f32x4*)out)[1] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -214,10 +217,10 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
   }
   __syncthreads();
 
-  f32x16 o[2][2];               // o[qb][db][i]: d = 32 db + 8 (i / 4) + 4 g + i % 4, q = 32 qb + n32
-  float m[2], l[2];             // reference of the row, this lane's share of its sum
+  f32x16 o[QB][2];              // o[qb][db][i]: d = 32 db + 8 (i / 4) + 4 g + i % 4, q = 32 qb + n32
+  float m[QB], l[QB];           // reference of the row, this lane's share of its sum
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
     m[qb] = -INFINITY;
     l[qb] = 0.f;
 #pragma unroll
@@ -238,9 +241,9 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
   for (int t = wave; t < n_tiles; t += kWaves) {
     LBM_LOADS_LEFT(9);
     // ---- S^T = K Q^T: s[qb][i] is kv = 8 (i / 4) + 4 g + i % 4, q = 32 qb + n32
-    f32x16 s[2], s_lo[2];
+    f32x16 s[QB], s_lo[QB];
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
+    for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[qb][i] = s_lo[qb][i] = 0.f;
 #pragma unroll
@@ -248,17 +251,17 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
       const int c = ks * 4 + g * 2;
       const f32x4 k0 = *(const f32x4*)(raw_k + n32 * 256 + ((c ^ (n32 & 15)) * 16));
       const f32x4 k1 = *(const f32x4*)(raw_k + n32 * 256 + (((c + 1) ^ (n32 & 15)) * 16));
-      bf16x8 kp[3], qp[2][3];
+      bf16x8 kp[3], qp[QB][3];
       split_truncated(f32x8{k0[0], k0[1], k0[2], k0[3], k1[0], k1[1], k1[2], k1[3]}, kp);
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb)
+      for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
         for (int k = 0; k < 3; ++k)
           qp[qb][k] = *(const bf16x8*)&lds_q[k * kQPlane + (qb * 32 + n32) * 64 + ((ks * 2 + g) ^ ((n32 >> 1) & 7)) * 8];
-      mfma_split(kp, qp[0], qp[1], s, s_lo);
+      mfma_split<QB>(kp, qp, s, s_lo);
     }
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
+    for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[qb][i] += s_lo[qb][i];
     // ---- the next K tile: its entries have landed, this one's fragments are read
@@ -271,14 +274,14 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
     const int n_valid = kv_tokens - t * kTile;
     if (n_valid < kTile) {   // the ragged last tile
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb)
+      for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
         for (int i = 0; i < 16; ++i)
           if (8 * (i >> 2) + 4 * g + (i & 3) >= n_valid) s[qb][i] = -INFINITY;
     }
-    float mx[2];
+    float mx[QB];
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
+    for (int qb = 0; qb < QB; ++qb) {
       float x = s[qb][0];
 #pragma unroll
       for (int i = 1; i < 16; ++i) x = fmaxf(x, s[qb][i]);
@@ -286,9 +289,9 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
       swap_halves(x, lo, hi);
       mx[qb] = fmaxf(lo, hi);
     }
-    if (__builtin_amdgcn_ballot_w64(mx[0] > m[0] + kSlack || mx[1] > m[1] + kSlack)) {   // (always on the first tile)
+    if (__builtin_amdgcn_ballot_w64(mx[0] > m[0] + kSlack || mx[QB - 1] > m[QB - 1] + kSlack)) {   // (always on the first tile)
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) {
+      for (int qb = 0; qb < QB; ++qb) {
         const float to = fmaxf(m[qb], mx[qb]);
         const float alpha = __builtin_amdgcn_exp2f(m[qb] - to);
         m[qb] = to;
@@ -299,9 +302,9 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
           for (int i = 0; i < 16; ++i) o[qb][db][i] *= alpha;
       }
     }
-    bf16x8 p[2][2][3];   // [qb][k-step][plane]: element j is kv = 16 kk + 4 g + j % 4 + 8 (j / 4)
+    bf16x8 p[2][QB][3];   // [k-step][qb][plane]: element j is kv = 16 kk + 4 g + j % 4 + 8 (j / 4)
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
+    for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         f32x8 x;
@@ -310,15 +313,15 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
           x[j] = __builtin_amdgcn_exp2f(s[qb][kk * 8 + j] - m[qb]);
         }
         l[qb] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
-        split_rounded(x, p[qb][kk]);
+        split_rounded(x, p[kk][qb]);
       }
     // ---- O^T += V^T P^T, the tile's sums in registers that held the scores before they join O
     LBM_LOADS_LEFT(9);
 #pragma unroll
     for (int db = 0; db < 2; ++db) {
-      f32x16 hi[2], lo[2];
+      f32x16 hi[QB], lo[QB];
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb)
+      for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) hi[qb][i] = lo[qb][i] = 0.f;
 #pragma unroll
@@ -331,10 +334,10 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
         }
         bf16x8 vp[3];
         split_truncated(x, vp);
-        mfma_split(vp, p[0][kk], p[1][kk], hi, lo);
+        mfma_split<QB>(vp, p[kk], hi, lo);
       }
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb)
+      for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[qb][db][i] += hi[qb][i] + lo[qb][i];
     }
@@ -346,10 +349,10 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
 
   // ---- merge the wavefronts' partial results through LDS
   float* so = (float*)lds + wave * (kRows * kOStride);
-  float* sl = (float*)lds + kWaves * (kRows * kOStride);   // [wave][64] row sums, then [wave][64] references
+  float* sl = (float*)lds + kWaves * (kRows * kOStride);   // [wave][row] row sums, then [wave][row] references
   float* sm = sl + kWaves * kRows;
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
 #pragma unroll
     for (int db = 0; db < 2; ++db)
 #pragma unroll
@@ -430,21 +433,42 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
   }
 }
 
-template <int S>
-int lbm_launch_attn_f32_d64(AttnArgsF32<S>& a, hipStream_t stream) {
+// Blocks of 32 query rows per workgroup: one where all such workgroups are one round of the 256 CUs (a workgroup of two takes half as
+// long again: K and V are split into bf16 for either), or where streams of one length take up to three rounds for two.
+// us, 16 heads, two blocks and one: 86 rows over 430 tokens 19.4, 13.1; 148 over 740 25.3, 16.5; 200 over 1,800 50.3, 31.4; 377 over 2,639
+// 68.6, 44.1; 512 over 4,608 114.6, 86.1; own rows 100 10.3, 7.9, 261 15.7, 10.5, 500 19.9, 14.5; three rounds for two: 1,100 over 5,500
+// 290, 267, 1,374 over 6,870 363, 337, two streams of 600 over 3,000 170, 157; two for one, which stay: 600 over 3,000 80, 100,
+// 1,004 over 8,032 241, 280, four streams of 148 over 740 28.6, 34.8.
+static int lbm_f32_row_blocks(const lbm_attn_stream* s, int n_streams, int num_heads) {
+  long long wgs2 = 0, wgs1 = 0;
+  bool alike = true;
+  for (int i = 0; i < n_streams; ++i) {
+    wgs2 += (long long)((s[i].q_rows + 63) / 64) * num_heads;
+    wgs1 += (long long)((s[i].q_rows + 31) / 32) * num_heads;
+    alike = alike && s[i].kv_tokens == s[0].kv_tokens;
+  }
+  if (wgs1 <= 256) return 1;
+  return alike && 3 * ((wgs1 + 255) / 256) < 5 * ((wgs2 + 255) / 256) ? 1 : 2;
+}
+template <int S, int QB>
+int lbm_launch_attn_f32_d64_rows(AttnArgsF32<S>& a, hipStream_t stream) {
   int wg = 0;
   for (int i = 0; i < S; ++i) {
     if (i < a.n_streams) wg = (wg + 7) & ~7;   // a stream starts on XCD 0, as the kernel's head -> XCD map assumes
     a.wg_begin[i] = wg;
-    if (i < a.n_streams) wg += (a.s[i].q_rows + kRows - 1) / kRows * a.num_heads;
+    if (i < a.n_streams) wg += (a.s[i].q_rows + 32 * QB - 1) / (32 * QB) * a.num_heads;
   }
   a.wg_begin[S] = wg;
   for (int i = a.n_streams; i < S; ++i) a.wg_begin[i] = wg;
   if (wg == 0) return LBM_OK;
   wg += (int)(((long long)a.append_tokens * a.num_heads * 16 + kThreads * kAppendPieces - 1) / (kThreads * kAppendPieces));
-  if (a.append_tokens > 0) hipLaunchKernelGGL((lbm_attn_f32_d64_kernel<S, true>), dim3(wg), dim3(kThreads), 0, stream, a);
-  else hipLaunchKernelGGL((lbm_attn_f32_d64_kernel<S, false>), dim3(wg), dim3(kThreads), 0, stream, a);
+  if (a.append_tokens > 0) hipLaunchKernelGGL((lbm_attn_f32_d64_kernel<S, true, QB>), dim3(wg), dim3(kThreads), 0, stream, a);
+  else hipLaunchKernelGGL((lbm_attn_f32_d64_kernel<S, false, QB>), dim3(wg), dim3(kThreads), 0, stream, a);
   return lbm_check_launch("lbm_attn_f32_d64_kernel");
+}
+template <int S>
+int lbm_launch_attn_f32_d64(AttnArgsF32<S>& a, hipStream_t stream) {
+  return lbm_f32_row_blocks(a.s, a.n_streams, a.num_heads) == 1 ? lbm_launch_attn_f32_d64_rows<S, 1>(a, stream) : lbm_launch_attn_f32_d64_rows<S, 2>(a, stream);
 }
 template int lbm_launch_attn_f32_d64<1>(AttnArgsF32<1>&, hipStream_t);
 template int lbm_launch_attn_f32_d64<LBM_MAX_STREAMS>(AttnArgsF32<LBM_MAX_STREAMS>&, hipStream_t);
