@@ -7,28 +7,37 @@
 #include "tables_logic.h"
 #include "lbm_internal.h"
 
+constexpr int kTableThreads = 1024;
 template <int S>   // streams that there is room for, 1 or LBM_MAX_STREAMS (arguments that nobody reads are copied all the same: 0.2 us of the host)
 struct LbmStepOps { lbm_step_op s[S]; };
 
 // RUN: lbm_rows_at_a_time.  A kernel for each: with both forms of the plan in one, steps of the one-row form take longer
 // (10,000 frames of one token 7.2 us apart, 7.4 in one; 2,000 5.7, 5.8).
+//
+// Between the phases.  A barrier that waits for the stores costs their trip to memory, and the plan's first load stands
+// behind it.  It is needed where a phase reads what one before it wrote; elsewhere a bare one orders the threads: every load of
+// a phase has come back when its stores leave, so no later phase overwrites what is still to be read (an eviction returns
+// pages to where the append took its own, the last thread of the step writes the header that all begin with).  An eviction reads
+// the appended frame only where no window is left; a plan that names the newest frame by the caller's rows reads none of its
+// pages, and of an eviction only the memory lists that one with tokens to keep extends.
 template <int S, int RUN>
-__global__ __launch_bounds__(1024) void lbm_tables_kernel(
-    int32_t* __restrict__ tables, lbm_cache_geom g, LbmStepOps<S> ops, int32_t* append_rows,
+__global__ __launch_bounds__(kTableThreads) void lbm_tables_kernel(
+    int32_t* __restrict__ tables, lbm_cache_geom g, LbmTablesLayout L, LbmPlanDeal deal, int nthr, LbmStepOps<S> ops, int32_t* append_rows,
     int32_t* kv_rows, int32_t* page_ids, int32_t* page_lens) {
   const int b = S == 1 ? 0 : blockIdx.x;
   const lbm_step_op op = ops.s[b];
   // (more than one workgroup per stream only where every stream's operation is a plan alone: the
   // phases in front of it need the barriers below)
-  const int tid = blockIdx.y * blockDim.x + threadIdx.x, nthr = gridDim.y * blockDim.x;
+  const int tid = blockIdx.y * kTableThreads + threadIdx.x;
   if (op.ops == 0) {
     if (append_rows)
       for (int t = tid; t < g.tokens_per_frame; t += nthr) append_rows[op.q_begin + t] = -1;
     return;
   }
-  const LbmTablesLayout L = lbm_tables_layout(g);
   int32_t* st = tables + (long long)b * L.words;
   LbmHdr h = lbm_hdr_load(st);
+  // (all of it here: a bare barrier does not wait for loads that nobody has used yet)
+  asm volatile("" : : "v"(h.fc), "v"(h.na), "v"(h.wh), "v"(h.wc), "v"(h.nf), "v"(h.nfs), "v"(h.nsp), "v"(h.stc), "v"(h.nm), "v"(h.nmp), "v"(h.err));
   if (op.ops & LBM_OP_RESET) {
     lbm_phase_reset(st, g, L, b * g.pages_per_stream, tid, nthr, h);
     __syncthreads();
@@ -39,15 +48,20 @@ __global__ __launch_bounds__(1024) void lbm_tables_kernel(
   }
   if (op.ops & LBM_OP_APPEND) {
     lbm_phase_append(st, g, L, append_rows ? append_rows + op.q_begin : nullptr, tid, nthr, h);
-    __syncthreads();
+    if ((op.ops & LBM_OP_EVICT) && op.sliding_window < 1) __syncthreads();
+    else asm volatile("s_barrier" ::: "memory");
   } else if (append_rows) {
     for (int t = tid; t < g.tokens_per_frame; t += nthr) append_rows[op.q_begin + t] = -1;
   }
   if (op.ops & LBM_OP_EVICT) {
     lbm_phase_evict(st, g, L, op.sliding_window, op.keep_tokens, tid, nthr, h);
-    __syncthreads();
+    asm volatile("s_barrier" ::: "memory");
   }
-  if (op.ops & LBM_OP_PLAN) lbm_phase_plan<RUN>(st, g, L, op, kv_rows, page_ids, page_lens, tid, nthr, h);
+  if (op.ops & LBM_OP_PLAN) {
+    const bool own = (op.ops & LBM_OP_PLAN_NEWEST_SELF) && g.layout != LBM_LAYOUT_TWO_STREAM && !page_ids;
+    if ((op.ops & (LBM_OP_APPEND | LBM_OP_EVICT)) && !(own && !((op.ops & LBM_OP_EVICT) && op.keep_tokens > 0))) __syncthreads();
+    lbm_phase_plan<RUN>(st, g, L, op, kv_rows, page_ids, page_lens, tid, nthr, h, &deal);
+  }
   if (tid == 0) lbm_hdr_store(st, h);
 }
 
@@ -124,18 +138,23 @@ static int lbm_launch_tables_of(int32_t* tables, const lbm_cache_geom& g, int n_
   constexpr int kRowsPerGroup = 4096, kSplitRows = 24576, kMostGroups = 64;
   const int groups = most_rows <= kRowsPerGroup ? 1 : (most_rows + kRowsPerGroup - 1) / kRowsPerGroup;
   const bool wide = groups > 1 && (!changes || most_rows > kSplitRows);
-  const auto kernel = lbm_rows_at_a_time(g) == 4 ? lbm_tables_kernel<S, 4> : lbm_tables_kernel<S, 1>;
+  const int run = lbm_rows_at_a_time(g);
+  const auto kernel = run == 4 ? lbm_tables_kernel<S, 4> : lbm_tables_kernel<S, 1>;
+  const LbmTablesLayout L = lbm_tables_layout(g);
+  auto launch = [&](int wgs, const LbmStepOps<S>& step, int32_t* rows) {
+    const int nthr = wgs * kTableThreads;
+    hipLaunchKernelGGL(kernel, dim3(n_streams, wgs), dim3(kTableThreads), 0, stream, tables, g, L, lbm_plan_deal(L, run, nthr), nthr, step, rows,
+                       kv_rows, page_ids, page_lens);
+    return lbm_check_launch("lbm_tables_kernel");
+  };
   if (changes || !wide) {
     if (wide)
       for (int i = 0; i < n_streams; ++i) o.s[i].ops &= ~kPlanBits;
-    hipLaunchKernelGGL(kernel, dim3(n_streams), dim3(1024), 0, stream, tables, g, o, append_rows, kv_rows, page_ids, page_lens);
-    const int rc = lbm_check_launch("lbm_tables_kernel");
+    const int rc = launch(1, o, append_rows);
     if (rc != LBM_OK || !wide) return rc;
   }
   // (append_rows was written by the launch in front, if it was asked for and there was one)
-  hipLaunchKernelGGL(kernel, dim3(n_streams, groups < kMostGroups ? groups : kMostGroups), dim3(1024), 0, stream,
-                     tables, g, plan, changes ? nullptr : append_rows, kv_rows, page_ids, page_lens);
-  return lbm_check_launch("lbm_tables_kernel");
+  return launch(groups < kMostGroups ? groups : kMostGroups, plan, changes ? nullptr : append_rows);
 }
 
 int lbm_launch_tables(int32_t* tables, const lbm_cache_geom& g, int n_streams,

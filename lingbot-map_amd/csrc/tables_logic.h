@@ -11,6 +11,7 @@
 #define LBM_TABLES_LOGIC_H
 
 #include "../../include/lbm_paged_attn.h"
+#include "tile_logic.h"
 
 #if defined(__HIPCC__)
 #define LBM_HD __host__ __device__ __forceinline__
@@ -23,12 +24,30 @@ struct LbmTablesLayout {
   int tpf;          // tokens of a frame stored in those pages
   int kpm;          // most pages a compacted frame keeps
   int ring_frames;  // capacity of the window ring, in frames
+  int shift;        // of a power-of-two page size, -1: it is none
   int off_free_patch, off_free_special, off_anchor, off_window, off_special;
   int off_mem_pages, off_mem_tcum, off_mem_pcum;
   long long words;
 };
 
 LBM_HD int lbm_ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// Sixteen wavefronts on one CU take the same instructions: a division is 40 of them, 0.3 us of a step that has a dozen.  So the
+// layout is the launch's, pages are found by shifts, frames of the ring without remainders and threads' frames by a
+// reciprocal.  With the barriers that lbm_tables_kernel no longer waits at, us a keyframe's step, before and now: 17 frames of 1,004 tokens
+// 6.8, 6.0, of 261 4.9, 4.1, 5 of 100 4.5, 3.6; 300 of one token 4.6, 3.8; four streams of 1,004 7.0, 6.3; a plan alone 3.7, 3.45.
+// The page and slot of token t of a page list; page sizes are powers of two in every configuration but one (page = patches per frame)
+LBM_HD int lbm_page_of(const LbmTablesLayout& L, int page_size, int t, int& slot) {
+  const int page = L.shift >= 0 ? t >> L.shift : t / page_size;
+  slot = t - page * page_size;
+  return page;
+}
+LBM_HD int lbm_pages_for(const LbmTablesLayout& L, int page_size, int tokens) {
+  int slot;
+  return lbm_page_of(L, page_size, tokens + page_size - 1, slot);
+}
+// a frame's place in the ring, i below twice its frames (head and count are at most its frames each)
+LBM_HD int lbm_ring(const LbmTablesLayout& L, int i) { return i >= L.ring_frames ? i - L.ring_frames : i; }
 
 LBM_HD bool lbm_geom_valid(const lbm_cache_geom& g) {
   if (g.layout != LBM_LAYOUT_TWO_STREAM && g.layout != LBM_LAYOUT_FRAME_PAGES) return false;
@@ -46,6 +65,7 @@ LBM_HD LbmTablesLayout lbm_tables_layout(const lbm_cache_geom& g) {
   L.ppf = lbm_ceil_div(L.tpf, g.page_size);
   L.kpm = two ? 0 : lbm_ceil_div(g.num_special_tokens, g.page_size);
   L.ring_frames = g.patch_pages / L.ppf;
+  L.shift = (g.page_size & (g.page_size - 1)) == 0 ? __builtin_ctz((unsigned)g.page_size) : -1;
   int off = LBM_HDR_WORDS;
   L.off_free_patch = off;   off += g.patch_pages;
   L.off_free_special = off; off += g.special_pages;
@@ -106,14 +126,14 @@ LBM_HD void lbm_phase_rollback(int32_t* st, const lbm_cache_geom& g, const LbmTa
   int new_count = h.stc, n_pop = 0;
   if (two) {
     new_count = h.stc - g.num_special_tokens;
-    n_pop = h.nsp - (new_count > 0 ? lbm_ceil_div(new_count, g.page_size) : 0);
+    n_pop = h.nsp - (new_count > 0 ? lbm_pages_for(L, g.page_size, new_count) : 0);
   }
   if (h.fc <= 0 || (from_window ? h.wc <= 0 : h.na <= 0) || new_count < 0) {
     h.err |= LBM_TERR_ROLLBACK;
     return;
   }
   const int32_t* src = from_window
-      ? st + L.off_window + ((h.wh + h.wc - 1) % L.ring_frames) * L.ppf
+      ? st + L.off_window + lbm_ring(L, h.wh + h.wc - 1) * L.ppf
       : st + L.off_anchor + (h.na - 1) * L.ppf;
   for (int j = tid; j < L.ppf; j += nthr) st[L.off_free_patch + h.nf + j] = src[L.ppf - 1 - j];
   for (int k = tid; k < n_pop; k += nthr)
@@ -134,7 +154,7 @@ LBM_HD void lbm_phase_append(int32_t* st, const lbm_cache_geom& g, const LbmTabl
   const bool two = g.layout == LBM_LAYOUT_TWO_STREAM;
   const int S = g.page_size, n_sp = g.num_special_tokens, T = g.tokens_per_frame;
   const bool to_anchor = h.na < g.scale_frames;
-  const int new_sp = two ? lbm_ceil_div(h.stc + n_sp, S) - h.nsp : 0;
+  const int new_sp = two ? lbm_pages_for(L, S, h.stc + n_sp) - h.nsp : 0;
   int err = 0;
   if (h.nf < L.ppf) err |= LBM_TERR_PATCH_POOL;
   if (!to_anchor && h.wc >= L.ring_frames) err |= LBM_TERR_WINDOW_RING;
@@ -146,19 +166,17 @@ LBM_HD void lbm_phase_append(int32_t* st, const lbm_cache_geom& g, const LbmTabl
   }
   const int32_t* fp = st + L.off_free_patch;
   int32_t* dst = to_anchor ? st + L.off_anchor + h.na * L.ppf
-                           : st + L.off_window + ((h.wh + h.wc) % L.ring_frames) * L.ppf;
+                           : st + L.off_window + lbm_ring(L, h.wh + h.wc) * L.ppf;
   for (int j = tid; j < L.ppf; j += nthr) dst[j] = fp[h.nf - 1 - j];
   if (rows_out) {
     for (int t = tid; t < T; t += nthr) {
       int page, slot;
       if (!two) {
-        page = fp[h.nf - 1 - t / S]; slot = t % S;
+        page = fp[h.nf - 1 - lbm_page_of(L, S, t, slot)];
       } else if (t >= n_sp) {
-        const int i = t - n_sp;
-        page = fp[h.nf - 1 - i / S]; slot = i % S;
+        page = fp[h.nf - 1 - lbm_page_of(L, S, t - n_sp, slot)];
       } else {
-        const int c = h.stc + t, pi = c / S;
-        slot = c % S;
+        const int pi = lbm_page_of(L, S, h.stc + t, slot);
         page = pi < h.nsp ? st[L.off_special + pi] : st[L.off_free_special + h.nfs - 1 - (pi - h.nsp)];
       }
       rows_out[t] = page * 2 * S + slot;
@@ -185,17 +203,17 @@ LBM_HD void lbm_phase_evict(int32_t* st, const lbm_cache_geom& g, const LbmTable
   const bool two = g.layout == LBM_LAYOUT_TWO_STREAM;
   if (two || keep < 0) keep = 0;
   if (keep > g.num_special_tokens) keep = g.num_special_tokens;
-  const int kp = keep ? lbm_ceil_div(keep, g.page_size) : 0;
+  const int kp = keep ? lbm_pages_for(L, g.page_size, keep) : 0;
   if (keep && h.nm + n_ev > g.memory_frames) { h.err |= LBM_TERR_MEMORY_FULL; return; }
   const int per = L.ppf - kp;
   const int32_t* win = st + L.off_window;
   for (int i = tid; i < n_ev * per; i += nthr) {
-    const int e = i / per, j = kp + i % per;
-    st[L.off_free_patch + h.nf + i] = win[((h.wh + e) % L.ring_frames) * L.ppf + j];
+    const int e = n_ev == 1 ? 0 : i / per, j = kp + i - e * per;
+    st[L.off_free_patch + h.nf + i] = win[lbm_ring(L, h.wh + e) * L.ppf + j];
   }
   for (int i = tid; i < n_ev * kp; i += nthr) {
-    const int e = i / kp, j = i % kp;
-    st[L.off_mem_pages + h.nmp + i] = win[((h.wh + e) % L.ring_frames) * L.ppf + j];
+    const int e = n_ev == 1 ? 0 : i / kp, j = i - e * kp;
+    st[L.off_mem_pages + h.nmp + i] = win[lbm_ring(L, h.wh + e) * L.ppf + j];
   }
   if (keep) {
     for (int e = tid; e < n_ev; e += nthr) {
@@ -206,7 +224,7 @@ LBM_HD void lbm_phase_evict(int32_t* st, const lbm_cache_geom& g, const LbmTable
     h.nmp += n_ev * kp;
     h.stc += n_ev * keep;
   }
-  h.wh = (h.wh + n_ev) % L.ring_frames;
+  h.wh = lbm_ring(L, h.wh + n_ev);
   h.wc -= n_ev;
   h.nf += n_ev * per;
 }
@@ -267,19 +285,26 @@ LBM_HD void lbm_plan_run(int32_t* out, const int32_t* anchor, const int32_t* win
 // one-token-per-frame cache by itself (10,000 frames: 1.4 ms).  Eight frames at a time; two where four-row runs leave a
 // thread no more, since a frame that is not there costs its addresses and compares all the same (one workgroup, us a step
 // with eight and with two: 197 tokens x 17 frames 6.1, 5.1; 261 x 17 5.9, 5.0; 1,004 x 5 6.3, 5.3).
+struct LbmPlanDeal { int runs, groups; unsigned per_runs; };
+LBM_HD LbmPlanDeal lbm_plan_deal(const LbmTablesLayout& L, int run, int nthr) {
+  const int runs = lbm_ceil_div(L.tpf, run);
+  return {runs, runs < nthr ? nthr / runs : 1, lbm_per(runs)};
+}
 template <int RUN>
-LBM_HD void lbm_plan_frames(int32_t* out, const int32_t* st, int S, int shift, const LbmTablesLayout& L, const LbmHdr& h,
-                            const lbm_step_op& op, bool newest_self, int limit, int tid, int nthr) {
+LBM_HD void lbm_plan_frames(int32_t* out, const int32_t* st, int S, const LbmTablesLayout& L, const LbmHdr& h, const lbm_step_op& op,
+                            const LbmPlanDeal& deal, bool newest_self, int limit, int tid, int nthr) {
   const int32_t* anchor = st + L.off_anchor;
   const int32_t* win = st + L.off_window;
-  const int runs = lbm_ceil_div(L.tpf, RUN);
-  const int groups = runs < nthr ? nthr / runs : 1;
-  const int my_group = groups > 1 ? tid / runs : 0;
-  const int u_first = groups > 1 ? (my_group < groups ? tid % runs : runs) : tid;
+  const int runs = deal.runs, groups = deal.groups;
+  int my_group = 0, u_first = tid;
+  if (groups > 1) {
+    my_group = lbm_divide(tid, runs, deal.per_runs, u_first);
+    if (my_group >= groups) u_first = runs;
+  }
   for (int u = u_first; u < runs; u += groups > 1 ? runs : nthr) {
     const int t = u * RUN, n_run = RUN == 1 || L.tpf - t >= RUN ? RUN : L.tpf - t;
-    const int pg = shift >= 0 ? t >> shift : t / S;
-    const int slot = t - pg * S;
+    int slot;
+    const int pg = lbm_page_of(L, S, t, slot);
     if (RUN > 1 && h.na + h.wc <= 2 * groups)
       lbm_plan_run<RUN, 2>(out, anchor, win, S, L, h, op.q_begin, newest_self, limit, t, n_run, pg, slot, my_group, groups);
     else
@@ -298,11 +323,11 @@ LBM_HD int lbm_rows_at_a_time(const lbm_cache_geom& g) { return (g.page_size & 3
 // capacity it gives instead) and publishes a count within that bound, so a host/device
 // disagreement cannot make the attention kernel read outside the table (it sets
 // LBM_TERR_KV_COUNT instead).
-// RUN: rows that a thread writes at a time, as lbm_rows_at_a_time says (0: asked here).
+// RUN: rows that a thread writes at a time, as lbm_rows_at_a_time says (0: asked here).  deal: lbm_plan_deal of them and of nthr, or null.
 template <int RUN = 0>
 LBM_HD void lbm_phase_plan(int32_t* st, const lbm_cache_geom& g, const LbmTablesLayout& L,
                            const lbm_step_op& op, int32_t* kv_rows, int32_t* page_ids,
-                           int32_t* page_lens, int tid, int nthr, LbmHdr& h) {
+                           int32_t* page_lens, int tid, int nthr, LbmHdr& h, const LbmPlanDeal* deal = nullptr) {
   const bool two = g.layout == LBM_LAYOUT_TWO_STREAM;
   const int S = g.page_size;
   const int nfr = h.na + h.wc;
@@ -321,24 +346,24 @@ LBM_HD void lbm_phase_plan(int32_t* st, const lbm_cache_geom& g, const LbmTables
   const int32_t* win = st + L.off_window;
   if (kv_rows) {
     int32_t* out = kv_rows + op.kv_row_begin;
-    // token t of a page list sits in page t / S, slot t % S; page sizes are powers of two in
-    // every configuration but one (page = patches per frame), so the common case is a shift
-    const int shift = (S & (S - 1)) == 0 ? __builtin_ctz((unsigned)S) : -1;
-    if (RUN == 4 || (RUN == 0 && lbm_rows_at_a_time(g) == 4)) lbm_plan_frames<4>(out, st, S, shift, L, h, op, newest_self, limit, tid, nthr);
-    else lbm_plan_frames<1>(out, st, S, shift, L, h, op, newest_self, limit, tid, nthr);
+    const int run = RUN ? RUN : lbm_rows_at_a_time(g);
+    const LbmPlanDeal dealt = deal ? *deal : lbm_plan_deal(L, run, nthr);
+    if (RUN == 4 || (RUN == 0 && run == 4)) lbm_plan_frames<4>(out, st, S, L, h, op, dealt, newest_self, limit, tid, nthr);
+    else lbm_plan_frames<1>(out, st, S, L, h, op, dealt, newest_self, limit, tid, nthr);
     if (two) {
       for (int c = tid; c < h.stc; c += nthr) {
-        const int pg = shift >= 0 ? c >> shift : c / S;
-        if (frame_tokens + c < limit) out[frame_tokens + c] = st[L.off_special + pg] * 2 * S + (c - pg * S);
+        int slot;
+        const int pg = lbm_page_of(L, S, c, slot);
+        if (frame_tokens + c < limit) out[frame_tokens + c] = st[L.off_special + pg] * 2 * S + slot;
       }
     } else {
       for (int e = tid; e < h.nm; e += nthr) {
         const int t0 = st[L.off_mem_tcum + e], t1 = st[L.off_mem_tcum + e + 1];
         const int p0 = st[L.off_mem_pcum + e];
         for (int t = 0; t < t1 - t0; ++t) {
-          const int pg = shift >= 0 ? t >> shift : t / S;
-          if (frame_tokens + t0 + t < limit)
-            out[frame_tokens + t0 + t] = st[L.off_mem_pages + p0 + pg] * 2 * S + (t - pg * S);
+          int slot;
+          const int pg = lbm_page_of(L, S, t, slot);
+          if (frame_tokens + t0 + t < limit) out[frame_tokens + t0 + t] = st[L.off_mem_pages + p0 + pg] * 2 * S + slot;
         }
       }
     }

@@ -5,6 +5,8 @@ import math
 import pytest
 import torch
 
+from test_tables_logic_cpu import host_lib  # noqa: F401  (a fixture)
+
 pytestmark = pytest.mark.gpu
 
 BF16_MAX_ABS, BF16_MEAN_ABS = 2e-2, 2e-3
@@ -456,3 +458,38 @@ def test_blocks_and_fixed_order_managers_add_in_the_order_of_the_native_call(fra
     assert torch.equal(a, flagged(fused, scaled, 0.0, k, v))
     assert torch.equal(b, flagged(split, q, 0.125, k, v))
     assert torch.equal(c, flagged(plain, q, 0.125, k, v)) and torch.equal(b, c)
+
+
+@pytest.mark.parametrize("layout,T,page_size,n_sp", [(1, 37, 16, 5), (1, 37, 5, 5), (1, 1, 16, 0), (1, 1500, 4, 3), (0, 37, 8, 5), (0, 20, 7, 6)])
+def test_table_steps_of_any_operations_as_on_one_host_thread(host_lib, layout, T, page_size, n_sp):
+    """300 launches of random operations together (windows down to none, frames evicted that the same step appended, kept
+    tokens, the newest frame as own rows, page tables asked for or not, pools that run out): every word of the tables and
+    of the outputs as the host build of the phases leaves it, one after the other."""
+    import ctypes as C
+    import random
+
+    import lingbot_map_amd._native as N
+    rng, dev, streams = random.Random(T * 100 + page_size), torch.device("cuda:0"), 2
+    ppf = -(-(T - (n_sp if layout == 0 else 0)) // page_size)
+    geom = N.CacheGeom(layout, T, n_sp, page_size, 2, 9 * ppf, 40, 40, 9 * ppf + 40)
+    words, cap = host_lib.lbm_tables_words_host(C.byref(geom)), 16384
+    arrays = [torch.full((n,), -9, dtype=torch.int32) for n in (streams * words, streams * T, streams * cap, streams * cap, streams * cap)]
+    there = [a.to(dev) for a in arrays]
+    for step in range(300):
+        ops = (N.StepOp * streams)()
+        pages = rng.random() < 0.3
+        for b in range(streams):
+            bits = N.OP_RESET if step == 0 or rng.random() < 0.01 else 0
+            bits |= (N.OP_ROLLBACK if rng.random() < 0.15 else 0) | (N.OP_APPEND if rng.random() < 0.7 else 0)
+            bits |= (N.OP_EVICT if rng.random() < 0.6 else 0) | (N.OP_PLAN if rng.random() < 0.7 else 0)
+            if layout == 1 and bits & N.OP_APPEND and bits & N.OP_PLAN and rng.random() < 0.7:
+                bits |= N.OP_PLAN_NEWEST_SELF
+            ops[b] = N.StepOp(bits, rng.choice([0, 1, 2, 2, 3, 5]), rng.choice([-1, 0, 0, n_sp, 1]), rng.choice([0, 0, T]), b * T, b * cap,
+                              -cap, b * cap)
+        p = lambda t, on: C.c_void_p(t.data_ptr()) if on else None
+        on = (True, True, True, pages, pages)
+        assert host_lib.lbm_tables_step_host(p(arrays[0], True), C.byref(geom), streams, ops, *[p(t, o) for t, o in zip(arrays[1:], on[1:])]) == N.OK
+        N.check(N.lib.lbm_tables_step(p(there[0], True), C.byref(geom), streams, ops, *[p(t, o) for t, o in zip(there[1:], on[1:])], None))
+        torch.cuda.synchronize()
+        for a, t in zip(arrays, there):
+            assert torch.equal(a, t.cpu()), (step, [o.ops for o in ops])
