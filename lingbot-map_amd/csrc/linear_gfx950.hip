@@ -607,14 +607,20 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
   // The producer's own inputs - q/k norm weights, every pass's rotary table entries and pool rows -
   // are asked for now as well.
   const int H = p.num_heads;
+  // 256 columns, four heads of q, k or v: the eight lanes of a head's row work on those columns of all four of a token, one set of
+  // entries for the four (the registers hold no more: the second of the tile's two passes asks for its own when it comes)
+  // (without norm and table rows of 512 bytes leave faster, as in the kernel below).
+  constexpr bool kByToken = EPI == kEpiQkvPrepare && TN == 256 && (ROPE != 0 || NORM);
+  constexpr int kTokens = kByToken ? kGM / 64 : kPasses, kRotary = kByToken ? 1 : kPasses;
   struct {
     int c, which, h, c8;
-    lbm_qkv::f32x4 w4[2], b4[2], cs4[kPasses][4];
-    int pool_row[kPasses];
+    lbm_qkv::f32x4 w4[2], b4[2], cs4[kRotary][4];
+    int pool_row[kTokens];
   } pq = {};
+  auto token_of = [&](int j) { return min(m0 + (kByToken ? j * 64 + (tid >> 3) : j * kRowsPerPass + tid / kPieces), p.M - 1); };
   if (EPI == kEpiQkvPrepare) {
     typedef lbm_qkv::f32x4 qf4;
-    pq.c = (tid % kPieces) * 8;
+    pq.c = kByToken ? (tid & 7) * 8 : (tid % kPieces) * 8;
     const int col = n0 + pq.c;                    // column of the projection: [q|k|v][head][64]
     pq.which = col / (H * 64);                    // uniform over the workgroup (H * 64 is a multiple of TN)
     pq.h = (col - pq.which * H * 64) >> 6;
@@ -626,9 +632,9 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
       pq.b4[0] = bp[0]; pq.b4[1] = bp[1];
     }
 #pragma unroll
-    for (int j = 0; j < kPasses; ++j) {
-      const int t = min(m0 + j * kRowsPerPass + tid / kPieces, p.M - 1);
-      if (pq.which < 2) ask_rotary<ROPE>(p, t, pq.c8, pq.cs4[j]);
+    for (int j = 0; j < kTokens; ++j) {
+      const int t = token_of(j);
+      if (pq.which < 2 && j < kRotary) ask_rotary<ROPE>(p, t, pq.c8, pq.cs4[j]);
       pq.pool_row[j] = -1;
       if (pq.which > 0 && p.append_rows) pq.pool_row[j] = p.append_rows[t];
     }
@@ -751,13 +757,28 @@ __global__ __launch_bounds__(lbm_linear_threads(TN), 1) void lbm_linear_bf16_ker
   __syncthreads();
   if (EPI == kEpiQkvPrepare) {
     unsigned short* const plain = produced_rows(p, pq.which);
+    if (kByToken) {
+#pragma unroll
+      for (int j = 0; j < kTokens; ++j) {
+        const int r = j * 64 + (tid >> 3);
+        if (j > 0 && pq.which < 2) ask_rotary<ROPE>(p, token_of(j), pq.c8, pq.cs4[0]);
+        if (pq.which < 2) lbm_qkv::ready_rotary<ROPE>(pq.cs4[0], pq.c8);
+#pragma unroll
+        for (int s = 0; s < TN / 64; ++s) {
+          const u32x2 lo = *(const u32x2*)&stage[r * kCStride + s * 64 + pq.c], hi = *(const u32x2*)&stage[r * kCStride + s * 64 + pq.c + 4];
+          const bf16x8 o8 = produce_row<ROPE, NORM, true>(u32x4{lo[0], lo[1], hi[0], hi[1]}, pq.which, pq.c8, pq.w4, pq.b4, pq.cs4[0], p.eps, pq.which == 0 ? p.q_scale : 1.0f);
+          if (m0 + r < p.M) store_produced(p, plain, o8, pq.which, m0 + r, pq.h + s, pq.c8, pq.pool_row[j]);
+        }
+      }
+      return;
+    }
 #pragma unroll
     for (int j = 0; j < kPasses; ++j) {
       const int r = j * kRowsPerPass + tid / kPieces;
       const u32x2 lo = *(const u32x2*)&stage[r * kCStride + pq.c], hi = *(const u32x2*)&stage[r * kCStride + pq.c + 4];
       // (rows past M are computed on the last token's entries and never stored)
-      const bf16x8 o8 = produce_row<ROPE, NORM>(u32x4{lo[0], lo[1], hi[0], hi[1]}, pq.which, pq.c8, pq.w4, pq.b4, pq.cs4[j], p.eps, pq.which == 0 ? p.q_scale : 1.0f);
-      if (m0 + r < p.M) store_produced(p, plain, o8, pq.which, m0 + r, pq.h, pq.c8, pq.pool_row[j]);
+      const bf16x8 o8 = produce_row<ROPE, NORM>(u32x4{lo[0], lo[1], hi[0], hi[1]}, pq.which, pq.c8, pq.w4, pq.b4, pq.cs4[kByToken ? 0 : j], p.eps, pq.which == 0 ? p.q_scale : 1.0f);
+      if (m0 + r < p.M) store_produced(p, plain, o8, pq.which, m0 + r, pq.h, pq.c8, pq.pool_row[kByToken ? 0 : j]);
     }
     return;
   }
@@ -1459,6 +1480,9 @@ int lbm_linear_rows_tiles(LinearArgs& p, int tn, int splits) {
 // takes 1.35-1.4 rounds of 128 x 128, so two for one gain (M x N x K 8,040 x 1,024 x 4,096: 61 us against
 // 72; 4,100 x 1,024 x 4,096: 44 against 55; 1,200 x 4,096 x 1,024: 21 against 24) and one for one (4,016 x
 // 1,024 x 4,096: 48 against 36) or three for two (8,200 x 1,024 x 4,096: 100 against 94) do not.
+// The qkv projection between one round of 128 x 128 tiles and the first size of the 192-row ones, us with two rounds and with one: without
+// norm and table, interleaved and half-split entries, 16 heads 1,285 rows 18.3, 20.7, 21.3 and 16.2, 19.8, 20.1, 1,900 rows 19.8, 22.5, 23.0 and
+// 16.3, 20.1, 20.4; 12 heads 1,800 rows 17.7, 19.4, 19.8 and 14.8, 18.1, 17.8, 2,600 rows 17.2, 21.9, 23.5 and 14.0, 17.7, 18.0.
 bool lbm_linear_wider(LinearArgs& p) {
   if (p.N % 256 != 0) return false;
   const long long tiles = (long long)p.m_tiles * (p.N / 256);
@@ -1611,7 +1635,7 @@ LinearForm lbm_linear_form(LinearArgs& p, int epilogue, int heads, bool may_spli
   }
   if (may_split) f.splits = lbm_linear_splits(p, epilogue);
   f.rows = lbm_linear_rows_tiles(p, f.tn, f.splits);
-  f.wider = !f.rows && !qkv && f.splits == 1 && f.tn == 128 && lbm_linear_wider(p);
+  f.wider = !f.rows && (!qkv || (heads & 3) == 0) && f.splits == 1 && f.tn == 128 && lbm_linear_wider(p);
   lbm_linear_panels(p, f.rows, f.splits);
   return f;
 }
@@ -1795,10 +1819,11 @@ int lbm_launch_qkv_linear_prepare(const void* a, const lbm_row_norm* a_norm, con
 #undef LBM_QKV_ROWS_T
     return lbm_check_launch("lbm_linear_bf16_rows_kernel<qkv prepare>");
   }
-  const dim3 grid = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles)), block(lbm_linear_threads(128));
+  const dim3 grid = lbm_touch_grid(p.touch, (unsigned)(p.m_tiles * p.n_tiles)), block(lbm_linear_threads(f.wider ? 256 : 128));
 #define LBM_QKV_LAUNCH_L(R, NRM, L)                                                                                   \
   {                                                                                                                   \
-    if (wide) hipLaunchKernelGGL((lbm_linear_bf16_kernel<kEpiQkvPrepare, 128, R, NRM, L>), grid, block, 0, stream, p); \
+    if (f.wider) hipLaunchKernelGGL((lbm_linear_bf16_kernel<kEpiQkvPrepare, 256, R, NRM, L>), grid, block, 0, stream, p); \
+    else if (wide) hipLaunchKernelGGL((lbm_linear_bf16_kernel<kEpiQkvPrepare, 128, R, NRM, L>), grid, block, 0, stream, p); \
     else hipLaunchKernelGGL((lbm_linear_bf16_kernel<kEpiQkvPrepare, 64, R, NRM, L>), grid, block, 0, stream, p);       \
   }
 #define LBM_QKV_LAUNCH(R, NRM)                                                                                        \

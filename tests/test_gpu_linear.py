@@ -244,11 +244,11 @@ def test_qkv_projection_with_the_producer_as_its_epilogue(M, H, K, norm, rope):
 
 
 @pytest.mark.parametrize("norm,rope", [(True, "half_split"), (True, "interleaved"), (False, "half_split"), (True, "none"), (False, "none")])
-@pytest.mark.parametrize("M,H", [(2008, 16), (8321, 4), (3649, 12), (4097, 16), (5377, 12)])
+@pytest.mark.parametrize("M,H", [(2008, 16), (8321, 4), (3649, 12), (4097, 16), (5377, 12), (1281, 16), (1920, 16), (2609, 12)])
 def test_producer_on_tiles_of_four_heads(M, H, norm, rope):
     """As above on tiles of 256 columns - q, k and v heads mixed where there is a norm or a table, four of a kind
     where there is neither - of 128 (2,008 and 8,321 rows), 192 (3,649) and 256 rows (4,097, and 5,377 with one row in the last
-    tile), with a factor on q."""
+    tile), and on 128 x 256 tiles that sum K in two halves (1,281, 1,920 and 2,609 rows; one kind each), with a factor on q."""
     test_qkv_projection_with_the_producer_as_its_epilogue(M, H, 128, norm, rope)
     N, dev, D, K = _native(), torch.device("cuda:0"), 64, 128
     g = torch.Generator().manual_seed(M + H)
