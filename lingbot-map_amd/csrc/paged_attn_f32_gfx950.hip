@@ -292,6 +292,8 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
     if (__builtin_amdgcn_ballot_w64(mx[0] > m[0] + kSlack || mx[QB - 1] > m[QB - 1] + kSlack)) {   // (always on the first tile)
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
+        // (block by block: what a row's sums are rounded against does not depend on how many blocks share its workgroup)
+        if (QB > 1 && !__builtin_amdgcn_ballot_w64(mx[qb] > m[qb] + kSlack)) continue;
         const float to = fmaxf(m[qb], mx[qb]);
         const float alpha = __builtin_amdgcn_exp2f(m[qb] - to);
         m[qb] = to;
@@ -388,15 +390,18 @@ __global__ __launch_bounds__(kThreads) void lbm_attn_f32_d64_kernel(AttnArgsF32<
     }
   }
   // A term of the split of an infinity is NaN, and so is every result that one had a part in - also where
-  // floats give a number (a key at -inf has no weight) or an infinity.  A workgroup that ends with such a
-  // value walks its rows once more, in plain fp32: eight lanes per row, token by token.  A launch with such a
-  // workgroup, or with nothing else, takes 0.44-0.48 ms at 1,004 rows x 1,004 tokens (39 us without) and
+  // floats give a number (a key at -inf has no weight) or an infinity.  A row that ends with such a
+  // value is walked once more, in plain fp32: by its eight lanes, token by token.  (That row alone: the others' bits do not
+  // depend on which rows share their workgroup.)  A launch with such a
+  // row, or with nothing else, takes 0.44-0.48 ms at 1,004 rows x 1,004 tokens (39 us without) and
   // 4.4-4.6 ms at 8,032 tokens (260 us).
   float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   unsigned top = bits(l_tot) & 0x7fffffffu;
 #pragma unroll
   for (int i = 0; i < 8; ++i) top = max(top, bits(acc[i]) & 0x7fffffffu);
-  if (__syncthreads_or(top >= 0x7f800000u)) {
+#pragma unroll
+  for (int x = 1; x < 8; x *= 2) top = max(top, (unsigned)__shfl_xor((int)top, x));
+  if (top >= 0x7f800000u) {
     const f32x4* qp = (const f32x4*)(a.q + ((size_t)(sp.q_begin + min(q_row0 + out_row, sp.q_rows - 1)) * H + head) * 64 + out_d);
     const f32x4 q0 = qp[0] * a.scale_log2, q1 = qp[1] * a.scale_log2;
     float m_row = -INFINITY;
