@@ -1768,6 +1768,7 @@ __device__ __forceinline__ float row_group_sum(float v) {
 // 12.0, 13.6 (two workgroups per CU); head_dim 64, 300 tokens 6.8, 6.2, 5.8.
 template <int S, int D, int NW, int NB, bool ONE, int VS = 1>
 __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs<S> a) {
+#pragma clang fp contract(off)   // (products are fused by name: a stream's result does not depend on how many share its launch)
   constexpr int LPR = D / 4;         // lanes per K/V row, 16 bytes each
   constexpr int RPW = 64 / LPR;      // row groups of a wavefront
   constexpr int G = NW * RPW;        // row groups of the workgroup
@@ -1834,7 +1835,7 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
     float s[NB], mx = m;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      s[j] = row_group_sum<LPR>(k[j][0] * q4[0] + k[j][1] * q4[1] + k[j][2] * q4[2] + k[j][3] * q4[3]);
+      s[j] = row_group_sum<LPR>(fmaf(k[j][3], q4[3], fmaf(k[j][2], q4[2], fmaf(k[j][0], q4[0], k[j][1] * q4[1]))));
       if (t0 + j * G + grp >= t_end) {
         s[j] = -INFINITY;
         v[j] = vec{};   // (the last token's values may be infinite: 0 x inf)
@@ -1845,13 +1846,12 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
     const float ref = mx > -INFINITY ? mx : 0.f;
     const float alpha = __builtin_amdgcn_exp2f(m - ref);
     m = mx;
-    acc *= alpha;
-    l *= alpha;
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       const float p = __builtin_amdgcn_exp2f(s[j] - ref);
-      l += p;
-      acc += v[j] * p;
+      l = j == 0 ? fmaf(l, alpha, p) : l + p;
+#pragma unroll
+      for (int i = 0; i < VE; ++i) acc[i] = j == 0 ? fmaf(acc[i], alpha, v[j][i] * p) : fmaf(v[j][i], p, acc[i]);
     }
   }
   // ---- the row groups of a wavefront, then the wavefronts
@@ -1861,8 +1861,8 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
     const float mt = fmaxf(m, m1), ref = mt > -INFINITY ? mt : 0.f;
     const float w0 = __builtin_amdgcn_exp2f(m - ref), w1 = __builtin_amdgcn_exp2f(m1 - ref);
 #pragma unroll
-    for (int i = 0; i < VE; ++i) acc[i] = acc[i] * w0 + __shfl_xor(acc[i], step) * w1;
-    l = l * w0 + l1 * w1;
+    for (int i = 0; i < VE; ++i) acc[i] = fmaf(acc[i], w0, __shfl_xor(acc[i], step) * w1);
+    l = fmaf(l, w0, l1 * w1);
     m = mt;
   }
   if (lane < LPR) *(vec*)&red_o[wave][VE * ln] = acc;
@@ -1882,8 +1882,8 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
       const float wgt = __builtin_amdgcn_exp2f(red_m[w] - ref);
-      ls[w % kSums] += red_l[w] * wgt;
-      os[w % kSums] += red_o[w][tid] * wgt;
+      ls[w % kSums] = fmaf(red_l[w], wgt, ls[w % kSums]);
+      os[w % kSums] = fmaf(red_o[w][tid], wgt, os[w % kSums]);
     }
     const float o = kSums == 1 ? os[0] : (os[0] + os[kSums / 2]) + (os[1 % kSums] + os[kSums - 1]);
     const float lt = kSums == 1 ? ls[0] : (ls[0] + ls[kSums / 2]) + (ls[1 % kSums] + ls[kSums - 1]);
@@ -1915,11 +1915,14 @@ __global__ __launch_bounds__(NW * 64) void lbm_attn_f32_decode_kernel(DecodeArgs
 // outputs are asked for beside the maxima, before a weight is known, the others' together (40 chunks of 128 floats: six
 // trips as batches of eight behind the weights 4.2 us, two so 4.0).  kBatch is the next of 8, 16 and 32 above the number of
 // chunks: loads of chunks that are not there cost their issue all the same (us a launch, always 32 and these: 8 chunks 3.9,
-// 3.4, 9 to 16 3.9, 3.55; 32 and more are the same either way).
+// 3.4, 9 to 16 3.9, 3.55; 32 and more are the same either way).  The sums have no branches and their products are fused by
+// name: behind a branch per chunk the compiler asked for some of the second batch's outputs only once the chunks before them had
+// been added, and rounded one chunk's products apart from the others'.
 constexpr int kDecMergeBatch = 32;
 static_assert(kDecMaxChunks <= 2 * kDecMergeBatch, "two batches hold every chunk");
 template <int D, int kBatch>
 __device__ __forceinline__ void lbm_decode_merge_row(const float* base, size_t stride, int nc, float* out, float* w, float (*red)[2]) {
+#pragma clang fp contract(off)
   const int tid = threadIdx.x;
   const int d = min(tid, D - 1), c_own = min(tid, nc - 1);      // (loads outside of conditional blocks: they go out together)
   float x[kBatch], m_c = base[c_own * stride + D], l_c = base[c_own * stride + D + 1];
@@ -1933,7 +1936,7 @@ __device__ __forceinline__ void lbm_decode_merge_row(const float* base, size_t s
   __syncthreads();
   m = fmaxf(red[0][0], red[0][1]);
   const float w_c = m_c > -INFINITY ? exp2f(m_c - m) : 0.f;   // a chunk without tokens weighs nothing
-  if (tid < nc) w[tid] = w_c;
+  if (tid < kDecMaxChunks) w[tid] = w_c;      // (0 for a chunk that is not there)
   float l = l_c * w_c;
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) l += __shfl_xor(l, o);
@@ -1943,14 +1946,12 @@ __device__ __forceinline__ void lbm_decode_merge_row(const float* base, size_t s
   if (tid >= D) return;
   float o = 0.f;
 #pragma unroll
-  for (int j = 0; j < kBatch; ++j)
-    if (j < nc) o += x[j] * w[j];
+  for (int j = 0; j < kBatch; ++j) o = fmaf(j < nc ? x[j] : 0.f, w[j], o);
   if (kBatch == kDecMergeBatch && nc > kBatch) {
 #pragma unroll
     for (int j = 0; j < kBatch; ++j) x[j] = base[min(kBatch + j, nc - 1) * stride + tid];
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j)
-      if (kBatch + j < nc) o += x[j] * w[kBatch + j];
+    for (int j = 0; j < kBatch; ++j) o = fmaf(kBatch + j < nc ? x[j] : 0.f, w[kBatch + j], o);
   }
   out[tid] = l > 0.f ? o / l : 0.f;
 }
