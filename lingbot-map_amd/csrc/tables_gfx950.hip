@@ -8,6 +8,10 @@
 #include "lbm_internal.h"
 
 constexpr int kTableThreads = 1024;
+// A barrier that waits for no stores.  It is handed the tables: a kernel's own __restrict__ argument is memory that an asm
+// statement may not touch unless it is given the address, clobbers or not, and loads and stores could move across.
+__device__ __forceinline__ void lbm_bare_barrier(const int32_t* tables) { asm volatile("s_barrier" : : "s"(tables) : "memory"); }
+
 template <int S>   // streams that there is room for, 1 or LBM_MAX_STREAMS (arguments that nobody reads are copied all the same: 0.2 us of the host)
 struct LbmStepOps { lbm_step_op s[S]; };
 
@@ -49,13 +53,13 @@ __global__ __launch_bounds__(kTableThreads) void lbm_tables_kernel(
   if (op.ops & LBM_OP_APPEND) {
     lbm_phase_append(st, g, L, append_rows ? append_rows + op.q_begin : nullptr, tid, nthr, h);
     if ((op.ops & LBM_OP_EVICT) && op.sliding_window < 1) __syncthreads();
-    else asm volatile("s_barrier" ::: "memory");
+    else lbm_bare_barrier(st);
   } else if (append_rows) {
     for (int t = tid; t < g.tokens_per_frame; t += nthr) append_rows[op.q_begin + t] = -1;
   }
   if (op.ops & LBM_OP_EVICT) {
     lbm_phase_evict(st, g, L, op.sliding_window, op.keep_tokens, tid, nthr, h);
-    asm volatile("s_barrier" ::: "memory");
+    lbm_bare_barrier(st);
   }
   if (op.ops & LBM_OP_PLAN) {
     const bool own = (op.ops & LBM_OP_PLAN_NEWEST_SELF) && g.layout != LBM_LAYOUT_TWO_STREAM && !page_ids;
