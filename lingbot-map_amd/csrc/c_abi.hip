@@ -219,6 +219,15 @@ size_t lbm_attn_workspace_bytes(const lbm_attn_stream* streams, int32_t n_stream
   return lbm_attn_schedule_bytes(sch, num_heads, head_dim, false);
 }
 
+// Whether rows that LBM_ATTN_OWN_ROWS promises may be read without their table
+static bool lbm_own_rows_usable(bool own_rows, const void* q, const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads, int32_t head_dim) {
+  // (q travels to LDS directly on the way without a table, 16 bytes a lane; elsewhere it is loaded, from any address)
+  own_rows = own_rows && ((uintptr_t)q & 15) == 0;
+  // (rows are addressed by 32-bit byte offsets from the stream's first)
+  for (int i = 0; own_rows && i < n_streams; ++i) own_rows = (long long)streams[i].kv_tokens * num_heads * head_dim * 2 < (1LL << 32);
+  return own_rows;
+}
+
 static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, void* out, const void* self_k,
                              const void* self_v, const int32_t* kv_rows, const int32_t* live_kv_tokens,
                              const lbm_attn_stream* streams, int32_t n_streams, int32_t num_heads,
@@ -235,10 +244,7 @@ static int lbm_attn_run_impl(const char* who, const void* q, const void* pool, v
   if (live_kv_tokens)
     for (int i = 0; i < n_streams; ++i)
       if (streams[i].live_at < 0) return lbm_fail(LBM_ERR_INVALID, "%s: stream %d has a negative live_at", who, i);
-  // (q travels to LDS directly on the way without a table, 16 bytes a lane; elsewhere it is loaded, from any address)
-  own_rows = own_rows && ((uintptr_t)q & 15) == 0;
-  // (rows are addressed by 32-bit byte offsets from the stream's first)
-  for (int i = 0; own_rows && i < n_streams; ++i) own_rows = (long long)streams[i].kv_tokens * num_heads * head_dim * 2 < (1LL << 32);
+  own_rows = lbm_own_rows_usable(own_rows, q, streams, n_streams, num_heads, head_dim);
   LbmAttnSchedule sch;
   lbm_attn_schedule(streams, n_streams, num_heads, &sch, fixed_order);
   const size_t need = lbm_attn_schedule_bytes(sch, num_heads, head_dim, true);
@@ -350,38 +356,22 @@ int lbm_block_run(const lbm_block_weights* w, const lbm_block_call* c, void* str
   const int tiles = lbm_linear_stats_tiles_for(c->rows, (int)dim);
   const lbm_row_norm norm1 = {c->stats, w->qkv_colsum, c->stats_tiles, w->norm1_eps};
   const lbm_row_norm norm2 = {stats1, w->fc1_colsum, tiles, w->norm2_eps};
-  // Which launch asks for which of the weights ahead (hints[r] is what launch 2 + r reads, the fourth the next block's
-  // first): the nearest of the three before it that can, but rather one of 256-column tiles with idle CUs than one that
-  // would do it by wavefronts beside the computing ones.  Three, since further ahead costs more than it saves once K/V and the
-  // rows of a few streams pass through the memory-side cache in between (ms a frame, three | any before it: two streams of 1,004
-  // rows 8.82 | 9.14, three anchor frames of 666 rows 7.37 | 7.68).  The nearest, since the 64 idle CUs of a qkv launch on 128 x 128
-  // tiles, which L2 binds, take from it what asking for all of them saves (1,004 rows 5.88, by wavefronts in between 5.86);
-  // 256-column tiles leave L2 the time (qkv projection, proj, fc1, fc2 of 2,008 rows: fc1's weights asked for by proj's wavefronts
-  // 66.5 us, by the qkv launch 64.9; of 3,000 rows 87.6, 86.7).
+  // (hints[r] is what launch 2 + r reads, the fourth the next block's first)
+  const bool own_rows = c->own_rows && c->keep_kv && !c->live_kv_tokens;
   int by[4] = {-1, -1, -1, -1};
   if (c->hints[0] || c->hints[1] || c->hints[2] || c->hints[3]) {
     bool attends = false;
     if (c->n_streams > 0 && lbm_check_attn_streams(c->streams, c->n_streams, "lbm_block_run") == LBM_OK) {
       LbmAttnSchedule sch;
       lbm_attn_schedule(c->streams, c->n_streams, w->num_heads, &sch, true);
-      attends = lbm_attention_asks(sch);
+      attends = lbm_attention_asks(sch, lbm_own_rows_usable(own_rows, q, c->streams, c->n_streams, w->num_heads, 64));
     }
     const bool split = c->split_workspace && c->split_workspace_bytes >= lbm_linear_workspace_for(c->rows, (int)dim, w->hidden, LBM_LINEAR_BIAS_RESIDUAL);
     const LbmAsks asks[5] = {lbm_linear_asks(c->rows, 3 * (int)dim, (int)dim, 0, w->num_heads, false), attends ? LBM_ASKS_IDLE : LBM_ASKS_NOT,
                          lbm_linear_asks(c->rows, (int)dim, (int)dim, LBM_LINEAR_BIAS_RESIDUAL, 0, false),
                          lbm_linear_asks(c->rows, w->hidden, (int)dim, LBM_LINEAR_BIAS_GELU, 0, false),
                          lbm_linear_asks(c->rows, (int)dim, w->hidden, LBM_LINEAR_BIAS_RESIDUAL, 0, split)};
-    for (int r = 0; r < 4; ++r) {
-      const int first = r > 0 ? r - 1 : 0;
-      for (int l = 1 + r; l >= first && by[r] < 0; --l)
-        if (asks[l] != LBM_ASKS_NOT) by[r] = l;
-      if (by[r] >= 0 && asks[by[r]] == LBM_ASKS_WAVES)
-        for (int l = by[r] - 1; l >= first; --l)
-          if (asks[l] == LBM_ASKS_WIDE_IDLE) {
-            by[r] = l;
-            break;
-          }
-    }
+    lbm_deal_hints(asks, by);
   }
   auto hint = [&](int launch) {
     lbm_set_prefetch_hint(nullptr, 0);
@@ -401,7 +391,7 @@ int lbm_block_run(const lbm_block_weights* w, const lbm_block_call* c, void* str
     rc = lbm_attn_run_impl("lbm_block_run", q, c->pool ? c->pool : k, heads, c->keep_kv ? k : nullptr, c->keep_kv ? v : nullptr,
                            c->kv_rows, c->live_kv_tokens, c->streams, c->n_streams, w->num_heads, 64, c->page_size, LBM_DTYPE_BF16,
                            0.f, c->attn_workspace, c->attn_workspace_bytes, stream, nullptr, 0, false,
-                           c->own_rows && c->keep_kv && !c->live_kv_tokens, true, &touch);
+                           own_rows, true, &touch);
     if (rc != LBM_OK) return rc;
   }
   hint(2);

@@ -46,9 +46,7 @@ void lbm_take_prefetch_hint(LbmTouch& t);
 // The grid of a launch of `wgs` workgroups, one a CU: with t.wgs more that ask for t's ranges where its last round leaves
 // kTouchIdle CUs without work (16 or 64: within 0.5 % of a frame for most sizes, but 16 three anchor frames of 666 rows 8 % slower).
 dim3 lbm_touch_grid(LbmTouch& t, unsigned wgs);
-// How lbm_linear_norm (heads 0) or the qkv projection of so many heads would ask for a hint: not at all, by wavefronts beside the
-// computing ones, by workgroups of their own on idle CUs, and that beside tiles of 256 columns
-enum LbmAsks { LBM_ASKS_NOT, LBM_ASKS_WAVES, LBM_ASKS_IDLE, LBM_ASKS_WIDE_IDLE };
+// How lbm_linear_norm (heads 0) or the qkv projection of so many heads would ask for a hint
 LbmAsks lbm_linear_asks(int M, int N, int K, int epilogue, int heads, bool may_split);
 size_t lbm_linear_workspace_for(int M, int N, int K, int epilogue);
 
@@ -116,8 +114,9 @@ int lbm_launch_attention(const void* q, const void* pool, void* out, const void*
                          void* workspace, size_t workspace_bytes, hipStream_t stream,
                          const int32_t* append_rows = nullptr, int append_tokens = 0, bool append_apart = false,
                          bool own_rows = false, const LbmTouch* touch = nullptr);
-// whether such a launch has CUs to spare for the workgroups that ask for a hint
-bool lbm_attention_asks(const LbmAttnSchedule& sch);
+// Whether such a launch (bf16, no live counts, nothing to append) carries workgroups that ask for a hint: its kernel has them
+// and CUs are idle
+bool lbm_attention_asks(const LbmAttnSchedule& sch, bool own_rows);
 
 #ifdef __HIPCC__
 // 16 or 8 bytes stored past the L2 (device scope), for results that whole lines of neighbouring lanes leave.  A kernel ends

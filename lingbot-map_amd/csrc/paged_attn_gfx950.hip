@@ -2356,7 +2356,31 @@ size_t lbm_attn_schedule_bytes(const LbmAttnSchedule& sch, int num_heads, int he
   return split_kv > few_q ? split_kv : few_q;
 }
 
-bool lbm_attention_asks(const LbmAttnSchedule& sch) { return lbm_idle_cus(sch.total_wgs) >= kTouchIdle; }
+namespace {
+// The kernel that a launch on the split-KV schedule takes; own_rows: in order, with no live counts and nothing to append.
+enum LbmSplitForm { kFormTable, kFormPair, kFormWhole };
+LbmSplitForm lbm_split_form(const LbmAttnSchedule& sch, bool own_rows) {
+  // Own rows in order, two splits per stream: both in one workgroup, no launch to merge (lbm_attn_split's PAIR).  us, two
+  // kernels and this one: 16 heads, four streams of 833 rows 28.7, 18.8, of 1,004 32.0, 22.3, of 3,000 154, 140, of 5,000
+  // 383, 361; 2 x 2,000 43.9, 34.9; 1 x 4,096 68.8, 61.0; four streams of 513 rows over 4,609 60.4, 56.1; from the line on,
+  // eight streams of 257 rows over 4,097 54.1, 48.8, 12 heads 51.8, 47.8, of 300 52.1, 49.2, of 448 56.8, 50.7; six of 257
+  // 58.8, 54.7; eight of 385 over 1,500 32.2, 25.9.  Up to 256 rows, which leave it half as many workgroups and those with half a
+  // load each, the two kernels stay: eight streams of 40 rows over 4,097 45.8, 54.6; 12 heads, 255 rows over 4,223 44.5, 51.9.
+  bool pair = own_rows;
+  for (int i = 0; i < sch.n_streams; ++i) pair = pair && sch.s[i].n_splits == 2 && 2 * sch.s[i].q_rows > kQTile;
+  if (pair) return kFormPair;
+  // The same in one split.  us, with the table and without, 16 heads: 6 streams of 600 rows 21.6, 20.7; 8 x 1,004
+  // 39.7, 38.7; 3 x 1,500 61.7, 58.3; 16 x 100 over 4,097 76.1, 71.6.
+  bool whole = own_rows;
+  for (int i = 0; i < sch.n_streams; ++i) whole = whole && sch.s[i].n_splits == 1;
+  return whole ? kFormWhole : kFormTable;
+}
+}  // namespace
+
+// (the kernels of own rows have no workgroups that ask)
+bool lbm_attention_asks(const LbmAttnSchedule& sch, bool own_rows) {
+  return (sch.small || lbm_split_form(sch, own_rows) == kFormTable) && lbm_idle_cus(sch.total_wgs) >= kTouchIdle;
+}
 
 namespace {
 int lbm_launch_attention_only(const void* q, const void* pool, void* out, const void* self_k,
@@ -2545,15 +2569,8 @@ int lbm_launch_bf16(const AttnCore& core, const LbmAttnSchedule& sch, hipStream_
     else hipLaunchKernelGGL((lbm_attn_bf16_d64_small_kernel<S, 1, false>), grid, block, 0, stream, a);
     return lbm_check_launch("lbm_attn_bf16_d64_small_kernel");
   }
-  // Own rows in order, two splits per stream: both in one workgroup, no launch to merge (lbm_attn_split's PAIR).  us, two
-  // kernels and this one: 16 heads, four streams of 833 rows 28.7, 18.8, of 1,004 32.0, 22.3, of 3,000 154, 140, of 5,000
-  // 383, 361; 2 x 2,000 43.9, 34.9; 1 x 4,096 68.8, 61.0; four streams of 513 rows over 4,609 60.4, 56.1; from the line on,
-  // eight streams of 257 rows over 4,097 54.1, 48.8, 12 heads 51.8, 47.8, of 300 52.1, 49.2, of 448 56.8, 50.7; six of 257
-  // 58.8, 54.7; eight of 385 over 1,500 32.2, 25.9.  Up to 256 rows, which leave it half as many workgroups and those with half a
-  // load each, the two kernels stay: eight streams of 40 rows over 4,097 45.8, 54.6; 12 heads, 255 rows over 4,223 44.5, 51.9.
-  bool pair = own_rows && !a.live_kv_tokens && append_tokens <= 0;
-  for (int i = 0; i < sch.n_streams; ++i) pair = pair && sch.s[i].n_splits == 2 && 2 * sch.s[i].q_rows > kQTile;
-  if (pair) {
+  const LbmSplitForm form = lbm_split_form(sch, own_rows && !a.live_kv_tokens && append_tokens <= 0);
+  if (form == kFormPair) {
     int wg = 0;
     for (int i = 0; i < sch.n_streams; ++i) {
       LbmAttnStreamPlan& p = a.s[i];
@@ -2566,11 +2583,7 @@ int lbm_launch_bf16(const AttnCore& core, const LbmAttnSchedule& sch, hipStream_
     hipLaunchKernelGGL(lbm_attn_bf16_d64_pair_kernel<S>, dim3((unsigned)wg), dim3(kThreads), 0, stream, a);
     return lbm_check_launch("lbm_attn_bf16_d64_pair_kernel");
   }
-  // The same in one split.  us, with the table and without, 16 heads: 6 streams of 600 rows 21.6, 20.7; 8 x 1,004
-  // 39.7, 38.7; 3 x 1,500 61.7, 58.3; 16 x 100 over 4,097 76.1, 71.6.
-  bool whole = own_rows && !a.live_kv_tokens && append_tokens <= 0;
-  for (int i = 0; i < sch.n_streams; ++i) whole = whole && sch.s[i].n_splits == 1;
-  if (whole) {
+  if (form == kFormWhole) {
     hipLaunchKernelGGL(lbm_attn_bf16_d64_own_kernel<S>, dim3((unsigned)sch.total_wgs), dim3(kThreads), 0, stream, a);
     return lbm_check_launch("lbm_attn_bf16_d64_own_kernel");
   }

@@ -22,6 +22,33 @@ struct LbmTouch {
 LBM_TOUCH_FN int lbm_idle_cus(long long wgs) { return (int)((256 - wgs % 256) % 256); }
 constexpr int kTouchIdle = 32;
 
+// How a launch would ask for a hint: not at all, by wavefronts beside the computing ones, by workgroups of their own on idle CUs,
+// and that beside tiles of 256 columns
+enum LbmAsks { LBM_ASKS_NOT, LBM_ASKS_WAVES, LBM_ASKS_IDLE, LBM_ASKS_WIDE_IDLE };
+// Which of a block's five launches (qkv projection, attention, proj, fc1, fc2) asks for which of the weights ahead, -1: none.  by[r]
+// is for what launch 2 + r reads, the fourth the next block's first: the nearest of the three before it that can, but
+// rather one of 256-column tiles with idle CUs than one that
+// would do it by wavefronts beside the computing ones.  Three, since further ahead costs more than it saves once K/V and the
+// rows of a few streams pass through the memory-side cache in between (ms a frame, three | any before it: two streams of 1,004
+// rows 8.82 | 9.14, three anchor frames of 666 rows 7.37 | 7.68).  The nearest, since the 64 idle CUs of a qkv launch on 128 x 128
+// tiles, which L2 binds, take from it what asking for all of them saves (1,004 rows 5.88, by wavefronts in between 5.86);
+// 256-column tiles leave L2 the time (qkv projection, proj, fc1, fc2 of 2,008 rows: fc1's weights asked for by proj's wavefronts
+// 66.5 us, by the qkv launch 64.9; of 3,000 rows 87.6, 86.7).
+LBM_TOUCH_FN void lbm_deal_hints(const LbmAsks (&asks)[5], int (&by)[4]) {
+  for (int r = 0; r < 4; ++r) {
+    const int first = r > 0 ? r - 1 : 0;
+    by[r] = -1;
+    for (int l = 1 + r; l >= first && by[r] < 0; --l)
+      if (asks[l] != LBM_ASKS_NOT) by[r] = l;
+    if (by[r] >= 0 && asks[by[r]] == LBM_ASKS_WAVES)
+      for (int l = by[r] - 1; l >= first; --l)
+        if (asks[l] == LBM_ASKS_WIDE_IDLE) {
+          by[r] = l;
+          break;
+        }
+  }
+}
+
 // A thread's place: every `step`-th line from `first` on of the part of an XCD (all lines where xcd_shift is 0, else its
 // eighth of each range); step 0: none.
 struct LbmTouchPlace { unsigned xcd, xcd_shift, first, step; };
