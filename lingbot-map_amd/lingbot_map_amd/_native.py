@@ -112,6 +112,9 @@ def _load():
         raise RuntimeError(
             f"HIP library {LIB_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
             "(there is no CPU fallback for this path)")
+    # torch's libraries first, its HIP runtime among them: loaded before it, the library brings ROCm's own, and of two
+    # runtimes in a process one finds no device
+    import torch  # noqa: F401
     lib = C.CDLL(LIB_PATH)
     p, i32, vp = C.POINTER, C.c_int32, C.c_void_p
     lib.lbm_abi_version.restype = C.c_int
@@ -181,7 +184,6 @@ def _load_host():
     """The extension module of the attention calls' host side (``csrc/host_calls.cpp``)."""
     if not os.path.exists(HOST_PATH):
         raise RuntimeError(f"{HOST_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'`")
-    import torch  # noqa: F401  (its libraries first)
     loader = importlib.machinery.ExtensionFileLoader("lbm_host", HOST_PATH)
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader("lbm_host", loader))
     loader.exec_module(module)

@@ -106,3 +106,13 @@ def test_workspace_query_is_zero_where_nothing_is_split():
     arr = (N.AttnStream * 8)(*[N.AttnStream(i * 1004, 1004, i * 5000, 5000, 0) for i in range(8)])
     assert N.lib.lbm_attn_workspace_bytes(arr, 8, 16, 64) == 0
     assert N.lib.lbm_attn_workspace_bytes((N.AttnStream * 1)(N.AttnStream(0, 1004, 0, 1004, 0)), 1, 16, 64) == 0
+
+
+def test_one_hip_runtime_whichever_is_imported_first():
+    """Imported before torch the package still uses torch's HIP runtime: of two in a process one finds no device."""
+    import subprocess
+    import sys
+    show = "import os; print(*{os.path.realpath(l.split()[-1]) for l in open('/proc/self/maps') if 'libamdhip64' in l}, sep='\\n')"
+    seen = [subprocess.run([sys.executable, "-c", f"import sys; sys.path.insert(0, {os.path.join(ROOT, 'lingbot-map_amd')!r}); {first}; {show}"],
+                           stdout=subprocess.PIPE, text=True, check=True).stdout.split() for first in ("import lingbot_map_amd", "import torch, lingbot_map_amd")]
+    assert len(seen[0]) == 1 and seen[0] == seen[1]
