@@ -389,7 +389,8 @@ typedef struct lbm_block_call {
                                /* keep_kv: kv_rows names rows of this call (negative entries);
                                 * n_streams 0: no attention, the caller filled its output */
   const void* hints[4];        /* memory to ask for ahead (lbm_linear_prefetch_hint): what proj, fc1, fc2 and the launch behind
-                                * this block read, each asked for by the one launch before it that can do so at least cost; NULL: none */
+                                * this block read, each asked for by the one launch before it that can do so at least cost; NULL: none.
+                                * None outlives the call. */
   size_t hint_bytes[4];
   int32_t own_rows;            /* ABI 11; 1: kv_rows is as LBM_ATTN_OWN_ROWS says (with keep_kv) */
 } lbm_block_call;

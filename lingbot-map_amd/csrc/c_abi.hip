@@ -141,7 +141,9 @@ int lbm_linear_norm(const void* a, const lbm_row_norm* a_norm, const void* w, co
 }
 
 int lbm_linear_prefetch_hint(const void* next_read, size_t bytes) {
-  lbm_set_prefetch_hint(next_read, next_read ? bytes : 0);
+  LbmTouch t = {};
+  lbm_add_touch(t, next_read, bytes);
+  lbm_set_prefetch_hint(t);
   return LBM_OK;
 }
 
@@ -373,38 +375,42 @@ int lbm_block_run(const lbm_block_weights* w, const lbm_block_call* c, void* str
                          lbm_linear_asks(c->rows, (int)dim, w->hidden, LBM_LINEAR_BIAS_RESIDUAL, 0, split)};
     lbm_deal_hints(asks, by);
   }
-  auto hint = [&](int launch) {
-    lbm_set_prefetch_hint(nullptr, 0);
+  // Nothing that the call names outlives it: the memory may not.
+  auto ahead = [&](int launch) {
+    LbmTouch t = {};
     for (int r = 0; r < 4; ++r)
-      if (by[r] == launch) lbm_add_prefetch_hint(c->hints[r], c->hint_bytes[r]);
+      if (by[r] == launch) lbm_add_touch(t, c->hints[r], c->hint_bytes[r]);
+    return t;
   };
-  hint(0);
+  auto ended = [&](int rc) {
+    if (rc != LBM_OK) lbm_set_prefetch_hint({});
+    return rc;
+  };
+  lbm_set_prefetch_hint(ahead(0));
   int rc = lbm_qkv_linear_prepare_norm(c->a, c->stats ? &norm1 : nullptr, w->qkv_w, w->qkv_b, c->rows, (int32_t)dim, w->q_norm_w,
                                        w->q_norm_b, w->k_norm_w, w->k_norm_b, w->qk_eps, c->q_scale, c->rope_cs, c->rope_layout, q,
                                        c->keep_kv ? k : nullptr, c->keep_kv ? v : nullptr, c->pool, c->append_rows, w->num_heads, 64,
                                        c->page_size, stream);
-  if (rc != LBM_OK) return rc;
+  if (ended(rc) != LBM_OK) return rc;
   if (c->n_streams > 0) {
-    hint(1);
-    LbmTouch touch;
-    lbm_take_prefetch_hint(touch);
+    const LbmTouch touch = ahead(1);
     rc = lbm_attn_run_impl("lbm_block_run", q, c->pool ? c->pool : k, heads, c->keep_kv ? k : nullptr, c->keep_kv ? v : nullptr,
                            c->kv_rows, c->live_kv_tokens, c->streams, c->n_streams, w->num_heads, 64, c->page_size, LBM_DTYPE_BF16,
                            0.f, c->attn_workspace, c->attn_workspace_bytes, stream, nullptr, 0, false,
                            own_rows, true, &touch);
     if (rc != LBM_OK) return rc;
   }
-  hint(2);
+  lbm_set_prefetch_hint(ahead(2));
   rc = lbm_linear_norm(heads, nullptr, w->proj_w, w->proj_b, w->ls1, c->x, x1, stats1, c->rows, (int32_t)dim, (int32_t)dim,
                        LBM_LINEAR_BIAS_RESIDUAL, nullptr, 0, stream);
-  if (rc != LBM_OK) return rc;
-  hint(3);
+  if (ended(rc) != LBM_OK) return rc;
+  lbm_set_prefetch_hint(ahead(3));
   rc = lbm_linear_norm(x1, &norm2, w->fc1_w, w->fc1_b, nullptr, nullptr, hidden, nullptr, c->rows, w->hidden, (int32_t)dim,
                        LBM_LINEAR_BIAS_GELU, nullptr, 0, stream);
-  if (rc != LBM_OK) return rc;
-  hint(4);
-  return lbm_linear_norm(hidden, nullptr, w->fc2_w, w->fc2_b, w->ls2, x1, c->out, c->out_stats, c->rows, (int32_t)dim, w->hidden,
-                         LBM_LINEAR_BIAS_RESIDUAL, c->split_workspace, c->split_workspace_bytes, stream);
+  if (ended(rc) != LBM_OK) return rc;
+  lbm_set_prefetch_hint(ahead(4));
+  return ended(lbm_linear_norm(hidden, nullptr, w->fc2_w, w->fc2_b, w->ls2, x1, c->out, c->out_stats, c->rows, (int32_t)dim, w->hidden,
+                               LBM_LINEAR_BIAS_RESIDUAL, c->split_workspace, c->split_workspace_bytes, stream));
 }
 
 }  // extern "C"

@@ -40,8 +40,7 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
                       void* workspace, size_t workspace_bytes, hipStream_t stream);
 int lbm_linear_stats_tiles_for(int M, int N);
 
-void lbm_set_prefetch_hint(const void* ptr, size_t bytes);   // the calling thread's next launch asks for this alone
-void lbm_add_prefetch_hint(const void* ptr, size_t bytes);   // for this too, up to kTouchRanges ranges
+void lbm_set_prefetch_hint(const LbmTouch& t);   // the calling thread's next launch asks for these ranges alone
 void lbm_take_prefetch_hint(LbmTouch& t);
 // The grid of a launch of `wgs` workgroups, one a CU: with t.wgs more that ask for t's ranges where its last round leaves
 // kTouchIdle CUs without work (16 or 64: within 0.5 % of a frame for most sizes, but 16 three anchor frames of 666 rows 8 % slower).

@@ -1578,19 +1578,7 @@ namespace {
 thread_local LbmTouch g_prefetch_hint = {};
 }  // namespace
 
-void lbm_set_prefetch_hint(const void* ptr, size_t bytes) {
-  g_prefetch_hint = {};
-  lbm_add_prefetch_hint(ptr, bytes);
-}
-void lbm_add_prefetch_hint(const void* ptr, size_t bytes) {
-  if (!ptr || bytes < 128) return;
-  for (int r = 0; r < kTouchRanges; ++r)
-    if (!g_prefetch_hint.lines[r]) {
-      g_prefetch_hint.at[r] = (const char*)ptr;
-      g_prefetch_hint.lines[r] = (unsigned)(bytes / 128);
-      return;
-    }
-}
+void lbm_set_prefetch_hint(const LbmTouch& t) { g_prefetch_hint = t; }
 void lbm_take_prefetch_hint(LbmTouch& t) {
   t = g_prefetch_hint;
   g_prefetch_hint = {};
@@ -1653,7 +1641,7 @@ int lbm_launch_linear(const void* a, const lbm_row_norm* a_norm, const void* w, 
                       const void* residual, void* out, float* out_stats, int M, int N, int K, int epilogue,
                       void* workspace, size_t workspace_bytes, hipStream_t stream) {
   if (M == 0) {
-    lbm_set_prefetch_hint(nullptr, 0);   // a hint is for the next call, whatever that call does
+    lbm_set_prefetch_hint({});   // a hint is for the next call, whatever that call does
     return LBM_OK;
   }
   if (K % kGK != 0 || N % 64 != 0)

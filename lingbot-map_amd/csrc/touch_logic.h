@@ -22,6 +22,17 @@ struct LbmTouch {
 LBM_TOUCH_FN int lbm_idle_cus(long long wgs) { return (int)((256 - wgs % 256) % 256); }
 constexpr int kTouchIdle = 32;
 
+// one range more, up to kTouchRanges
+LBM_TOUCH_FN void lbm_add_touch(LbmTouch& t, const void* ptr, size_t bytes) {
+  if (!ptr || bytes < 128) return;
+  for (int r = 0; r < kTouchRanges; ++r)
+    if (!t.lines[r]) {
+      t.at[r] = (const char*)ptr;
+      t.lines[r] = (unsigned)(bytes / 128);
+      return;
+    }
+}
+
 // How a launch would ask for a hint: not at all, by wavefronts beside the computing ones, by workgroups of their own on idle CUs,
 // and that beside tiles of 256 columns
 enum LbmAsks { LBM_ASKS_NOT, LBM_ASKS_WAVES, LBM_ASKS_IDLE, LBM_ASKS_WIDE_IDLE };

@@ -10,6 +10,17 @@ extern "C" void lbm_hints_deal(const int* asks, int* by) {
   for (int r = 0; r < 4; ++r) by[r] = to[r];
 }
 
+// The calling thread's pending hint: its ranges' addresses and 128-byte lines; it stays pending.
+extern "C" void lbm_hints_pending(long long* at, unsigned* lines) {
+  LbmTouch t;
+  lbm_take_prefetch_hint(t);
+  for (int r = 0; r < kTouchRanges; ++r) {
+    at[r] = t.lines[r] ? (long long)(size_t)t.at[r] : 0;
+    lines[r] = t.lines[r];
+  }
+  lbm_set_prefetch_hint(t);
+}
+
 // One attention launch in a fixed order: its rows per workgroup on the short-KV kernel (0: the split-KV schedule), its workgroups
 // and each stream's splits; whether it asks for a hint.
 extern "C" int lbm_hints_attention(const lbm_attn_stream* streams, int n, int heads, int own_rows, int* small, int* wgs, int* splits) {

@@ -1,4 +1,4 @@
-"""Which launch of a block asks for which of the weights ahead (csrc/touch_logic.h, ``lbm_attention_asks``), on the CPU: a hint goes to
+"""Which launch of a block asks for which of the weights ahead (csrc/touch_logic.h, ``lbm_attention_asks``): a hint goes to
 a launch that asks for it, whenever one of those that may can."""
 import ctypes as C
 import itertools
@@ -61,3 +61,46 @@ def test_attention_of_several_frames_leaves_hints_to_others(host):
     arr = (N.AttnStream * 6)(*[N.AttnStream(i * 1004, 1004, i * 1004, 1004, 0) for i in range(6)])
     assert host.lbm_hints_attention(arr, 6, 16, 0, C.byref(small), C.byref(wgs), splits) == 1 and not small.value
     assert host.lbm_hints_attention(arr, 6, 16, 1, C.byref(small), C.byref(wgs), splits) == 0
+
+
+def _pending(host):
+    at, lines = (C.c_longlong * 4)(), (C.c_uint * 4)()
+    host.lbm_hints_pending(at, lines)
+    return [(a, n) for a, n in zip(at, lines) if n]
+
+
+def _refused_block(hints):
+    """A block of one head, whose 64 columns the first linear refuses; nothing is launched and no address read."""
+    p = 1 << 40
+    w = N.BlockWeights(*[p] * 8, None, p, *[None] * 6, 0.0, 1e-5, 1e-5, 1, 256)
+    call = N.BlockCall(p, p, None, p, None, p, None, None, None, p, None, None, p, None, 1 << 30, 0, 0, 1.0, 4, 0, 0, 1, 0, 16, hints, (4096,) * 4, 1)
+    assert N.lib.lbm_block_run(w, call, None) != N.OK
+    assert b"multiple of 128" in N.lib.lbm_last_error()
+
+
+def test_a_refused_block_leaves_no_hint_of_its_own(host):
+    N.lib.lbm_linear_prefetch_hint(None, 0)
+    _refused_block(tuple((2 << 40) + i * 4096 for i in range(4)))
+    assert _pending(host) == []
+    _refused_block((None,) + tuple((2 << 40) + i * 4096 for i in range(3)))
+    assert _pending(host) == []
+
+
+@pytest.mark.gpu
+def test_a_block_refused_at_its_last_linear_leaves_no_hint(host):
+    """192 hidden columns: fc1 takes them, fc2 does not; the first three launches have run."""
+    import torch
+    dev = torch.device("cuda:0")
+    rows, dim, hidden = 8, 128, 192
+    mem = torch.zeros(1 << 22, dtype=torch.uint8, device=dev)
+    p = mem.data_ptr()
+    w = N.BlockWeights(*[p] * 4, None, None, None, None, None, p, *[None] * 6, 0.0, 1e-5, 1e-5, 2, hidden)
+    need = int(N.lib.lbm_block_scratch_bytes(rows, 2, hidden))
+    scratch = torch.zeros(need, dtype=torch.uint8, device=dev)
+    out = torch.zeros(rows, dim, dtype=torch.bfloat16, device=dev)
+    for hints in ((p,) * 4, (None,) * 3 + (p,)):
+        call = N.BlockCall(p, p, None, out.data_ptr(), None, scratch.data_ptr(), None, None, None, p, None, None, None, None, need, 0, 0, 1.0,
+                           rows, 0, 0, 1, 0, 16, hints, (4096,) * 4, 1)
+        assert N.lib.lbm_block_run(w, call, None) != N.OK and b"multiple of 128" in N.lib.lbm_last_error()
+        torch.cuda.synchronize()
+        assert _pending(host) == []
