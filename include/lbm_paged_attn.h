@@ -390,7 +390,7 @@ typedef struct lbm_block_call {
                                 * n_streams 0: no attention, the caller filled its output */
   const void* hints[4];        /* memory to ask for ahead (lbm_linear_prefetch_hint): what proj, fc1, fc2 and the launch behind
                                 * this block read, each asked for by the one launch before it that can do so at least cost; NULL: none.
-                                * None outlives the call. */
+                                * With hints[0] NULL the first launch takes a hint given beforehand.  None outlives the call. */
   size_t hint_bytes[4];
   int32_t own_rows;            /* ABI 11; 1: kv_rows is as LBM_ATTN_OWN_ROWS says (with keep_kv) */
 } lbm_block_call;

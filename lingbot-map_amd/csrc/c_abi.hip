@@ -375,9 +375,11 @@ int lbm_block_run(const lbm_block_weights* w, const lbm_block_call* c, void* str
                          lbm_linear_asks(c->rows, (int)dim, w->hidden, LBM_LINEAR_BIAS_RESIDUAL, 0, split)};
     lbm_deal_hints(asks, by);
   }
-  // Nothing that the call names outlives it: the memory may not.
-  auto ahead = [&](int launch) {
-    LbmTouch t = {};
+  // A hint that the caller gave beforehand is for the first linear, unless the call names proj's weights itself; refused, it
+  // leaves that hint as it was.  Nothing that the call named itself outlives it: the memory may not.
+  LbmTouch callers = {};
+  if (!c->hints[0]) lbm_take_prefetch_hint(callers);
+  auto ahead = [&](int launch, LbmTouch t = {}) {
     for (int r = 0; r < 4; ++r)
       if (by[r] == launch) lbm_add_touch(t, c->hints[r], c->hint_bytes[r]);
     return t;
@@ -386,12 +388,17 @@ int lbm_block_run(const lbm_block_weights* w, const lbm_block_call* c, void* str
     if (rc != LBM_OK) lbm_set_prefetch_hint({});
     return rc;
   };
-  lbm_set_prefetch_hint(ahead(0));
+  lbm_set_prefetch_hint(ahead(0, callers));
   int rc = lbm_qkv_linear_prepare_norm(c->a, c->stats ? &norm1 : nullptr, w->qkv_w, w->qkv_b, c->rows, (int32_t)dim, w->q_norm_w,
                                        w->q_norm_b, w->k_norm_w, w->k_norm_b, w->qk_eps, c->q_scale, c->rope_cs, c->rope_layout, q,
                                        c->keep_kv ? k : nullptr, c->keep_kv ? v : nullptr, c->pool, c->append_rows, w->num_heads, 64,
                                        c->page_size, stream);
-  if (ended(rc) != LBM_OK) return rc;
+  if (rc != LBM_OK) {
+    LbmTouch left;
+    lbm_take_prefetch_hint(left);
+    if (left.lines[0]) lbm_set_prefetch_hint(callers);
+    return rc;
+  }
   if (c->n_streams > 0) {
     const LbmTouch touch = ahead(1);
     rc = lbm_attn_run_impl("lbm_block_run", q, c->pool ? c->pool : k, heads, c->keep_kv ? k : nullptr, c->keep_kv ? v : nullptr,

@@ -86,9 +86,20 @@ def test_a_refused_block_leaves_no_hint_of_its_own(host):
     assert _pending(host) == []
 
 
+def test_a_hint_given_before_a_block_is_its_first_linears(host):
+    """A block with no hint for proj does not withdraw it: refused, it leaves it as it was."""
+    for own in ((None,) * 4, (None, 3 << 40, 3 << 40, 3 << 40)):
+        N.lib.lbm_linear_prefetch_hint(2 << 40, 8192)
+        _refused_block(own)
+        assert _pending(host) == [(2 << 40, 64)]
+    _refused_block((3 << 40,) + (None,) * 3)      # (the block's own takes its place)
+    assert _pending(host) == []
+    N.lib.lbm_linear_prefetch_hint(None, 0)
+
+
 @pytest.mark.gpu
 def test_a_block_refused_at_its_last_linear_leaves_no_hint(host):
-    """192 hidden columns: fc1 takes them, fc2 does not; the first three launches have run."""
+    """192 hidden columns: fc1 takes them, fc2 does not; the first three launches have run.  And a hint given beforehand has been taken."""
     import torch
     dev = torch.device("cuda:0")
     rows, dim, hidden = 8, 128, 192
@@ -98,7 +109,8 @@ def test_a_block_refused_at_its_last_linear_leaves_no_hint(host):
     need = int(N.lib.lbm_block_scratch_bytes(rows, 2, hidden))
     scratch = torch.zeros(need, dtype=torch.uint8, device=dev)
     out = torch.zeros(rows, dim, dtype=torch.bfloat16, device=dev)
-    for hints in ((p,) * 4, (None,) * 3 + (p,)):
+    for hints in ((p,) * 4, (None,) * 4):
+        N.lib.lbm_linear_prefetch_hint(p, 4096)
         call = N.BlockCall(p, p, None, out.data_ptr(), None, scratch.data_ptr(), None, None, None, p, None, None, None, None, need, 0, 0, 1.0,
                            rows, 0, 0, 1, 0, 16, hints, (4096,) * 4, 1)
         assert N.lib.lbm_block_run(w, call, None) != N.OK and b"multiple of 128" in N.lib.lbm_last_error()
