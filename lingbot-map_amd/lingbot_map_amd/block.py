@@ -674,8 +674,10 @@ class HipPagedBlock(nn.Module):
     #: hold, so a layer would find its own in HBM): proj's, fc1's and fc2's and the next block's qkv weights, which
     #: ``lbm_block_run`` asks for from launches before theirs.  ms per frame without and with, replayed: 86 rows 3.31,
     #: 2.78; 261 rows 3.61, 3.22; 1,004 rows 6.74, 6.37; eager, where the frame waits for the host: 187 rows 3.51, 3.22,
-    #: 86 rows 3.26, 3.26.  A switch for measurements - results do not depend on it.
+    #: 86 rows 3.26, 3.26.  ``HINT_ROWS``: eager frames of fewer rows name none.  Switches for measurements - results do not
+    #: depend on them.
     PREFETCH_HINTS = os.environ.get("LBM_PREFETCH_HINTS", "1") != "0"
+    HINT_ROWS = 0
 
     def __init__(self, dim: int, num_heads: int, mlp_ratio: float = 4.0, qkv_bias: bool = True,
                  proj_bias: bool = True, ffn_bias: bool = True, drop: float = 0.0, attn_drop: float = 0.0,
@@ -824,7 +826,7 @@ class HipPagedBlock(nn.Module):
             if append is None:
                 return None
         hints = ((None,) * 4, (0,) * 4)
-        if self.PREFETCH_HINTS:
+        if self.PREFETCH_HINTS and (rows >= self.HINT_ROWS or torch.cuda.is_current_stream_capturing()):
             hints = native.hints_with(next_norm)
         call = N.BlockCall(
             x.data_ptr(), a.data_ptr(), stats_ptr, out.data_ptr(), None if stats_out is None else stats_out.data_ptr(),

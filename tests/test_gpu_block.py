@@ -743,3 +743,21 @@ def test_weights_asked_for_ahead_change_no_result(rows, monkeypatch):
         got.append(outs)
     for a, b in zip(*got):
         assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
+def test_eager_frames_below_a_line_name_no_weights(monkeypatch):
+    """``HipPagedBlock.HINT_ROWS``, 0 unless it is set: eager frames of fewer rows give no hints, others do."""
+    from lingbot_map_amd import HipPagedBlock
+    from lingbot_map_amd.block import _NativeBlock
+    dev, asked = torch.device("cuda:0"), []
+    block = HipPagedBlock(1024, 16).to(dev, torch.bfloat16).eval()
+    hints_with = _NativeBlock.hints_with
+    monkeypatch.setattr(_NativeBlock, "hints_with", lambda self, next_norm: asked.append(1) or hints_with(self, next_norm))
+    counts = []
+    for line in (None, 100, 101):
+        if line is not None:
+            monkeypatch.setattr(HipPagedBlock, "HINT_ROWS", line)
+        with torch.no_grad():
+            block(torch.randn(1, 100, 1024, device=dev).to(torch.bfloat16))
+        counts.append(len(asked))
+    assert counts == [1, 2, 2]
