@@ -11,6 +11,7 @@ N(0,1) tensors already resident in HBM.  Prints one JSON line.
 from __future__ import annotations
 
 import argparse
+import gc
 import json
 import math
 import os
@@ -61,14 +62,22 @@ def kernel_time_ms(fn, iters: int, torch) -> float:
 
 
 def event_time_ms(fn, iters: int, torch) -> float:
-    """Average duration of fn() in ms from one HIP event pair on the launch stream."""
+    """Average duration of fn() in ms from one HIP event pair on the launch stream.  Python's collector is off meanwhile: a
+    full collection takes 40 ms with torch loaded, the launches run out and the pause counts as theirs (four ragged streams,
+    100 launches of 190 us: 536 and 629 us when one fell between the events)."""
     start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    torch.cuda.synchronize()
-    start.record()
-    for _ in range(iters):
-        fn()
-    stop.record()
-    stop.synchronize()
+    collects = gc.isenabled()
+    gc.disable()
+    try:
+        torch.cuda.synchronize()
+        start.record()
+        for _ in range(iters):
+            fn()
+        stop.record()
+        stop.synchronize()
+    finally:
+        if collects:
+            gc.enable()
     return start.elapsed_time(stop) / iters
 
 
